@@ -31,7 +31,14 @@ struct GemmProblem {
   int activation;    // srtActivation
   float coef;
   int tile_n;        // kernel-specific: columns per workgroup when a launcher narrows its tile (0: the kernel's own)
+  int row_padding;   // 1: operands in the library's own workspace, whose rows are readable up to a multiple of 8 elements
 };
+
+// Whether every 16-byte chunk of a 16-bit result lies on a 16-byte boundary and whole inside its row: what the kernels
+// that store such chunks through a buffer descriptor need.
+__host__ __device__ __forceinline__ bool c_whole_chunks(const GemmProblem& p) {
+  return p.scn == 1 && ((p.N | (int)p.scm | (int)p.scb) & 7) == 0 && (reinterpret_cast<uintptr_t>(p.C) & 15u) == 0;
+}
 
 // ---- element codecs ---------------------------------------------------------------------
 struct BF16 {
@@ -306,6 +313,10 @@ int mfma_select(const GemmProblem& p);
 int mfma_config(const GemmProblem& p, int tile);
 const char* mfma_name(int config);
 hipError_t launch_mfma(const GemmProblem& p, int config, hipStream_t stream);
+// Operands copied into aligned, zero-padded workspace first (gemm_pack.hip), and the plan the heuristic picks for the copies.
+bool pack_preferred(const GemmProblem& p);
+hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErrorOutOfMemory: no workspace, nothing was launched
+hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream);
 // Split-K over the 256 x 256 kernel: number of k parts (0: the problem does not qualify) and launch.
 int mfma_splitk_parts(const GemmProblem& p);
 bool mfma_prefers_splitk(const GemmProblem& p);

@@ -33,6 +33,7 @@ namespace srt {
 
 // 256 x 256 ring kernels, one translation unit per (type, layout): gemm_ring_inst.hip
 bool ring_fits_problem(const GemmProblem& p, bool a_kc, bool b_kc);
+bool ring_reach_problem(const GemmProblem& p, bool a_kc, bool b_kc);   // without the rules on the result
 hipError_t launch_kc64_BF16(const GemmProblem& p, hipStream_t stream);
 hipError_t launch_kc64_F16(const GemmProblem& p, hipStream_t stream);
 #define SRT_RING_DECL(T) \
@@ -421,11 +422,12 @@ __global__ __launch_bounds__(NT) void gemm_mfma_kernel(GemmProblem p) {
 
   // epilogue: the MFMA took the B fragment first, so each 32 x 32 accumulator tile is C^T: a lane
   // holds row l % 32 and, per group of four registers, the four consecutive columns
-  // 8 (v / 4) + 4 (l / 32) + 0..3 -- one 8-byte store per group where the row pitch and base of C
-  // keep it aligned and the group lies inside N, element stores otherwise.
+  // 8 (v / 4) + 4 (l / 32) + 0..3 -- one 8-byte store per group that lies inside N where C's rows are contiguous,
+  // element stores otherwise.
   Epilogue<T> ep(p);
   uint16_t* C = (uint16_t*)p.C + (long long)bz * p.scb;
-  const bool wide = p.scn == 1 && (p.scm % 4) == 0 && (reinterpret_cast<uintptr_t>(C) & 7u) == 0;
+  const bool rows = p.scn == 1;
+  const bool wide = rows && (p.scm % 4) == 0 && (reinterpret_cast<uintptr_t>(C) & 7u) == 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int m = m0 + wm0 + 32 * i + (lane & 31);
@@ -444,11 +446,13 @@ __global__ __launch_bounds__(NT) void gemm_mfma_kernel(GemmProblem p) {
           const float bv = ep.per_row ? brow : (n + e < p.N ? ep.bias_at(0, n + e) : 0.0f);
           h[e] = ep.finish(acc[i][j][4 * q + e], bv);
         }
-        if (wide && n + 3 < p.N) {
+        if (rows && n + 3 < p.N) {
+          // eight bytes at whatever alignment the row has (64 x 511 x 511 x 63 x . W^T: 50 us with element stores, 31 with these)
           uint2 w;
           w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
           w.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
-          *reinterpret_cast<uint2*>(crow + n) = w;
+          if (wide) *reinterpret_cast<uint2*>(crow + n) = w;
+          else __builtin_memcpy(crow + n, &w, 8);
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -652,10 +656,10 @@ static int mfma_layout(const GemmProblem& p) {
   if (p.batch > 65535) return -1;
   bool a_kc, b_kc;
   if (p.sak == 1 && (p.K % 8) == 0) a_kc = true;
-  else if (p.sam == 1 && (p.M % 8) == 0) a_kc = false;
+  else if (p.sam == 1 && ((p.M % 8) == 0 || p.row_padding)) a_kc = false;
   else return -1;
   if (p.sbk == 1 && (p.K % 8) == 0) b_kc = true;
-  else if (p.sbn == 1 && (p.N % 8) == 0) b_kc = false;
+  else if (p.sbn == 1 && ((p.N % 8) == 0 || p.row_padding)) b_kc = false;
   else return -1;
   const long long lda = a_kc ? p.sam : p.sak, ldb = b_kc ? p.sbn : p.sbk;
   // a single row/column operand may carry any leading stride; otherwise rows must stay aligned
@@ -679,7 +683,10 @@ int mfma_config(const GemmProblem& p, int tile) {
   }
   const int layout = mfma_layout(p);
   if (layout < 0 || tile < 1 || (tile > 6 && (tile < 9 || tile > 14))) return 0;
-  if ((tile == 1 || tile >= 4) && !ring_fits_problem(p, (layout & 2) != 0, (layout & 1) != 0)) return 0;
+  // (the 64- and 128-deep kernels of the 16x16x32 family store any contiguous rows, the others whole aligned chunks only)
+  const bool stores_any = tile == 9 || (tile >= 12 && tile <= 14);
+  if ((tile == 1 || tile >= 4) && !(stores_any ? ring_reach_problem(p, (layout & 2) != 0, (layout & 1) != 0)
+                                               : ring_fits_problem(p, (layout & 2) != 0, (layout & 1) != 0))) return 0;
   if ((tile == 9 || tile == 12 || tile == 13) && !(p.K % 64 == 0 && p.K >= 256)) return 0;   // whole 64-deep units, at least four
   if (tile == 14 && !(p.K % 128 == 0 && p.K >= 256)) return 0;   // whole 128-deep units, at least two
   if (tile == 10) {   // left-over tiles to share, k in whole quads, no transcendental activation
@@ -728,6 +735,25 @@ static bool narrow_round(const GemmProblem& p, int layout) {
   return tn >= 64;
 }
 
+// The tile of a problem whose result rows are not whole aligned chunks (an odd number of columns): one of the kernels that
+// store such rows, by rounds of the persistent grid -- a whole tile takes 6 + 24 us per 1024 k, a half tile 0.6 and a quarter
+// tile 0.29 of that per round, fitted to the figures above -- or the register-staged kernels when K is not in their units.
+static int ragged_store_config(const GemmProblem& p) {
+  const long long cus = compute_units();
+  auto rounds = [&](int tm, int tn) {
+    const long long t = (long long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn) * p.batch;
+    return (double)((t + cus - 1) / cus);
+  };
+  const int configs[4] = {mfma_config(p, 9), mfma_config(p, 12), mfma_config(p, 13), mfma_config(p, 14)};
+  const double times[4] = {rounds(256, 256), 0.6 * rounds(128, 256), 0.6 * rounds(256, 128), 0.29 * rounds(128, 128)};
+  int best = -1;
+  for (int i = 0; i < 4; ++i)
+    if (configs[i] && (best < 0 || times[i] < times[best])) best = i;
+  if (best >= 0) return configs[best];
+  const long long t128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+  return mfma_config(p, t128 >= cus ? 2 : 3);
+}
+
 int mfma_select(const GemmProblem& p) {
   const int layout = mfma_layout(p);
   auto tiles = [&](int t) { return (long long)((p.M + t - 1) / t) * ((p.N + t - 1) / t) * p.batch; };
@@ -759,6 +785,7 @@ int mfma_select(const GemmProblem& p) {
   //    the 256 x 256 kernels' preconditions but have at least one such tile per CU.
   const bool big_ok = ring_fits_problem(p, (layout & 2) != 0, (layout & 1) != 0);
   const long long t256 = tiles(256);
+  if (!big_ok && !c_whole_chunks(p)) return ragged_store_config(p);
   //  * with a k-contiguous A the 16x16x32 kernel also comes with 128 x 256 tiles: twice the
   //    workgroups, which is what a problem that leaves compute units idle needs (2048^3: 29 us
   //    against 42 us; 512 x 14336 x 4096: 59 against 82; 256 x 1024 x 1024: 15 against 19 for 64 x 64
@@ -1216,6 +1243,11 @@ const char* mfma_name(int config) {
 hipError_t launch_mfma(const GemmProblem& p, int config, hipStream_t stream) {
   const int tile = config >> 2;
   const bool a_kc = (config & 2) != 0, b_kc = (config & 1) != 0;
+  if ((tile == 7 || tile == 8) && pack_preferred(p)) {
+    const hipError_t e = launch_packed(p, stream);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();   // no room for the copies (nothing was launched): the operands as they are
+  }
   if (p.dtype == srtReal16BF) return launch_tile<BF16>(p, tile, a_kc, b_kc, stream);
   return launch_tile<F16>(p, tile, a_kc, b_kc, stream);
 }

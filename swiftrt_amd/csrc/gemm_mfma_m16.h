@@ -228,11 +228,24 @@ __device__ __forceinline__ void load_bias(const GemmProblem& p, int wave_m0, int
       if (m < p.M) b[i].x = bias[(long long)m * p.sbias];
     }
   } else if (p.sbias == 1 && (reinterpret_cast<uintptr_t>(bias) & 7u) == 0) {
-    // N is a multiple of 8 and n of 4: a lane's four columns are all inside or all outside
+    // a lane's four columns are all inside, all outside, or (N not a multiple of 4) across the end of the row
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int n = wave_n0 + 16 * j + 4 * g;
-      if (n < p.N) b[j] = *reinterpret_cast<const u32x2_t*>(bias + n);
+      if (n + 4 <= p.N) b[j] = *reinterpret_cast<const u32x2_t*>(bias + n);
+    }
+    if ((p.N & 3) != 0) {
+      const int n = p.N & ~3;   // the lane that holds the last, partial group
+      const int j = (n - wave_n0) >> 4;
+      if (n >= wave_n0 && ((n >> 2) & 3) == g) {
+        uint32_t h[3] = {0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (n + e < p.N) h[e] = bias[n + e];
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          if (t == j) b[t] = u32x2_t{h[0] | (h[1] << 16), h[2]};
+      }
     }
   } else {
 #pragma unroll
@@ -266,7 +279,7 @@ __device__ __forceinline__ void load_bias(const GemmProblem& p, int wave_m0, int
 // otherwise).
 // TN: column tiles per wave (8; 6 for the 192-wide workgroup tile, whose wave covers 96 columns).  n_end: columns at
 // or beyond it belong to another tile and are not stored (a workgroup tile narrower than its MFMA footprint).
-template <typename T, int TM, bool HAS_BIAS, int CLAMP, bool FLIP = false, int TN = 8>
+template <typename T, int TM, bool HAS_BIAS, int CLAMP, bool FLIP = false, int TN = 8, bool WHOLE = true>
 __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (&acc)[TM][TN], int wave_m0, int wave_n0,
                                            int bz, int lane, uint32_t stage, const u32x2_t (&b)[8], int n_end = 0x7fffffff) {
   static_assert(!FLIP || (TM == 8 && TN == 8), "a square block of accumulator tiles");
@@ -283,7 +296,8 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
   const int jn = lane & 15, g = lane >> 4;
   const int rd_chunk = lane & 15, rd_row = lane >> 4;   // read side: chunk of rows rd_row + 4 it
   const int n_rd = wave_n0 + 8 * rd_chunk;
-  // N is a multiple of 8 (checked on the host): the chunk is whole
+  // WHOLE: N is a multiple of 8 and rows are aligned (checked on the host).  Otherwise the result is stored through its
+  // address instead of a descriptor: 16 bytes at 2-byte alignment where the chunk lies inside the row, elements at its end
   const bool n_rd_ok = n_rd < p.N && (TN == 8 || (rd_chunk < 2 * TN && n_rd < n_end));
 
   // staging address of accumulator tile (ii, j): row 16 ii + jn, chunk (2 j + g / 2) ^ jn -- the lane's part of
@@ -352,12 +366,35 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
       for (int q = 0; q < 4; ++q) {
         const int row = rd_row + 4 * (4 * it4 + q);
         const int m = wave_m0 + ROWS * half + row;
-        const uint32_t off = (n_rd_ok && m < p.M) ? (uint32_t)(m * ldc2 + n_rd * 2) : OOB;
-        __builtin_amdgcn_raw_buffer_store_b128(v[q], rc, (int)off, 0, SRT_STORE_AUX);
+        if constexpr (WHOLE) {
+          const uint32_t off = (n_rd_ok && m < p.M) ? (uint32_t)(m * ldc2 + n_rd * 2) : OOB;
+          __builtin_amdgcn_raw_buffer_store_b128(v[q], rc, (int)off, 0, SRT_STORE_AUX);
+        } else if (n_rd_ok && m < p.M) {
+          S* dst = C + (long long)m * p.scm + n_rd;
+          if (n_rd + 8 <= p.N) {
+            __builtin_memcpy(dst, &v[q], 16);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 7; ++e)
+              if (n_rd + e < p.N) dst[e] = (S)(v[q][e >> 1] >> (16 * (e & 1)));
+          }
+        }
       }
       SRT_FENCE();
     }
   }
+}
+
+// store_tile for an epilogue kind, on results of either alignment: two copies of the code behind one uniform branch (a choice
+// at every store cost the launch 0.8 us, 1000 x 1000 x 1000 18.3 -> 19.1).
+template <typename T, int TM, int EPI, bool FLIP, int TN>
+__device__ __forceinline__ void store_tile_any(const GemmProblem& p, const f32x4_t (&acc)[TM][TN], int wave_m0, int wave_n0,
+                                               int bz, int lane, uint32_t stage, const u32x2_t (&b)[8], int n_end) {
+  constexpr bool HAS_BIAS = EPI != EPI_PLAIN && EPI != EPI_RELU;
+  constexpr int CLAMP = EPI == EPI_RELU || EPI == EPI_BIAS_RELU ? 1 : EPI == EPI_CLIPPED ? 2
+                      : EPI == EPI_SIGMOID ? 3 : EPI == EPI_TANH ? 4 : EPI == EPI_ELU ? 5 : 0;
+  if (c_whole_chunks(p)) store_tile<T, TM, HAS_BIAS, CLAMP, FLIP, TN, true>(p, acc, wave_m0, wave_n0, bz, lane, stage, b, n_end);
+  else store_tile<T, TM, HAS_BIAS, CLAMP, FLIP, TN, false>(p, acc, wave_m0, wave_n0, bz, lane, stage, b, n_end);
 }
 
 // sigmoid / tanh / elu: acc + bias goes to the staging area as fp32 (passes of ROWS = 32 or 16 rows:
@@ -557,8 +594,8 @@ __global__ __launch_bounds__(NT) void gemm_m16_kernel(GemmProblem p) {
 
   const long long lda = A_KC ? p.sam : p.sak;
   const long long ldb = B_KC ? p.sbn : p.sbk;
-  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + p.M;
-  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + p.N;
+  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + ((p.M + 7) & ~7);
+  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + ((p.N + 7) & ~7);
   const u32x4_t ra = ring::make_rsrc(p.A, (uint32_t)(((long long)(p.batch - 1) * p.sab + a_view) * 2));
   const u32x4_t rb = ring::make_rsrc(p.B, (uint32_t)(((long long)(p.batch - 1) * p.sbb + b_view) * 2));
   const uint32_t kstep_a = A_KC ? (uint32_t)(BK * 2) : (uint32_t)(BK * lda * 2);   // bytes per k stage

@@ -441,8 +441,8 @@ __device__ __forceinline__ void gemm_m16d_body(const GemmProblem& p, const TailS
 
   const long long lda = A_KC ? p.sam : p.sak;
   const long long ldb = B_KC ? p.sbn : p.sbk;
-  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + p.M;
-  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + p.N;
+  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + ((p.M + 7) & ~7);
+  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + ((p.N + 7) & ~7);
   const u32x4_t ra = ring::make_rsrc(p.A, (uint32_t)(((long long)(p.batch - 1) * p.sab + a_view) * 2));
   const u32x4_t rb = ring::make_rsrc(p.B, (uint32_t)(((long long)(p.batch - 1) * p.sbb + b_view) * 2));
   // tile number -> position and operand offsets (the narrow tile's columns lie tile_w apart)
@@ -862,14 +862,7 @@ __device__ __forceinline__ void gemm_m16d_body(const GemmProblem& p, const TailS
     } else if constexpr (EPI == EPI_PARTIAL) {
       m16::store_tile_partial<TM>(p, acc, em0, en0, bz, le, stage);
     } else {
-      if (EPI == EPI_BIAS) m16::store_tile<T, TM, true, 0, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else if (EPI == EPI_RELU) m16::store_tile<T, TM, false, 1, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else if (EPI == EPI_BIAS_RELU) m16::store_tile<T, TM, true, 1, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else if (EPI == EPI_CLIPPED) m16::store_tile<T, TM, true, 2, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else if (EPI == EPI_SIGMOID) m16::store_tile<T, TM, true, 3, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else if (EPI == EPI_TANH) m16::store_tile<T, TM, true, 4, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else if (EPI == EPI_ELU) m16::store_tile<T, TM, true, 5, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-      else m16::store_tile<T, TM, false, 0, FLIP>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
+      m16::store_tile_any<T, TM, EPI, FLIP, TN>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
     }
     if (!has_next) break;
 

@@ -150,8 +150,8 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
 
   const long long lda = A_KC ? p.sam : p.sak;
   const long long ldb = B_KC ? p.sbn : p.sbk;
-  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + p.M;
-  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + p.N;
+  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + ((p.M + 7) & ~7);
+  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + ((p.N + 7) & ~7);
   const u32x4_t ra = ring::make_rsrc(p.A, (uint32_t)(((long long)(p.batch - 1) * p.sab + a_view) * 2));
   const u32x4_t rb = ring::make_rsrc(p.B, (uint32_t)(((long long)(p.batch - 1) * p.sbb + b_view) * 2));
   // tile number -> position and operand offsets (the walk's own columns are 256 apart)
@@ -360,14 +360,7 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
     uint32_t sb = x < lds + UNIT ? x + 4 * UNIT : x - UNIT;
     const uint32_t stage = ((wave & 2) ? sb : sa) + (uint32_t)(wave & 1) * (uint32_t)(UNIT / 2);
 
-    if (EPI == EPI_BIAS) m16::store_tile<T, 4, true, 0, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else if (EPI == EPI_RELU) m16::store_tile<T, 4, false, 1, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else if (EPI == EPI_BIAS_RELU) m16::store_tile<T, 4, true, 1, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else if (EPI == EPI_CLIPPED) m16::store_tile<T, 4, true, 2, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else if (EPI == EPI_SIGMOID) m16::store_tile<T, 4, true, 3, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else if (EPI == EPI_TANH) m16::store_tile<T, 4, true, 4, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else if (EPI == EPI_ELU) m16::store_tile<T, 4, true, 5, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
-    else m16::store_tile<T, 4, false, 0, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
+    m16::store_tile_any<T, 4, EPI, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
     if (!has_next) break;
 
     // every wave has finished reading its staging area before any wave's loads overwrite it

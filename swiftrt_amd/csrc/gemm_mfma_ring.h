@@ -544,8 +544,8 @@ __global__ __launch_bounds__(NT) void gemm_ring_kernel(GemmProblem p) {
   // batch's view reads as zero.  Inside the tensor nothing is masked by the descriptor: rows of a
   // partial tile beyond M (columns beyond N) read whatever follows and only reach accumulators
   // that are never stored; k beyond K is masked by the loaders (ragged last stage).
-  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + p.M;
-  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + p.N;
+  const long long a_view = A_KC ? (long long)(p.M - 1) * lda + p.K : (long long)(p.K - 1) * lda + ((p.M + 7) & ~7);
+  const long long b_view = B_KC ? (long long)(p.N - 1) * ldb + p.K : (long long)(p.K - 1) * ldb + ((p.N + 7) & ~7);
   const u32x4_t ra = make_rsrc(p.A, (uint32_t)(((long long)(p.batch - 1) * p.sab + a_view) * 2));
   const u32x4_t rb = make_rsrc(p.B, (uint32_t)(((long long)(p.batch - 1) * p.sbb + b_view) * 2));
   const uint32_t kstep_a = A_KC ? (uint32_t)(BK * 2) : (uint32_t)(BK * lda * 2);   // bytes per k stage
@@ -799,7 +799,7 @@ __global__ __launch_bounds__(NT) void gemm_ring_kernel(GemmProblem p) {
 // batches) must span less than 1 Gi elements so 32-bit byte offsets reach it (including the rows
 // of a partial last tile), and C
 // must take aligned 16-byte stores of eight whole columns.
-inline bool ring_fits(const GemmProblem& p, bool a_kc, bool b_kc) {
+inline bool ring_reach(const GemmProblem& p, bool a_kc, bool b_kc) {
   const long long lda = a_kc ? p.sam : p.sak, ldb = b_kc ? p.sbn : p.sbk;
   const long long nb = p.batch - 1;
   const long long a_reach = nb * p.sab + (a_kc ? ((long long)p.M + BM) * lda + p.K : ((long long)p.K + BK) * lda + p.M + BM);
@@ -807,11 +807,9 @@ inline bool ring_fits(const GemmProblem& p, bool a_kc, bool b_kc) {
   const long long c_reach = ((long long)p.M + BM) * p.scm + p.N + BN;
   const long long lim = 0x7fffffffLL / 2 - 4096;   // in elements: byte offsets stay below 2^31
   if (!(a_reach < lim && b_reach < lim && c_reach < lim)) return false;
-  if (p.sab < 0 || p.sbb < 0) return false;
-  if ((p.N % 8) != 0 || (p.scm % 8) != 0 || (p.scb % 8) != 0) return false;
-  if ((reinterpret_cast<uintptr_t>(p.C) & 15u) != 0) return false;
-  return true;
+  return p.sab >= 0 && p.sbb >= 0;
 }
+inline bool ring_fits(const GemmProblem& p, bool a_kc, bool b_kc) { return c_whole_chunks(p) && ring_reach(p, a_kc, b_kc); }
 
 // Workgroups of the persistent grid: one per compute unit (a workgroup takes a whole unit's LDS),
 // a multiple of 8 because the XCD-aware tile order wants the stride between a workgroup's tiles

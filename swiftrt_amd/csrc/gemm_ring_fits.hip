@@ -2,5 +2,6 @@
 #include "gemm_mfma_ring.h"
 
 namespace srt {
+bool ring_reach_problem(const GemmProblem& p, bool a_kc, bool b_kc) { return ring::ring_reach(p, a_kc, b_kc); }
 bool ring_fits_problem(const GemmProblem& p, bool a_kc, bool b_kc) { return ring::ring_fits(p, a_kc, b_kc); }
 }  // namespace srt

@@ -59,7 +59,7 @@ srtStatus build_problem(const void* a, const srtTensorDescriptor* ad, int tA,
   p->scm = (long long)od->strides[r]; p->scn = (long long)od->strides[r + 1];
   p->scb = rank == 3 ? (long long)od->strides[0] : 0;
   p->bias = nullptr; p->sbias = 0; p->bias_per_row = 0;
-  p->activation = activation; p->coef = (float)coef; p->tile_n = 0;
+  p->activation = activation; p->coef = (float)coef; p->tile_n = 0; p->row_padding = 0;
   if (bias) {
     if (!biasd || !biasd->shape || !biasd->strides) return srtErrorInvalidValue;
     if (biasd->type != od->type) return srtErrorNotSupported;
@@ -240,6 +240,22 @@ hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
   }
 }
 
+hipError_t launch_or_fall_back(const GemmProblem& p, Plan plan, hipStream_t stream) {
+  hipError_t e = launch_plan(p, plan, stream);
+  if ((plan == kPlanSplitK || plan == kPlanM16DTail) && e == hipErrorOutOfMemory) {
+    // no room for the workspace (nothing was launched): the plan that needs none
+    (void)hipGetLastError();
+    const int c = plan == kPlanM16DTail ? srt::mfma_config(p, 9) : srt::mfma_select(p);
+    e = c ? srt::launch_mfma(p, c, stream) : srt::launch_generic(p, stream);
+  }
+  if (plan == kPlanF32Parts && e == hipErrorOutOfMemory) {
+    // likewise for the fp32 parts: the whole k range per tile, no workspace
+    (void)hipGetLastError();
+    e = srt::f32_ring_fits(p) ? srt::launch_f32_ring(p, stream, 0) : srt::launch_f32_mfma_variant(p, false, stream);
+  }
+  return e;
+}
+
 struct PlanKey {
   int dtype, M, N, K, batch, layout, epilogue;
   bool operator<(const PlanKey& o) const {
@@ -405,22 +421,16 @@ srtStatus run(const GemmProblem& p, hipStream_t stream) {
   }
   const Plan plan = select(p);
   if (plan == kPlanGeneric && !srt::generic_supported(p)) return srtErrorNotSupported;
-  hipError_t e = launch_plan(p, plan, stream);
-  if ((plan == kPlanSplitK || plan == kPlanM16DTail) && e == hipErrorOutOfMemory) {
-    // no room for the workspace (nothing was launched): the plan that needs none
-    (void)hipGetLastError();
-    const int c = plan == kPlanM16DTail ? srt::mfma_config(p, 9) : srt::mfma_select(p);
-    e = c ? srt::launch_mfma(p, c, stream) : srt::launch_generic(p, stream);
-  }
-  if (plan == kPlanF32Parts && e == hipErrorOutOfMemory) {
-    // likewise for the fp32 parts: the whole k range per tile, no workspace
-    (void)hipGetLastError();
-    e = srt::f32_ring_fits(p) ? srt::launch_f32_ring(p, stream, 0) : srt::launch_f32_mfma_variant(p, false, stream);
-  }
-  return srt::from_hip(e);
+  return srt::from_hip(launch_or_fall_back(p, plan, stream));
 }
-
 }  // namespace
+
+namespace srt {
+// The heuristic's plan for a problem built inside the library (operands copied into its workspace).
+hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream) {
+  return launch_or_fall_back(p, heuristic_plan(p), stream);
+}
+}  // namespace srt
 
 extern "C" {
 

@@ -1,0 +1,69 @@
+"""Operands copied into aligned workspace (gemm_pack.hip) and results whose rows are not whole aligned 16-byte chunks.
+
+Integer operands, exact comparison (every partial sum is representable, so the kernel and its order of summation do not
+matter); operands framed by NaNs, results by a sentinel, so that a copy or a store past an edge shows."""
+import numpy as np
+import pytest
+
+import swiftrt_amd as srt
+from tests import helpers as H
+from tests.test_gpu_canaries import NAN_BITS, run_matmul_case
+from tests.test_gpu_matmul import query_kernel
+
+pytestmark = pytest.mark.gpu
+
+ANY = ("mfma_128x128_any", "mfma_64x64_any")
+
+
+@pytest.fixture(autouse=True)
+def clean_cache():
+    srt.PlanCache.clear()
+    yield
+    srt.PlanCache.clear()
+
+
+# k extents either side of a staging unit and of the rule's short ones; one and several tiles; each layout; a batch
+@pytest.mark.parametrize("M,N,K,batch", [(129, 257, 129, 1), (127, 513, 257, 1), (65, 70, 1023, 1), (300, 333, 127, 1),
+                                         (2049, 2047, 65, 1), (2047, 2050, 255, 1), (71, 131, 385, 5)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_copied_operands(tmp_path, M, N, K, batch, ta, tb):
+    ran = run_matmul_case(tmp_path, H.BF16, M, N, K, batch, ta, tb, ANY, 900 + M + K, left=3, right=2, operand_sentinel=NAN_BITS)
+    assert ran == list(ANY)
+
+
+def test_copied_views_without_a_unit_stride_and_shared_matrices():
+    g = H.rng(901)
+    a = g.integers(-2, 3, (600, 900)).astype(np.float32)
+    b = g.integers(-2, 3, (900, 800)).astype(np.float32)
+    at, bt = srt.Tensor(H.encode(a, H.F16)), srt.Tensor(H.encode(b, H.F16))
+    got = srt.matmul(at[1:599:2, 3:897:3], bt[2:896:3, 1:799:2])
+    want = a[1:599:2, 3:897:3].astype(np.float64) @ b[2:896:3, 1:799:2].astype(np.float64)
+    assert np.array_equal(got.array(), H.encode(want.astype(np.float32), H.F16))
+    # one right operand under every matrix of a batch (stride 0), odd extents
+    x = g.integers(-2, 3, (6, 257, 301)).astype(np.float32)
+    w = g.integers(-2, 3, (301, 515)).astype(np.float32)
+    wt = srt.Tensor.repeating(srt.Tensor(H.encode(w, H.BF16)), [6, 301, 515])
+    got = srt.matmul(srt.Tensor(H.encode(x, H.BF16)), wt)
+    want = x.astype(np.float64) @ w.astype(np.float64)
+    assert np.array_equal(H.to64(got.array()), H.to64(H.encode(want.astype(np.float32), H.BF16)))
+
+
+# aligned operands, an odd number of result columns: every kernel that stores such rows, edges of its tile in both directions
+@pytest.mark.parametrize("dt", [H.BF16, H.F16])
+@pytest.mark.parametrize("M,N,K,batch", [(256, 257, 256, 1), (136, 127, 384, 1), (264, 391, 512, 1), (72, 129, 256, 3)])
+def test_results_with_ragged_rows(tmp_path, dt, M, N, K, batch):
+    ran = set()
+    for ta in (False, True):
+        for bias, relu in ((False, False), (True, True), (True, False)):
+            ran |= set(run_matmul_case(tmp_path, dt, M, N, K, batch, ta, True,
+                                       ("mfma_256x256_m16_k64", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128",
+                                        "mfma_128x128", "mfma_64x64"), 910 + N, with_bias=bias, relu=relu))
+    assert ran == {"mfma_256x256_m16_k64", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128", "mfma_128x128",
+                   "mfma_64x64"}
+
+
+def test_the_choice_for_ragged_rows():
+    for (M, N, K, kernel) in [(2048, 50257, 768, "mfma_256x256_m16_k64"), (512, 1001, 1024, "mfma_128x128_m16_k128"),
+                              (512, 1001, 200, "mfma_64x64")]:
+        a, b = srt.Tensor(shape=[M, K], dtype=np.uint16), srt.Tensor(shape=[N, K], dtype=np.uint16)
+        assert query_kernel(a, False, b, True, srt.Tensor(shape=[M, N], dtype=np.uint16)) == kernel
