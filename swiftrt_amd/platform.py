@@ -13,6 +13,7 @@ from . import native
 from .native import check
 
 _queue_ids = itertools.count(1)
+IDENTITY = 5   # srtActivationIdentity: no activation
 
 
 class HipEvent:
@@ -117,6 +118,9 @@ class HipQueue:
         check(native.lib().srtMemcpyAsync(ctypes.c_void_p(host_ptr), ctypes.c_void_p(src.pointer), byte_count,
                                           native.D2H, self.stream), "srtMemcpyAsync(D2H)")
 
+    def zero(self, dst, byte_count):
+        check(native.lib().srtMemsetAsync(ctypes.c_void_p(dst.pointer), 0, byte_count, self.stream), "srtMemsetAsync")
+
     def copy_async(self, src, dst):
         n = min(src.byte_count, dst.byte_count)
         check(native.lib().srtMemcpyAsync(ctypes.c_void_p(dst.pointer), ctypes.c_void_p(src.pointer), n,
@@ -146,32 +150,22 @@ class HipQueue:
         Tensor.deviceRead), descriptors are built per call and the native entry point is invoked
         on this queue's stream.  srtErrorNotSupported surfaces as NotSupportedError: a Swift
         caller would run its own cpu_matmul there; this module has no CPU arithmetic."""
-        from .tensor import ActivationType
         self.select()
         a_ptr = lhs.device_read(self)
         b_ptr = rhs.device_read(self)
         bias_ptr = bias.device_read(self) if bias is not None else None
-        o_ptr = result.device_read_write(self)
-        ad, ka = lhs.descriptor()
-        bd, kb = rhs.descriptor()
-        od, ko = result.descriptor()
+        o_ptr = result.device_write(self)
         L = native.lib()
-        if bias is None and activation in (None, ActivationType.identity):
-            st = L.srtMatmul(a_ptr, ctypes.byref(ad), int(transpose_lhs), b_ptr, ctypes.byref(bd), int(transpose_rhs),
-                             o_ptr, ctypes.byref(od), self.stream)
+        if bias is None and activation in (None, IDENTITY):
+            st = L.srtMatmul(a_ptr, lhs.descriptor_ref(), int(transpose_lhs), b_ptr, rhs.descriptor_ref(), int(transpose_rhs),
+                             o_ptr, result.descriptor_ref(), self.stream)
         else:
-            act = ActivationType.identity if activation is None else activation
-            if bias is not None:
-                biasd, kbias = bias.descriptor()
-                biasd_ref = ctypes.byref(biasd)
-            else:
-                biasd_ref, kbias = None, None
-            st = L.srtMatmulBiasActivation(a_ptr, ctypes.byref(ad), int(transpose_lhs), b_ptr, ctypes.byref(bd),
-                                           int(transpose_rhs), bias_ptr, biasd_ref, int(act), float(coef),
-                                           o_ptr, ctypes.byref(od), self.stream)
-            del kbias
-        del ka, kb, ko
+            act = IDENTITY if activation is None else int(activation)
+            st = L.srtMatmulBiasActivation(a_ptr, lhs.descriptor_ref(), int(transpose_lhs), b_ptr, rhs.descriptor_ref(),
+                                           int(transpose_rhs), bias_ptr, bias.descriptor_ref() if bias is not None else None,
+                                           act, float(coef), o_ptr, result.descriptor_ref(), self.stream)
         check(st, "srtMatmul")
+        result.device_written()
 
     def tune_matmul(self, lhs, transpose_lhs, rhs, transpose_rhs, result, bias=None, activation=None, coef=0.0):
         """Role of CudaMatmul2.tune (CudaMatmul.swift:112-120): measures every kernel plan the problem
@@ -212,37 +206,33 @@ class HipQueue:
                 and lhs.shape == out.shape and lhs.type_id == out.type_id and lhs.order == out.order:
             if not hasattr(rhs, "device_read"):
                 element = lhs.element_storage(rhs)
-                o_ptr = out.device_read_write(self)
+                o_ptr = out.device_write(self)
                 check(getattr(L, "srt" + name + "TEFlat")(a_ptr, lhs.type_id, ctypes.c_void_p(element.ctypes.data),
                                                           o_ptr, out.count, self.stream), "srt" + name + "TEFlat")
+                out.device_written()
                 return
             if rhs.is_contiguous and rhs.shape == out.shape and rhs.type_id == out.type_id and rhs.order == out.order:
                 b_ptr = rhs.device_read(self)
-                o_ptr = out.device_read_write(self)
+                o_ptr = out.device_write(self)
                 check(getattr(L, "srt" + name + "Flat")(out.type_id, a_ptr, b_ptr, o_ptr, out.count, self.stream),
                       "srt" + name + "Flat")
+                out.device_written()
                 return
-        ad, ka = lhs.descriptor()
         if rhs is None:
-            o_ptr = out.device_read_write(self)
-            od, ko = out.descriptor()
-            st = getattr(L, "srt" + name)(a_ptr, ctypes.byref(ad), o_ptr, ctypes.byref(od), self.stream)
+            o_ptr = out.device_write(self)
+            st = getattr(L, "srt" + name)(a_ptr, lhs.descriptor_ref(), o_ptr, out.descriptor_ref(), self.stream)
         elif hasattr(rhs, "device_read"):
             b_ptr = rhs.device_read(self)
-            o_ptr = out.device_read_write(self)
-            bd, kb = rhs.descriptor()
-            od, ko = out.descriptor()
-            st = getattr(L, "srt" + name)(a_ptr, ctypes.byref(ad), b_ptr, ctypes.byref(bd), o_ptr, ctypes.byref(od),
+            o_ptr = out.device_write(self)
+            st = getattr(L, "srt" + name)(a_ptr, lhs.descriptor_ref(), b_ptr, rhs.descriptor_ref(), o_ptr, out.descriptor_ref(),
                                           self.stream)
-            del kb
         else:
             element = lhs.element_storage(rhs)          # one element in the tensor's storage format
-            o_ptr = out.device_read_write(self)
-            od, ko = out.descriptor()
-            st = getattr(L, "srt" + name + "TE")(a_ptr, ctypes.byref(ad), ctypes.c_void_p(element.ctypes.data),
-                                                 o_ptr, ctypes.byref(od), self.stream)
-        del ka, ko
+            o_ptr = out.device_write(self)
+            st = getattr(L, "srt" + name + "TE")(a_ptr, lhs.descriptor_ref(), ctypes.c_void_p(element.ctypes.data),
+                                                 o_ptr, out.descriptor_ref(), self.stream)
         check(st, "srt" + name)
+        out.device_written()
 
     def add(self, lhs, rhs, out): self._elementwise("Add", lhs, rhs, out)
     def subtract(self, lhs, rhs, out): self._elementwise("Sub", lhs, rhs, out)
@@ -265,9 +255,10 @@ class HipQueue:
         element = out.element_storage(value)
         if not out.is_contiguous:
             raise native.NotSupportedError(native.ERROR_NOT_SUPPORTED, "fill of a strided view")
-        o_ptr = out.device_read_write(self)
+        o_ptr = out.device_write(self)
         check(native.lib().srtFillFlat(out.type_id, o_ptr, ctypes.c_void_p(element.ctypes.data), out.count,
                                        self.stream), "srtFillFlat")
+        out.device_written()
 
     def activation_backward(self, y, dy, activation, coef, dx, dbias=None, no_alloc=False):
         """Role of CudaActivation.backward (platform/cuda/layers/CudaActivation.swift:101-127) fused
@@ -276,22 +267,16 @@ class HipQueue:
         already be resident on the device, or the mirror's own staging would allocate)."""
         self.select()
         y_ptr, dy_ptr = y.device_read(self), dy.device_read(self)
-        dx_ptr = dx.device_read_write(self)
-        yd, k1 = y.descriptor()
-        dyd, k2 = dy.descriptor()
-        dxd, k3 = dx.descriptor()
-        if dbias is not None:
-            db_ptr = dbias.device_read_write(self)
-            dbd, k4 = dbias.descriptor()
-            dbd_ref = ctypes.byref(dbd)
-        else:
-            db_ptr, dbd_ref, k4 = None, None, None
+        dx_ptr = dx.device_write(self)
+        db_ptr = dbias.device_write(self) if dbias is not None else None
         name = "srtActivationBackwardBiasNoAlloc" if no_alloc else "srtActivationBackwardBias"
-        st = getattr(native.lib(), name)(y_ptr, ctypes.byref(yd), dy_ptr, ctypes.byref(dyd),
-                                         int(activation), float(coef), dx_ptr, ctypes.byref(dxd),
-                                         db_ptr, dbd_ref, self.stream)
-        del k1, k2, k3, k4
+        st = getattr(native.lib(), name)(y_ptr, y.descriptor_ref(), dy_ptr, dy.descriptor_ref(), int(activation), float(coef),
+                                         dx_ptr, dx.descriptor_ref(),
+                                         db_ptr, dbias.descriptor_ref() if dbias is not None else None, self.stream)
         check(st, name)
+        dx.device_written()
+        if dbias is not None:
+            dbias.device_written()
 
     def __del__(self):
         try:

@@ -5,7 +5,9 @@ Tensor.swift:26-54), `.t` (tensor/TensorInit.swift:844-890), the matmul operator
 (operators/Matmul.swift:29-72) and Dense (Sources/SwiftRTLayers/Dense.swift:21-71).
 All arithmetic happens in the native module; this file only carries layout and dispatch.
 """
+import ctypes
 import enum
+import math
 
 import numpy as np
 
@@ -52,15 +54,31 @@ class Tensor:
     version-based migration, platform/common/DiscreteStorage.swift:211-381)."""
 
     class _Storage:
-        def __init__(self, host):
-            self.host = host            # flat numpy array (authoritative when host_version is newest)
+        """The flat buffer: a host replica made on first use (zeros, when no values were given) and a device replica
+        made on first use.  A result never touched by the host has no host replica at all."""
+        __slots__ = ("_host", "dtype", "itemsize", "size", "nbytes", "device", "host_version", "device_version", "last_queue",
+                     "last_copy")
+
+        def __init__(self, host=None, dtype=None, size=None):
+            self._host = host           # flat numpy array (authoritative when host_version is newest), or None: zeros
+            self.dtype = host.dtype if host is not None else np.dtype(dtype)
+            self.itemsize = self.dtype.itemsize
+            self.size = host.size if host is not None else size
+            self.nbytes = self.size * self.itemsize
             self.device = None          # HipDeviceMemory
             self.host_version = 0
             self.device_version = -1
             self.last_queue = None
             self.last_copy = None       # "h2d" / "d2h": DiscreteStorage.testLastAccessCopiedDeviceMemory role
 
+        @property
+        def host(self):
+            if self._host is None:
+                self._host = np.zeros(self.size, dtype=self.dtype)
+            return self._host
+
     def __init__(self, array=None, shape=None, dtype=None, order=Order.row, _storage=None, _offset=0, _strides=None):
+        self._descriptor = None
         if _storage is not None:
             self.storage, self.offset = _storage, _offset
             self.shape, self.strides, self.order = tuple(shape), tuple(_strides), order
@@ -72,14 +90,14 @@ class Tensor:
             if arr.dtype not in _DTYPES:
                 raise TypeError(f"unsupported element storage {arr.dtype}")
             shape = arr.shape
-            flat = np.ascontiguousarray(arr).reshape(-1).copy()
             if order == Order.col and arr.ndim >= 2:
                 # lay the logical values out column-major in the last two dims
                 flat = np.ascontiguousarray(np.swapaxes(arr, -1, -2)).reshape(-1).copy()
+            else:
+                flat = np.ascontiguousarray(arr).reshape(-1).copy()
+            self.storage = Tensor._Storage(flat)
         else:
-            n = int(np.prod(shape)) if len(shape) else 1
-            flat = np.zeros(n, dtype=np.dtype(dtype))
-        self.storage = Tensor._Storage(flat)
+            self.storage = Tensor._Storage(dtype=dtype, size=math.prod(int(s) for s in shape))
         self.offset = 0
         self.shape = tuple(int(s) for s in shape)
         self.strides = tuple(strides_for(self.shape, order))
@@ -88,7 +106,7 @@ class Tensor:
     # -- layout ------------------------------------------------------------------------------
     @property
     def dtype(self):
-        return self.storage.host.dtype
+        return self.storage.dtype
 
     @property
     def rank(self):
@@ -96,7 +114,7 @@ class Tensor:
 
     @property
     def count(self):
-        return int(np.prod(self.shape)) if self.shape else 1
+        return math.prod(self.shape)
 
     @property
     def t(self):
@@ -125,6 +143,14 @@ class Tensor:
 
     def descriptor(self):
         return native.make_descriptor(_DTYPES[self.dtype], self.shape, self.strides, self.order.value)
+
+    def descriptor_ref(self):
+        """The descriptor as an argument of a native call: made once (a tensor's layout never changes) and kept with the
+        tensor.  For this module's own calls, which do not write to it; descriptor() makes one that the caller owns."""
+        if self._descriptor is None:
+            d, keep = self.descriptor()
+            self._descriptor = (ctypes.byref(d), d, keep)
+        return self._descriptor[0]
 
     @property
     def type_id(self):
@@ -190,11 +216,12 @@ class Tensor:
     def _ensure_device(self, queue):
         s = self.storage
         if s.device is None:
-            s.device = queue.allocate(s.host.nbytes)
-        if s.last_queue is not None and s.last_queue is not queue:
-            queue.wait(s.last_queue.record_event())   # cross-queue sync, DiscreteStorage.swift:271-296
-        s.last_queue = queue
-        s.device.last_queue = queue
+            s.device = queue.allocate(s.nbytes)
+        if s.last_queue is not queue:
+            if s.last_queue is not None:
+                queue.wait(s.last_queue.record_event())   # cross-queue sync, DiscreteStorage.swift:271-296
+            s.last_queue = queue
+            s.device.last_queue = queue
 
     def device_read(self, queue):
         """Pointer to this view's first element on the queue's device, copying host->device when
@@ -203,17 +230,33 @@ class Tensor:
         self._ensure_device(queue)
         s.last_copy = None
         if s.device_version < s.host_version:
-            queue.copy_to_device(s.host.ctypes.data, s.device, s.host.nbytes)
-            queue.wait_for_completion()      # the pageable host buffer may change after return
+            if s._host is None:                  # zeros: made where they are read
+                queue.zero(s.device, s.nbytes)
+            else:
+                queue.copy_to_device(s.host.ctypes.data, s.device, s.nbytes)
+                queue.wait_for_completion()      # the pageable host buffer may change after return
+                s.last_copy = "h2d"
             s.device_version = s.host_version
-            s.last_copy = "h2d"
-        return s.device.pointer + self.offset * s.host.itemsize
+        return s.device.pointer + self.offset * s.itemsize
 
     def device_read_write(self, queue):
         ptr = self.device_read(queue)
+        self.device_written()
+        return ptr
+
+    def device_write(self, queue):
+        """Pointer to this view's first element on the queue's device, for a call that writes every element of the view and
+        reads none: when the view is the whole buffer, nothing is copied or cleared first (the values a 4096 x 11008 result
+        was born with took three milliseconds to make and move).  device_written() follows once the call has been accepted."""
+        s = self.storage
+        if self.offset == 0 and self.is_contiguous and self.count == s.size:
+            self._ensure_device(queue)
+            return s.device.pointer
+        return self.device_read(queue)
+
+    def device_written(self):
         s = self.storage
         s.device_version = max(s.device_version, s.host_version) + 1
-        return ptr
 
     def array(self):
         """Logical values as a numpy array in storage dtype, syncing device->host first if the
@@ -222,11 +265,13 @@ class Tensor:
         s.last_copy = None
         if s.device is not None and s.device_version > s.host_version:
             q = s.last_queue
-            q.copy_to_host(s.device, s.host.ctypes.data, s.host.nbytes)
+            if s._host is None:
+                s._host = np.empty(s.size, dtype=s.dtype)
+            q.copy_to_host(s.device, s.host.ctypes.data, s.nbytes)
             q.wait_for_completion()
             s.host_version = s.device_version
             s.last_copy = "d2h"
-        item = s.host.itemsize
+        item = s.itemsize
         return np.lib.stride_tricks.as_strided(s.host[self.offset:], shape=self.shape,
                                                strides=[st * item for st in self.strides]).copy()
 
