@@ -405,6 +405,18 @@ srtStatus srtCopy(const void* a, const srtTensorDescriptor* aDesc,
 srtStatus srtCopyFlat(srtDataType atype, const void* a, srtDataType otype, void* out, size_t count,
                       srtStream stream);
 srtStatus srtFillFlat(srtDataType type, void* out, const void* element, size_t count, srtStream stream);
+/* out = a and b joined along dimension `axis` (concatenate(_:_:axis:) of two tensors): out.shape[axis] =
+ * a.shape[axis] + b.shape[axis], every other extent equal, one element type, any strides. */
+srtStatus srtConcat(const void* a, const srtTensorDescriptor* aDesc, const void* b, const srtTensorDescriptor* bDesc,
+                    int32_t axis, void* out, const srtTensorDescriptor* oDesc, srtStream stream);
+/* The gate arithmetic of an LSTM cell (LSTMCell, Sources/SwiftRTLayers/Recurrent.swift:255-266) in one call.
+ * gates [B, 4H] = input, update, forget, output parts side by side; cell, newCell, newHidden [B, H]:
+ *   newCell = cell * sigmoid(forget) + sigmoid(input) * tanh(update);  newHidden = tanh(newCell) * sigmoid(output)
+ * Every intermediate is rounded to the element type: the results are bit for bit those of the srtSigmoid, srtTanh,
+ * srtMul and srtAdd calls it stands for.  Element types 32F, 16F, 16BF, one for all; any strides. */
+srtStatus srtLstmGates(const void* gates, const srtTensorDescriptor* gatesDesc, const void* cell,
+                       const srtTensorDescriptor* cellDesc, void* newCell, const srtTensorDescriptor* newCellDesc,
+                       void* newHidden, const srtTensorDescriptor* newHiddenDesc, srtStream stream);
 
 /* ---- test helper ------------------------------------------------------------------------- */
 /* Replaces srtDelayStream, Modules/SwiftRTCuda/utilities_api.h:28: occupies `stream` for about

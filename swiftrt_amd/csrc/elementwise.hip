@@ -12,6 +12,7 @@
 // :1369-1377 `1 / (1 + exp(-x))`, ...).  This file is compiled with floating-point contraction
 // off so the four basic operations match a C restatement bit for bit.
 #include <cstring>
+#include <type_traits>
 
 #include "gemm_common.h"
 #include "status.h"
@@ -21,6 +22,12 @@ namespace ew {
 
 constexpr int MAX_RANK = 4;   // after collapsing adjacent dimensions
 constexpr int kVectorsPerLane = 4;   // (two: sigmoid 32.2 -> 30.7 us, bias-broadcast add 33.3 -> 36.8, the rest unchanged)
+// Up to this much traffic a lane takes one vector, without the streaming hint: a small map is a launch and a memory round trip,
+// four vectors one after the other are four round trips on a quarter of the lanes, and its bytes were most likely just written
+// and stay in the caches for whatever reads them next.  One each / four each, us: add bf16 2048^2 (25 MB) 5.4 / 8.3, bias add bf16 1000
+// x 4096 (16 MB) 4.3 / 7.2, sigmoid f32 2048 x 2000 (33 MB) 6.8 / 8.7, bias add and tanh bf16 4096^2 (67 MB) 12.2 / 13.9 and 11.9 /
+// 13.2, add bf16 4096^2 (100 MB) 18.5 / 17.9, cast bf16 4096^2 to f32 (100 MB) 19.8 / 18.0, add f32 4096^2 (201 MB) 36.9 / 33.2.
+constexpr unsigned long long kOneVectorBytes = 80000000;
 
 // ---- operations -----------------------------------------------------------------------------
 struct Add { static constexpr bool binary = true; static __device__ __forceinline__ float apply(float a, float b) { return a + b; } };
@@ -87,8 +94,8 @@ __device__ __forceinline__ Pack<T, V> load_pack(const typename T::storage* p) {
   }
 }
 
-template <typename TI, typename TO, typename Op, int V, bool B_CACHED = false>
-__global__ __launch_bounds__(256) void map_kernel(Map m) {
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE>
+__device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
   using SI = typename TI::storage;
   using SO = typename TO::storage;
   const SI* a = (const SI*)m.a;
@@ -99,9 +106,9 @@ __global__ __launch_bounds__(256) void map_kernel(Map m) {
   // this device the memory parallelism of a streaming kernel comes from the waves: the same kernel with all
   // four vectors' loads issued before the first use needs 92 registers (five waves) and ran 15-20 % slower,
   // and four consecutive rows per lane with a row-broadcast operand loaded once were no faster either.
-  const unsigned long long base = (unsigned long long)blockIdx.x * (256 * kVectorsPerLane) + threadIdx.x;
+  const unsigned long long base = (unsigned long long)block * (256 * PER_LANE) + threadIdx.x;
 #pragma unroll
-  for (int u = 0; u < kVectorsPerLane; ++u) {
+  for (int u = 0; u < PER_LANE; ++u) {
     const unsigned long long id = base + (unsigned long long)u * 256;
     if (id >= m.total) break;
     // decompose the vector id over the collapsed dimensions
@@ -128,7 +135,7 @@ __global__ __launch_bounds__(256) void map_kernel(Map m) {
 #pragma unroll
       for (int i = 0; i < V; ++i) fa[i] = m.element;
     } else if (V > 1 && m.sa[inner] == 1) {
-      const Pack<TI, V> pa = load_pack<TI, V, true>(a + oa);
+      const Pack<TI, V> pa = load_pack<TI, V, PER_LANE != 1>(a + oa);
 #pragma unroll
       for (int i = 0; i < V; ++i) fa[i] = TI::to_float(pa.v[i]);
     } else {
@@ -143,7 +150,7 @@ __global__ __launch_bounds__(256) void map_kernel(Map m) {
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = 0.0f;
     } else if (V > 1 && m.sb[inner] == 1) {
-      const Pack<TI, V> pb = load_pack<TI, V, !B_CACHED>(b + ob);
+      const Pack<TI, V> pb = load_pack<TI, V, !B_CACHED && PER_LANE != 1>(b + ob);
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = TI::to_float(pb.v[i]);
     } else {
@@ -168,11 +175,31 @@ __global__ __launch_bounds__(256) void map_kernel(Map m) {
   }
 }
 
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED = false, int PER_LANE = kVectorsPerLane>
+__global__ __launch_bounds__(256) void map_kernel(Map m) {
+  map_block<TI, TO, Op, V, B_CACHED, PER_LANE>(m, blockIdx.x);
+}
+
+// Two copies in one launch (the halves of a concatenation).
+template <typename T, int V>
+__global__ __launch_bounds__(256) void copy_pair_kernel(Map m0, Map m1, uint32_t blocks0) {
+  if (blockIdx.x < blocks0) map_block<T, T, Copy, V, false, 1>(m0, blockIdx.x);
+  else map_block<T, T, Copy, V, false, 1>(m1, blockIdx.x - blocks0);
+}
+
 template <typename TI, typename TO, typename Op, int V>
 hipError_t launch_v(const Map& m, hipStream_t stream) {
-  const unsigned long long blocks = (m.total + 256 * kVectorsPerLane - 1) / (256 * kVectorsPerLane);
+  unsigned long long vector_bytes = V * sizeof(typename TO::storage);
+  if (!m.fill) vector_bytes += V * sizeof(typename TI::storage) * (m.b && !m.b_reused ? 2 : 1);
+  // (single elements, 2-byte accesses: from a million of them four each, bias add bf16 4095^2 34.0 us against 37.8)
+  const int per_lane = m.total * vector_bytes <= (V == 1 ? kOneVectorBytes / 16 : kOneVectorBytes) ? 1 : kVectorsPerLane;
+  const unsigned long long blocks = (m.total + 256 * per_lane - 1) / (256 * per_lane);
   if (blocks == 0) return hipSuccess;
   if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  if (per_lane == 1) {
+    hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, false, 1>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
+    return launch_status(stream);
+  }
   // (a run-time choice between the two kinds of load inside one kernel cost every operation 14 %)
   if constexpr (V > 1 && Op::binary) {
     if (m.b_reused) {
@@ -261,6 +288,89 @@ hipError_t launch_convert(int itype, int otype, const Map& m, hipStream_t stream
   if (itype == srtReal16BF && otype == srtReal16F) return launch_t<BF16, F16, Copy>(m, stream);
   if (itype == srtReal16F && otype == srtReal16BF) return launch_t<F16, BF16, Copy>(m, stream);
   return hipErrorNotSupported;
+}
+
+template <typename T>
+hipError_t launch_copy_pair(Map m0, Map m1, hipStream_t stream) {
+  constexpr int V = 16 / sizeof(typename T::storage);
+  auto go = [&](auto width) {
+    constexpr int W = decltype(width)::value;
+    const unsigned long long b0 = (m0.total + 255) / 256, b1 = (m1.total + 255) / 256;
+    if (b0 + b1 > 0x7fffffffull) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((copy_pair_kernel<T, W>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, m0, m1, (uint32_t)b0);
+    return launch_status(stream);
+  };
+  if (vector_width<T, T>(m0) == V && vector_width<T, T>(m1) == V) {
+    for (Map* m : {&m0, &m1}) {
+      m->shape[m->rank - 1] /= V;
+      m->total /= V;
+    }
+    return go(std::integral_constant<int, V>{});
+  }
+  return go(std::integral_constant<int, 1>{});
+}
+
+// ---- the gate arithmetic of an LSTM cell ---------------------------------------------------------
+// From gates = [input, update, forget, output] (one row of 4 H per batch row) and the cell state:
+//   cell' = cell * sigmoid(forget) + sigmoid(input) * tanh(update),  hidden' = tanh(cell') * sigmoid(output)
+// with every intermediate rounded to the element type, i.e. bit for bit what the nine element-wise launches it replaces give.
+// Those were launches and round trips, not bytes: 64 x 512 fp32 is 0.9 MB in all and took 9 x 7 us; here it is one launch, each
+// value read and written once, a lane one 16-byte vector of the H dimension (one element when the layout does not allow it).
+struct GateProblem {
+  uint32_t rows, columns;            // columns counted in vectors of V elements
+  const void* gates;
+  const void* cell;
+  void* new_cell;
+  void* new_hidden;
+  long long part;                    // elements between the gates of one column
+  long long gates_row, gates_col, cell_row, cell_col, new_cell_row, new_cell_col, new_hidden_row, new_hidden_col;
+};
+
+template <typename T, int V>
+__global__ __launch_bounds__(256) void lstm_gates_kernel(GateProblem p) {
+  using S = typename T::storage;
+  using SigmoidT = std::conditional_t<T::dtype == srtReal32F, Sigmoid, SigmoidFast>;
+  using TanhT = std::conditional_t<T::dtype == srtReal32F, Tanh, TanhFast>;
+  const uint32_t id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= p.rows * p.columns) return;
+  const uint32_t row = id / p.columns, col = (id - row * p.columns) * V;
+  const S* g = (const S*)p.gates + (long long)row * p.gates_row + (long long)col * p.gates_col;
+  const Pack<T, V> gi = load_pack<T, V, false>(g), gu = load_pack<T, V, false>(g + p.part),
+                   gf = load_pack<T, V, false>(g + 2 * p.part), go = load_pack<T, V, false>(g + 3 * p.part);
+  const Pack<T, V> c = load_pack<T, V, false>((const S*)p.cell + (long long)row * p.cell_row + (long long)col * p.cell_col);
+  Pack<T, V> nc, nh;
+  auto round = [](float x) { return T::to_float(T::from_float(x)); };
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const float in = round(SigmoidT::apply(T::to_float(gi.v[i]), 0.0f)), up = round(TanhT::apply(T::to_float(gu.v[i]), 0.0f));
+    const float forget = round(SigmoidT::apply(T::to_float(gf.v[i]), 0.0f)), out = round(SigmoidT::apply(T::to_float(go.v[i]), 0.0f));
+    const float kept = round(T::to_float(c.v[i]) * forget), added = round(in * up);
+    nc.v[i] = T::from_float(kept + added);
+    nh.v[i] = T::from_float(round(TanhT::apply(T::to_float(nc.v[i]), 0.0f)) * out);
+  }
+  *reinterpret_cast<Pack<T, V>*>((S*)p.new_cell + (long long)row * p.new_cell_row + (long long)col * p.new_cell_col) = nc;
+  *reinterpret_cast<Pack<T, V>*>((S*)p.new_hidden + (long long)row * p.new_hidden_row + (long long)col * p.new_hidden_col) = nh;
+}
+
+template <typename T>
+hipError_t launch_lstm_gates(GateProblem p, hipStream_t stream) {
+  constexpr int V = 16 / sizeof(typename T::storage);
+  auto go = [&](auto width) {
+    constexpr int W = decltype(width)::value;
+    p.columns /= W;
+    const unsigned long long lanes = (unsigned long long)p.rows * p.columns;
+    if (lanes > 0x7fffffffull) return hipErrorNotSupported;
+    hipLaunchKernelGGL((lstm_gates_kernel<T, W>), dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, stream, p);
+    return launch_status(stream);
+  };
+  const bool dense = p.gates_col == 1 && p.cell_col == 1 && p.new_cell_col == 1 && p.new_hidden_col == 1;
+  const bool whole = p.columns % V == 0 && p.part % V == 0 && p.gates_row % V == 0 && p.cell_row % V == 0 && p.new_cell_row % V == 0 &&
+                     p.new_hidden_row % V == 0;
+  const bool aligned = (((uintptr_t)p.gates | (uintptr_t)p.cell | (uintptr_t)p.new_cell | (uintptr_t)p.new_hidden) & 15u) == 0;
+  // (a small cell has more to gain from lanes than from wide accesses: the transcendental chain of a lane is serial)
+  const bool few = (unsigned long long)p.rows * p.columns <= 256ull * 1024;
+  if (dense && whole && aligned && !few) return go(std::integral_constant<int, V>{});
+  return go(std::integral_constant<int, 1>{});
 }
 
 // ---- host side: descriptors -> collapsed index space -------------------------------------------
@@ -524,6 +634,74 @@ srtStatus srtFillFlat(srtDataType type, void* out, const void* element, size_t c
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   return flat_pieces(count, type_size(type), type_size(type), m,
                      [&](const Map& p) { return launch_op(kCopy, type, p, hs); });
+}
+
+
+// out = a and b joined along `axis`: the two copies of a concatenation in one launch.
+srtStatus srtConcat(const void* a, const srtTensorDescriptor* aDesc, const void* b, const srtTensorDescriptor* bDesc, int32_t axis,
+                    void* out, const srtTensorDescriptor* oDesc, srtStream stream) {
+  if (!desc_ok(aDesc) || !desc_ok(bDesc) || !desc_ok(oDesc)) return srtErrorInvalidValue;
+  if (!float_type(oDesc->type) || aDesc->type != oDesc->type || bDesc->type != oDesc->type) return srtErrorNotSupported;
+  const uint32_t rank = oDesc->rank;
+  if (rank > 8) return srtErrorNotSupported;
+  if (aDesc->rank != rank || bDesc->rank != rank || axis < 0 || (uint32_t)axis >= rank) return srtErrorInvalidValue;
+  if (aDesc->shape[axis] + bDesc->shape[axis] != oDesc->shape[axis]) return srtErrorInvalidValue;
+  Map m[2]{};
+  bool empty[2];
+  for (int i = 0; i < 2; ++i) {
+    const srtTensorDescriptor* d = i ? bDesc : aDesc;
+    srtTensorDescriptor part = *oDesc;   // the piece of the result that this input fills
+    size_t shape[8];
+    for (uint32_t k = 0; k < rank; ++k) shape[k] = k == (uint32_t)axis ? d->shape[k] : oDesc->shape[k];
+    part.shape = shape;
+    if (srtStatus s = build_map(d, nullptr, &part, &m[i], &empty[i]); s != srtSuccess) return s;
+    if (!empty[i] && (!(i ? b : a) || !out)) return srtErrorInvalidValue;
+    m[i].a = i ? b : a;
+    m[i].o = (char*)out + (i ? aDesc->shape[axis] * oDesc->strides[axis] * type_size(oDesc->type) : 0);
+  }
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  if (empty[0] && empty[1]) return srtSuccess;
+  if (empty[0] || empty[1]) return srt::from_hip(launch_op(kCopy, oDesc->type, m[empty[0] ? 1 : 0], hs));
+  if ((m[0].total + m[1].total) * 2 * type_size(oDesc->type) > kOneVectorBytes) {   // bytes, not launches: the plain copy's shape
+    if (srtStatus s = srt::from_hip(launch_op(kCopy, oDesc->type, m[0], hs)); s != srtSuccess) return s;
+    return srt::from_hip(launch_op(kCopy, oDesc->type, m[1], hs));
+  }
+  switch (oDesc->type) {
+    case srtReal32F: return srt::from_hip(launch_copy_pair<srt::F32>(m[0], m[1], hs));
+    case srtReal16F: return srt::from_hip(launch_copy_pair<srt::F16>(m[0], m[1], hs));
+    default: return srt::from_hip(launch_copy_pair<srt::BF16>(m[0], m[1], hs));
+  }
+}
+
+srtStatus srtLstmGates(const void* gates, const srtTensorDescriptor* gatesDesc, const void* cell, const srtTensorDescriptor* cellDesc,
+                       void* newCell, const srtTensorDescriptor* newCellDesc, void* newHidden,
+                       const srtTensorDescriptor* newHiddenDesc, srtStream stream) {
+  const srtTensorDescriptor* all[4] = {gatesDesc, cellDesc, newCellDesc, newHiddenDesc};
+  for (const srtTensorDescriptor* d : all) {
+    if (!desc_ok(d)) return srtErrorInvalidValue;
+    if (!float_type(d->type) || d->type != gatesDesc->type) return srtErrorNotSupported;
+    if (d->rank != 2 || d->shape[0] != gatesDesc->shape[0]) return srtErrorInvalidValue;
+  }
+  const size_t rows = cellDesc->shape[0], columns = cellDesc->shape[1];
+  if (gatesDesc->shape[1] != 4 * columns || newCellDesc->shape[1] != columns || newHiddenDesc->shape[1] != columns)
+    return srtErrorInvalidValue;
+  if (rows == 0 || columns == 0) return srtSuccess;
+  if (rows > 0x7fffffffull || columns > 0x7fffffffull) return srtErrorNotSupported;
+  if (!gates || !cell || !newCell || !newHidden) return srtErrorInvalidValue;
+  GateProblem p{};
+  p.rows = (uint32_t)rows; p.columns = (uint32_t)columns;
+  p.gates = gates; p.cell = cell; p.new_cell = newCell; p.new_hidden = newHidden;
+  p.part = (long long)(columns * gatesDesc->strides[1]);
+  p.gates_row = (long long)gatesDesc->strides[0]; p.gates_col = (long long)gatesDesc->strides[1];
+  p.cell_row = (long long)cellDesc->strides[0]; p.cell_col = (long long)cellDesc->strides[1];
+  p.new_cell_row = (long long)newCellDesc->strides[0]; p.new_cell_col = (long long)newCellDesc->strides[1];
+  p.new_hidden_row = (long long)newHiddenDesc->strides[0]; p.new_hidden_col = (long long)newHiddenDesc->strides[1];
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  switch (gatesDesc->type) {
+    case srtReal32F: return srt::from_hip(launch_lstm_gates<srt::F32>(p, hs));
+    case srtReal16F: return srt::from_hip(launch_lstm_gates<srt::F16>(p, hs));
+    default: return srt::from_hip(launch_lstm_gates<srt::BF16>(p, hs));
+  }
 }
 
 }  // extern "C"

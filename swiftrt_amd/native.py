@@ -5,6 +5,7 @@ is missing, or a call returns a hard error, an exception is raised.
 """
 import ctypes
 import os
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # SWIFTRT_HIP_LIBRARY selects another build of the same library (e.g. lib/debug/libSwiftRTHip.so from
@@ -103,6 +104,8 @@ SIGNATURES = {
     "srtPlanCacheLoad": (_i32, [ctypes.c_char_p]),
     "srtCopyFlat": (_i32, [_i32, _vp, _i32, _vp, ctypes.c_size_t, _vp]),
     "srtFillFlat": (_i32, [_i32, _vp, _vp, ctypes.c_size_t, _vp]),
+    "srtConcat": (_i32, [_vp, _descp, _vp, _descp, _i32, _vp, _descp, _vp]),
+    "srtLstmGates": (_i32, [_vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _vp]),
 }
 # element-wise neighbours: tensor-tensor, tensor-element and unary forms share three signatures
 for _name in ("Add", "Sub", "Mul", "Div", "Max", "Min"):
@@ -151,24 +154,34 @@ def check(status, what="srt call"):
     raise SrtError(status, what)
 
 
+_U64 = (1 << 64) - 1
+# rank -> (packer of a descriptor followed by its three arrays, buffer type): the header is 56 bytes, then shape, strides and
+# logical strides, to which the header's three pointers point
+_DESCRIPTOR_LAYOUTS = {}
+
+
+def _descriptor_layout(rank):
+    packer = struct.Struct(f"=iIi4x{5 + 3 * rank}Q")
+    assert packer.size == ctypes.sizeof(TensorDescriptor) + 24 * rank
+    _DESCRIPTOR_LAYOUTS[rank] = packer, ctypes.c_char * packer.size
+    return _DESCRIPTOR_LAYOUTS[rank]
+
+
 def make_descriptor(dtype, shape, strides, order):
     """Build an srtTensorDescriptor; returns (descriptor, keepalive) -- keep `keepalive`
     referenced for the duration of the call, like the stack arrays in Tensor.withTensor."""
     rank = len(shape)
-    arr_t = ctypes.c_size_t * rank
-    shp = arr_t(*[int(s) for s in shape])
-    std = arr_t(*[int(s) for s in strides])
-    dense = [1] * rank
-    for i in range(rank - 2, -1, -1):
-        dense[i] = dense[i + 1] * int(shape[i + 1])
-    lst = arr_t(*dense)
-    count = 1
-    span = 1
-    for s, st in zip(shape, strides):
-        count *= int(s)
-        span += (int(s) - 1) * int(st) if int(s) > 0 else 0
-    d = TensorDescriptor(int(dtype), rank, int(order), count, span if count else 0,
-                         ctypes.cast(shp, ctypes.POINTER(ctypes.c_size_t)),
-                         ctypes.cast(std, ctypes.POINTER(ctypes.c_size_t)),
-                         ctypes.cast(lst, ctypes.POINTER(ctypes.c_size_t)))
-    return d, (shp, std, lst)
+    packer, buffer = _DESCRIPTOR_LAYOUTS.get(rank) or _descriptor_layout(rank)
+    shape = [int(s) for s in shape]
+    strides = [int(s) for s in strides]
+    count, span, dense = 1, 1, [1] * rank
+    for i in range(rank - 1, -1, -1):
+        dense[i] = count
+        count *= shape[i]
+        if shape[i] > 0:
+            span += (shape[i] - 1) * strides[i]
+    buf = buffer()
+    at = ctypes.addressof(buf) + 56
+    packer.pack_into(buf, 0, int(dtype), rank, int(order), count & _U64, (span if count else 0) & _U64, at, at + 8 * rank,
+                     at + 16 * rank, *[s & _U64 for s in shape], *[s & _U64 for s in strides], *[s & _U64 for s in dense])
+    return TensorDescriptor.from_buffer(buf), buf

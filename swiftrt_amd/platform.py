@@ -249,6 +249,25 @@ class HipQueue:
         """Role of CudaQueue.copy / cast: element types may differ (srtCopy converts)."""
         self._elementwise("Copy", x, None, out)
 
+    def concatenate(self, a, b, axis, out):
+        """out = a and b joined along `axis`, one launch."""
+        self.select()
+        a_ptr, b_ptr = a.device_read(self), b.device_read(self)
+        o_ptr = out.device_write(self)
+        check(native.lib().srtConcat(a_ptr, a.descriptor_ref(), b_ptr, b.descriptor_ref(), axis, o_ptr, out.descriptor_ref(),
+                                     self.stream), "srtConcat")
+        out.device_written()
+
+    def lstm_gates(self, gates, cell, new_cell, new_hidden):
+        """The gate arithmetic of LSTMCell (SwiftRTLayers/Recurrent.swift:255-266), one launch."""
+        self.select()
+        g_ptr, c_ptr = gates.device_read(self), cell.device_read(self)
+        nc_ptr, nh_ptr = new_cell.device_write(self), new_hidden.device_write(self)
+        check(native.lib().srtLstmGates(g_ptr, gates.descriptor_ref(), c_ptr, cell.descriptor_ref(), nc_ptr,
+                                        new_cell.descriptor_ref(), nh_ptr, new_hidden.descriptor_ref(), self.stream), "srtLstmGates")
+        new_cell.device_written()
+        new_hidden.device_written()
+
     def fill(self, out, value):
         """Role of CudaQueue.fill(_:with:) (platform/cuda/functions/CudaFill.swift): dense `out`."""
         self.select()

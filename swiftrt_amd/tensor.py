@@ -78,7 +78,7 @@ class Tensor:
             return self._host
 
     def __init__(self, array=None, shape=None, dtype=None, order=Order.row, _storage=None, _offset=0, _strides=None):
-        self._descriptor = None
+        self._descriptor = self._contiguous = None   # made on first use: a tensor's layout never changes
         if _storage is not None:
             self.storage, self.offset = _storage, _offset
             self.shape, self.strides, self.order = tuple(shape), tuple(_strides), order
@@ -102,6 +102,7 @@ class Tensor:
         self.shape = tuple(int(s) for s in shape)
         self.strides = tuple(strides_for(self.shape, order))
         self.order = order
+        self._contiguous = True
 
     # -- layout ------------------------------------------------------------------------------
     @property
@@ -145,8 +146,7 @@ class Tensor:
         return native.make_descriptor(_DTYPES[self.dtype], self.shape, self.strides, self.order.value)
 
     def descriptor_ref(self):
-        """The descriptor as an argument of a native call: made once (a tensor's layout never changes) and kept with the
-        tensor.  For this module's own calls, which do not write to it; descriptor() makes one that the caller owns."""
+        """The descriptor as an argument of a native call: made once and kept with the tensor.  For this module's own calls, which do not write to it; descriptor() makes one that the caller owns."""
         if self._descriptor is None:
             d, keep = self.descriptor()
             self._descriptor = (ctypes.byref(d), d, keep)
@@ -158,7 +158,9 @@ class Tensor:
 
     @property
     def is_contiguous(self):
-        return tuple(self.strides) == tuple(strides_for(self.shape, self.order))
+        if self._contiguous is None:
+            self._contiguous = tuple(self.strides) == tuple(strides_for(self.shape, self.order))
+        return self._contiguous
 
     def element_storage(self, value):
         """One scalar in this tensor's storage format (a 1-element array): what
@@ -356,19 +358,14 @@ def filled(shape, value, dtype, order=Order.row):
 
 
 def concatenate(a, b, axis):
-    """concatenate(_:_:axis:) of two tensors: two strided device copies into views of the result."""
+    """concatenate(_:_:axis:) of two tensors, one device call."""
     if a.rank != b.rank or a.dtype != b.dtype:
         raise ValueError("concatenate: rank and element type must agree")
+    axis %= a.rank
     shape = list(a.shape)
     shape[axis] += b.shape[axis]
     out = Tensor(shape=shape, dtype=a.dtype, order=a.order)
-    lo = [slice(None)] * a.rank
-    hi = [slice(None)] * a.rank
-    lo[axis] = slice(0, a.shape[axis])
-    hi[axis] = slice(a.shape[axis], shape[axis])
-    q = current_queue()
-    q.copy(a, out[tuple(lo)])
-    q.copy(b, out[tuple(hi)])
+    current_queue().concatenate(a, b, axis, out)
     return out
 
 
@@ -441,10 +438,7 @@ class LSTMCell:
     def __call__(self, x, cell, hidden):
         gate_input = concatenate(x, hidden, axis=1)
         fused = matmul(gate_input, self.fused_weight, bias=self.fused_bias)
-        input_gate = sigmoid(self.part(0, fused))
-        update_gate = tanh(self.part(1, fused))
-        forget_gate = sigmoid(self.part(2, fused))
-        output_gate = sigmoid(self.part(3, fused))
-        new_cell = cell * forget_gate + input_gate * update_gate
-        new_hidden = tanh(new_cell) * output_gate
+        new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
+        new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
+        current_queue().lstm_gates(fused, cell, new_cell, new_hidden)
         return new_cell, new_hidden
