@@ -13,6 +13,7 @@
 // off so the four basic operations match a C restatement bit for bit.
 #include <cstring>
 #include <type_traits>
+#include <utility>
 
 #include "gemm_common.h"
 #include "status.h"
@@ -70,6 +71,7 @@ struct Map {
   int b_is_element;
   int fill;                      // no input at all: out = element
   int b_reused;                  // the second operand is broadcast along some dimension: its lines are read again and again
+  uint32_t inner_elements;       // extent of the innermost dimension in elements
 };
 
 template <typename T, int V>
@@ -81,11 +83,15 @@ struct alignas(V * sizeof(typename T::storage)) Pack {
 // is read once, and without the hint its lines stay in L2 until evicted (the same hint raised a
 // bare streaming read of this device from 5.7 to 6.2 TB/s).  A broadcast operand (a bias row under
 // every row of the other operand) is the opposite case: its few lines are wanted in the caches.
-template <typename T, int V, bool STREAM>
+// ANYWHERE: from any element's address (global memory takes 16 bytes at element alignment).
+template <typename T, int V, bool STREAM, bool ANYWHERE = false>
 __device__ __forceinline__ Pack<T, V> load_pack(const typename T::storage* p) {
-  constexpr int BYTES = V * (int)sizeof(typename T::storage);
+  using S = typename T::storage;
+  constexpr int BYTES = V * (int)sizeof(S);
   if constexpr (BYTES >= 8) {
-    typedef uint32_t words_t __attribute__((ext_vector_type(BYTES / 4)));
+    typedef uint32_t whole_t __attribute__((ext_vector_type(BYTES / 4)));
+    typedef uint32_t loose_t __attribute__((ext_vector_type(BYTES / 4), aligned(sizeof(S))));
+    using words_t = std::conditional_t<ANYWHERE, loose_t, whole_t>;
     const words_t w = STREAM ? __builtin_nontemporal_load(reinterpret_cast<const words_t*>(p))
                              : *reinterpret_cast<const words_t*>(p);
     return __builtin_bit_cast(Pack<T, V>, w);
@@ -93,8 +99,32 @@ __device__ __forceinline__ Pack<T, V> load_pack(const typename T::storage* p) {
     return *reinterpret_cast<const Pack<T, V>*>(p);
   }
 }
+template <typename T, int V>
+__device__ __forceinline__ void store_pack_anywhere(typename T::storage* p, const Pack<T, V>& v) {
+  __builtin_memcpy(p, &v, sizeof(v));
+}
 
-template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE>
+// V results of an operation, rounded to the element type.
+template <typename TO, typename Op, int V>
+__device__ __forceinline__ Pack<TO, V> apply_pack(const float (&fa)[V], const float (&fb)[V]) {
+  Pack<TO, V> po;
+  if constexpr (V > 1 && TO::dtype == srtReal16BF) {
+    float r[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) r[i] = Op::apply(fa[i], fb[i]);
+    uint32_t w[V / 2];
+    encode_bf16<V>(r, w);
+    po = __builtin_bit_cast(Pack<TO, V>, w);
+  } else {
+#pragma unroll
+    for (int i = 0; i < V; ++i) po.v[i] = TO::from_float(Op::apply(fa[i], fb[i]));
+  }
+  return po;
+}
+
+// RAGGED: rows that are no whole number of aligned vectors (odd extents, pitches or bases): the last vector of a row is partial and
+// goes by elements, the others at element alignment.
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE, bool RAGGED = false>
 __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
   using SI = typename TI::storage;
   using SO = typename TO::storage;
@@ -112,7 +142,7 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
     const unsigned long long id = base + (unsigned long long)u * 256;
     if (id >= m.total) break;
     // decompose the vector id over the collapsed dimensions
-    uint32_t rest = (uint32_t)id;
+    uint32_t rest = (uint32_t)id, count = V;
     long long oa = 0, ob = 0, oo = 0;
 #pragma unroll
     for (int d = MAX_RANK - 1; d >= 0; --d) {
@@ -126,16 +156,25 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
         rest = q;
       }
       const long long scale = (d == inner) ? V : 1;
+      if (RAGGED && d == inner) count = m.inner_elements - idx * V;
       oa += (long long)idx * m.sa[d] * scale;
       ob += (long long)idx * m.sb[d] * scale;
       oo += (long long)idx * m.so[d] * scale;
     }
     float fa[V], fb[V];
+    if (RAGGED && count < V) {
+      for (uint32_t i = 0; i < count; ++i) {
+        const float x = m.fill ? m.element : TI::to_float(a[oa + (long long)i * m.sa[inner]]);
+        const float y = m.b_is_element ? m.element : b == nullptr ? 0.0f : TI::to_float(b[ob + (long long)i * m.sb[inner]]);
+        o[oo + i] = TO::from_float(Op::apply(x, y));
+      }
+      continue;
+    }
     if (m.fill) {
 #pragma unroll
       for (int i = 0; i < V; ++i) fa[i] = m.element;
     } else if (V > 1 && m.sa[inner] == 1) {
-      const Pack<TI, V> pa = load_pack<TI, V, PER_LANE != 1>(a + oa);
+      const Pack<TI, V> pa = load_pack<TI, V, PER_LANE != 1, RAGGED>(a + oa);
 #pragma unroll
       for (int i = 0; i < V; ++i) fa[i] = TI::to_float(pa.v[i]);
     } else {
@@ -150,34 +189,22 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = 0.0f;
     } else if (V > 1 && m.sb[inner] == 1) {
-      const Pack<TI, V> pb = load_pack<TI, V, !B_CACHED && PER_LANE != 1>(b + ob);
+      const Pack<TI, V> pb = load_pack<TI, V, !B_CACHED && PER_LANE != 1, RAGGED>(b + ob);
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = TI::to_float(pb.v[i]);
     } else {
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = TI::to_float(b[ob + (long long)i * m.sb[inner]]);
     }
-    if constexpr (V > 1 && TO::dtype == srtReal16BF) {
-      float r[V];
-#pragma unroll
-      for (int i = 0; i < V; ++i) r[i] = Op::apply(fa[i], fb[i]);
-      uint32_t w[V / 2];
-      encode_bf16<V>(r, w);
-      *reinterpret_cast<Pack<TO, V>*>(o + oo) = __builtin_bit_cast(Pack<TO, V>, w);
-    } else if (V > 1) {
-      Pack<TO, V> po;
-#pragma unroll
-      for (int i = 0; i < V; ++i) po.v[i] = TO::from_float(Op::apply(fa[i], fb[i]));
-      *reinterpret_cast<Pack<TO, V>*>(o + oo) = po;
-    } else {
-      o[oo] = TO::from_float(Op::apply(fa[0], fb[0]));
-    }
+    const Pack<TO, V> po = apply_pack<TO, Op, V>(fa, fb);
+    if constexpr (RAGGED) store_pack_anywhere<TO, V>(o + oo, po);
+    else *reinterpret_cast<Pack<TO, V>*>(o + oo) = po;
   }
 }
 
-template <typename TI, typename TO, typename Op, int V, bool B_CACHED = false, int PER_LANE = kVectorsPerLane>
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED = false, int PER_LANE = kVectorsPerLane, bool RAGGED = false>
 __global__ __launch_bounds__(256) void map_kernel(Map m) {
-  map_block<TI, TO, Op, V, B_CACHED, PER_LANE>(m, blockIdx.x);
+  map_block<TI, TO, Op, V, B_CACHED, PER_LANE, RAGGED>(m, blockIdx.x);
 }
 
 // Two copies in one launch (the halves of a concatenation).
@@ -187,7 +214,139 @@ __global__ __launch_bounds__(256) void copy_pair_kernel(Map m0, Map m1, uint32_t
   else map_block<T, T, Copy, V, false, 1>(m1, blockIdx.x - blocks0);
 }
 
-template <typename TI, typename TO, typename Op, int V>
+// ---- operands that walk memory across the result's rows --------------------------------------------
+// An input whose unit stride lies along another dimension than the result's (`x.t` against a row-major result) made the kernel above
+// read one element per line and lane: 4096^2 bf16 66 us, 1.0 TB/s.  Here a workgroup takes 64 x 64 elements of the two dimensions: it
+// reads such an operand along its own rows (16 bytes per lane), turns it in LDS and writes the result along the result's rows;
+// an operand that needs no turning is read where the result is written.
+//   bound   memory, both sides in whole 128-byte (16-bit) or 256-byte (fp32) row segments
+//   LDS     [64 rows of the result's dimension][64 + pad], one element per bank word or half word: pad 2 (16-bit) and 1 (fp32) put the
+//           eight (four) elements a lane gathers, and its neighbours', on different banks
+constexpr int TURN = 64;
+
+struct TurnMap {
+  Map m;
+  int across;                       // the dimension of the operands' unit stride (the result's is the innermost one)
+  int turn_a, turn_b;               // which operands are turned
+  uint32_t tiles_inner, tiles_across;
+};
+
+//   STREAM  the turned operand's reads carry the streaming hint once the map is past kOneVectorBytes: f32 4096^2 32.5 -> 28.5 us, but
+//           bf16 4096^2 13.0 -> 15.3
+template <typename TI, typename TO, typename Op, bool STREAM>
+__global__ __launch_bounds__(256) void turn_kernel(TurnMap t) {
+  using SI = typename TI::storage;
+  using SO = typename TO::storage;
+  constexpr int VI = 16 / sizeof(SI);                                  // elements of a 16-byte read
+  constexpr int V = 16 / (sizeof(SI) > sizeof(SO) ? sizeof(SI) : sizeof(SO));   // elements a lane writes at once
+  constexpr int PITCH = TURN + (sizeof(SI) == 2 ? 2 : 1);
+  __shared__ SI lds[Op::binary ? 2 : 1][TURN * PITCH];
+  const Map& m = t.m;
+  const int inner = m.rank - 1;
+  // workgroup -> tile of the two dimensions, index of the others
+  uint32_t rest = blockIdx.x;
+  const uint32_t ti = rest % t.tiles_inner;
+  rest /= t.tiles_inner;
+  const uint32_t ta = (rest + ti) % t.tiles_across;   // along a diagonal: neighbours of a power-of-two pitch share no channel (4096^2 bf16 15.0 -> 12.9 us)
+  rest /= t.tiles_across;
+  long long oa = 0, ob = 0, oo = 0;
+#pragma unroll
+  for (int d = MAX_RANK - 2; d >= 0; --d) {
+    if (d >= inner || d == t.across) continue;
+    const uint32_t q = rest / m.shape[d], idx = rest - q * m.shape[d];
+    rest = q;
+    oa += (long long)idx * m.sa[d];
+    ob += (long long)idx * m.sb[d];
+    oo += (long long)idx * m.so[d];
+  }
+  const uint32_t i0 = ti * TURN, a0 = ta * TURN;
+  const uint32_t ni = min((uint32_t)TURN, m.shape[inner] - i0), na = min((uint32_t)TURN, m.shape[t.across] - a0);
+  const SI* a = (const SI*)m.a + oa + (long long)i0 * m.sa[inner] + (long long)a0 * m.sa[t.across];
+  const SI* b = m.b ? (const SI*)m.b + ob + (long long)i0 * m.sb[inner] + (long long)a0 * m.sb[t.across] : nullptr;
+  SO* o = (SO*)m.o + oo + i0 + (long long)a0 * m.so[t.across];
+  const int tid = threadIdx.x;
+
+  auto turn_in = [&](const SI* src, long long row_stride, SI* to) {
+    constexpr int CH = TURN / VI;   // reads per row
+#pragma unroll
+    for (int u = 0; u < TURN * CH / 256; ++u) {
+      const uint32_t id = tid + u * 256, row = id / CH, col = (id % CH) * VI;
+      if (row < ni && col < na) {
+        const SI* p = src + (long long)row * row_stride + col;
+        Pack<TI, VI> x;
+        if (col + VI <= na) {
+          x = load_pack<TI, VI, STREAM, true>(p);
+        } else {
+#pragma unroll
+          for (int e = 0; e < VI; ++e) x.v[e] = p[min((uint32_t)e, na - 1 - col)];
+        }
+#pragma unroll
+        for (int e = 0; e < VI; ++e) to[row * PITCH + col + e] = x.v[e];
+      }
+    }
+  };
+  if (t.turn_a) turn_in(a, m.sa[inner], lds[0]);
+  if (Op::binary && t.turn_b) turn_in(b, m.sb[inner], lds[Op::binary ? 1 : 0]);
+  __syncthreads();
+
+  constexpr int CO = TURN / V;      // writes per row of the result
+#pragma unroll
+  for (int u = 0; u < TURN * CO / 256; ++u) {
+    const uint32_t id = tid + u * 256, row = id / CO, col = (id % CO) * V;   // row: along `across`, col: along the result's rows
+    if (row >= na || col >= ni) continue;
+    float fa[V], fb[V];
+    auto gather = [&](bool turned, const SI* from, const SI* direct, long long s_inner, long long s_across, float (&f)[V]) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const uint32_t c = min(col + e, ni - 1);
+        f[e] = TI::to_float(turned ? from[c * PITCH + row] : direct[(long long)c * s_inner + (long long)row * s_across]);
+      }
+    };
+    gather(t.turn_a, lds[0], a, m.sa[inner], m.sa[t.across], fa);
+    if (m.b_is_element) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) fb[e] = m.element;
+    } else if (Op::binary && b) {
+      gather(t.turn_b, lds[Op::binary ? 1 : 0], b, m.sb[inner], m.sb[t.across], fb);
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e) fb[e] = 0.0f;
+    }
+    const Pack<TO, V> po = apply_pack<TO, Op, V>(fa, fb);
+    SO* dst = o + (long long)row * m.so[t.across] + col;
+    if (col + V <= ni) {
+      store_pack_anywhere<TO, V>(dst, po);
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e)
+        if (col + e < ni) dst[e] = po.v[e];
+    }
+  }
+}
+
+// Whether an operand is turned: its unit stride along another dimension than the innermost, and tiles that are mostly full.
+template <typename TI, typename TO, typename Op>
+bool plan_turn(const Map& m, TurnMap* t) {
+  const int inner = m.rank - 1;
+  if (m.fill || m.rank < 2 || m.so[inner] != 1 || m.shape[inner] < 16) return false;
+  auto unit_dim = [&](const void* p, const long long* s) {
+    if (!p || s[inner] == 0 || s[inner] == 1) return -1;
+    for (int d = 0; d < inner; ++d)
+      if (s[d] == 1 && m.shape[d] >= 16) return d;
+    return -1;
+  };
+  const int da = unit_dim(m.a, m.sa), db = Op::binary && !m.b_is_element ? unit_dim(m.b, m.sb) : -1;
+  if (da < 0 && db < 0) return false;
+  t->m = m;
+  t->across = da >= 0 ? da : db;
+  t->turn_a = da >= 0;
+  t->turn_b = db >= 0 && db == t->across;
+  t->tiles_inner = (m.shape[inner] + TURN - 1) / TURN;
+  t->tiles_across = (m.shape[t->across] + TURN - 1) / TURN;
+  return true;
+}
+
+template <typename TI, typename TO, typename Op, int V, bool RAGGED>
 hipError_t launch_v(const Map& m, hipStream_t stream) {
   unsigned long long vector_bytes = V * sizeof(typename TO::storage);
   if (!m.fill) vector_bytes += V * sizeof(typename TI::storage) * (m.b && !m.b_reused ? 2 : 1);
@@ -197,56 +356,78 @@ hipError_t launch_v(const Map& m, hipStream_t stream) {
   if (blocks == 0) return hipSuccess;
   if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
   if (per_lane == 1) {
-    hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, false, 1>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
+    hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, false, 1, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
     return launch_status(stream);
   }
   // (a run-time choice between the two kinds of load inside one kernel cost every operation 14 %)
   if constexpr (V > 1 && Op::binary) {
     if (m.b_reused) {
-      hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, true>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
+      hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, true, kVectorsPerLane, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
       return launch_status(stream);
     }
   }
-  hipLaunchKernelGGL((map_kernel<TI, TO, Op, V>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
+  hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, false, kVectorsPerLane, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
   return launch_status(stream);
 }
 
 // Vector width the layout allows: the innermost dimension must be contiguous in the result and
-// contiguous or broadcast in the inputs, its extent and every other stride of a vector-accessed
-// operand a multiple of V, and the base pointers aligned to the vector.
+// contiguous or broadcast in the inputs.  *ragged: its extent, some other stride or a base pointer is no multiple of the vector.
 template <typename TI, typename TO>
-int vector_width(const Map& m) {
+int vector_width(const Map& m, bool* ragged) {
   constexpr int V = 16 / (sizeof(typename TI::storage) > sizeof(typename TO::storage) ? sizeof(typename TI::storage)
                                                                                       : sizeof(typename TO::storage));
+  *ragged = false;
   const int inner = m.rank - 1;
-  if (m.so[inner] != 1 || m.shape[inner] % V) return 1;
+  if (m.so[inner] != 1) return 1;
+  if (m.shape[inner] % V) *ragged = true;
   auto operand_ok = [&](const void* p, const long long* s, size_t esize, bool is_out) {
     if (!p) return true;
     if (s[inner] != 1 && (is_out || s[inner] != 0)) return false;
     if (s[inner] == 1) {
-      if ((uintptr_t)p % (V * esize)) return false;
+      if ((uintptr_t)p % (V * esize)) *ragged = true;
       for (int d = 0; d < inner; ++d)
-        if (s[d] % V) return false;
+        if (s[d] % V) *ragged = true;
     }
     return true;
   };
   if (!operand_ok(m.o, m.so, sizeof(typename TO::storage), true)) return 1;
   if (!m.fill && !operand_ok(m.a, m.sa, sizeof(typename TI::storage), false)) return 1;
   if (!m.fill && !m.b_is_element && !operand_ok(m.b, m.sb, sizeof(typename TI::storage), false)) return 1;
-  return V;
+  // rows of hardly more than a vector leave most of a ragged row to the element loop
+  return *ragged && m.shape[inner] < 2 * V ? 1 : V;
+}
+
+// The map with its innermost extent counted in vectors.
+inline void count_vectors(Map* m, int v) {
+  const int inner = m->rank - 1;
+  const uint32_t vectors = (m->shape[inner] + v - 1) / v;
+  m->inner_elements = m->shape[inner];
+  m->total = m->total / m->shape[inner] * vectors;
+  m->shape[inner] = vectors;
 }
 
 template <typename TI, typename TO, typename Op>
 hipError_t launch_t(Map m, hipStream_t stream) {
   constexpr int V = 16 / (sizeof(typename TI::storage) > sizeof(typename TO::storage) ? sizeof(typename TI::storage)
                                                                                       : sizeof(typename TO::storage));
-  if (vector_width<TI, TO>(m) == V) {
-    const int inner = m.rank - 1;
-    m.shape[inner] /= V;
-    m.total /= V;
-    return launch_v<TI, TO, Op, V>(m, stream);
+  bool ragged;
+  if (vector_width<TI, TO>(m, &ragged) == V) {
+    count_vectors(&m, V);
+    return ragged ? launch_v<TI, TO, Op, V, true>(m, stream) : launch_v<TI, TO, Op, V, false>(m, stream);
   }
-  return launch_v<TI, TO, Op, 1>(m, stream);
+  TurnMap t;
+  if (plan_turn<TI, TO, Op>(m, &t)) {
+    const int inner = m.rank - 1;
+    const unsigned long long others = m.total / m.shape[inner] / m.shape[t.across];
+    const unsigned long long blocks = others * t.tiles_inner * t.tiles_across;
+    if (blocks <= 0x7fffffffull) {
+      const unsigned long long bytes = m.total * (sizeof(typename TO::storage) + sizeof(typename TI::storage) * (m.b && !m.b_reused ? 2 : 1));
+      if (bytes > kOneVectorBytes) hipLaunchKernelGGL((turn_kernel<TI, TO, Op, true>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+      else hipLaunchKernelGGL((turn_kernel<TI, TO, Op, false>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+      return launch_status(stream);
+    }
+  }
+  return launch_v<TI, TO, Op, 1, false>(m, stream);
 }
 
 template <typename Op>
@@ -300,11 +481,10 @@ hipError_t launch_copy_pair(Map m0, Map m1, hipStream_t stream) {
     hipLaunchKernelGGL((copy_pair_kernel<T, W>), dim3((unsigned)(b0 + b1)), dim3(256), 0, stream, m0, m1, (uint32_t)b0);
     return launch_status(stream);
   };
-  if (vector_width<T, T>(m0) == V && vector_width<T, T>(m1) == V) {
-    for (Map* m : {&m0, &m1}) {
-      m->shape[m->rank - 1] /= V;
-      m->total /= V;
-    }
+  bool r0, r1;
+  if (vector_width<T, T>(m0, &r0) == V && !r0 && vector_width<T, T>(m1, &r1) == V && !r1) {
+    count_vectors(&m0, V);
+    count_vectors(&m1, V);
     return go(std::integral_constant<int, V>{});
   }
   return go(std::integral_constant<int, 1>{});
@@ -424,6 +604,14 @@ srtStatus build_map(const srtTensorDescriptor* ad, const srtTensorDescriptor* bd
   }
   if (total == 0) { *empty = true; return srtSuccess; }
   if (n == 0) { shape[0] = 1; sa[0] = sb[0] = 0; so[0] = 1; n = 1; }
+  // the result's storage order: its smallest stride innermost (a column-major result is a row-major walk of its storage)
+  for (int d = 1; d < n; ++d)
+    for (int e = d; e > 0 && so[e - 1] < so[e]; --e) {
+      std::swap(shape[e - 1], shape[e]);
+      std::swap(sa[e - 1], sa[e]);
+      std::swap(sb[e - 1], sb[e]);
+      std::swap(so[e - 1], so[e]);
+    }
   // merge d into d + 1 where stride[d] == shape[d + 1] * stride[d + 1] for every operand
   int w = 0;
   for (int d = 1; d < n; ++d) {

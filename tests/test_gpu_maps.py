@@ -1,0 +1,77 @@
+"""Element-wise maps whose operands walk memory across the result's rows (turned through LDS in 64 x 64 tiles) and maps whose rows are
+no whole number of aligned vectors: exact against numpy on small integers, at the edges of the tile and of the vector."""
+import numpy as np
+import pytest
+
+import swiftrt_amd as srt
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+DTS = [H.F32, H.F16, H.BF16]
+
+
+def ints(g, shape, dt):
+    return H.encode(g.integers(-8, 9, shape), dt)
+
+
+def check(got, want, dt):
+    assert np.array_equal(H.to64(got.array()), H.to64(H.encode(want, dt)))
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("m,n", [(16, 16), (15, 200), (63, 65), (64, 128), (129, 17), (300, 1001)])
+def test_turned_operands(dt, m, n):
+    g = H.rng(m * n)
+    at, bt, a, b = ints(g, (n, m), dt), ints(g, (n, m), dt), ints(g, (m, n), dt), ints(g, (n,), dt)
+    A, B = H.to64(at).T, H.to64(bt).T
+    T = srt.Tensor
+    out = lambda: srt.Tensor(shape=[m, n], dtype=at.dtype)   # noqa: E731
+    q = srt.current_queue()
+    for lhs, rhs, want in [(T(at).t, T(a), A + H.to64(a)), (T(a), T(bt).t, H.to64(a) + B), (T(at).t, T(bt).t, A + B),
+                           (T(at).t, T.repeating(T(b), [m, n]), A + H.to64(b)), (T(at).t, 3.0, A + 3)]:
+        o = out()
+        q.add(lhs, rhs, o)
+        check(o, want, dt)
+    o = out()
+    q.neg(T(at).t, o)
+    check(o, -A, dt)
+    other = H.BF16 if dt == H.F32 else H.F32
+    o = srt.Tensor(shape=[m, n], dtype=H.NP_STORAGE[other])
+    q.copy(T(at).t, o)                                       # with conversion
+    check(o, A, other)
+
+
+@pytest.mark.parametrize("dt", DTS)
+def test_turned_inside_a_batch_and_a_frame(dt):
+    g = H.rng(3)
+    x = ints(g, (3, 70, 90), dt)
+    frame = srt.Tensor(H.encode(np.full((3, 100, 80), 5), dt))
+    view = frame[:, 4:94, 3:73]
+    srt.current_queue().copy(srt.Tensor(x).t, view)
+    want = np.full((3, 100, 80), 5.0)
+    want[:, 4:94, 3:73] = np.swapaxes(H.to64(x), 1, 2)
+    check(frame, want, dt)
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("n", [7, 15, 16, 17, 33, 1001])
+def test_ragged_rows(dt, n):
+    g = H.rng(n)
+    a, b = ints(g, (37, n), dt), ints(g, (n,), dt)
+    frame = srt.Tensor(H.encode(np.full((37, n + 5), 5), dt))
+    srt.current_queue().mul(srt.Tensor(a), srt.Tensor.repeating(srt.Tensor(b), [37, n]), frame[:, 3:3 + n])
+    want = np.full((37, n + 5), 5.0)
+    want[:, 3:3 + n] = H.to64(a) * H.to64(b)
+    check(frame, want, dt)
+    check(srt.Tensor(a) + srt.Tensor(a), 2 * H.to64(a), dt)
+    flat = srt.Tensor(np.ascontiguousarray(a.reshape(-1)[1:]))
+    check(flat + flat, 2 * H.to64(a).reshape(-1)[1:], dt)
+
+
+@pytest.mark.parametrize("dt", DTS)
+def test_column_major_results_are_walked_in_their_storage_order(dt):
+    g = H.rng(4)
+    a, b = ints(g, (65, 130), dt), ints(g, (65, 130), dt)
+    col = lambda x: srt.Tensor(x, order=srt.Order.col)       # noqa: E731
+    check(col(a) + col(b), H.to64(a) + H.to64(b), dt)
+    check(col(a) + srt.Tensor(b), H.to64(a) + H.to64(b), dt)   # row-major into column-major
