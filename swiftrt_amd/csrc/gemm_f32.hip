@@ -8,9 +8,9 @@
 //                       16-byte global loads, 8-byte operand reads (4096^3: ~120 TFLOP/s)
 //   128 x 128 / 64 x 64 element-wise loads with the caller's strides (views, column-major, odd
 //                       pitches all land here); the small tile when the large one would leave CUs idle
-//   32 x 32 split-K     launch-latency-sized problems (512^3 = 64 tiles of 64 x 64): the 4 waves split
-//                       K between them and sum through LDS; row-major operands take a variant that
-//                       keeps a wave's whole k range in flight
+//   32 x 32 split-K     launch-latency-sized problems (512^3 = 64 tiles of 64 x 64): the waves split
+//                       K between them and sum through LDS; operands with a unit stride take a variant
+//                       of 8 waves with 16-byte loads
 #include "gemm_common.h"
 #include "gemm_f32_ring.h"
 
@@ -378,52 +378,114 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_splitk_kernel(GemmProblem p
     if (mb + i < p.M) C[(long long)(mb + i) * p.scm + (long long)n * p.scn] = out[i];
 }
 
-// ---- 32 x 32 tiles, the 4 waves split K; row-major operands, whole k range in flight ------------
-// The variant above keeps one 16-deep slab in flight per wave, so a launch-latency-sized problem
-// (512^3: 8 slabs per wave) pays one memory round trip per slab.  When both operands are row-major
-// with 16-byte aligned rows (A k-contiguous, B n-contiguous) a wave instead requests up to
-// SV_SLABS slabs of its k range at once with 16-byte loads (4 per slab and lane), and multiplies
-// them as they arrive; wave w owns a contiguous quarter of K.
-//   A slab  32 rows x 16 k: lane f (two per lane) loads 4 k of row f / 4; transposed into LDS
+// ---- 32 x 32 tiles, 8 waves split K; operands with a unit stride -------------------------------------------
+// The variant above walks k element by element, one slab in flight per wave.  When both operands
+// have a unit stride, along k or along m / n, a wave requests SV_SLABS slabs of its k range at once
+// with 16-byte loads (4 per slab and lane) and multiplies them as they arrive; wave w owns a
+// contiguous eighth of K.  Rows may start anywhere and end anywhere: the loads need element
+// alignment only, and a piece that would cross a row's end is loaded from the row's last four
+// elements and shifted into place when it is stored to LDS.
+//   bound   latency: a round trip to memory and the matrix time of a unit's tiles (512^3: one tile per unit, 1.7 us of
+//           MFMAs at their peak).  Two waves per SIMD, so that one multiplies while the other waits or stores to LDS.
+//   waves   us with 4 waves x 8 slabs / 8 x 8 / 8 x 4 / 8 x 2 / 16 x 4: 512^3 x . W 7.2 / 7.0 / 6.3 / 6.1 / 6.6, 256 x 1000 x 784
+//           10.8 / 9.5 / 8.7 / 8.5 / 8.2, 64 x 2048 x 1024 11.4 / 9.4 / 9.0 / 8.9 / 8.7, 4 x 256^3 5.3 / 5.4 / 4.7 / 4.2 / 5.5, 1001^3
+//           35.2 / 40.3 / 30.2 / 30.7 / 36.7: more slabs than a wave has are loads for nothing, and registers that
+//           keep a second workgroup off the unit
+//   before  (4 waves x 8 slabs for aligned row-major operands, by elements otherwise) 512^3 x . W 6.7, x . W^T 11.5, x^T . W 11.5;
+//           256 x 1000 x 784 10.0, 16.7, 16.7; 64 x 2048 x 1024 10.7, 19.6, 19.7; 1001^3 41; 33 x 4093 x 2047 35.
+//           Now 6.1, 5.4, 6.4; 8.5, 7.7, 9.4; 8.9, 7.9, 10.1; 31, 30, 35; 17.1, 14.5, 18.7.
+//   k-contiguous slab   32 rows x 16 k: lane f (two per lane) loads 4 k of row f / 4; transposed into LDS
 //           k-major [k][m], pitch 36: the four ds_write_b32 of a lane pair are conflict-free.
-//   B slab  16 k x 32 n: lane f loads 4 n of k row f / 8; LDS [k][n], pitch 32: even k rows sit
+//   mn-contiguous slab  16 k x 32 mn: lane f loads 4 mn of k row f / 8; LDS [k][mn], pitch 32: even k rows sit
 //           in banks 0-31 and odd ones in 32-63, which is exactly the split of the MFMA operand
 //           read (lanes 0-31 take k = 2 kk, lanes 32-63 k = 2 kk + 1).
-constexpr int SV_SLABS = 8;
+constexpr int SV_WAVES = 8, SV_SLABS = 2;
 
-__global__ __launch_bounds__(256) void gemm_f32_mfma_splitk_vec_kernel(GemmProblem p) {
-  __shared__ float As[4][2][FK][36];
-  __shared__ __attribute__((aligned(16))) float Bs[4][2][FK][32];
-  __shared__ float red[4][16][64];
+typedef f32x4v_t f32x4u_t __attribute__((aligned(4)));
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// v's elements s .. 3 moved to the front, zeros behind them (s >= 4: all zeros)
+__device__ __forceinline__ f32x4v_t shifted(f32x4v_t v, int s) {
+  if (s & 1) v = f32x4v_t{v[1], v[2], v[3], 0.0f};
+  if (s & 2) v = f32x4v_t{v[2], v[3], 0.0f, 0.0f};
+  if (s >= 4) v = f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f};
+  return v;
+}
+
+template <bool KC>
+struct SlabStage {
+  static constexpr int PITCH = KC ? 36 : 32;
+  const float* row[2];   // KC: the row's start; MN: the piece's place in k row 0
+  int k[2], mn[2];       // the piece's place in a slab
+  int over[2];           // MN: elements the piece was moved back to end inside its row
+  long long ld;
+  int K, last_k;         // last_k: the largest k (MN) or piece start (KC) this wave may read
+  bool edge;             // MN, workgroup-uniform: some piece crosses the rows' end
+
+  // extent: M or N (MN: at least 4); k_end: where this wave's k range ends (KC: K at least 4)
+  __device__ __forceinline__ void init(const float* base, int lane, int mn0, int extent, long long stride, int K_, int k_end) {
+    ld = stride;
+    K = K_;
+    last_k = min(k_end, K_) - (KC ? 4 : 1);
+    edge = !KC && mn0 + 32 > extent;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int f = lane + 64 * i;
+      if (KC) {
+        mn[i] = f >> 2; k[i] = (f & 3) * 4; over[i] = 0;
+        // (a row past the extent repeats the last one: it feeds results that are not stored)
+        row[i] = base + (long long)min(mn0 + mn[i], extent - 1) * stride;
+      } else {
+        k[i] = f >> 3; mn[i] = (f & 7) * 4;
+        const int at = min(mn0 + mn[i], extent - 4);
+        over[i] = mn0 + mn[i] - at;
+        row[i] = base + at;
+      }
+    }
+  }
+  __device__ __forceinline__ f32x4v_t load(int i, int k0) const {
+    const int at = min(k0 + k[i], last_k);
+    return *reinterpret_cast<const f32x4u_t*>(row[i] + (KC ? (long long)at : (long long)at * ld));
+  }
+  __device__ __forceinline__ void store(int i, int k0, f32x4v_t v, float (*dst)[PITCH]) const {
+    if (KC) {
+      if (k0 + FK > K) v = shifted(v, max(0, k0 + k[i] - (K - 4)));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[k[i] + e][mn[i]] = v[e];
+    } else {
+      if (edge) v = shifted(v, over[i]);
+      if (k0 + FK > K && k0 + k[i] >= K) v = f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f};
+      *reinterpret_cast<f32x4v_t*>(&dst[k[i]][mn[i]]) = v;
+    }
+  }
+};
+
+template <bool A_KC, bool B_KC>
+__global__ __launch_bounds__(64 * SV_WAVES) void gemm_f32_mfma_splitk_vec_kernel(GemmProblem p) {
+  using StageA = SlabStage<A_KC>;
+  using StageB = SlabStage<B_KC>;
+  union Lds {
+    struct {
+      float a[SV_WAVES][FK][StageA::PITCH], b[SV_WAVES][FK][StageB::PITCH];
+    } slab;
+    float red[SV_WAVES][16][64];   // the waves' partial tiles, once every wave is done with its slabs
+  };
+  __shared__ __attribute__((aligned(16))) Lds lds;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, kh = lane >> 5;
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32, bz = blockIdx.z;
-  const float* A = (const float*)p.A + (long long)bz * p.sab;
-  const float* B = (const float*)p.B + (long long)bz * p.sbb;
   float* C = (float*)p.C + (long long)bz * p.scb;
 
-  // this wave's slabs: a contiguous quarter of the k range
+  // this wave's slabs: a contiguous part of the k range
   const int slabs = (p.K + FK - 1) / FK;
-  const int per_wave = (slabs + 3) / 4;
+  const int per_wave = (slabs + SV_WAVES - 1) / SV_WAVES;
   const int first = wave * per_wave;
   const int last = min(slabs, first + per_wave);   // exclusive
 
-  // lane -> 16-byte piece of a slab (two pieces per operand)
-  int am[2], ak[2], bk[2], bn[2];
-  const float* ap[2];
-  const float* bp[2];
-  bool a_row_ok[2], b_col_ok[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int f = lane + 64 * i;
-    am[i] = f >> 2; ak[i] = (f & 3) * 4;
-    bk[i] = f >> 3; bn[i] = (f & 7) * 4;
-    a_row_ok[i] = m0 + am[i] < p.M;
-    b_col_ok[i] = n0 + bn[i] < p.N;   // N is a multiple of 4: the piece is whole
-    ap[i] = A + (long long)(m0 + am[i]) * p.sam + ak[i];
-    bp[i] = B + (long long)bk[i] * p.sbk + n0 + bn[i];
-  }
+  StageA sa;
+  StageB sb;
+  sa.init((const float*)p.A + (long long)bz * p.sab, lane, m0, p.M, A_KC ? p.sam : p.sak, p.K, last * FK);
+  sb.init((const float*)p.B + (long long)bz * p.sbb, lane, n0, p.N, B_KC ? p.sbn : p.sbk, p.K, last * FK);
 
   f32x16_t acc;
 #pragma unroll
@@ -431,56 +493,58 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_splitk_vec_kernel(GemmProbl
 
   for (int s0 = first; s0 < last; s0 += SV_SLABS) {
     f32x4v_t ra[SV_SLABS][2], rb[SV_SLABS][2];
+    // (slabs past the wave's range repeat its last piece: no branch between the loads)
 #pragma unroll
     for (int s = 0; s < SV_SLABS; ++s) {
-      const int k0 = (s0 + s) * FK;
-      const bool live = s0 + s < last;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const f32x4v_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        // K is a multiple of 4: a piece lies wholly inside or outside the k range
-        ra[s][i] = (live && a_row_ok[i] && k0 + ak[i] < p.K) ? *reinterpret_cast<const f32x4v_t*>(ap[i] + k0) : zero;
-        rb[s][i] = (live && b_col_ok[i] && k0 + bk[i] < p.K)
-                       ? *reinterpret_cast<const f32x4v_t*>(bp[i] + (long long)k0 * p.sbk) : zero;
+        ra[s][i] = sa.load(i, (s0 + s) * FK);
+        rb[s][i] = sb.load(i, (s0 + s) * FK);
       }
     }
 #pragma unroll
     for (int s = 0; s < SV_SLABS; ++s) {
       if (s0 + s >= last) break;
-      const int buf = s & 1;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) As[wave][buf][ak[i] + e][am[i]] = ra[s][i][e];
-        *reinterpret_cast<f32x4v_t*>(&Bs[wave][buf][bk[i]][bn[i]]) = rb[s][i];
+        sa.store(i, (s0 + s) * FK, ra[s][i], lds.slab.a[wave]);
+        sb.store(i, (s0 + s) * FK, rb[s][i], lds.slab.b[wave]);
       }
       // the slab is written and read by this wave only: LDS operations of one wave execute in
-      // order, so a wave-level fence (for the compiler) is all that is needed; the other buffer
-      // may still be read by the MFMAs issued for the previous slab
+      // order (the next slab's writes behind this one's reads, too), so a wave-level fence (for
+      // the compiler) is all that is needed
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int kk = 0; kk < FK / 2; ++kk)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[wave][buf][2 * kk + kh][r], Bs[wave][buf][2 * kk + kh][r], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(lds.slab.a[wave][2 * kk + kh][r], lds.slab.b[wave][2 * kk + kh][r], acc, 0, 0, 0);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     }
   }
 
+  __syncthreads();
 #pragma unroll
-  for (int v = 0; v < 16; ++v) red[wave][v][lane] = acc[v];
+  for (int v = 0; v < 16; ++v) lds.red[wave][v][lane] = acc[v];
   __syncthreads();
 
-  // wave w finishes accumulator registers 4 w .. 4 w + 3: rows 8 w + 4 kh + i, column r
+  // wave w finishes accumulator registers R w .. R w + R - 1; register v is row 8 (v / 4) + 4 kh + v % 4, column r
+  constexpr int R = 16 / SV_WAVES;
   Epilogue<F32> ep(p);
   const int n = n0 + r;
   if (n >= p.N) return;
-  const int mb = m0 + 8 * wave + 4 * kh;
-  float out[4];
+  const int mb = m0 + 8 * (R * wave / 4) + 4 * kh + (R * wave) % 4;
+  float out[R];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int v = 4 * wave + i;
-    out[i] = (red[0][v][lane] + red[1][v][lane]) + (red[2][v][lane] + red[3][v][lane]);
+  for (int i = 0; i < R; ++i) {
+    float part[SV_WAVES];
+#pragma unroll
+    for (int w = 0; w < SV_WAVES; ++w) part[w] = lds.red[w][R * wave + i][lane];
+#pragma unroll
+    for (int step = 1; step < SV_WAVES; step *= 2)
+#pragma unroll
+      for (int w = 0; w < SV_WAVES; w += 2 * step) part[w] += part[w + step];
+    out[i] = part[0];
   }
   ep.finish_run(out, [&](int i, int* m, int* nn) {
     *m = mb + i;
@@ -488,17 +552,25 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_splitk_vec_kernel(GemmProbl
     return *m < p.M;
   });
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < R; ++i)
     if (mb + i < p.M) C[(long long)(mb + i) * p.scm + (long long)n * p.scn] = out[i];
 }
 
-// Preconditions of the vector variant: both operands row-major with 16-byte aligned rows.
+// Preconditions of the vector variant: both operands have a unit stride, with at least one whole vector along it.
 bool splitk_vec_fits(const GemmProblem& p) {
-  if (p.sak != 1 || p.sbn != 1) return false;
-  if ((p.K % 4) != 0 || (p.N % 4) != 0) return false;
-  if ((p.sam % 4) != 0 || (p.sbk % 4) != 0 || (p.sab % 4) != 0 || (p.sbb % 4) != 0) return false;
-  if ((reinterpret_cast<uintptr_t>(p.A) & 15u) != 0 || (reinterpret_cast<uintptr_t>(p.B) & 15u) != 0) return false;
+  if (p.sak == 1 ? p.K < 4 : (p.sam != 1 || p.M < 4)) return false;
+  if (p.sbn == 1 ? p.N < 4 : (p.sbk != 1 || p.K < 4)) return false;
   return true;
+}
+
+hipError_t launch_f32_splitk_vec(const GemmProblem& p, hipStream_t stream) {
+  const dim3 grid((p.N + 31) / 32, (p.M + 31) / 32, p.batch), block(64 * SV_WAVES);
+  const bool a_kc = p.sak == 1, b_kc = p.sbn != 1;
+  if (a_kc && b_kc) hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<true, true>), grid, block, 0, stream, p);
+  else if (a_kc) hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<true, false>), grid, block, 0, stream, p);
+  else if (b_kc) hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<false, true>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<false, false>), grid, block, 0, stream, p);
+  return launch_status(stream);
 }
 
 // ---- split-K over the 128 x 128 vector kernel -----------------------------------------------------
@@ -673,9 +745,9 @@ bool f32_mfma_supported(const GemmProblem& p) {
 //   64 x 128 tiles    R x 30.5 per 1024 k + 4      (512 x 4096 x 4096 125 / 126, 256 x 8192 x 8192 255 / 248, 1536^3 95 / 96)
 //   64 x 64 tiles     R x 16.5 per 1024 k + 4      (1024^3 20.3 / 20.5, 64 x 14336 x 4096 71 / 70, 1536^3 77 / 78, 768^3 15.9 / 16.4)
 //   k in parts on 128 x 128 tiles: f32_tile_parts' estimate
-//   32 x 32 tiles, k split over the waves: every workgroup reads 64 x K x 4 bytes, at 32 bytes/ns alone on its unit and 31
-//   per unit when they share (both operands row-major: 16-byte loads), 16 and 21.5 otherwise, + 3
-//                      (512^3 6.7 / 7.1, 1024^3 31 / 37 and 42 / 52, 32 x 14336 x 4096 59 / 62 and 90 / 88, 128 x 512 x 4096 35 / 36 and 68 / 69)
+//   32 x 32 tiles, k split over the waves: every workgroup reads 64 x K x 4 bytes, at 42 / 50 / 38 / 43 bytes/ns (x . W /
+//   x . W^T / x^T . W / x^T . W^T) alone on its unit and 36 / 37 / 33 / 38 per unit when they share, + 3
+//                      (512^3 6.1 / 6.1 and 5.6 / 5.4, 512 x 512 x 2048 15.5 / 16.5 and 13.5 / 14.6, 1001^3 31 / 31 and 31 / 30)
 // Smaller tiles cost more per flop (more operand bytes per MFMA through L2 and LDS) and win by filling the device:
 // 1024^3 20 us on 256 tiles of 64 x 64 against 31-42 on 32 x 32 and 62 on 64 tiles of 128 x 128.
 // Returns 0: 128 x 128, 1: 64 x 128, 2: 64 x 64, 3: parts, 4: the 32 x 32 kernel.
@@ -704,8 +776,9 @@ int f32_ring_choice(const GemmProblem& p) {
   if (f32_mfma_supported(p)) {
     const double tiles32 = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch;
     const double bytes = 64.0 * (double)p.K * 4.0;   // per workgroup
-    const bool vec = splitk_vec_fits(p);
-    const double alone = bytes / (vec ? 32.0e3 : 16.0e3), shared = tiles32 / cus * bytes / (vec ? 31.0e3 : 21.5e3);
+    const int layout = (p.sak == 1 ? 0 : 2) + (p.sbn == 1 ? 0 : 1);
+    constexpr double kAlone[4] = {42.0e3, 50.0e3, 38.0e3, 43.0e3}, kShared[4] = {36.0e3, 37.0e3, 33.0e3, 38.0e3};
+    const double alone = bytes / kAlone[layout], shared = tiles32 / cus * bytes / kShared[layout];
     offer(4, (alone > shared ? alone : shared) + 3.0);
   }
   return choice;
@@ -722,9 +795,9 @@ bool f32_mfma_prefers_splitk(const GemmProblem& p) {
 
 hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_t stream) {
   if (splitk) {
+    if (splitk_vec_fits(p)) return launch_f32_splitk_vec(p, stream);
     dim3 grid((p.N + 31) / 32, (p.M + 31) / 32, p.batch);
-    if (splitk_vec_fits(p)) hipLaunchKernelGGL(gemm_f32_mfma_splitk_vec_kernel, grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(gemm_f32_mfma_splitk_kernel, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(gemm_f32_mfma_splitk_kernel, grid, dim3(256), 0, stream, p);
   } else {
     // the 128 x 128 tile once it gives every CU a workgroup, the 64 x 64 tile below that
     const long long tiles128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
