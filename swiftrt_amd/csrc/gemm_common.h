@@ -315,6 +315,10 @@ const char* mfma_name(int config);
 hipError_t launch_mfma(const GemmProblem& p, int config, hipStream_t stream);
 // Operands copied into aligned, zero-padded workspace first (gemm_pack.hip), and the plan the heuristic picks for the copies.
 bool pack_preferred(const GemmProblem& p);
+double packed_us(const GemmProblem& p);   // estimate of an fp32 problem's time that way, copies included (0: it cannot)
+double f32_ring_us(const GemmProblem& p);   // and of the ring kernel's plans alone
+enum class F32Any { kTile, kSplitK, kParts, kPacked };
+F32Any f32_any_choice(const GemmProblem& p, double packed_us);   // for a problem the ring kernel does not read
 hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErrorOutOfMemory: no workspace, nothing was launched
 hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream);
 // Split-K over the 256 x 256 kernel: number of k parts (0: the problem does not qualify) and launch.
@@ -329,7 +333,6 @@ bool skinny_preferred(const GemmProblem& p);   // the heuristic's choice among t
 hipError_t launch_skinny(const GemmProblem& p, hipStream_t stream);
 
 bool f32_mfma_supported(const GemmProblem& p);
-hipError_t launch_f32_mfma(const GemmProblem& p, hipStream_t stream);
 bool f32_mfma_prefers_splitk(const GemmProblem& p);
 hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_t stream);
 bool f32_ring_fits(const GemmProblem& p);

@@ -278,7 +278,7 @@ bool mfma128_vec_fits(const GemmProblem& p) {
   if (!(a_kf || a_mf) || !(b_kf || b_nf)) return false;
   const long long lda = a_kf ? p.sam : p.sak, ldb = b_kf ? p.sbn : p.sbk;
   if ((lda % 4) != 0 || (ldb % 4) != 0 || (p.sab % 4) != 0 || (p.sbb % 4) != 0) return false;
-  if ((a_kf ? p.K : p.M) % 4 != 0 || (b_kf ? p.K : p.N) % 4 != 0) return false;
+  if (!p.row_padding && ((a_kf ? p.K : p.M) % 4 != 0 || (b_kf ? p.K : p.N) % 4 != 0)) return false;
   if ((reinterpret_cast<uintptr_t>(p.A) & 15u) != 0 || (reinterpret_cast<uintptr_t>(p.B) & 15u) != 0) return false;
   return true;
 }
@@ -739,6 +739,17 @@ bool f32_mfma_supported(const GemmProblem& p) {
   return true;
 }
 
+// The 32 x 32 kernel's time in microseconds (f32_ring_choice below has the figures).
+static double splitk_us(const GemmProblem& p) {
+  const double cus = compute_units();
+  const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch;
+  const double bytes = 64.0 * (double)p.K * 4.0;   // per workgroup
+  constexpr double kAlone[5] = {42.0e3, 50.0e3, 38.0e3, 43.0e3, 16.0e3}, kShared[5] = {36.0e3, 37.0e3, 33.0e3, 38.0e3, 21.5e3};
+  const int layout = !splitk_vec_fits(p) ? 4 : (p.sak == 1 ? 0 : 2) + (p.sbn == 1 ? 0 : 1);
+  const double alone = bytes / kAlone[layout], shared = tiles / cus * bytes / kShared[layout];
+  return (alone > shared ? alone : shared) + 3.0;
+}
+
 // Which fp32 kernel a problem the ring kernel reads should run on, by estimates of the time in microseconds (each
 // fitted to measurements on one device, 256 units; R(t) = rounds of t tiles over the units):
 //   128 x 128 tiles   R x 59 per 1024 k + 4        (2048^3 124 / 122, 1024 x 4096 x 4096 239 / 240, 1536^3 92 / 92)
@@ -751,18 +762,18 @@ bool f32_mfma_supported(const GemmProblem& p) {
 // Smaller tiles cost more per flop (more operand bytes per MFMA through L2 and LDS) and win by filling the device:
 // 1024^3 20 us on 256 tiles of 64 x 64 against 31-42 on 32 x 32 and 62 on 64 tiles of 128 x 128.
 // Returns 0: 128 x 128, 1: 64 x 128, 2: 64 x 64, 3: parts, 4: the 32 x 32 kernel.
-int f32_ring_choice(const GemmProblem& p) {
+static int ring_choice(const GemmProblem& p, double* us) {
   const int cus = compute_units();
   auto rounds = [&](int tm, int tn) {
     const long long t = (long long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn) * p.batch;
     return (double)((t + cus - 1) / cus);
   };
   const double k = (double)p.K / 1024.0;
-  double best = rounds(128, 128) * 59.0 * k + 4.0;
+  *us = rounds(128, 128) * 59.0 * k + 4.0;
   int choice = 0;
-  auto offer = [&](int c, double us) {
-    if (us < best) {
-      best = us;
+  auto offer = [&](int c, double t) {
+    if (t < *us) {
+      *us = t;
       choice = c;
     }
   };
@@ -773,17 +784,19 @@ int f32_ring_choice(const GemmProblem& p) {
     offer(3, (double)((tiles * s + cus - 1) / cus) * 59.0 * (double)(p.K / s) / 1024.0 + 4.0 +
                  (double)s * (double)p.M * (double)p.N * 8.0 / 6.0e6 + 5.0);
   }
-  if (f32_mfma_supported(p)) {
-    const double tiles32 = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch;
-    const double bytes = 64.0 * (double)p.K * 4.0;   // per workgroup
-    const int layout = (p.sak == 1 ? 0 : 2) + (p.sbn == 1 ? 0 : 1);
-    constexpr double kAlone[4] = {42.0e3, 50.0e3, 38.0e3, 43.0e3}, kShared[4] = {36.0e3, 37.0e3, 33.0e3, 38.0e3};
-    const double alone = bytes / kAlone[layout], shared = tiles32 / cus * bytes / kShared[layout];
-    offer(4, (alone > shared ? alone : shared) + 3.0);
-  }
+  if (f32_mfma_supported(p)) offer(4, splitk_us(p));
   return choice;
 }
 
+int f32_ring_choice(const GemmProblem& p) {
+  double us;
+  return ring_choice(p, &us);
+}
+double f32_ring_us(const GemmProblem& p) {
+  double us;
+  (void)ring_choice(p, &us);
+  return us;
+}
 
 // The split-K variant pays when 64 x 64 tiles alone would leave most CUs idle.
 // With up to 64 rows it pays whatever the tile count: larger tiles would be mostly padding (32 x 14336 x 4096: 60 us
@@ -799,6 +812,11 @@ hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_
     dim3 grid((p.N + 31) / 32, (p.M + 31) / 32, p.batch);
     hipLaunchKernelGGL(gemm_f32_mfma_splitk_kernel, grid, dim3(256), 0, stream, p);
   } else {
+    if (pack_preferred(p)) {
+      const hipError_t e = launch_packed(p, stream);
+      if (e != hipErrorOutOfMemory) return e;
+      (void)hipGetLastError();   // no room for the copies (nothing was launched): the operands as they are
+    }
     // the 128 x 128 tile once it gives every CU a workgroup, the 64 x 64 tile below that
     const long long tiles128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
     if (tiles128 >= 256) {
@@ -815,8 +833,30 @@ hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_
   return launch_status(stream);
 }
 
-hipError_t launch_f32_mfma(const GemmProblem& p, hipStream_t stream) {
-  return launch_f32_mfma_variant(p, f32_mfma_prefers_splitk(p), stream);
+// Where a problem the ring kernel does not read, and that is too large for the rule above, runs, by estimates in
+// microseconds:
+//   as it is   64 x 64 tiles at 30.8 per 1024 k and tile of a unit; from 256 tiles of 128 x 128 on those at 92 (120 when a unit
+//              has one only), or at 78 (86) with 16-byte loads; + 4
+//   32 x 32    splitk_us and 0.45 per tile of a unit for its fill and store
+//   copied     (packed_us > 0, from gemm_pack.hip) the ring kernel's estimate, 5 for the extra launch and the wait between the
+//              two, the copies and the result's stores at their bandwidth
+// measured, x . W (as it is / 32 x 32 / copied): 1000 x 2000 x 1000 64 / 60 / 46, 1023 x 2047 x 2047 126 / 114 / 76, 2000^3 172 / 212 /
+// 135, 2001 x 3003 x 1501 268 / 326 / 155, 2001 x 2001 x 300 41 / 41 / 34, 300 x 10001 x 500 57 / 55 / 46, 4096 x 3000 x 1000 230 / 383 /
+// 197, 8 x 300 x 500 x 700 46 / 28 / 34, 16 x 511 x 511 x 63 x . W^T 14.7 / 17.0 / 22.2, 3000 x 3000 x 100 36.5 / 41.7 / 35.9.
+// (The rule above and the parts pass stay ahead of the copies: the ring kernel sums a tile's k in one chain, they in several,
+// and 1001^3 is off by 5.7e-7 against 2.1e-7 that way.)
+F32Any f32_any_choice(const GemmProblem& p, double packed_us) {
+  if (f32_mfma_prefers_splitk(p)) return F32Any::kSplitK;
+  if (f32_tile_parts(p) >= 2) return F32Any::kParts;
+  const double cus = compute_units();
+  auto tiles = [&](int s) { return (double)((p.M + s - 1) / s) * (double)((p.N + s - 1) / s) * (double)p.batch; };
+  const double t128 = __builtin_ceil(tiles(128) / cus), t64 = __builtin_ceil(tiles(64) / cus);
+  double per_k = 30.8 * t64;
+  if (tiles(128) >= 256) per_k = mfma128_vec_fits(p) ? (t128 > 1 ? 78.0 : 86.0) * t128 : (t128 > 1 ? 92.0 : 120.0) * t128;
+  const double as_is = per_k * (double)p.K / 1024.0 + 4.0;
+  const double split = splitk_us(p) + 0.45 * tiles(32) / cus;
+  if (packed_us > 0.0 && packed_us < as_is && packed_us < split) return F32Any::kPacked;
+  return split < as_is ? F32Any::kSplitK : F32Any::kTile;
 }
 
 }  // namespace srt

@@ -73,6 +73,7 @@ inline long long round_up(long long v, long long unit) { return (v + unit - 1) /
 // The k extent of the copies: whole 128-deep units where one round of 128 x 128 tiles holds the problem, else whole 64-deep
 // ones; short k loops (no such kernel) in whole 64-deep units too, which the register-staged kernels read.
 int pack_depth(const GemmProblem& p) {
+  if (p.dtype == srtReal32F) return p.K <= 128 ? 128 : (int)round_up(p.K, 64);   // gemm_f32_ring.h: whole 64-deep units, two at least
   const long long t128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
   const bool quarter = t128 <= compute_units() && p.K > 128;
   const long long k = round_up(p.K, quarter ? 128 : 64);
@@ -117,26 +118,34 @@ struct PackPlan {
   size_t bytes_a, bytes_b;
 };
 bool plan_pack(const GemmProblem& p, PackPlan* t) {
-  if (p.dtype != srtReal16BF && p.dtype != srtReal16F) return false;
+  if (p.dtype != srtReal16BF && p.dtype != srtReal16F && p.dtype != srtReal32F) return false;
   if (p.scn != 1 || p.scm < 0 || p.K < 1 || p.batch > 65535) return false;
   if (p.sam < 0 || p.sak < 0 || p.sab < 0 || p.sbk < 0 || p.sbn < 0 || p.sbb < 0) return false;
-  const int depth = pack_depth(p);
+  const int depth = pack_depth(p), es = p.dtype == srtReal32F ? 4 : 2;
   Operand a{p.A, p.sam, p.sak, p.sab}, b{p.B, p.sbn, p.sbk, p.sbb};
-  t->bytes_a = plan_operand(&a, p.M, p.K, depth, p.batch, 2, &t->a);
-  t->bytes_b = plan_operand(&b, p.N, p.K, depth, p.batch, 2, &t->b);
+  t->bytes_a = plan_operand(&a, p.M, p.K, depth, p.batch, es, &t->a);
+  t->bytes_b = plan_operand(&b, p.N, p.K, depth, p.batch, es, &t->b);
   if (t->bytes_a == ~(size_t)0 || t->bytes_b == ~(size_t)0) return false;
   t->q = p;
   t->q.K = depth;
   t->q.sam = a.s_mn; t->q.sak = a.s_k; t->q.sab = a.s_batch;
   t->q.sbn = b.s_mn; t->q.sbk = b.s_k; t->q.sbb = b.s_batch;
   t->q.row_padding = 1;
+  if (t->bytes_a) t->q.A = nullptr;   // (workspace: aligned)
+  if (t->bytes_b) t->q.B = nullptr;
   return t->bytes_a + t->bytes_b != 0;
 }
 
 }  // namespace
 
-// Whether copying pays: always once the problem fills the device with 128 x 128 tiles; below that by two estimates in
-// microseconds.
+double packed_us(const GemmProblem& p) {
+  PackPlan t;
+  if (p.dtype != srtReal32F || p.row_padding || !plan_pack(p, &t) || !f32_ring_fits(t.q)) return 0.0;
+  return 5.0 + (double)(t.bytes_a + t.bytes_b) / 3.0e6 + (double)p.batch * p.M * p.N * 4.0 / 8.0e6 + f32_ring_us(t.q);
+}
+
+// Whether copying pays (fp32: f32_any_choice in gemm_f32.hip).  16-bit types: always once the problem fills the device with
+// 128 x 128 tiles; below that by two estimates in microseconds.
 //   as it is   4 + its 64-deep stages at 1.0 (both operands contiguous along k), 2.5 (B along n) or 5 (A along m, or views
 //              without a unit stride), once per 512 tiles of 64 x 64
 //   copied     8 for the extra launch and the wait between the two, the copies' bytes at 6 TB/s, and a round of 128 x 128
@@ -148,6 +157,7 @@ bool plan_pack(const GemmProblem& p, PackPlan* t) {
 bool pack_preferred(const GemmProblem& p) {
   PackPlan t;
   if (p.row_padding || !plan_pack(p, &t)) return false;
+  if (p.dtype == srtReal32F) return !f32_ring_fits(p) && f32_any_choice(p, packed_us(p)) == F32Any::kPacked;
   auto tiles = [&](int s) { return (double)((p.M + s - 1) / s) * ((p.N + s - 1) / s) * p.batch; };
   const double cus = compute_units();
   if (tiles(128) >= cus) return true;
@@ -169,7 +179,9 @@ hipError_t launch_packed(const GemmProblem& p, hipStream_t stream) {
   if (t.bytes_a) t.q.A = t.a.dst = workspace;
   if (t.bytes_b) t.q.B = t.b.dst = (char*)workspace + at_b;
   auto blocks = [](const PackJob& j) { return (j.total + 256 * kChunksPerLane - 1) / (256 * kChunksPerLane); };
-  hipLaunchKernelGGL(pack_kernel<2>, dim3(blocks(t.a) + blocks(t.b)), dim3(256), 0, stream, t.a, t.b, blocks(t.a));
+  const dim3 grid(blocks(t.a) + blocks(t.b));
+  if (p.dtype == srtReal32F) hipLaunchKernelGGL(pack_kernel<4>, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a));
+  else hipLaunchKernelGGL(pack_kernel<2>, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a));
   hipError_t e = launch_status(stream);
   if (e == hipSuccess) e = launch_heuristic(t.q, stream);
   (void)srtDeviceFree(workspace);   // stream-ordered: reused only by work queued after the kernels above

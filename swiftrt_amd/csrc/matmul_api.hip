@@ -203,11 +203,14 @@ Plan heuristic_plan(const GemmProblem& p) {
         default: return kPlanF32SplitK;
       }
     }
-    // launch-sized problems and up to 64 rows: 32 x 32 tiles whose four waves split K
-    if (srt::f32_mfma_prefers_splitk(p)) return kPlanF32SplitK;
-    // a single matrix of too few 128 x 128 tiles for the device: its k range in parts on those tiles
-    if (srt::f32_tile_parts(p) >= 2) return kPlanF32Parts;
-    return kPlanF32Tile64;
+    switch (srt::f32_any_choice(p, srt::packed_us(p))) {
+      // launch-sized problems and up to 64 rows: 32 x 32 tiles whose waves split K
+      case srt::F32Any::kSplitK: return kPlanF32SplitK;
+      // a single matrix of too few 128 x 128 tiles for the device: its k range in parts on those tiles
+      case srt::F32Any::kParts: return kPlanF32Parts;
+      // (operands the ring kernel would read once copied into its layout are copied by the launch)
+      default: return kPlanF32Tile64;
+    }
   }
   return kPlanGeneric;
 }

@@ -67,3 +67,22 @@ def test_the_choice_for_ragged_rows():
                               (512, 1001, 200, "mfma_64x64")]:
         a, b = srt.Tensor(shape=[M, K], dtype=np.uint16), srt.Tensor(shape=[N, K], dtype=np.uint16)
         assert query_kernel(a, False, b, True, srt.Tensor(shape=[M, N], dtype=np.uint16)) == kernel
+
+
+# fp32 operands the 64-deep kernel reads only from a copy: k either side of its units, ragged rows and columns, each layout, a batch
+@pytest.mark.parametrize("M,N,K,batch", [(1023, 2047, 1001, 1), (2049, 1155, 515, 1), (1500, 2050, 129, 1), (700, 1500, 1001, 2),
+                                         (1200, 2000, 1004, 1)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_copied_fp32_operands(tmp_path, M, N, K, batch, ta, tb):
+    ran = run_matmul_case(tmp_path, H.F32, M, N, K, batch, ta, tb, ("f32_mfma_64x64",), 920 + M + K, left=3, right=2,
+                          operand_sentinel=NAN_BITS)
+    assert ran == ["f32_mfma_64x64"]
+
+
+def test_copied_fp32_views_without_a_unit_stride():
+    g = H.rng(921)
+    a = g.integers(-2, 3, (2100, 1100)).astype(np.float32)
+    b = g.integers(-2, 3, (1100, 4100)).astype(np.float32)
+    got = srt.matmul(srt.Tensor(a)[1:2051, 3:1099:2], srt.Tensor(b)[2:1098:2, 1:4097:2])
+    want = a[1:2051, 3:1099:2].astype(np.float64) @ b[2:1098:2, 1:4097:2].astype(np.float64)
+    assert np.array_equal(got.array(), want.astype(np.float32))
