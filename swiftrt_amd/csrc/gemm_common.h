@@ -320,6 +320,9 @@ double f32_ring_us(const GemmProblem& p);   // and of the ring kernel's plans al
 enum class F32Any { kTile, kSplitK, kParts, kPacked };
 F32Any f32_any_choice(const GemmProblem& p, double packed_us);   // for a problem the ring kernel does not read
 hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErrorOutOfMemory: no workspace, nothing was launched
+// 32 x 32 tiles whose waves split k (gemm_waves.hip): whether that is the choice, and the launch.
+bool waves_preferred(const GemmProblem& p);
+hipError_t launch_waves(const GemmProblem& p, hipStream_t stream);
 hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream);
 // Split-K over the 256 x 256 kernel: number of k parts (0: the problem does not qualify) and launch.
 int mfma_splitk_parts(const GemmProblem& p);

@@ -152,6 +152,8 @@ bool plan_supported(const GemmProblem& p, Plan plan) {
 }
 
 Plan heuristic_plan(const GemmProblem& p) {
+  // 16-bit problems of few tiles: 32 x 32 ones whose waves split k (the launch of this plan picks them by the same rule)
+  if (srt::waves_preferred(p)) return kPlanAny64;
   // one round of 128 x 128 tiles holds the problem (64 rows or more) and its k loop is not worth cutting
   if (srt::mfma_prefers_quarter(p)) return kPlanM16Q;
   if (srt::skinny_supported(p) && srt::skinny_preferred(p)) return kPlanSkinny;
