@@ -14,8 +14,7 @@
 //           one ds_read_b128; mn-contiguous [32 k][32 mn], 64 bytes per k row: two ds_read_b64_tr_b16, whose four k rows
 //           per half wave are 256 contiguous bytes
 //   sums    fp32; the eight partial tiles meet in LDS and are added pairwise, in a fixed order
-//   measured (before / now, us, bf16; before: 128 x 128 and 64 x 64 tiles, split-K, the streaming kernel): 256 x 256 x 1024 9.5 / 4.1,
-//           512^3 7.2 / 3.8, 512 x 512 x 4096 23.9 / 12.2, 192 x 1536 x 2240 26.2 / 10.5, 128 x 112 x 8000 46 / 16, 152 x 257 x 1529 x . W^T 19.0 /
+//   measured (before / now, us, bf16; before: 128 x 128 and 64 x 64 tiles, split-K, the streaming kernel): 136 x 448 x 576 9.9 / 3.8, 192 x 1536 x 2240 26.2 / 10.5, 128 x 112 x 8000 46 / 16, 152 x 257 x 1529 x . W^T 19.0 /
 //           6.3, 1176 x 384 x 3280 44 / 22, 1001^3 17.7 / 15.0, 32 x 2304 x 1469 13.7 / 5.3
 #include "gemm_common.h"
 
@@ -249,9 +248,9 @@ bool fits(const GemmProblem& p) {
 //            operands off the 16-byte rules; 5 + 7 where k is in neither's units (register-staged tiles).  A lower bound:
 //            more rounds cost more.  Measured / estimated: 512^3 7.2 / 7.5, 256 x 256 x 1024 9.5 / 10, 1001^3 17.7 / 14.9,
 //            136 x 448 x 576 8.5-11.6 / 8.9, 1176 x 384 x 3280 34-66 / 27
-// Problems the streaming kernel prefers stay with it (its rows of the weight arrive in whole lines: 64 x 2048 x 8192 x . W 19.6 there,
-// 25.7 here; 2 x 7808 x 2304 x . W 9.9 and 12.2), and so does what is in the 128 x 128 tiles' units in a batch, in more than one
-// round of tiles, below 512 k or beyond 3072 (a matrix of a short k loop keeps the bits it has in a batch; long ones have split-K).
+// Problems the streaming kernel prefers, or long k loops it takes, stay with it (its rows of the weight arrive in whole lines: 64 x 2048 x 8192 x . W 19.6 there,
+// 25.7 here; 2 x 7808 x 2304 x . W 9.9 and 12.2), and whole 128-deep units with the 128 x 128 tiles that
+// read them: a matrix keeps the bits it has in a batch, where those are ahead (32 x 256^3 6.3 against 9.3).
 bool waves_preferred(const GemmProblem& p) {
   if (p.row_padding || !fits(p)) return false;
   const double cus = compute_units(), k = (double)p.K / 1024.0, bytes = 128.0 * (double)p.K;
@@ -263,10 +262,10 @@ bool waves_preferred(const GemmProblem& p) {
   const double whole = 5.0 + 5.0 * k, cut = 17.0 + 2.5 * k;
   double others = whole < cut ? whole : cut;
   if (here >= others + 5.0 && here >= 5.0 + 7.0 * k) return false;   // (whatever the operands are)
-  if (skinny_supported(p) && skinny_preferred(p)) return false;
+  if (skinny_supported(p) && (skinny_preferred(p) || p.K >= 2048)) return false;
   if (mfma_config(p, 3) == 0) others += 5.0;
-  else if (mfma_config(p, 14) == 0) others = mfma_splitk_parts(p) >= 2 ? others : 5.0 + 7.0 * k;
-  else if (p.batch > 1 || rounds > 1.0 || p.K < 512 || p.K > 3072) return false;
+  else if (mfma_config(p, 14) != 0) return false;
+  else if (mfma_splitk_parts(p) < 2) others = 5.0 + 7.0 * k;
   return here < others;
 }
 

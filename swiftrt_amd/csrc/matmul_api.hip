@@ -152,8 +152,9 @@ bool plan_supported(const GemmProblem& p, Plan plan) {
 }
 
 Plan heuristic_plan(const GemmProblem& p) {
-  // 16-bit problems of few tiles: 32 x 32 ones whose waves split k (the launch of this plan picks them by the same rule)
-  if (srt::waves_preferred(p)) return kPlanAny64;
+  // 16-bit problems of few tiles off the 16-byte rules: 32 x 32 tiles whose waves split k (the launches of the 64 x 64 plans pick
+  // them by this rule; aligned operands keep the choices below and run them where that is the 64 x 64 plan)
+  if (srt::waves_preferred(p) && srt::mfma_config(p, 3) == 0) return kPlanAny64;
   // one round of 128 x 128 tiles holds the problem (64 rows or more) and its k loop is not worth cutting
   if (srt::mfma_prefers_quarter(p)) return kPlanM16Q;
   if (srt::skinny_supported(p) && srt::skinny_preferred(p)) return kPlanSkinny;

@@ -64,7 +64,7 @@ def test_results_with_ragged_rows(tmp_path, dt, M, N, K, batch):
 
 def test_the_choice_for_ragged_rows():
     for (M, N, K, kernel) in [(2048, 50257, 768, "mfma_256x256_m16_k64"), (512, 1001, 1024, "mfma_128x128_m16_k128"),
-                              (2048, 1001, 72, "mfma_64x64")]:
+                              (512, 1001, 200, "mfma_64x64")]:
         a, b = srt.Tensor(shape=[M, K], dtype=np.uint16), srt.Tensor(shape=[N, K], dtype=np.uint16)
         assert query_kernel(a, False, b, True, srt.Tensor(shape=[M, N], dtype=np.uint16)) == kernel
 
