@@ -361,6 +361,8 @@ def concatenate(a, b, axis):
     """concatenate(_:_:axis:) of two tensors, one device call."""
     if a.rank != b.rank or a.dtype != b.dtype:
         raise ValueError("concatenate: rank and element type must agree")
+    if not -a.rank <= axis < a.rank:
+        raise IndexError(f"concatenate: axis {axis} of rank {a.rank}")
     axis %= a.rank
     shape = list(a.shape)
     shape[axis] += b.shape[axis]

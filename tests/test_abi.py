@@ -514,6 +514,14 @@ def test_matmul_shape_rules_raise_before_any_native_call():
         srt.Dense(srt.Tensor(np.zeros((2, 4), np.float32)), bias=srt.Tensor(np.zeros(3, np.float32)))
 
 
+def test_concatenate_refuses_an_axis_out_of_range():
+    for rank, axes in ((1, (1, 2, -2)), (2, (2, 3, 5, -3)), (3, (3, -4))):
+        t = srt.Tensor(np.zeros((2,) * rank, np.float32))
+        for axis in axes:
+            with pytest.raises(IndexError):
+                srt.concatenate(t, t, axis)
+
+
 def test_activation_enum_matches_reference_case_order():
     assert [a.name for a in srt.ActivationType] == ["sigmoid", "relu", "tanh", "clippedRelu", "elu", "identity"]
     assert [int(a) for a in srt.ActivationType] == list(range(6))
