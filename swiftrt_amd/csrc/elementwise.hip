@@ -400,7 +400,7 @@ int vector_width(const Map& m, bool* ragged) {
 // The map with its innermost extent counted in vectors.
 inline void count_vectors(Map* m, int v) {
   const int inner = m->rank - 1;
-  const uint32_t vectors = (m->shape[inner] + v - 1) / v;
+  const uint32_t vectors = (uint32_t)(((unsigned long long)m->shape[inner] + v - 1) / v);   // (extents reach 2^32 - 1)
   m->inner_elements = m->shape[inner];
   m->total = m->total / m->shape[inner] * vectors;
   m->shape[inner] = vectors;

@@ -514,6 +514,20 @@ def test_matmul_shape_rules_raise_before_any_native_call():
         srt.Dense(srt.Tensor(np.zeros((2, 4), np.float32)), bias=srt.Tensor(np.zeros(3, np.float32)))
 
 
+@pytest.mark.parametrize("extent", [0xfffffff9, 0xffffffff])
+def test_extents_just_below_32_bits_reach_a_launch(extent):
+    """The innermost extent in vectors is counted in 64 bits: a count that wraps to zero would answer success without a launch.
+    Without a device a launch is an error, so success can only mean that none was tried."""
+    L = native.lib()
+    n = ctypes.c_int32(0)
+    if L.srtGetDeviceCount(ctypes.byref(n)) == 0 and n.value:
+        pytest.skip("placeholder pointers: for machines without a device")
+    d, keep = native.make_descriptor(native.REAL16BF, (extent,), (1,), native.ORDER_ROW)
+    p = ctypes.c_void_p(256)
+    for name in ("srtNeg", "srtCopy", "srtSigmoid"):
+        assert getattr(L, name)(p, ctypes.byref(d), p, ctypes.byref(d), None) != 0, name
+
+
 def test_concatenate_refuses_an_axis_out_of_range():
     for rank, axes in ((1, (1, 2, -2)), (2, (2, 3, 5, -3)), (3, (3, -4))):
         t = srt.Tensor(np.zeros((2,) * rank, np.float32))

@@ -1,9 +1,12 @@
 """Element-wise maps whose operands walk memory across the result's rows (turned through LDS in 64 x 64 tiles) and maps whose rows are
 no whole number of aligned vectors: exact against numpy on small integers, at the edges of the tile and of the vector."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import swiftrt_amd as srt
+from swiftrt_amd import native
 from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +78,22 @@ def test_column_major_results_are_walked_in_their_storage_order(dt):
     col = lambda x: srt.Tensor(x, order=srt.Order.col)       # noqa: E731
     check(col(a) + col(b), H.to64(a) + H.to64(b), dt)
     check(col(a) + srt.Tensor(b), H.to64(a) + H.to64(b), dt)   # row-major into column-major
+
+
+@pytest.mark.parametrize("count", [0xfffffff9, 0xffffffff])
+def test_extents_just_below_32_bits(count):
+    """One dense 16-bit row whose extent rounded up to whole vectors passes 2^32 (two buffers of 8.6 GB): read back at both ends and
+    in the middle."""
+    L, q = native.lib(), srt.current_queue()
+    d, keep = native.make_descriptor(native.REAL16BF, (count,), (1,), native.ORDER_ROW)
+    src, dst = q.allocate(2 * count), q.allocate(2 * count)
+    element = np.array([0x3FC0], np.uint16)              # 1.5
+    native.check(L.srtFillFlat(native.REAL16BF, src.pointer, ctypes.c_void_p(element.ctypes.data), count, q.stream))
+    q.zero(dst, 2 * count)
+    native.check(L.srtNeg(src.pointer, ctypes.byref(d), dst.pointer, ctypes.byref(d), q.stream))
+    for at in (0, count // 2, count - 4096):
+        got = np.zeros(4096, np.uint16)
+        native.check(L.srtMemcpyAsync(ctypes.c_void_p(got.ctypes.data), ctypes.c_void_p(dst.pointer + 2 * at), 8192, native.D2H,
+                                      q.stream))
+        q.wait_for_completion()
+        assert np.all(got == 0xBFC0), at
