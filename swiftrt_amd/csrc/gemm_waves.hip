@@ -229,8 +229,9 @@ hipError_t launch_as(const GemmProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
-// Both operands have a unit stride, with at least one whole vector along it.
+// Both operands have a unit stride, with at least one whole vector along it, and there is something to sum.
 bool fits(const GemmProblem& p) {
+  if (p.K < 1) return false;
   if (p.dtype != srtReal16BF && p.dtype != srtReal16F) return false;
   if (p.sak == 1 ? p.K < 8 : (p.sam != 1 || p.M < 8)) return false;
   if (p.sbn == 1 ? p.N < 8 : (p.sbk != 1 || p.K < 8)) return false;

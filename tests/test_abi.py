@@ -444,6 +444,22 @@ def test_kernel_selection_is_queryable_without_gpu():
     assert query(native.REAL16BF, 8, 65664, 32768, tb=True) == "skinny/pieces"
 
 
+def test_an_empty_sum_runs_on_the_generic_kernel():
+    """K = 0 (the result is the activation of the bias): no matrix-core kernel qualifies, in any layout, type or size."""
+    L = native.lib()
+    buf = ctypes.create_string_buffer(64)
+    p = ctypes.c_void_p(256)
+    for dt in (native.REAL16BF, native.REAL16F, native.REAL32F):
+        for M, N in ((8, 8), (33, 33), (64, 512), (2048, 2048)):
+            for ta in (0, 1):
+                for tb in (0, 1):
+                    ad, k1 = native.make_descriptor(dt, (0, M) if ta else (M, 0), (M if ta else 1, 1), native.ORDER_ROW)
+                    bd, k2 = native.make_descriptor(dt, (N, 0) if tb else (0, N), (1 if tb else N, 1), native.ORDER_ROW)
+                    od, k3 = native.make_descriptor(dt, (M, N), (N, 1), native.ORDER_ROW)
+                    assert L.srtMatmulQueryKernel(ctypes.byref(ad), ta, ctypes.byref(bd), tb, ctypes.byref(od), p, p, p, buf, 64) == 0
+                    assert buf.value.decode() == "generic", (dt, M, N, ta, tb)
+
+
 def test_kernel_selection_answers_for_any_problem():
     """Random shapes, types, layouts, pitches, batches and alignments (zero extents included): the selection logic
     answers every one with success and a known plan name.  (Run against the host-sanitizer build of the library, this is

@@ -2,6 +2,7 @@
 
 Integer operands, exact comparison (every partial sum is representable, so the kernel and its order of summation do not
 matter); operands framed by NaNs, results by a sentinel, so that a load or a store past an edge shows."""
+import numpy as np
 import pytest
 
 import swiftrt_amd as srt
@@ -30,3 +31,18 @@ def test_rows_of_any_extent_and_alignment(tmp_path, dt, M, N, K, batch, ta, tb, 
     ran = run_matmul_case(tmp_path, dt, M, N, K, batch, ta, tb, ("mfma_64x64_any",), 800 + M + K, left=left, right=right,
                           operand_sentinel=NAN_BITS, with_bias=M % 2 == 0)
     assert ran == ["mfma_64x64_any"]
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("dt", [H.BF16, H.F16])
+def test_an_empty_sum_is_the_bias(dt, ta, tb):
+    """K = 0: nothing is read, every element of the result is written."""
+    M, N = 40, 72
+    T = srt.Tensor
+    bias = T(H.encode(np.arange(N) - 30.0, dt))
+    a, b = T(shape=[0, M] if ta else [M, 0], dtype=bias.dtype), T(shape=[N, 0] if tb else [0, N], dtype=bias.dtype)
+    for with_bias, want in ((False, np.zeros((M, N))), (True, np.maximum(np.tile(np.arange(N) - 30.0, (M, 1)), 0.0))):
+        out = T(H.encode(np.full((M, N), 5.0), dt))
+        srt.current_queue().matmul(a, ta, b, tb, out, bias=bias if with_bias else None,
+                                   activation=srt.ActivationType.relu if with_bias else None)
+        assert np.array_equal(H.to64(out.array()), want), with_bias
