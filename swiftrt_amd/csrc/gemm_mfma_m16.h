@@ -212,7 +212,8 @@ struct FragReader {
 // (5.5 us of a 95 us tile at K = 4096).  A dense, 8-byte-aligned bias is read as eight 8-byte loads.
 // They wait in their stored 16-bit form, two to a register (16 registers per lane): b[j] holds the four
 // per-column values of column tile j; in the per-row case b[i].x holds row tile i's value.
-template <typename T, int TM>
+// WHOLE: N is a multiple of 8 (checked on the host).
+template <typename T, int TM, bool WHOLE = true>
 __device__ __forceinline__ void load_bias(const GemmProblem& p, int wave_m0, int wave_n0, int lane, u32x2_t (&b)[8]) {
   using S = typename T::storage;
   static_assert(sizeof(S) == 2 && TM <= 8, "16-bit element types, at most 8 row tiles");
@@ -228,13 +229,13 @@ __device__ __forceinline__ void load_bias(const GemmProblem& p, int wave_m0, int
       if (m < p.M) b[i].x = bias[(long long)m * p.sbias];
     }
   } else if (p.sbias == 1 && (reinterpret_cast<uintptr_t>(bias) & 7u) == 0) {
-    // a lane's four columns are all inside, all outside, or (N not a multiple of 4) across the end of the row
+    // a lane's four columns are all inside, all outside, or (not WHOLE) across the end of the row
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int n = wave_n0 + 16 * j + 4 * g;
       if (n + 4 <= p.N) b[j] = *reinterpret_cast<const u32x2_t*>(bias + n);
     }
-    if ((p.N & 3) != 0) {
+    if (!WHOLE && (p.N & 3) != 0) {
       const int n = p.N & ~3;   // the lane that holds the last, partial group
       const int j = (n - wave_n0) >> 4;
       if (n >= wave_n0 && ((n >> 2) & 3) == g) {
@@ -385,16 +386,16 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
   }
 }
 
-// store_tile for an epilogue kind, on results of either alignment: two copies of the code behind one uniform branch (a choice
-// at every store cost the launch 0.8 us, 1000 x 1000 x 1000 18.3 -> 19.1).
-template <typename T, int TM, int EPI, bool FLIP, int TN>
-__device__ __forceinline__ void store_tile_any(const GemmProblem& p, const f32x4_t (&acc)[TM][TN], int wave_m0, int wave_n0,
-                                               int bz, int lane, uint32_t stage, const u32x2_t (&b)[8], int n_end) {
+// store_tile for an epilogue kind.  Whether the result is stored in whole aligned chunks is a property of the kernel, not of the
+// call: with both copies of the code behind one uniform branch in every kernel, aligned results paid 0.2-0.8 us a launch
+// (4096 x 4096 x 256 13.7 -> 14.2, 3072 x 3072 x 1024 22.9 -> 23.7), and with a choice at every store more.
+template <typename T, int TM, int EPI, bool FLIP, int TN, bool WHOLE>
+__device__ __forceinline__ void store_tile_as(const GemmProblem& p, const f32x4_t (&acc)[TM][TN], int wave_m0, int wave_n0,
+                                              int bz, int lane, uint32_t stage, const u32x2_t (&b)[8], int n_end) {
   constexpr bool HAS_BIAS = EPI != EPI_PLAIN && EPI != EPI_RELU;
   constexpr int CLAMP = EPI == EPI_RELU || EPI == EPI_BIAS_RELU ? 1 : EPI == EPI_CLIPPED ? 2
                       : EPI == EPI_SIGMOID ? 3 : EPI == EPI_TANH ? 4 : EPI == EPI_ELU ? 5 : 0;
-  if (c_whole_chunks(p)) store_tile<T, TM, HAS_BIAS, CLAMP, FLIP, TN, true>(p, acc, wave_m0, wave_n0, bz, lane, stage, b, n_end);
-  else store_tile<T, TM, HAS_BIAS, CLAMP, FLIP, TN, false>(p, acc, wave_m0, wave_n0, bz, lane, stage, b, n_end);
+  store_tile<T, TM, HAS_BIAS, CLAMP, FLIP, TN, WHOLE>(p, acc, wave_m0, wave_n0, bz, lane, stage, b, n_end);
 }
 
 // sigmoid / tanh / elu: acc + bias goes to the staging area as fp32 (passes of ROWS = 32 or 16 rows:

@@ -411,7 +411,8 @@ constexpr int TAIL_MAX_PARTS = 3;
 // B's k rows are fetched whole (the tile's neighbour's columns ride along).
 // TM: row tiles per wave.  8: 256 rows per workgroup tile.  4: the 128 x 256 half tile (waves of 64 x 128) for problems that
 // leave compute units idle with whole tiles; its A unit is 128 rows of a k-contiguous A (in a slot of the same size).
-template <typename T, bool A_KC, bool B_KC, int EPI, bool SK, bool FLIP = false, int TN = 8, int TM = 8>
+// WHOLE: the result's rows are whole aligned 16-byte chunks (c_whole_chunks), stored through a descriptor; false: any rows.
+template <typename T, bool A_KC, bool B_KC, int EPI, bool SK, bool FLIP = false, int TN = 8, int TM = 8, bool WHOLE = true>
 __device__ __forceinline__ void gemm_m16d_body(const GemmProblem& p, const TailShare& ts) {
   static_assert(EPI != EPI_TRANS, "sigmoid / tanh / elu have epilogue kinds of their own here");
   static_assert(!FLIP || EPI != EPI_PARTIAL, "flipped: the store_tile epilogues only");
@@ -779,7 +780,7 @@ __device__ __forceinline__ void gemm_m16d_body(const GemmProblem& p, const TailS
     constexpr bool LINEAR_BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_RELU || EPI == EPI_CLIPPED || EPI == EPI_SIGMOID ||
                                  EPI == EPI_TANH || EPI == EPI_ELU;
     u32x2_t bias_regs[8];
-    if (LINEAR_BIAS) m16::load_bias<T, TM>(pe, em0, en0, le, bias_regs);   // lands during the wait below
+    if (LINEAR_BIAS) m16::load_bias<T, TM, WHOLE>(pe, em0, en0, le, bias_regs);   // lands during the wait below
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier\n\ts_nop 7\n\ts_nop 7" ::: "memory");
     if (LINEAR_BIAS || SK) m16::pin_all<TM>(acc);
     const int n_end = cur_tile.n0 + tile_w;   // (the narrow tile: its valid columns end here)
@@ -862,7 +863,7 @@ __device__ __forceinline__ void gemm_m16d_body(const GemmProblem& p, const TailS
     } else if constexpr (EPI == EPI_PARTIAL) {
       m16::store_tile_partial<TM>(p, acc, em0, en0, bz, le, stage);
     } else {
-      m16::store_tile_any<T, TM, EPI, FLIP, TN>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
+      m16::store_tile_as<T, TM, EPI, FLIP, TN, WHOLE>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
     }
     if (!has_next) break;
 
@@ -874,9 +875,9 @@ __device__ __forceinline__ void gemm_m16d_body(const GemmProblem& p, const TailS
   }
 }
 
-template <typename T, bool A_KC, bool B_KC, int EPI, bool FLIP = false>
+template <typename T, bool A_KC, bool B_KC, int EPI, bool FLIP = false, bool WHOLE = true>
 __global__ __launch_bounds__(NT) void gemm_m16d_kernel(GemmProblem p) {
-  gemm_m16d_body<T, A_KC, B_KC, EPI, false, FLIP>(p, TailShare{});
+  gemm_m16d_body<T, A_KC, B_KC, EPI, false, FLIP, 8, 8, WHOLE>(p, TailShare{});
 }
 
 template <typename T, bool A_KC, bool B_KC, int EPI, bool FLIP = false>
@@ -885,15 +886,15 @@ __global__ __launch_bounds__(NT) void gemm_m16d_tail_kernel(GemmProblem p, TailS
 }
 
 // The 128 x 256 half tile (k-contiguous A), for problems that leave compute units idle with whole tiles.
-template <typename T, bool B_KC, int EPI>
+template <typename T, bool B_KC, int EPI, bool WHOLE = true>
 __global__ __launch_bounds__(NT) void gemm_m16d_half_kernel(GemmProblem p) {
-  gemm_m16d_body<T, true, B_KC, EPI, false, false, 8, 4>(p, TailShare{});
+  gemm_m16d_body<T, true, B_KC, EPI, false, false, 8, 4, WHOLE>(p, TailShare{});
 }
 
 // The 256 x 128 half tile, for an A that is not k-contiguous.
-template <typename T, bool B_KC, int EPI>
+template <typename T, bool B_KC, int EPI, bool WHOLE>
 __global__ __launch_bounds__(NT) void gemm_m16d_narrow_kernel(GemmProblem p) {
-  gemm_m16d_body<T, false, B_KC, EPI, false, false, 4, 8>(p, TailShare{});
+  gemm_m16d_body<T, false, B_KC, EPI, false, false, 4, 8, WHOLE>(p, TailShare{});
 }
 
 // Two tile walks in one launch, for a tile count that leaves the last round of the persistent grid between half
@@ -917,9 +918,9 @@ __global__ __launch_bounds__(NT) void gemm_m16d_split_kernel(GemmProblem wide, G
 // Host-side admission beyond the 32-deep kernel's: whole super-stages, at least four of them.
 inline bool deep_fits(const GemmProblem& p) { return p.K % DK == 0 && p.K >= 4 * DK; }
 
-template <typename T, bool A_KC, bool B_KC, int EPI, bool FLIP = false>
+template <typename T, bool A_KC, bool B_KC, int EPI, bool FLIP = false, bool WHOLE = true>
 hipError_t launch_kernel(const GemmProblem& p, hipStream_t stream) {
-  auto kernel = gemm_m16d_kernel<T, A_KC, B_KC, EPI, FLIP>;
+  auto kernel = gemm_m16d_kernel<T, A_KC, B_KC, EPI, FLIP, WHOLE>;
   constexpr int lds_bytes = UNITS * UNIT;
   static std::atomic<uint32_t> configured{0};
   if (hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kernel), lds_bytes, configured); e != hipSuccess) return e;
@@ -1073,30 +1074,35 @@ hipError_t launch_tail(const GemmProblem& p, hipStream_t stream) {
   return launch_tail_kernel<T, A_KC, B_KC, EPI_PLAIN>(p, stream);
 }
 
-template <typename T, bool A_KC, bool B_KC>
-hipError_t launch(const GemmProblem& p, hipStream_t stream) {
+template <typename T, bool A_KC, bool B_KC, bool WHOLE>
+hipError_t launch_as(const GemmProblem& p, hipStream_t stream) {
   // x . W runs as (W^T . x^T)^T: the flipped problem has an m-contiguous A and a k-contiguous B.  Whatever qualifies
   // this way round qualifies flipped: the operands' reaches and alignments exchange places, an n-contiguous B's N is a
   // multiple of 8 as an m-contiguous A's M must be, and the result is addressed as before.
   constexpr bool FLIP = A_KC && !B_KC;
   constexpr bool KA = FLIP ? false : A_KC, KB = FLIP ? true : B_KC;
   const GemmProblem q = FLIP ? flipped(p) : p;
-  if (p.activation == srtActivationSigmoid) return launch_kernel<T, KA, KB, EPI_SIGMOID, FLIP>(q, stream);
-  if (p.activation == srtActivationTanh) return launch_kernel<T, KA, KB, EPI_TANH, FLIP>(q, stream);
-  if (p.activation == srtActivationElu) return launch_kernel<T, KA, KB, EPI_ELU, FLIP>(q, stream);
-  if (p.activation == srtActivationClippedRelu) return launch_kernel<T, KA, KB, EPI_CLIPPED, FLIP>(q, stream);
+  if (p.activation == srtActivationSigmoid) return launch_kernel<T, KA, KB, EPI_SIGMOID, FLIP, WHOLE>(q, stream);
+  if (p.activation == srtActivationTanh) return launch_kernel<T, KA, KB, EPI_TANH, FLIP, WHOLE>(q, stream);
+  if (p.activation == srtActivationElu) return launch_kernel<T, KA, KB, EPI_ELU, FLIP, WHOLE>(q, stream);
+  if (p.activation == srtActivationClippedRelu) return launch_kernel<T, KA, KB, EPI_CLIPPED, FLIP, WHOLE>(q, stream);
   if (p.activation == srtActivationRelu) {
-    if (p.bias) return launch_kernel<T, KA, KB, EPI_BIAS_RELU, FLIP>(q, stream);
-    return launch_kernel<T, KA, KB, EPI_RELU, FLIP>(q, stream);
+    if (p.bias) return launch_kernel<T, KA, KB, EPI_BIAS_RELU, FLIP, WHOLE>(q, stream);
+    return launch_kernel<T, KA, KB, EPI_RELU, FLIP, WHOLE>(q, stream);
   }
-  if (p.bias) return launch_kernel<T, KA, KB, EPI_BIAS, FLIP>(q, stream);
-  return launch_kernel<T, KA, KB, EPI_PLAIN, FLIP>(q, stream);
+  if (p.bias) return launch_kernel<T, KA, KB, EPI_BIAS, FLIP, WHOLE>(q, stream);
+  return launch_kernel<T, KA, KB, EPI_PLAIN, FLIP, WHOLE>(q, stream);
+}
+
+template <typename T, bool A_KC, bool B_KC>
+hipError_t launch(const GemmProblem& p, hipStream_t stream) {
+  return c_whole_chunks(p) ? launch_as<T, A_KC, B_KC, true>(p, stream) : launch_as<T, A_KC, B_KC, false>(p, stream);
 }
 
 // ---- the half tile ------------------------------------------------------------------------------------------------
-template <typename T, bool B_KC, int EPI>
+template <typename T, bool B_KC, int EPI, bool WHOLE = true>
 hipError_t launch_half_kernel(const GemmProblem& p, hipStream_t stream) {
-  auto kernel = gemm_m16d_half_kernel<T, B_KC, EPI>;
+  auto kernel = gemm_m16d_half_kernel<T, B_KC, EPI, WHOLE>;
   constexpr int lds_bytes = UNITS * UNIT;
   static std::atomic<uint32_t> configured{0};
   if (hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kernel), lds_bytes, configured); e != hipSuccess) return e;
@@ -1106,24 +1112,29 @@ hipError_t launch_half_kernel(const GemmProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
+template <typename T, bool B_KC, bool WHOLE>
+hipError_t launch_half_as(const GemmProblem& p, hipStream_t stream) {
+  if (p.activation == srtActivationSigmoid) return launch_half_kernel<T, B_KC, EPI_SIGMOID, WHOLE>(p, stream);
+  if (p.activation == srtActivationTanh) return launch_half_kernel<T, B_KC, EPI_TANH, WHOLE>(p, stream);
+  if (p.activation == srtActivationElu) return launch_half_kernel<T, B_KC, EPI_ELU, WHOLE>(p, stream);
+  if (p.activation == srtActivationClippedRelu) return launch_half_kernel<T, B_KC, EPI_CLIPPED, WHOLE>(p, stream);
+  if (p.activation == srtActivationRelu) {
+    if (p.bias) return launch_half_kernel<T, B_KC, EPI_BIAS_RELU, WHOLE>(p, stream);
+    return launch_half_kernel<T, B_KC, EPI_RELU, WHOLE>(p, stream);
+  }
+  if (p.bias) return launch_half_kernel<T, B_KC, EPI_BIAS, WHOLE>(p, stream);
+  return launch_half_kernel<T, B_KC, EPI_PLAIN, WHOLE>(p, stream);
+}
+
 template <typename T, bool B_KC>
 hipError_t launch_half(const GemmProblem& p, hipStream_t stream) {
-  if (p.activation == srtActivationSigmoid) return launch_half_kernel<T, B_KC, EPI_SIGMOID>(p, stream);
-  if (p.activation == srtActivationTanh) return launch_half_kernel<T, B_KC, EPI_TANH>(p, stream);
-  if (p.activation == srtActivationElu) return launch_half_kernel<T, B_KC, EPI_ELU>(p, stream);
-  if (p.activation == srtActivationClippedRelu) return launch_half_kernel<T, B_KC, EPI_CLIPPED>(p, stream);
-  if (p.activation == srtActivationRelu) {
-    if (p.bias) return launch_half_kernel<T, B_KC, EPI_BIAS_RELU>(p, stream);
-    return launch_half_kernel<T, B_KC, EPI_RELU>(p, stream);
-  }
-  if (p.bias) return launch_half_kernel<T, B_KC, EPI_BIAS>(p, stream);
-  return launch_half_kernel<T, B_KC, EPI_PLAIN>(p, stream);
+  return c_whole_chunks(p) ? launch_half_as<T, B_KC, true>(p, stream) : launch_half_as<T, B_KC, false>(p, stream);
 }
 
 // the 256 x 128 half tile (A not k-contiguous)
-template <typename T, bool B_KC, int EPI>
+template <typename T, bool B_KC, int EPI, bool WHOLE>
 hipError_t launch_narrow_kernel(const GemmProblem& p, hipStream_t stream) {
-  auto kernel = gemm_m16d_narrow_kernel<T, B_KC, EPI>;
+  auto kernel = gemm_m16d_narrow_kernel<T, B_KC, EPI, WHOLE>;
   constexpr int lds_bytes = UNITS * UNIT;
   static std::atomic<uint32_t> configured{0};
   if (hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kernel), lds_bytes, configured); e != hipSuccess) return e;
@@ -1135,18 +1146,23 @@ hipError_t launch_narrow_kernel(const GemmProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
+template <typename T, bool B_KC, bool WHOLE>
+hipError_t launch_narrow_as(const GemmProblem& p, hipStream_t stream) {
+  if (p.activation == srtActivationSigmoid) return launch_narrow_kernel<T, B_KC, EPI_SIGMOID, WHOLE>(p, stream);
+  if (p.activation == srtActivationTanh) return launch_narrow_kernel<T, B_KC, EPI_TANH, WHOLE>(p, stream);
+  if (p.activation == srtActivationElu) return launch_narrow_kernel<T, B_KC, EPI_ELU, WHOLE>(p, stream);
+  if (p.activation == srtActivationClippedRelu) return launch_narrow_kernel<T, B_KC, EPI_CLIPPED, WHOLE>(p, stream);
+  if (p.activation == srtActivationRelu) {
+    if (p.bias) return launch_narrow_kernel<T, B_KC, EPI_BIAS_RELU, WHOLE>(p, stream);
+    return launch_narrow_kernel<T, B_KC, EPI_RELU, WHOLE>(p, stream);
+  }
+  if (p.bias) return launch_narrow_kernel<T, B_KC, EPI_BIAS, WHOLE>(p, stream);
+  return launch_narrow_kernel<T, B_KC, EPI_PLAIN, WHOLE>(p, stream);
+}
+
 template <typename T, bool B_KC>
 hipError_t launch_narrow(const GemmProblem& p, hipStream_t stream) {
-  if (p.activation == srtActivationSigmoid) return launch_narrow_kernel<T, B_KC, EPI_SIGMOID>(p, stream);
-  if (p.activation == srtActivationTanh) return launch_narrow_kernel<T, B_KC, EPI_TANH>(p, stream);
-  if (p.activation == srtActivationElu) return launch_narrow_kernel<T, B_KC, EPI_ELU>(p, stream);
-  if (p.activation == srtActivationClippedRelu) return launch_narrow_kernel<T, B_KC, EPI_CLIPPED>(p, stream);
-  if (p.activation == srtActivationRelu) {
-    if (p.bias) return launch_narrow_kernel<T, B_KC, EPI_BIAS_RELU>(p, stream);
-    return launch_narrow_kernel<T, B_KC, EPI_RELU>(p, stream);
-  }
-  if (p.bias) return launch_narrow_kernel<T, B_KC, EPI_BIAS>(p, stream);
-  return launch_narrow_kernel<T, B_KC, EPI_PLAIN>(p, stream);
+  return c_whole_chunks(p) ? launch_narrow_as<T, B_KC, true>(p, stream) : launch_narrow_as<T, B_KC, false>(p, stream);
 }
 
 // The split-K pass on half tiles (a k-contiguous A of at most 128 rows): fp32 accumulators to a workspace.

@@ -128,7 +128,10 @@ struct FragReader<false> {
   }
 };
 
-template <typename T, bool A_KC, bool B_KC, int EPI>
+#define SRT_ARGS __attribute__((address_space(4)))
+
+// WHOLE: the result's rows are whole aligned 16-byte chunks (c_whole_chunks), stored through a descriptor; false: any rows.
+template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE>
 __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];
   const uint32_t lds = (uint32_t)(uintptr_t)(SRT_LDS unsigned char*)lds_raw;
@@ -350,8 +353,15 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
     const int le = lane_id();
     constexpr bool LINEAR_BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_RELU || EPI == EPI_CLIPPED || EPI == EPI_SIGMOID ||
                                  EPI == EPI_TANH || EPI == EPI_ELU;
+    // What the epilogue needs of the problem is read from the kernel's arguments here: held from the start, it spilled scalar
+    // registers in the prologue, and two or three 128-deep units are mostly prologue and epilogue (us, held / read here: F16
+    // 32 x 256^3 x . W^T 6.37 / 6.28, 512 x 4096 x 256 x . W 6.60 / 6.52, 640 x 896 x 768 8.67 / 8.55).  x^T . W has registers to
+    // spare and is 1 % better off without (512^3 7.43 / 7.50).
+    const SRT_ARGS GemmProblem* args = (const SRT_ARGS GemmProblem*)__builtin_amdgcn_kernarg_segment_ptr();
+    if (A_KC || B_KC) asm volatile("" : "+s"(args));
+    const GemmProblem pe = A_KC || B_KC ? *(const GemmProblem*)args : p;
     u32x2_t bias_regs[8];
-    if (LINEAR_BIAS) m16::load_bias<T, 4>(p, em0, en0, le, bias_regs);   // lands during the wait below
+    if (LINEAR_BIAS) m16::load_bias<T, 4, WHOLE>(pe, em0, en0, le, bias_regs);   // lands during the wait below
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier\n\ts_nop 7\n\ts_nop 7" ::: "memory");
     if (LINEAR_BIAS) m16::pin_all<4, 4>(acc);
     const int n_end = cur_tile.n0 + TILE;
@@ -360,7 +370,7 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
     uint32_t sb = x < lds + UNIT ? x + 4 * UNIT : x - UNIT;
     const uint32_t stage = ((wave & 2) ? sb : sa) + (uint32_t)(wave & 1) * (uint32_t)(UNIT / 2);
 
-    m16::store_tile_any<T, 4, EPI, false, 4>(p, acc, em0, en0, bz, le, stage, bias_regs, n_end);
+    m16::store_tile_as<T, 4, EPI, false, 4, WHOLE>(pe, acc, em0, en0, bz, le, stage, bias_regs, n_end);
     if (!has_next) break;
 
     // every wave has finished reading its staging area before any wave's loads overwrite it
@@ -372,15 +382,15 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
 
 #undef SRT_FENCE
 
-template <typename T, bool A_KC, bool B_KC, int EPI>
+template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE>
 __global__ __launch_bounds__(NT) void gemm_m16q_kernel(GemmProblem p) {
-  gemm_m16q_body<T, A_KC, B_KC, EPI>(p);
+  gemm_m16q_body<T, A_KC, B_KC, EPI, WHOLE>(p);
 }
 
 // ---- host side ---------------------------------------------------------------------------------------
-template <typename T, bool A_KC, bool B_KC, int EPI>
+template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE>
 hipError_t launch_kernel(const GemmProblem& p, hipStream_t stream) {
-  auto kernel = gemm_m16q_kernel<T, A_KC, B_KC, EPI>;
+  auto kernel = gemm_m16q_kernel<T, A_KC, B_KC, EPI, WHOLE>;
   constexpr int lds_bytes = UNITS * UNIT;
   static std::atomic<uint32_t> configured{0};
   if (hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kernel), lds_bytes, configured); e != hipSuccess) return e;
@@ -390,18 +400,23 @@ hipError_t launch_kernel(const GemmProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
+template <typename T, bool A_KC, bool B_KC, bool WHOLE>
+hipError_t launch_as(const GemmProblem& p, hipStream_t stream) {
+  if (p.activation == srtActivationSigmoid) return launch_kernel<T, A_KC, B_KC, EPI_SIGMOID, WHOLE>(p, stream);
+  if (p.activation == srtActivationTanh) return launch_kernel<T, A_KC, B_KC, EPI_TANH, WHOLE>(p, stream);
+  if (p.activation == srtActivationElu) return launch_kernel<T, A_KC, B_KC, EPI_ELU, WHOLE>(p, stream);
+  if (p.activation == srtActivationClippedRelu) return launch_kernel<T, A_KC, B_KC, EPI_CLIPPED, WHOLE>(p, stream);
+  if (p.activation == srtActivationRelu) {
+    if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS_RELU, WHOLE>(p, stream);
+    return launch_kernel<T, A_KC, B_KC, EPI_RELU, WHOLE>(p, stream);
+  }
+  if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS, WHOLE>(p, stream);
+  return launch_kernel<T, A_KC, B_KC, EPI_PLAIN, WHOLE>(p, stream);
+}
+
 template <typename T, bool A_KC, bool B_KC>
 hipError_t launch(const GemmProblem& p, hipStream_t stream) {
-  if (p.activation == srtActivationSigmoid) return launch_kernel<T, A_KC, B_KC, EPI_SIGMOID>(p, stream);
-  if (p.activation == srtActivationTanh) return launch_kernel<T, A_KC, B_KC, EPI_TANH>(p, stream);
-  if (p.activation == srtActivationElu) return launch_kernel<T, A_KC, B_KC, EPI_ELU>(p, stream);
-  if (p.activation == srtActivationClippedRelu) return launch_kernel<T, A_KC, B_KC, EPI_CLIPPED>(p, stream);
-  if (p.activation == srtActivationRelu) {
-    if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS_RELU>(p, stream);
-    return launch_kernel<T, A_KC, B_KC, EPI_RELU>(p, stream);
-  }
-  if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS>(p, stream);
-  return launch_kernel<T, A_KC, B_KC, EPI_PLAIN>(p, stream);
+  return c_whole_chunks(p) ? launch_as<T, A_KC, B_KC, true>(p, stream) : launch_as<T, A_KC, B_KC, false>(p, stream);
 }
 
 }  // namespace m16q

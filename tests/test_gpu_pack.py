@@ -7,7 +7,7 @@ import pytest
 
 import swiftrt_amd as srt
 from tests import helpers as H
-from tests.test_gpu_canaries import NAN_BITS, run_matmul_case
+from tests.test_gpu_canaries import NAN_BITS, pin, run_matmul_case
 from tests.test_gpu_matmul import query_kernel
 
 pytestmark = pytest.mark.gpu
@@ -60,6 +60,26 @@ def test_results_with_ragged_rows(tmp_path, dt, M, N, K, batch):
                                         "mfma_128x128", "mfma_64x64"), 910 + N, with_bias=bias, relu=relu))
     assert ran == {"mfma_256x256_m16_k64", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128", "mfma_128x128",
                    "mfma_64x64"}
+
+
+@pytest.mark.parametrize("act,coef", [("sigmoid", 0.0), ("tanh", 0.0), ("elu", 0.7), ("clippedRelu", 0.5)])
+@pytest.mark.parametrize("dt", [H.BF16, H.F16])
+def test_ragged_rows_under_every_activation(tmp_path, dt, act, coef):
+    """The kernels' ragged and whole forms differ in how they store: the first 257 of 264 columns, bit for bit."""
+    M, N, WIDE, K, code = 136, 257, 264, 512, srt.ActivationType[act]
+    g = H.rng(940)
+    for plan, ta in (("mfma_256x256_m16_k64", False), ("mfma_256x256_m16_k64", True), ("mfma_128x256_m16_k64", False),
+                     ("mfma_256x128_m16_k64", True), ("mfma_128x128_m16_k128", False), ("mfma_128x128_m16_k128", True)):
+        a = srt.Tensor(H.encode(g.standard_normal((K, M) if ta else (M, K)), dt))
+        w, bias = H.encode(g.standard_normal((WIDE, K)) / 16, dt), H.encode(g.standard_normal(WIDE), dt)
+        results = []
+        for n in (N, WIDE):
+            out, b = srt.Tensor(shape=[M, n], dtype=w.dtype), srt.Tensor(w[:n])
+            pin(tmp_path, dt, M, n, K, 1, (2 if ta else 1) | 4 | 16 | (64 if n % 8 == 0 else 0), {10, 1 | (int(code) << 1)}, plan)
+            assert query_kernel(a, ta, b, True, out) == plan
+            srt.current_queue().matmul(a, ta, b, True, out, bias=srt.Tensor(bias[:n]), activation=code, coef=coef)
+            results.append(out.array().view(np.uint16))
+        assert np.array_equal(results[0], results[1][:, :N]), (plan, ta)
 
 
 def test_the_choice_for_ragged_rows():
