@@ -440,6 +440,10 @@ class LSTMCell:
     def __call__(self, x, cell, hidden):
         gate_input = concatenate(x, hidden, axis=1)
         fused = matmul(gate_input, self.fused_weight, bias=self.fused_bias)
+        if cell.rank != 2 or fused.shape != (cell.shape[0], 4 * cell.shape[1]):
+            # gates broadcast against the cell's shape, or a weight with columns past the fourth part: operator by operator
+            new_cell = (cell * sigmoid(self.part(2, fused)) + sigmoid(self.part(0, fused)) * tanh(self.part(1, fused)))
+            return new_cell, tanh(new_cell) * sigmoid(self.part(3, fused))
         new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
         new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
         current_queue().lstm_gates(fused, cell, new_cell, new_hidden)

@@ -53,6 +53,22 @@ def test_gates_on_views_and_refusals():
 
 
 @pytest.mark.parametrize("dt", DTS)
+def test_cells_the_gate_kernel_does_not_take(dt):
+    """A weight with columns past the fourth part; one row of gates under several rows of state, or under a stack of them."""
+    g = H.rng(6)
+    make = lambda *shape: srt.Tensor(H.encode(g.standard_normal(shape), dt))   # noqa: E731
+    h = 24
+    for columns, batch, state in ((4 * h + 3, 5, (5, h)), (4 * h, 1, (5, h)), (4 * h, 5, (3, 5, h))):
+        weight, bias, x, hidden, cell = make(16 + h, columns), make(columns), make(batch, 16), make(batch, h), make(*state)
+        new_cell, new_hidden = srt.LSTMCell(weight, bias)(x, cell, hidden)
+        fused = srt.matmul(srt.concatenate(x, hidden, 1), weight, bias=bias)
+        part = [fused[:, i * h:(i + 1) * h] for i in range(4)]
+        want_cell = cell * srt.sigmoid(part[2]) + srt.sigmoid(part[0]) * srt.tanh(part[1])
+        assert new_cell.shape == state and np.array_equal(bits(new_cell), bits(want_cell))
+        assert np.array_equal(bits(new_hidden), bits(srt.tanh(want_cell) * srt.sigmoid(part[3])))
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("shapes,axis", [(((4, 8), (4, 16)), 1), (((3, 5), (3, 7)), 1), (((5, 9), (2, 9)), 0),
                                          (((2, 3, 8), (2, 4, 8)), 1), (((1024, 3000), (1024, 3000)), 1), (((4, 0), (4, 3)), 1)])
 def test_concatenate(dt, shapes, axis):
