@@ -538,10 +538,19 @@ hipError_t launch_lstm_gates(GateProblem p, hipStream_t stream) {
   auto go = [&](auto width) {
     constexpr int W = decltype(width)::value;
     p.columns /= W;
-    const unsigned long long lanes = (unsigned long long)p.rows * p.columns;
-    if (lanes > 0x7fffffffull) return hipErrorNotSupported;
-    hipLaunchKernelGGL((lstm_gates_kernel<T, W>), dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, stream, p);
-    return launch_status(stream);
+    // the lanes of a launch are counted in 31 bits: a larger cell goes in pieces of whole rows
+    const uint32_t rows = p.rows, most = 0x7fffffffu / p.columns;
+    hipError_t e = hipSuccess;
+    for (uint32_t done = 0; done < rows && e == hipSuccess; done += p.rows) {
+      auto at = [&](const void* base, long long row) { return (char*)base + (long long)done * row * (long long)sizeof(typename T::storage); };
+      GateProblem q = p;
+      q.rows = p.rows = rows - done < most ? rows - done : most;
+      q.gates = at(p.gates, p.gates_row); q.cell = at(p.cell, p.cell_row);
+      q.new_cell = at(p.new_cell, p.new_cell_row); q.new_hidden = at(p.new_hidden, p.new_hidden_row);
+      hipLaunchKernelGGL((lstm_gates_kernel<T, W>), dim3((q.rows * q.columns + 255) / 256), dim3(256), 0, stream, q);
+      e = launch_status(stream);
+    }
+    return e;
   };
   const bool dense = p.gates_col == 1 && p.cell_col == 1 && p.new_cell_col == 1 && p.new_hidden_col == 1;
   const bool whole = p.columns % V == 0 && p.part % V == 0 && p.gates_row % V == 0 && p.cell_row % V == 0 && p.new_cell_row % V == 0 &&

@@ -37,6 +37,23 @@ def test_gates_are_the_unfused_chain(dt, b, h):
     assert np.array_equal(bits(nc), bits(want_cell)) and np.array_equal(bits(nh), bits(want_hidden))
 
 
+def test_gates_beyond_31_bits_of_lanes():
+    """The odd width goes lane per element; 2^31 of them take a second launch.  One value everywhere but in the last row."""
+    rows, h = 0x80000000 // 1023 + 2, 1023
+    q = srt.current_queue()
+    filled = lambda shape, value: srt.filled(shape, value, np.uint16)          # noqa: E731
+    gates, cell = filled([rows, 4 * h], 0.5), filled([rows, h], 0.25)
+    q.fill(last := srt.Tensor(shape=[1, 4 * h], dtype=np.uint16), -1.0)
+    q.copy(last, gates[rows - 1:rows])
+    nc, nh = srt.Tensor(shape=[rows, h], dtype=np.uint16), srt.Tensor(shape=[rows, h], dtype=np.uint16)
+    q.lstm_gates(gates, cell, nc, nh)
+    for at in (0, rows // 2, rows - 2, rows - 1):
+        row = slice(at, at + 1)
+        dense = lambda t: (o := srt.Tensor(shape=[1, t.shape[1]], dtype=np.uint16), q.copy(t[row], o))[0]   # noqa: E731
+        want_cell, want_hidden = unfused(dense(gates), dense(cell))
+        assert np.array_equal(bits(dense(nc)), bits(want_cell)) and np.array_equal(bits(dense(nh)), bits(want_hidden)), at
+
+
 def test_gates_on_views_and_refusals():
     g = H.rng(5)
     wide = srt.Tensor(g.standard_normal((9, 200)).astype(np.float32))
