@@ -313,14 +313,17 @@ int mfma_select(const GemmProblem& p);
 int mfma_config(const GemmProblem& p, int tile);
 const char* mfma_name(int config);
 hipError_t launch_mfma(const GemmProblem& p, int config, hipStream_t stream);
-// Operands copied into aligned, zero-padded workspace first (gemm_pack.hip), and the plan the heuristic picks for the copies.
+// Operands copied into aligned, zero-padded workspace first (gemm_pack.hip): whether they can be, whether that is the choice, and
+// the launch, which runs the plan the heuristic picks for the copies.
+bool pack_supported(const GemmProblem& p);
 bool pack_preferred(const GemmProblem& p);
 double packed_us(const GemmProblem& p);   // estimate of an fp32 problem's time that way, copies included (0: it cannot)
 double f32_ring_us(const GemmProblem& p);   // and of the ring kernel's plans alone
 enum class F32Any { kTile, kSplitK, kParts, kPacked };
 F32Any f32_any_choice(const GemmProblem& p, double packed_us);   // for a problem the ring kernel does not read
 hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErrorOutOfMemory: no workspace, nothing was launched
-// 32 x 32 tiles whose waves split k (gemm_waves.hip): whether that is the choice, and the launch.
+// 32 x 32 tiles whose waves split k (gemm_waves.hip): whether they read the problem, whether they are the choice, and the launch.
+bool waves_supported(const GemmProblem& p);
 bool waves_preferred(const GemmProblem& p);
 hipError_t launch_waves(const GemmProblem& p, hipStream_t stream);
 hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream);

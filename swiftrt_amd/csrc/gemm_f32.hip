@@ -812,11 +812,6 @@ hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_
     dim3 grid((p.N + 31) / 32, (p.M + 31) / 32, p.batch);
     hipLaunchKernelGGL(gemm_f32_mfma_splitk_kernel, grid, dim3(256), 0, stream, p);
   } else {
-    if (pack_preferred(p)) {
-      const hipError_t e = launch_packed(p, stream);
-      if (e != hipErrorOutOfMemory) return e;
-      (void)hipGetLastError();   // no room for the copies (nothing was launched): the operands as they are
-    }
     // the 128 x 128 tile once it gives every CU a workgroup, the 64 x 64 tile below that
     const long long tiles128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
     if (tiles128 >= 256) {

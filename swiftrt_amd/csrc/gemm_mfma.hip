@@ -1243,12 +1243,6 @@ const char* mfma_name(int config) {
 hipError_t launch_mfma(const GemmProblem& p, int config, hipStream_t stream) {
   const int tile = config >> 2;
   const bool a_kc = (config & 2) != 0, b_kc = (config & 1) != 0;
-  if ((tile == 3 || tile == 8) && waves_preferred(p)) return launch_waves(p, stream);
-  if ((tile == 7 || tile == 8) && pack_preferred(p)) {
-    const hipError_t e = launch_packed(p, stream);
-    if (e != hipErrorOutOfMemory) return e;
-    (void)hipGetLastError();   // no room for the copies (nothing was launched): the operands as they are
-  }
   if (p.dtype == srtReal16BF) return launch_tile<BF16>(p, tile, a_kc, b_kc, stream);
   return launch_tile<F16>(p, tile, a_kc, b_kc, stream);
 }

@@ -138,13 +138,18 @@ bool plan_pack(const GemmProblem& p, PackPlan* t) {
 
 }  // namespace
 
+bool pack_supported(const GemmProblem& p) {
+  PackPlan t;
+  return !p.row_padding && plan_pack(p, &t) && (p.dtype != srtReal32F || f32_ring_fits(t.q));
+}
+
 double packed_us(const GemmProblem& p) {
   PackPlan t;
   if (p.dtype != srtReal32F || p.row_padding || !plan_pack(p, &t) || !f32_ring_fits(t.q)) return 0.0;
   return 5.0 + (double)(t.bytes_a + t.bytes_b) / 3.0e6 + (double)p.batch * p.M * p.N * 4.0 / 8.0e6 + f32_ring_us(t.q);
 }
 
-// Whether copying pays (fp32: f32_any_choice in gemm_f32.hip).  16-bit types: always once the problem fills the device with
+// Whether copying 16-bit operands pays (fp32: f32_any_choice in gemm_f32.hip): always once the problem fills the device with
 // 128 x 128 tiles; below that by two estimates in microseconds.
 //   as it is   4 + its 64-deep stages at 1.0 (both operands contiguous along k), 2.5 (B along n) or 5 (A along m, or views
 //              without a unit stride), once per 512 tiles of 64 x 64
@@ -156,8 +161,7 @@ double packed_us(const GemmProblem& p) {
 // 1520 / 177; 2048 x 50257 x 768 x . W 880 / 186 (34 of them the copy of W).
 bool pack_preferred(const GemmProblem& p) {
   PackPlan t;
-  if (p.row_padding || !plan_pack(p, &t)) return false;
-  if (p.dtype == srtReal32F) return !f32_ring_fits(p) && f32_any_choice(p, packed_us(p)) == F32Any::kPacked;
+  if (p.dtype == srtReal32F || p.row_padding || !plan_pack(p, &t)) return false;
   auto tiles = [&](int s) { return (double)((p.M + s - 1) / s) * ((p.N + s - 1) / s) * p.batch; };
   const double cus = compute_units();
   if (tiles(128) >= cus) return true;

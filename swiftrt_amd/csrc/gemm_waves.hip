@@ -240,6 +240,8 @@ bool fits(const GemmProblem& p) {
 
 }  // namespace
 
+bool waves_supported(const GemmProblem& p) { return fits(p); }
+
 // Whether these tiles are the choice, by two estimates in microseconds (256 units):
 //   here     3 + rounds of a unit's tiles at 128 K bytes each: 60 bytes/ns up to 300 KB of a unit, 50 for one tile alone, 42 else;
 //            0.55 a tile at least (its fill, sums and store).  Measured / estimated: 512 x 512 x 4096 10.8-14.2 / 13.5, 1024 x 1024 x

@@ -114,14 +114,14 @@ srtStatus build_problem(const void* a, const srtTensorDescriptor* ad, int tA,
 // (the role of ExecutionPlanCache / ExecutionPlanner, platform/common/ExecutionPlanner.swift:20-29,
 // and of the empty CudaMatmul2.tune, platform/cuda/functions/CudaMatmul.swift:112-120).
 enum Plan { kPlanGeneric, kPlanSkinny, kPlanRing256, kPlanMfma128, kPlanMfma64, kPlanF32Tile64, kPlanF32SplitK,
-            kPlanKc64, kPlanM16, kPlanSplitK, kPlanM16H, kPlanAny128, kPlanAny64, kPlanM16D, kPlanM16DTail, kPlanM16DSplit, kPlanM16DH, kPlanM16DN, kPlanM16Q, kPlanF32Parts, kPlanF32Ring, kPlanF32Ring64x128, kPlanF32Ring64, kPlanCount };
+            kPlanKc64, kPlanM16, kPlanSplitK, kPlanM16H, kPlanAny128, kPlanAny64, kPlanM16D, kPlanM16DTail, kPlanM16DSplit, kPlanM16DH, kPlanM16DN, kPlanM16Q, kPlanF32Parts, kPlanF32Ring, kPlanF32Ring64x128, kPlanF32Ring64, kPlanWaves, kPlanCopied, kPlanCount };
 
 const char* const kPlanNames[kPlanCount] = {"generic", "skinny", "mfma_256x256", "mfma_128x128", "mfma_64x64",
                                             "f32_mfma_64x64", "f32_mfma_splitk", "mfma_256x256_k64",
                                             "mfma_256x256_m16", "mfma_256x256_splitk", "mfma_128x256_m16",
                                             "mfma_128x128_any", "mfma_64x64_any", "mfma_256x256_m16_k64",
                                             "mfma_256x256_m16_k64_tail", "mfma_256x256_m16_k64_split",
-                                            "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128", "f32_mfma_128x128_parts", "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring"};
+                                            "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128", "f32_mfma_128x128_parts", "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring", "mfma_32x32_waves", "copied"};
 
 bool plan_supported(const GemmProblem& p, Plan plan) {
   switch (plan) {
@@ -147,14 +147,38 @@ bool plan_supported(const GemmProblem& p, Plan plan) {
     case kPlanF32Ring64: return srt::f32_ring_fits(p);
     case kPlanF32Tile64: return srt::f32_mfma_supported(p) && (p.M + 63) / 64 <= 65535;
     case kPlanF32SplitK: return srt::f32_mfma_supported(p);
+    case kPlanWaves: return srt::waves_supported(p);
+    case kPlanCopied: return srt::pack_supported(p);
     default: return srt::generic_supported(p);
   }
 }
 
-Plan heuristic_plan(const GemmProblem& p) {
-  // 16-bit problems of few tiles off the 16-byte rules: 32 x 32 tiles whose waves split k (the launches of the 64 x 64 plans pick
-  // them by this rule; aligned operands keep the choices below and run them where that is the 64 x 64 plan)
-  if (srt::waves_preferred(p) && srt::mfma_config(p, 3) == 0) return kPlanAny64;
+// The plan of the tile that mfma_select picks (kPlanGeneric: none qualifies).  copies: operands off the 16-byte rules may be
+// copied into workspace.
+Plan tile_plan(const GemmProblem& p, bool copies) {
+  const int c = srt::mfma_select(p);
+  if (c == 0) return kPlanGeneric;
+  switch (c >> 2) {
+    case 1: return kPlanRing256;
+    case 2: return kPlanMfma128;
+    case 4: return kPlanKc64;
+    case 5: return kPlanM16;
+    case 6: return kPlanM16H;
+    case 7: return copies && srt::pack_preferred(p) ? kPlanCopied : kPlanAny128;
+    case 8: return copies && srt::pack_preferred(p) ? kPlanCopied : kPlanAny64;
+    case 9: return kPlanM16D;
+    case 10: return kPlanM16DTail;
+    case 12: return kPlanM16DH;
+    case 13: return kPlanM16DN;
+    case 14: return kPlanM16Q;
+    default: return srt::waves_preferred(p) ? kPlanWaves : kPlanMfma64;
+  }
+}
+
+Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
+  // 16-bit problems of few tiles off the 16-byte rules: 32 x 32 tiles whose waves split k (aligned operands keep the choices
+  // below and run them where that is the 64 x 64 plan)
+  if (srt::waves_preferred(p) && srt::mfma_config(p, 3) == 0) return kPlanWaves;
   // one round of 128 x 128 tiles holds the problem (64 rows or more) and its k loop is not worth cutting
   if (srt::mfma_prefers_quarter(p)) return kPlanM16Q;
   if (srt::skinny_supported(p) && srt::skinny_preferred(p)) return kPlanSkinny;
@@ -176,24 +200,8 @@ Plan heuristic_plan(const GemmProblem& p) {
   // few 256 x 256 tiles and a long k loop: K split over the idle compute units
   if (srt::mfma_prefers_splitk(p)) return kPlanSplitK;
   if (streams) return kPlanSkinny;
-  const int c = srt::mfma_select(p);
-  if (c) {
-    switch (c >> 2) {
-      case 1: return kPlanRing256;
-      case 2: return kPlanMfma128;
-      case 4: return kPlanKc64;
-      case 5: return kPlanM16;
-      case 6: return kPlanM16H;
-      case 7: return kPlanAny128;
-      case 8: return kPlanAny64;
-      case 9: return kPlanM16D;
-      case 10: return kPlanM16DTail;
-      case 12: return kPlanM16DH;
-      case 13: return kPlanM16DN;
-      case 14: return kPlanM16Q;
-      default: return kPlanMfma64;
-    }
-  }
+  const Plan tile = tile_plan(p, copies);
+  if (tile != kPlanGeneric) return tile;
   if (srt::f32_mfma_supported(p)) {
     // what the ring kernel reads: the fastest of its three tile shapes, the k range in parts and the 32 x 32 kernel,
     // by their time estimates
@@ -206,12 +214,13 @@ Plan heuristic_plan(const GemmProblem& p) {
         default: return kPlanF32SplitK;
       }
     }
-    switch (srt::f32_any_choice(p, srt::packed_us(p))) {
+    switch (srt::f32_any_choice(p, copies ? srt::packed_us(p) : 0.0)) {
       // launch-sized problems and up to 64 rows: 32 x 32 tiles whose waves split K
       case srt::F32Any::kSplitK: return kPlanF32SplitK;
       // a single matrix of too few 128 x 128 tiles for the device: its k range in parts on those tiles
       case srt::F32Any::kParts: return kPlanF32Parts;
-      // (operands the ring kernel would read once copied into its layout are copied by the launch)
+      // operands the ring kernel reads once copied into its layout
+      case srt::F32Any::kPacked: return kPlanCopied;
       default: return kPlanF32Tile64;
     }
   }
@@ -242,24 +251,26 @@ hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
     case kPlanF32Ring64: return srt::launch_f32_ring(p, stream, 2);
     case kPlanF32Tile64: return srt::launch_f32_mfma_variant(p, false, stream);
     case kPlanF32SplitK: return srt::launch_f32_mfma_variant(p, true, stream);
+    case kPlanWaves: return srt::launch_waves(p, stream);
+    case kPlanCopied: return srt::launch_packed(p, stream);
     default: return srt::launch_generic(p, stream);
   }
 }
 
+// A plan that finds no room for its workspace (nothing that matters was launched) gives way to the plan that needs none.
 hipError_t launch_or_fall_back(const GemmProblem& p, Plan plan, hipStream_t stream) {
-  hipError_t e = launch_plan(p, plan, stream);
-  if ((plan == kPlanSplitK || plan == kPlanM16DTail) && e == hipErrorOutOfMemory) {
-    // no room for the workspace (nothing was launched): the plan that needs none
-    (void)hipGetLastError();
-    const int c = plan == kPlanM16DTail ? srt::mfma_config(p, 9) : srt::mfma_select(p);
-    e = c ? srt::launch_mfma(p, c, stream) : srt::launch_generic(p, stream);
+  const hipError_t e = launch_plan(p, plan, stream);
+  if (e != hipErrorOutOfMemory) return e;
+  Plan next;
+  switch (plan) {
+    case kPlanSplitK: next = tile_plan(p, false); break;
+    case kPlanM16DTail: next = kPlanM16D; break;
+    case kPlanF32Parts: next = srt::f32_ring_fits(p) ? kPlanF32Ring : kPlanF32Tile64; break;   // the whole k range per tile
+    case kPlanCopied: next = heuristic_plan(p, false); break;   // the operands as they are
+    default: return e;
   }
-  if (plan == kPlanF32Parts && e == hipErrorOutOfMemory) {
-    // likewise for the fp32 parts: the whole k range per tile, no workspace
-    (void)hipGetLastError();
-    e = srt::f32_ring_fits(p) ? srt::launch_f32_ring(p, stream, 0) : srt::launch_f32_mfma_variant(p, false, stream);
-  }
-  return e;
+  (void)hipGetLastError();
+  return launch_plan(p, plan_supported(p, next) ? next : kPlanGeneric, stream);
 }
 
 struct PlanKey {
@@ -524,7 +535,7 @@ srtStatus srtMatmulTune(const void* a, const srtTensorDescriptor* aDesc, int32_t
     if (plan == kPlanGeneric && fallback != kPlanGeneric && 2.0 * p.M * p.N * p.K * p.batch > 1e9) continue;
     const int warm = 2, reps = 8;
     for (int i = 0; i < warm && err == hipSuccess; ++i) err = launch_plan(p, plan, hs);
-    if ((plan == kPlanSplitK || plan == kPlanM16DTail || plan == kPlanF32Parts) && err == hipErrorOutOfMemory) {
+    if ((plan == kPlanSplitK || plan == kPlanM16DTail || plan == kPlanF32Parts || plan == kPlanCopied) && err == hipErrorOutOfMemory) {
       // no room for this plan's workspace (nothing was launched): it is not a candidate, as in run()
       (void)hipGetLastError();
       err = hipSuccess;
@@ -544,7 +555,7 @@ srtStatus srtMatmulTune(const void* a, const srtTensorDescriptor* aDesc, int32_t
   if (best_ms < 0.0f) return srtErrorNotSupported;   // no kernel qualifies: the caller's CPU path
   plan_cache().put(key_of(p), best);
   // leave `out` written by the chosen plan
-  err = launch_plan(p, best, hs);
+  err = launch_or_fall_back(p, best, hs);
   if (chosen && chosenCapacity) std::snprintf(chosen, chosenCapacity, "%s", kPlanNames[best]);
   return srt::from_hip(err);
 }

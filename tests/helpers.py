@@ -1,4 +1,8 @@
-"""Shared helpers for the parity tests: seeded inputs, storage codecs, error metrics."""
+"""Shared helpers for the parity tests: seeded inputs, storage codecs, error metrics, pinned kernel plans."""
+import contextlib
+import os
+import tempfile
+
 import numpy as np
 
 from oracle import srt_oracle as ora
@@ -9,6 +13,21 @@ NP_STORAGE = {F32: np.float32, F16: np.float16, BF16: np.uint16}
 TOL = {F32: 1e-5, F16: 2e-2, BF16: 2e-2}
 # unit roundoff of the stored result, used for the tighter element-wise bound
 ULP = {F32: 2.0 ** -24, F16: 2.0 ** -11, BF16: 2.0 ** -8}
+
+
+@contextlib.contextmanager
+def pinned(plan, dt, M, N, K, layout, epilogues=(10,), batch=1):
+    """Products of this key run on `plan` inside the block (layout and epilogue codes: srt_hip.h, plan / tune cache)."""
+    import swiftrt_amd as srt
+    with tempfile.TemporaryDirectory() as d:
+        path = os.path.join(d, "plans.txt")
+        with open(path, "w") as f:
+            f.writelines(f"{dt} {M} {N} {K} {batch} {layout} {e} {plan}\n" for e in epilogues)
+        srt.PlanCache.load(path)
+    try:
+        yield plan
+    finally:
+        srt.PlanCache.clear()
 
 
 def rng(seed):

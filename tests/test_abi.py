@@ -361,7 +361,7 @@ def test_kernel_selection_is_queryable_without_gpu():
     assert query(native.REAL16BF, 512, 4096, 256) == "mfma_128x128_m16_k128"              # short k loops too (two 128-deep units)
     assert query(native.REAL16BF, 512, 4096, 192) == "mfma_128x256_m16"                   # (8.4 us against 10.0 in whole tiles)
     assert query(native.REAL16F, 256, 256, 256, tb=True) == "mfma_128x128_m16_k128"
-    assert query(native.REAL16F, 256, 256, 192, tb=True) == "mfma_64x64"
+    assert query(native.REAL16F, 256, 256, 192, tb=True) == "mfma_32x32_waves"
     assert query(native.REAL16BF, 1, 14336, 4096, tb=True) == "skinny"
     assert query(native.REAL16BF, 32, 14336, 4096, tb=True) == "skinny"
     # 33..64 rows: the streaming kernel when its workgroups make one round that fills the device
@@ -421,18 +421,20 @@ def test_kernel_selection_is_queryable_without_gpu():
     assert query_batched(native.REAL16BF, 4, 256, 256, 4096, ta=True) == "mfma_128x128_m16_k128"       # 16 quarter tiles (24 us against 40 shared: a batch has no split-K)
     assert query_batched(native.REAL16BF, 16, 256, 256, 2048, ta=True, tb=True) == "mfma_128x128_m16_k128"
     assert query_batched(native.REAL16BF, 4, 128, 128, 4096, tb=True) == "mfma_128x128_m16_k128"
-    assert query_batched(native.REAL16BF, 4, 128, 128, 4032, tb=True) == "mfma_64x64"                  # mostly padding, both k-contiguous
+    assert query_batched(native.REAL16BF, 4, 128, 128, 4032, tb=True) == "mfma_32x32_waves"                  # mostly padding, both k-contiguous
     assert query_batched(native.REAL16BF, 16, 512, 512, 4096) == "mfma_256x256_m16_k64_tail"           # 256 quarter tiles of small problems: operand traffic
     assert query_batched(native.REAL16BF, 64, 256, 256, 1024, tb=True) == "mfma_128x256_m16_k64"           # 128 half tiles in one round
     assert query_batched(native.REAL16BF, 64, 256, 1024, 256, tb=True) == "mfma_256x256_m16_k64"       # 512 half tiles: whole tiles
     assert query_batched(native.REAL16BF, 64, 384, 384, 4096, tb=True) == "mfma_256x256_k64"           # a last row of tiles half padding
     assert query_batched(native.REAL16BF, 28, 8, 88, 7680) == "skinny"                                 # ahead of sharing padded tiles
     assert query_batched(native.REAL16BF, 41, 1480, 72, 1248, tb=True) == "mfma_256x256_k64"           # a device's worth of padded whole tiles
-    assert query_batched(native.REAL16BF, 36, 8, 768, 328, tb=True) == "mfma_64x64"                    # 864 streaming workgroups: not worth it
-    # 16-bit operands that miss the 16-byte rules: the matrix-core kernel with element-wise staging
-    assert query(native.REAL16BF, 33, 33, 33) == "mfma_64x64_any"
-    assert query(native.REAL16BF, 64, 64, 64, align=2) == "mfma_64x64_any"            # misaligned view
-    assert query(native.REAL16F, 2048, 50257, 768) == "mfma_128x128_any"              # odd row pitch of B and C
+    assert query_batched(native.REAL16BF, 36, 8, 768, 328, tb=True) == "mfma_32x32_waves"                    # 864 streaming workgroups: not worth it
+    # 16-bit operands that miss the 16-byte rules: tiles whose waves split k, copies into aligned workspace, staging kernels
+    assert query(native.REAL16BF, 33, 33, 33) == "mfma_32x32_waves"
+    assert query(native.REAL16BF, 64, 64, 64, align=2) == "mfma_32x32_waves"            # misaligned view
+    assert query(native.REAL16F, 2048, 50257, 768) == "copied"                        # odd row pitch of B and C
+    assert query(native.REAL16BF, 300, 200, 5) == "mfma_64x64_any"                    # a k loop shorter than a vector
+    assert query(native.REAL32F, 1000, 2000, 1001) == "copied"
     assert query(native.REAL32F, 512, 512, 512) in ("generic", "f32_mfma")
     # operands of 1 Gi elements or more: halves of M (N for a k-contiguous B, the batch first) that the
     # 256 x 256 kernels' 32-bit offsets reach; a k walk out of reach keeps the small tiles
@@ -469,7 +471,8 @@ def test_kernel_selection_answers_for_any_problem():
     buf = ctypes.create_string_buffer(64)
     known = {"empty", "generic", "skinny", "f32_mfma", "mfma_256x256", "mfma_128x128", "mfma_64x64", "mfma_256x256_k64",
              "mfma_256x256_m16", "mfma_256x256_splitk", "mfma_128x256_m16", "mfma_128x128_any", "mfma_64x64_any",
-             "mfma_256x256_m16_k64", "mfma_256x256_m16_k64_tail", "mfma_256x256_m16_k64_split", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128"}
+             "mfma_256x256_m16_k64", "mfma_256x256_m16_k64_tail", "mfma_256x256_m16_k64_split", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128",
+             "mfma_32x32_waves", "copied"}
 
     def logu(lo, hi):
         return int(np.exp(g.uniform(np.log(lo), np.log(hi))))
@@ -503,7 +506,7 @@ def test_kernel_selection_answers_for_any_problem():
         name = buf.value.decode()
         assert name.split("/")[0] in known and name.split("/")[-1] in known | {"pieces"}, name
         seen.add(name.split("/")[0])
-    assert {"skinny", "mfma_64x64", "mfma_256x256_m16", "mfma_128x256_m16", "f32_mfma"} <= seen
+    assert {"skinny", "mfma_64x64", "mfma_256x256_m16", "mfma_128x256_m16", "f32_mfma", "mfma_32x32_waves", "copied"} <= seen
 
 
 def test_tensor_layout_and_views():

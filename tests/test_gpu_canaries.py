@@ -24,8 +24,8 @@ NAN_BITS = {np.dtype(np.uint16): 0x7FC0, np.dtype(np.float16): 0x7E00, np.dtype(
 
 ALL_PLANS_16 = ("mfma_256x256_m16_k64", "mfma_256x256_m16_k64_tail", "mfma_256x256_m16_k64_split", "mfma_256x256_m16", "mfma_256x256", "mfma_256x256_k64",
                 "mfma_256x256_splitk", "mfma_128x256_m16", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128", "mfma_128x128", "mfma_64x64", "mfma_128x128_any",
-                "mfma_64x64_any", "skinny", "generic")
-ALL_PLANS_32 = ("f32_mfma_64x64", "f32_mfma_splitk", "f32_mfma_128x128_parts", "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring", "generic")
+                "mfma_64x64_any", "mfma_32x32_waves", "copied", "skinny", "generic")
+ALL_PLANS_32 = ("f32_mfma_64x64", "f32_mfma_splitk", "f32_mfma_128x128_parts", "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring", "copied", "generic")
 
 
 @pytest.fixture(autouse=True)
@@ -164,13 +164,12 @@ def test_quarter_tile_keeps_inside_small_and_batched_views(tmp_path):
 
 
 def test_plans_for_unaligned_views_keep_inside(tmp_path):
-    """N not a multiple of 8, odd row pitches and bases off a 16-byte boundary: the element-wise staging kernels
-    and the generic kernel (the 16-byte store paths do not qualify and must not be chosen)."""
+    """N not a multiple of 8, odd row pitches and bases off a 16-byte boundary: the element-wise staging kernels, the
+    wave-split tiles, the copies and the generic kernel (the 16-byte store paths do not qualify and must not be chosen)."""
     for (M, N, K, left, right) in [(200, 265, 72, 3, 2), (130, 72, 136, 1, 4), (257, 129, 65, 8, 3)]:
         for ta, tb in [(False, False), (True, False), (False, True)]:
             ran = run_matmul_case(tmp_path, H.BF16, M, N, K, 1, ta, tb, ALL_PLANS_16, 740 + M, left=left, right=right)
-            assert set(ran) <= {"mfma_128x128_any", "mfma_64x64_any", "generic"} and "generic" in ran, ran
-            assert "mfma_64x64_any" in ran, ran
+            assert set(ran) == {"mfma_128x128_any", "mfma_64x64_any", "mfma_32x32_waves", "copied", "generic"}, ran
 
 
 def test_streaming_kernel_keeps_inside_including_its_56_column_tiles(tmp_path):
@@ -205,7 +204,7 @@ def test_nothing_outside_an_operand_view_reaches_a_sum(tmp_path):
         for ta, tb in [(False, False), (True, False), (False, True), (True, True)]:
             ran = run_matmul_case(tmp_path, H.BF16, M, N, K, 1, ta, tb, ALL_PLANS_16, 820 + M, left=left, right=right,
                                   operand_sentinel=NAN_BITS)
-            assert "mfma_64x64_any" in ran, ran
+            assert {"mfma_64x64_any", "mfma_128x128_any", "mfma_32x32_waves", "copied"} <= set(ran), ran
     for (M, N, K, tb) in [(32, 14336, 256, True), (24, 14328, 136, True), (8, 1000, 520, True), (8, 1096, 264, False), (40, 2056, 136, False)]:
         for dt in (H.BF16, H.F32):
             if dt == H.F32 and M > 32:

@@ -538,18 +538,24 @@ def test_unaligned_operands_run_on_the_matrix_cores(dt):
         b = r.integers(-3, 4, (N, K) if tb else (K, N)).astype(np.float32)
         bias = r.integers(-3, 4, N).astype(np.float32)
         at, bt, biast = srt.Tensor(H.encode(a, dt)), srt.Tensor(H.encode(b, dt)), srt.Tensor(H.encode(bias, dt))
-        out = srt.Tensor(shape=[M, N], dtype=at.dtype)
-        assert query_kernel(at, ta, bt, tb, out) == ("mfma_128x128_any" if M > 2000 else "mfma_64x64_any")
-        srt.current_queue().matmul(at, ta, bt, tb, out, bias=biast, activation=relu)
         exact = np.maximum((a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64) + bias[None, :], 0)
+        out = srt.Tensor(shape=[M, N], dtype=at.dtype)
+        assert query_kernel(at, ta, bt, tb, out) == ("copied" if M > 2000 else "mfma_32x32_waves")   # the choice
+        with H.pinned("mfma_128x128_any" if M > 2000 else "mfma_64x64_any", dt, M, N, K, (2 if ta else 1) | (4 if tb else 8) | 16,
+                      (10, 1 | (int(relu) << 1))) as plan:
+            assert query_kernel(at, ta, bt, tb, out) == plan
+            srt.current_queue().matmul(at, ta, bt, tb, out, bias=biast, activation=relu)
+            assert np.array_equal(out.array().view(np.uint16), H.encode(exact.astype(np.float32), dt).view(np.uint16)), (M, N, K, ta, tb)
+        srt.current_queue().matmul(at, ta, bt, tb, out, bias=biast, activation=relu)
         assert np.array_equal(out.array().view(np.uint16), H.encode(exact.astype(np.float32), dt).view(np.uint16)), (M, N, K, ta, tb)
     # views: both strides non-unit, odd starts; then a batch of odd-pitch matrices
     big_a = r.integers(-3, 4, (300, 200)).astype(np.float32)
     big_b = r.integers(-3, 4, (200, 400)).astype(np.float32)
     ta_, tb_ = srt.Tensor(H.encode(big_a, dt)), srt.Tensor(H.encode(big_b, dt))
     va, vb = ta_[1:291:2, 3:198:3], tb_[5:70, 1:391:3]
-    got = srt.matmul(va, vb)
-    assert query_kernel(va, False, vb, False, got) == "mfma_64x64_any"
+    with H.pinned("mfma_64x64_any", dt, 145, 130, 65, 16) as plan:
+        got = srt.matmul(va, vb)
+        assert query_kernel(va, False, vb, False, got) == plan
     exact = big_a[1:291:2, 3:198:3].astype(np.float64) @ big_b[5:70, 1:391:3].astype(np.float64)
     assert np.array_equal(got.array().view(np.uint16), H.encode(exact.astype(np.float32), dt).view(np.uint16))
     x = r.integers(-3, 4, (3, 70, 45)).astype(np.float32)
@@ -561,7 +567,8 @@ def test_unaligned_operands_run_on_the_matrix_cores(dt):
     a = (r.standard_normal((M, K)) / np.sqrt(K)).astype(np.float32)
     b = r.standard_normal((K, N)).astype(np.float32)
     a_st, b_st = H.encode(a, dt), H.encode(b, dt)
-    check_against_fp64(gpu_matmul(a_st, b_st, want_kernel="mfma_64x64_any"), a_st, b_st, False, False, dt)
+    with H.pinned("mfma_64x64_any", dt, M, N, K, 1 | 8 | 16) as plan:
+        check_against_fp64(gpu_matmul(a_st, b_st, want_kernel=plan), a_st, b_st, False, False, dt)
 
 
 def test_column_major_bias_broadcast_direction():

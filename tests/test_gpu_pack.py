@@ -2,17 +2,20 @@
 
 Integer operands, exact comparison (every partial sum is representable, so the kernel and its order of summation do not
 matter); operands framed by NaNs, results by a sentinel, so that a copy or a store past an edge shows."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import swiftrt_amd as srt
+from swiftrt_amd import native
 from tests import helpers as H
 from tests.test_gpu_canaries import NAN_BITS, pin, run_matmul_case
 from tests.test_gpu_matmul import query_kernel
 
 pytestmark = pytest.mark.gpu
 
-ANY = ("mfma_128x128_any", "mfma_64x64_any")
+ANY = ("copied", "mfma_128x128_any", "mfma_64x64_any")   # the copies, and the kernels that stage the operands as they are
 
 
 @pytest.fixture(autouse=True)
@@ -36,16 +39,23 @@ def test_copied_views_without_a_unit_stride_and_shared_matrices():
     a = g.integers(-2, 3, (600, 900)).astype(np.float32)
     b = g.integers(-2, 3, (900, 800)).astype(np.float32)
     at, bt = srt.Tensor(H.encode(a, H.F16)), srt.Tensor(H.encode(b, H.F16))
-    got = srt.matmul(at[1:599:2, 3:897:3], bt[2:896:3, 1:799:2])
+    av, bv = at[1:599:2, 3:897:3], bt[2:896:3, 1:799:2]
+    with H.pinned("copied", H.F16, 299, 399, 298, 16):
+        got = srt.matmul(av, bv)
+        assert query_kernel(av, False, bv, False, got) == "copied"
     want = a[1:599:2, 3:897:3].astype(np.float64) @ b[2:896:3, 1:799:2].astype(np.float64)
     assert np.array_equal(got.array(), H.encode(want.astype(np.float32), H.F16))
     # one right operand under every matrix of a batch (stride 0), odd extents
     x = g.integers(-2, 3, (6, 257, 301)).astype(np.float32)
     w = g.integers(-2, 3, (301, 515)).astype(np.float32)
     wt = srt.Tensor.repeating(srt.Tensor(H.encode(w, H.BF16)), [6, 301, 515])
-    got = srt.matmul(srt.Tensor(H.encode(x, H.BF16)), wt)
+    xt = srt.Tensor(H.encode(x, H.BF16))
     want = x.astype(np.float64) @ w.astype(np.float64)
-    assert np.array_equal(H.to64(got.array()), H.to64(H.encode(want.astype(np.float32), H.BF16)))
+    for plan in ("copied", "mfma_32x32_waves"):
+        with H.pinned(plan, H.BF16, 257, 515, 301, 1 | 8 | 16, batch=6):
+            got = srt.matmul(xt, wt)
+            assert query_kernel(xt, False, wt, False, got) == plan
+        assert np.array_equal(H.to64(got.array()), H.to64(H.encode(want.astype(np.float32), H.BF16))), plan
 
 
 # aligned operands, an odd number of result columns: every kernel that stores such rows, edges of its tile in both directions
@@ -84,7 +94,7 @@ def test_ragged_rows_under_every_activation(tmp_path, dt, act, coef):
 
 def test_the_choice_for_ragged_rows():
     for (M, N, K, kernel) in [(2048, 50257, 768, "mfma_256x256_m16_k64"), (512, 1001, 1024, "mfma_128x128_m16_k128"),
-                              (512, 1001, 200, "mfma_64x64")]:
+                              (512, 1001, 200, "mfma_32x32_waves")]:
         a, b = srt.Tensor(shape=[M, K], dtype=np.uint16), srt.Tensor(shape=[N, K], dtype=np.uint16)
         assert query_kernel(a, False, b, True, srt.Tensor(shape=[M, N], dtype=np.uint16)) == kernel
 
@@ -94,15 +104,17 @@ def test_the_choice_for_ragged_rows():
                                          (1200, 2000, 1004, 1)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 def test_copied_fp32_operands(tmp_path, M, N, K, batch, ta, tb):
-    ran = run_matmul_case(tmp_path, H.F32, M, N, K, batch, ta, tb, ("f32_mfma_64x64",), 920 + M + K, left=3, right=2,
+    ran = run_matmul_case(tmp_path, H.F32, M, N, K, batch, ta, tb, ("copied", "f32_mfma_64x64"), 920 + M + K, left=3, right=2,
                           operand_sentinel=NAN_BITS)
-    assert ran == ["f32_mfma_64x64"]
+    assert ran == ["copied", "f32_mfma_64x64"]
 
 
 def test_copied_fp32_views_without_a_unit_stride():
     g = H.rng(921)
     a = g.integers(-2, 3, (2100, 1100)).astype(np.float32)
     b = g.integers(-2, 3, (1100, 4100)).astype(np.float32)
-    got = srt.matmul(srt.Tensor(a)[1:2051, 3:1099:2], srt.Tensor(b)[2:1098:2, 1:4097:2])
+    av, bv = srt.Tensor(a)[1:2051, 3:1099:2], srt.Tensor(b)[2:1098:2, 1:4097:2]
+    got = srt.matmul(av, bv)
+    assert query_kernel(av, False, bv, False, got) == "copied"
     want = a[1:2051, 3:1099:2].astype(np.float64) @ b[2:1098:2, 1:4097:2].astype(np.float64)
     assert np.array_equal(got.array(), want.astype(np.float32))
