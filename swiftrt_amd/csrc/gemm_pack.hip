@@ -19,6 +19,10 @@ namespace srt {
 namespace {
 
 constexpr int kChunksPerLane = 4;
+// The copies of a call take at most this much, in blocks of a power of two: the allocator keeps a freed block for the next call of
+// its size, so calls of many odd shapes share a dozen blocks instead of leaving one each (two operands that the 256 x 256 kernels'
+// 32-bit offsets reach are 4 GiB; larger ones run as they are).
+constexpr size_t kCopiesMost = (size_t)4 << 30;
 
 struct PackJob {
   const void* src;
@@ -116,6 +120,12 @@ struct PackPlan {
   GemmProblem q;      // the problem over the copies, once their addresses are filled in
   PackJob a, b;
   size_t bytes_a, bytes_b;
+  size_t at_b() const { return (bytes_a + 255) / 256 * 256; }   // B's copy follows A's
+  size_t workspace() const {
+    size_t block = 256;
+    while (block < at_b() + bytes_b) block *= 2;
+    return block;
+  }
 };
 bool plan_pack(const GemmProblem& p, PackPlan* t) {
   if (p.dtype != srtReal16BF && p.dtype != srtReal16F && p.dtype != srtReal32F) return false;
@@ -133,7 +143,7 @@ bool plan_pack(const GemmProblem& p, PackPlan* t) {
   t->q.row_padding = 1;
   if (t->bytes_a) t->q.A = nullptr;   // (workspace: aligned)
   if (t->bytes_b) t->q.B = nullptr;
-  return t->bytes_a + t->bytes_b != 0;
+  return t->bytes_a + t->bytes_b != 0 && t->workspace() <= kCopiesMost;
 }
 
 }  // namespace
@@ -178,10 +188,9 @@ hipError_t launch_packed(const GemmProblem& p, hipStream_t stream) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return hipErrorOutOfMemory;
   void* workspace = nullptr;
-  const size_t at_b = (t.bytes_a + 255) / 256 * 256;
-  if (srtDeviceAllocate(&workspace, at_b + t.bytes_b, reinterpret_cast<srtStream>(stream)) != srtSuccess) return hipErrorOutOfMemory;
+  if (srtDeviceAllocate(&workspace, t.workspace(), reinterpret_cast<srtStream>(stream)) != srtSuccess) return hipErrorOutOfMemory;
   if (t.bytes_a) t.q.A = t.a.dst = workspace;
-  if (t.bytes_b) t.q.B = t.b.dst = (char*)workspace + at_b;
+  if (t.bytes_b) t.q.B = t.b.dst = (char*)workspace + t.at_b();
   auto blocks = [](const PackJob& j) { return (j.total + 256 * kChunksPerLane - 1) / (256 * kChunksPerLane); };
   const dim3 grid(blocks(t.a) + blocks(t.b));
   if (p.dtype == srtReal32F) hipLaunchKernelGGL(pack_kernel<4>, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a));

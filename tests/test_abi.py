@@ -434,6 +434,7 @@ def test_kernel_selection_is_queryable_without_gpu():
     assert query(native.REAL16BF, 64, 64, 64, align=2) == "mfma_32x32_waves"            # misaligned view
     assert query(native.REAL16F, 2048, 50257, 768) == "copied"                        # odd row pitch of B and C
     assert query(native.REAL16BF, 300, 200, 5) == "mfma_64x64_any"                    # a k loop shorter than a vector
+    assert query(native.REAL16BF, 65536, 65600, 16385, tb=True) == "mfma_128x128_any"   # copies of over 4 GiB: as they are
     assert query(native.REAL32F, 1000, 2000, 1001) == "copied"
     assert query(native.REAL32F, 512, 512, 512) in ("generic", "f32_mfma")
     # operands of 1 Gi elements or more: halves of M (N for a k-contiguous B, the batch first) that the

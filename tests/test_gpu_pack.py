@@ -118,3 +118,45 @@ def test_copied_fp32_views_without_a_unit_stride():
     assert query_kernel(av, False, bv, False, got) == "copied"
     want = a[1:2051, 3:1099:2].astype(np.float64) @ b[2:1098:2, 1:4097:2].astype(np.float64)
     assert np.array_equal(got.array(), want.astype(np.float32))
+
+
+# device-filling and small 16-bit products, fp32: the choice is the copies, and a stream under capture gives them no workspace
+@pytest.mark.parametrize("dt,M,N,K", [(H.BF16, 2049, 2051, 135), (H.F16, 2047, 2049, 257), (H.BF16, 1025, 1023, 1501),
+                                      (H.F32, 1023, 2047, 1001)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_without_workspace_the_operands_run_as_they_are(dt, M, N, K, ta, tb):
+    g, L, q = H.rng(950), native.lib(), srt.current_queue()
+    a = g.integers(-2, 3, (K, M) if ta else (M, K)).astype(np.float32)
+    b = g.integers(-2, 3, (N, K) if tb else (K, N)).astype(np.float32)
+    exact = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
+    want = H.encode(exact.astype(np.float32), dt)
+    at, bt, out = srt.Tensor(H.encode(a, dt)), srt.Tensor(H.encode(b, dt)), srt.Tensor(shape=[M, N], dtype=want.dtype)
+    assert query_kernel(at, ta, bt, tb, out) == "copied"
+    (ad, k1), (bd, k2), (od, k3) = at.descriptor(), bt.descriptor(), out.descriptor()
+
+    def call(stream):
+        native.check(L.srtMatmul(at.device_read(q), ctypes.byref(ad), int(ta), bt.device_read(q), ctypes.byref(bd), int(tb),
+                                 out.device_read_write(q), ctypes.byref(od), stream))
+    for plan in ("mfma_128x128_any", "mfma_64x64_any", "f32_mfma_64x64", "f32_mfma_splitk"):   # loaded before the capture
+        if (dt == H.F32) == plan.startswith("f32"):
+            with H.pinned(plan, dt, M, N, K, (2 if ta else 1) | (4 if tb else 8) | 16):
+                assert np.array_equal(srt.matmul(at, bt, ta, tb).array(), want), plan
+    call(q.stream)                                                                 # eager: copied
+    assert np.array_equal(out.array(), want)
+    # hipStreamCaptureModeThreadLocal; the runtime's symbols through the library that links it
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    assert L.hipStreamBeginCapture(q.stream, 1) == 0
+    try:
+        call(q.stream)
+    finally:
+        assert L.hipStreamEndCapture(q.stream, ctypes.byref(graph)) == 0
+    assert L.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        q.fill(out, 0.0)
+        assert L.hipGraphLaunch(run, q.stream) == 0
+        out.device_written()
+        assert np.array_equal(out.array(), want)
+        q.fill(out, 0.0)
+        call(q.stream)                                                             # and eager between the replays
+        assert np.array_equal(out.array(), want)
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
