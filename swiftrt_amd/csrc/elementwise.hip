@@ -74,6 +74,13 @@ struct Map {
   uint32_t inner_elements;       // extent of the innermost dimension in elements
 };
 
+// Operations of many instructions an element.
+template <typename Op>
+constexpr bool long_chain() {
+  return std::is_same_v<Op, Exp> || std::is_same_v<Op, ExpFast> || std::is_same_v<Op, Sigmoid> || std::is_same_v<Op, SigmoidFast> ||
+         std::is_same_v<Op, Tanh> || std::is_same_v<Op, TanhFast>;
+}
+
 template <typename T, int V>
 struct alignas(V * sizeof(typename T::storage)) Pack {
   typename T::storage v[V];
@@ -122,9 +129,31 @@ __device__ __forceinline__ Pack<TO, V> apply_pack(const float (&fa)[V], const fl
   return po;
 }
 
-// RAGGED: rows that are no whole number of aligned vectors (odd extents, pitches or bases): the last vector of a row is partial and
-// goes by elements, the others at element alignment.
-template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE, bool RAGGED = false>
+// `v` moved to the front by `over` elements (0 .. V - 1); what follows them is left over.
+template <int V>
+__device__ __forceinline__ void shift_front(float (&v)[V], uint32_t over) {
+#pragma unroll
+  for (int s = V / 2; s > 0; s /= 2)
+    if (over & s) {
+#pragma unroll
+      for (int i = 0; i + s < V; ++i) v[i] = v[i + s];
+    }
+}
+
+// The first V - over elements of `v`.
+template <typename T, int V>
+__device__ __forceinline__ void store_front(typename T::storage* p, const Pack<T, V>& v, uint32_t over) {
+#pragma unroll
+  for (int i = 0; i < V - 1; ++i)
+    if (i + over < (uint32_t)V) p[i] = v.v[i];
+}
+
+// RAGGED: rows that are no whole number of aligned vectors (odd extents, pitches or bases), read at element alignment.  The last,
+// partial vector of a row is read whole, from the row's last V elements, moved to the front (what it read of its neighbour's elements,
+// which that lane may be overwriting, falls off), and its `V - over` results are stored one by one.  Rows of fewer than 1000 elements (RAGGED 1) are read without the streaming hint: a line that two waves share is wanted
+// twice (bias add f32 2^24 elements in rows of 255 36 -> 28 us; 5001 x 7001 f32 add with the hint 64, without 79).  Read by elements too, one after the other, it held a launch up by 0.2 us an element (bias add bf16 1040 x 63 4.6 us; element
+// by element throughout 3.6).
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE, int RAGGED = 0>
 __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
   using SI = typename TI::storage;
   using SO = typename TO::storage;
@@ -142,7 +171,7 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
     const unsigned long long id = base + (unsigned long long)u * 256;
     if (id >= m.total) break;
     // decompose the vector id over the collapsed dimensions
-    uint32_t rest = (uint32_t)id, count = V;
+    uint32_t rest = (uint32_t)id, over = 0;   // over: elements the vector was moved back to end inside its row
     long long oa = 0, ob = 0, oo = 0;
 #pragma unroll
     for (int d = MAX_RANK - 1; d >= 0; --d) {
@@ -156,25 +185,21 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
         rest = q;
       }
       const long long scale = (d == inner) ? V : 1;
-      if (RAGGED && d == inner) count = m.inner_elements - idx * V;
+      if (RAGGED && d == inner && m.inner_elements - idx * V < (uint32_t)V) over = V - (m.inner_elements - idx * V);
       oa += (long long)idx * m.sa[d] * scale;
       ob += (long long)idx * m.sb[d] * scale;
       oo += (long long)idx * m.so[d] * scale;
     }
-    float fa[V], fb[V];
-    if (RAGGED && count < V) {
-      for (uint32_t i = 0; i < count; ++i) {
-        const float x = m.fill ? m.element : TI::to_float(a[oa + (long long)i * m.sa[inner]]);
-        const float y = m.b_is_element ? m.element : b == nullptr ? 0.0f : TI::to_float(b[ob + (long long)i * m.sb[inner]]);
-        o[oo + i] = TO::from_float(Op::apply(x, y));
-      }
-      continue;
+    if (RAGGED && over) {   // (an inner stride is 0 or 1 here)
+      oa -= (long long)over * m.sa[inner];
+      ob -= (long long)over * m.sb[inner];
     }
+    float fa[V], fb[V];
     if (m.fill) {
 #pragma unroll
       for (int i = 0; i < V; ++i) fa[i] = m.element;
     } else if (V > 1 && m.sa[inner] == 1) {
-      const Pack<TI, V> pa = load_pack<TI, V, PER_LANE != 1, RAGGED>(a + oa);
+      const Pack<TI, V> pa = load_pack<TI, V, PER_LANE != 1 && RAGGED != 1, RAGGED != 0>(a + oa);
 #pragma unroll
       for (int i = 0; i < V; ++i) fa[i] = TI::to_float(pa.v[i]);
     } else {
@@ -189,20 +214,25 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = 0.0f;
     } else if (V > 1 && m.sb[inner] == 1) {
-      const Pack<TI, V> pb = load_pack<TI, V, !B_CACHED && PER_LANE != 1, RAGGED>(b + ob);
+      const Pack<TI, V> pb = load_pack<TI, V, !B_CACHED && PER_LANE != 1 && RAGGED != 1, RAGGED != 0>(b + ob);
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = TI::to_float(pb.v[i]);
     } else {
 #pragma unroll
       for (int i = 0; i < V; ++i) fb[i] = TI::to_float(b[ob + (long long)i * m.sb[inner]]);
     }
+    if (RAGGED && over) {
+      shift_front<V>(fa, over);
+      if (Op::binary) shift_front<V>(fb, over);
+    }
     const Pack<TO, V> po = apply_pack<TO, Op, V>(fa, fb);
-    if constexpr (RAGGED) store_pack_anywhere<TO, V>(o + oo, po);
+    if (RAGGED && over) store_front<TO, V>(o + oo, po, over);
+    else if constexpr (RAGGED) store_pack_anywhere<TO, V>(o + oo, po);
     else *reinterpret_cast<Pack<TO, V>*>(o + oo) = po;
   }
 }
 
-template <typename TI, typename TO, typename Op, int V, bool B_CACHED = false, int PER_LANE = kVectorsPerLane, bool RAGGED = false>
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED = false, int PER_LANE = kVectorsPerLane, int RAGGED = 0>
 __global__ __launch_bounds__(256) void map_kernel(Map m) {
   map_block<TI, TO, Op, V, B_CACHED, PER_LANE, RAGGED>(m, blockIdx.x);
 }
@@ -296,6 +326,12 @@ __global__ __launch_bounds__(256) void turn_kernel(TurnMap t) {
     if (row >= na || col >= ni) continue;
     float fa[V], fb[V];
     auto gather = [&](bool turned, const SI* from, const SI* direct, long long s_inner, long long s_across, float (&f)[V]) {
+      if (!turned && s_inner == 1 && col + V <= ni) {
+        const Pack<TI, V> x = load_pack<TI, V, false, true>(direct + (long long)row * s_across + col);
+#pragma unroll
+        for (int e = 0; e < V; ++e) f[e] = TI::to_float(x.v[e]);
+        return;
+      }
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         const uint32_t c = min(col + e, ni - 1);
@@ -324,7 +360,11 @@ __global__ __launch_bounds__(256) void turn_kernel(TurnMap t) {
   }
 }
 
-// Whether an operand is turned: its unit stride along another dimension than the innermost, and tiles that are mostly full.
+// Whether operands are turned: a unit stride along another dimension than the innermost, tiles that are full enough, and enough of them.
+// The kernel above, whose lanes share the lines they read, is ahead of tiles on small maps (a quarter of the workgroups, and one trip
+// to memory after another) and on narrow ones.  Turned / not, us: x.t bf16 256 x 256 3.3 / 3.1, 2^20 3.5 / 4.1 (64 x 64 matrices), 2^24 12.8 / 43, but
+// 65536 of 16 x 16 89 / 35, 3970 of 65 x 65 56 / 48 with an addend; f32 2^18 4.3 / 3.3, 2^20 (96 x 96) 5.2 / 4.6, 2^24 39 / 55, 16384 of 32 x
+// 32 40 / 36, 508400 rows of 33 with an addend 74 / 42; rows of 4096 2^20 3.4 / 6.2 (bf16, 256 of them), rows of 2^20 62 / 632 (f32, 32).
 template <typename TI, typename TO, typename Op>
 bool plan_turn(const Map& m, TurnMap* t) {
   const int inner = m.rank - 1;
@@ -343,10 +383,17 @@ bool plan_turn(const Map& m, TurnMap* t) {
   t->turn_b = db >= 0 && db == t->across;
   t->tiles_inner = (m.shape[inner] + TURN - 1) / TURN;
   t->tiles_across = (m.shape[t->across] + TURN - 1) / TURN;
-  return true;
+  constexpr bool halves = sizeof(typename TI::storage) == 2 && sizeof(typename TO::storage) == 2;
+  const double fill = (double)m.shape[inner] * m.shape[t->across] / ((double)t->tiles_inner * t->tiles_across * TURN * TURN);
+  // long rows of the result: its neighbours along the operands' rows come a whole row later, when their lines may have left the caches
+  if (m.shape[inner] >= 256) return m.total >= 750000 && fill >= (halves || m.total >= 12000000 ? 0.2 : 0.3);
+  if (m.total < 2000000) return false;
+  const bool whole = m.shape[inner] % 8 == 0 && m.shape[t->across] % 8 == 0;   // rows of whole 16-byte pieces, either way
+  const bool all_turned = t->turn_a && (!m.b || t->turn_b);
+  return fill >= (!halves ? 0.55 : whole && (all_turned || m.total >= 4000000) ? 0.25 : all_turned ? 0.5 : 0.6);
 }
 
-template <typename TI, typename TO, typename Op, int V, bool RAGGED>
+template <typename TI, typename TO, typename Op, int V, int RAGGED>
 hipError_t launch_v(const Map& m, hipStream_t stream) {
   unsigned long long vector_bytes = V * sizeof(typename TO::storage);
   if (!m.fill) vector_bytes += V * sizeof(typename TI::storage) * (m.b && !m.b_reused ? 2 : 1);
@@ -393,8 +440,27 @@ int vector_width(const Map& m, bool* ragged) {
   if (!operand_ok(m.o, m.so, sizeof(typename TO::storage), true)) return 1;
   if (!m.fill && !operand_ok(m.a, m.sa, sizeof(typename TI::storage), false)) return 1;
   if (!m.fill && !m.b_is_element && !operand_ok(m.b, m.sb, sizeof(typename TI::storage), false)) return 1;
-  // rows of hardly more than a vector leave most of a ragged row to the element loop
-  return *ragged && m.shape[inner] < 2 * V ? 1 : V;
+  return V;
+}
+
+// Whether ragged rows are worth vectors: from four vectors a row (two of eight elements on a large map) and a few hundred thousand
+// elements, more where a result is a long
+// chain of arithmetic (eight in a row on one lane take longer than a small launch); fp32 with two whole operands not from 80 MB to
+// what the last-level cache holds, where single elements, whole lines to a wave, are ahead.  Vectors / single elements, us: add bf16 16384 x 16 rows
+// of 31 4.1 / 4.3, 63 3.6 / 4.4; bias add bf16 2^16 elements 3.4 / 3.3, 2^20 3.5 / 3.8, 2^22 6.4 / 9.4, 2^24 14 / 33; tanh bf16 rows of 63 2^18
+// 3.9 / 3.4, 2^20 3.9 / 3.5, 2^22 6.9 / 8.8; add f32 rows of 255 2^20 3.5 / 4.1, 2^22 9.4 / 9.7, 2^23 22 / 17, 2^24 38 / 31, 5001
+// x 7001 64 / 75.
+template <typename TI, typename TO, typename Op>
+bool ragged_pays(const Map& m, int v) {
+  const uint32_t row = m.shape[m.rank - 1];
+  if (row < 4u * (uint32_t)v && (v < 8 || row < 2u * (uint32_t)v || m.total < 6000000u)) return false;
+  if (m.total < (long_chain<Op>() ? 2000000u : 750000u)) return false;
+  if (sizeof(typename TI::storage) == 4 && m.b && !m.b_is_element && !m.b_reused)
+  {
+    const unsigned long long bytes = m.total * (8 + sizeof(typename TO::storage));
+    return bytes <= kOneVectorBytes || (bytes > 300000000 && row >= 1000);
+  }
+  return true;
 }
 
 // The map with its innermost extent counted in vectors.
@@ -411,9 +477,10 @@ hipError_t launch_t(Map m, hipStream_t stream) {
   constexpr int V = 16 / (sizeof(typename TI::storage) > sizeof(typename TO::storage) ? sizeof(typename TI::storage)
                                                                                       : sizeof(typename TO::storage));
   bool ragged;
-  if (vector_width<TI, TO>(m, &ragged) == V) {
+  if (vector_width<TI, TO>(m, &ragged) == V && (!ragged || ragged_pays<TI, TO, Op>(m, V))) {
     count_vectors(&m, V);
-    return ragged ? launch_v<TI, TO, Op, V, true>(m, stream) : launch_v<TI, TO, Op, V, false>(m, stream);
+    if (!ragged) return launch_v<TI, TO, Op, V, 0>(m, stream);
+    return m.inner_elements < 1000 ? launch_v<TI, TO, Op, V, 1>(m, stream) : launch_v<TI, TO, Op, V, 2>(m, stream);
   }
   TurnMap t;
   if (plan_turn<TI, TO, Op>(m, &t)) {
@@ -427,7 +494,7 @@ hipError_t launch_t(Map m, hipStream_t stream) {
       return launch_status(stream);
     }
   }
-  return launch_v<TI, TO, Op, 1, false>(m, stream);
+  return launch_v<TI, TO, Op, 1, 0>(m, stream);
 }
 
 template <typename Op>

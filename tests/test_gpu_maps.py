@@ -1,5 +1,6 @@
-"""Element-wise maps whose operands walk memory across the result's rows (turned through LDS in 64 x 64 tiles) and maps whose rows are
-no whole number of aligned vectors: exact against numpy on small integers, at the edges of the tile and of the vector."""
+"""Element-wise maps whose operands walk memory across the result's rows (turned through LDS in 64 x 64 tiles where that is ahead) and
+maps whose rows are no whole number of aligned vectors: exact against numpy on small integers, at the edges of the tile and of the
+vector, on maps small enough for the element-by-element kernel and large enough for the others."""
 import ctypes
 
 import numpy as np
@@ -44,6 +45,32 @@ def test_turned_operands(dt, m, n):
     check(o, A, other)
 
 
+# enough full tiles to be turned: a tile less a row or column, whole ones, several with remainders, rows of whole pieces that fill a
+# third of their tiles (16-bit), long rows of a few
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("m,n", [(61, 62), (64, 64), (48, 56), (127, 190), (300, 1001), (40, 40), (16, 1028), (33, 2049)])
+def test_turned_operands_of_large_maps(dt, m, n):
+    g = H.rng(m * n + 1)
+    batch = -(-2_100_000 // (m * n))
+    at, bt, a, b = ints(g, (batch, n, m), dt), ints(g, (batch, n, m), dt), ints(g, (batch, m, n), dt), ints(g, (n,), dt)
+    A, B = np.swapaxes(H.to64(at), 1, 2), np.swapaxes(H.to64(bt), 1, 2)
+    T, q = srt.Tensor, srt.current_queue()
+    for lhs, rhs, want in [(T(at).t, T(a), A + H.to64(a)), (T(a), T(bt).t, H.to64(a) + B), (T(at).t, T(bt).t, A + B),
+                           (T(at).t, T.repeating(T(b), [batch, m, n]), A + H.to64(b)), (T(at).t, 3.0, A + 3)]:
+        o = T(shape=[batch, m, n], dtype=at.dtype)
+        q.add(lhs, rhs, o)
+        check(o, want, dt)
+    other = H.BF16 if dt == H.F32 else H.F32
+    o = T(shape=[batch, m, n], dtype=H.NP_STORAGE[other])
+    q.copy(T(at).t, o)                                       # with conversion
+    check(o, A, other)
+    frame = T(H.encode(np.full((batch, m + 3, n + 5), 5), dt))
+    q.copy(T(at).t, frame[:, 1:1 + m, 3:3 + n])
+    want = np.full((batch, m + 3, n + 5), 5.0)
+    want[:, 1:1 + m, 3:3 + n] = A
+    check(frame, want, dt)
+
+
 @pytest.mark.parametrize("dt", DTS)
 def test_turned_inside_a_batch_and_a_frame(dt):
     g = H.rng(3)
@@ -69,6 +96,43 @@ def test_ragged_rows(dt, n):
     check(srt.Tensor(a) + srt.Tensor(a), 2 * H.to64(a), dt)
     flat = srt.Tensor(np.ascontiguousarray(a.reshape(-1)[1:]))
     check(flat + flat, 2 * H.to64(a).reshape(-1)[1:], dt)
+
+
+# every remainder of a vector, rows from the fewest vectors that go this way; maps past the size from which ragged rows take vectors,
+# past the one for long chains of arithmetic, and past the one from which a lane takes four vectors
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("n,elements", [*((n, 2_100_000) for n in (16, 17, 19, 31, 32, 33, 34, 35, 36, 37, 38, 39, 47, 1001)),
+                                        (17, 6_100_000), (23, 6_100_000), (63, 800_000), (999, 41_000_000), (1001, 41_000_000)])
+def test_ragged_rows_of_large_maps(dt, n, elements):
+    g = H.rng(n)
+    m = -(-elements // n)
+    a, c, b = ints(g, (m, n), dt), ints(g, (m, n), dt), ints(g, (n,), dt)
+    T, q = srt.Tensor, srt.current_queue()
+    frame = T(H.encode(np.full((m, n + 5), 5), dt))
+    view, row = frame[:, 3:3 + n], T.repeating(T(b), [m, n])
+    want = np.full((m, n + 5), 5.0)
+    want[:, 3:3 + n] = H.to64(a) * H.to64(b)
+    q.mul(T(a), row, view)
+    check(frame, want, dt)
+    want[:, 3:3 + n] = want[:, 3:3 + n] - H.to64(c)
+    q.subtract(view, T(c), view)                             # in place: a vector moved back to end inside its row reads its neighbour's
+    check(frame, want, dt)
+    if elements > 10_000_000:
+        return
+    want[:, 3:3 + n] = H.to64(H.encode(H.to64(b) - want[:, 3:3 + n], dt))
+    q.subtract(row, view, view)
+    check(frame, want, dt)
+    dense, got = T(shape=[m, n], dtype=a.dtype), T(H.encode(np.full((m, n + 5), 5), dt))
+    scaled = T(H.encode(g.standard_normal((m, n)), dt))
+    q.tanh(scaled, dense)                                    # (dense: aligned vectors)
+    q.tanh(scaled, got[:, 3:3 + n])
+    full = got.array()
+    assert np.array_equal(full[:, 3:3 + n].view(np.uint16), dense.array().view(np.uint16))
+    assert np.all(H.to64(full[:, :3]) == 5) and np.all(H.to64(full[:, 3 + n:]) == 5)
+    other = H.BF16 if dt == H.F32 else H.F32
+    o = T(shape=[m, n], dtype=H.NP_STORAGE[other])
+    q.copy(view, o)                                          # with conversion
+    check(o, want[:, 3:3 + n], other)
 
 
 @pytest.mark.parametrize("dt", DTS)
