@@ -320,7 +320,7 @@ bool pack_preferred(const GemmProblem& p);
 double packed_us(const GemmProblem& p);   // estimate of an fp32 problem's time that way, copies included (0: it cannot)
 double f32_ring_us(const GemmProblem& p);   // and of the ring kernel's plans alone
 enum class F32Any { kTile, kSplitK, kParts, kPacked };
-F32Any f32_any_choice(const GemmProblem& p, double packed_us);   // for a problem the ring kernel does not read
+F32Any f32_any_choice(const GemmProblem& p, bool copies);   // for a problem the ring kernel does not read
 hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErrorOutOfMemory: no workspace, nothing was launched
 // 32 x 32 tiles whose waves split k (gemm_waves.hip): whether they read the problem, whether they are the choice, and the launch.
 bool waves_supported(const GemmProblem& p);

@@ -833,14 +833,14 @@ hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_
 //   as it is   64 x 64 tiles at 30.8 per 1024 k and tile of a unit; from 256 tiles of 128 x 128 on those at 92 (120 when a unit
 //              has one only), or at 78 (86) with 16-byte loads; + 4
 //   32 x 32    splitk_us and 0.45 per tile of a unit for its fill and store
-//   copied     (packed_us > 0, from gemm_pack.hip) the ring kernel's estimate, 5 for the extra launch and the wait between the
+//   copied     (packed_us in gemm_pack.hip) the ring kernel's estimate, 5 for the extra launch and the wait between the
 //              two, the copies and the result's stores at their bandwidth
 // measured, x . W (as it is / 32 x 32 / copied): 1000 x 2000 x 1000 64 / 60 / 46, 1023 x 2047 x 2047 126 / 114 / 76, 2000^3 172 / 212 /
 // 135, 2001 x 3003 x 1501 268 / 326 / 155, 2001 x 2001 x 300 41 / 41 / 34, 300 x 10001 x 500 57 / 55 / 46, 4096 x 3000 x 1000 230 / 383 /
 // 197, 8 x 300 x 500 x 700 46 / 28 / 34, 16 x 511 x 511 x 63 x . W^T 14.7 / 17.0 / 22.2, 3000 x 3000 x 100 36.5 / 41.7 / 35.9.
 // (The rule above and the parts pass stay ahead of the copies: the ring kernel sums a tile's k in one chain, they in several,
 // and 1001^3 is off by 5.7e-7 against 2.1e-7 that way.)
-F32Any f32_any_choice(const GemmProblem& p, double packed_us) {
+F32Any f32_any_choice(const GemmProblem& p, bool copies) {
   if (f32_mfma_prefers_splitk(p)) return F32Any::kSplitK;
   if (f32_tile_parts(p) >= 2) return F32Any::kParts;
   const double cus = compute_units();
@@ -850,7 +850,8 @@ F32Any f32_any_choice(const GemmProblem& p, double packed_us) {
   if (tiles(128) >= 256) per_k = mfma128_vec_fits(p) ? (t128 > 1 ? 78.0 : 86.0) * t128 : (t128 > 1 ? 92.0 : 120.0) * t128;
   const double as_is = per_k * (double)p.K / 1024.0 + 4.0;
   const double split = splitk_us(p) + 0.45 * tiles(32) / cus;
-  if (packed_us > 0.0 && packed_us < as_is && packed_us < split) return F32Any::kPacked;
+  const double copied = copies ? packed_us(p) : 0.0;
+  if (copied > 0.0 && copied < as_is && copied < split) return F32Any::kPacked;
   return split < as_is ? F32Any::kSplitK : F32Any::kTile;
 }
 

@@ -738,6 +738,13 @@ static bool narrow_round(const GemmProblem& p, int layout) {
 // The tile of a problem whose result rows are not whole aligned chunks (an odd number of columns): one of the kernels that
 // store such rows, by rounds of the persistent grid -- a whole tile takes 6 + 24 us per 1024 k, a half tile 0.6 and a quarter
 // tile 0.29 of that per round, fitted to the figures above -- or the register-staged kernels when K is not in their units.
+// A problem of less than a device's worth of 128 x 128 tiles (the caller's own operands: a k-contiguous B) stays with 64 x 64 ones
+// where those are ahead, by estimates in microseconds:
+//   64 x 64      4 + its 64-deep stages at 0.5 (k-contiguous A) or 1.05, more from 400 tiles on
+//   the others   7.5 + 4.9 per 1024 k in quarter tiles, 7 (11: A not k-contiguous) + 9.8 in half tiles, 7 + 18 in whole ones
+// measured (64 x 64 / the others' best): x . W^T 128 x 1809 x 320 7.3 / 10.4, 1728 x 93 x 448 8.0 / 11.8, 128 x 5003 x 832 11.1 / 15.1, 304 x
+// 630 x 1024 11.9 / 12.2, 512 x 1809 x 2048 20.5 / 17.5, 128 x 93 x 4096 32 / 26; x^T . W^T 200 x 630 x 320 9.4 / 14.3, 64 x 17 x 768
+// 14.5 / 11.1, 1000 x 309 x 1536 in two 32.6 / 15.7.
 static int ragged_store_config(const GemmProblem& p) {
   const long long cus = compute_units();
   auto rounds = [&](int tm, int tn) {
@@ -745,13 +752,20 @@ static int ragged_store_config(const GemmProblem& p) {
     return (double)((t + cus - 1) / cus);
   };
   const int configs[4] = {mfma_config(p, 9), mfma_config(p, 12), mfma_config(p, 13), mfma_config(p, 14)};
-  const double times[4] = {rounds(256, 256), 0.6 * rounds(128, 256), 0.6 * rounds(256, 128), 0.29 * rounds(128, 128)};
+  const double r[4] = {rounds(256, 256), rounds(128, 256), rounds(256, 128), rounds(128, 128)};
+  const double times[4] = {r[0], 0.6 * r[1], 0.6 * r[2], 0.29 * r[3]};
   int best = -1;
   for (int i = 0; i < 4; ++i)
     if (configs[i] && (best < 0 || times[i] < times[best])) best = i;
-  if (best >= 0) return configs[best];
   const long long t128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-  return mfma_config(p, t128 >= cus ? 2 : 3);
+  if (best < 0) return mfma_config(p, t128 >= cus ? 2 : 3);
+  if (t128 < cus && !p.row_padding) {
+    constexpr double kFixed[4] = {7.0, 7.0, 11.0, 7.5}, kPerK[4] = {18.0, 9.8, 9.8, 4.9};
+    const double tiles64 = (double)((p.M + 63) / 64) * (double)((p.N + 63) / 64) * (double)p.batch;
+    const double small = 4.0 + (p.K + 63) / 64 * (p.sak == 1 ? 0.5 : 1.05) * (tiles64 > 400.0 ? tiles64 / 400.0 : 1.0);
+    if (small <= kFixed[best] + kPerK[best] * r[best] * p.K / 1024.0) return mfma_config(p, 3);
+  }
+  return configs[best];
 }
 
 int mfma_select(const GemmProblem& p) {
@@ -1063,6 +1077,7 @@ bool mfma_prefers_quarter(const GemmProblem& p) {
   const int config = mfma_config(p, 14);
   const bool a_kc = (config & 2) != 0, b_kc = (config & 1) != 0;
   if (config == 0 || p.N < 64) return false;
+  if (!c_whole_chunks(p) && !p.row_padding) return false;   // (ragged_store_config weighs it against 64 x 64 tiles)
   // (33-63 rows against an n-contiguous weight and a k loop of two or three units: 48 x 4712 x 256 6.6 us against 7.7 in half
   // tiles, 43 x 472 x 256 6.2 against 7.2 streamed; at K = 640 the streaming kernel is ahead again, 24 x 384 x 640 6.3 against 8.1)
   const bool short_nn = a_kc && !b_kc && p.M > 32 && p.K <= 384;

@@ -178,7 +178,7 @@ Plan tile_plan(const GemmProblem& p, bool copies) {
 Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
   // 16-bit problems of few tiles off the 16-byte rules: 32 x 32 tiles whose waves split k (aligned operands keep the choices
   // below and run them where that is the 64 x 64 plan)
-  if (srt::waves_preferred(p) && srt::mfma_config(p, 3) == 0) return kPlanWaves;
+  if (srt::mfma_config(p, 3) == 0 && srt::waves_preferred(p)) return kPlanWaves;
   // one round of 128 x 128 tiles holds the problem (64 rows or more) and its k loop is not worth cutting
   if (srt::mfma_prefers_quarter(p)) return kPlanM16Q;
   if (srt::skinny_supported(p) && srt::skinny_preferred(p)) return kPlanSkinny;
@@ -214,7 +214,7 @@ Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
         default: return kPlanF32SplitK;
       }
     }
-    switch (srt::f32_any_choice(p, copies ? srt::packed_us(p) : 0.0)) {
+    switch (srt::f32_any_choice(p, copies)) {
       // launch-sized problems and up to 64 rows: 32 x 32 tiles whose waves split K
       case srt::F32Any::kSplitK: return kPlanF32SplitK;
       // a single matrix of too few 128 x 128 tiles for the device: its k range in parts on those tiles

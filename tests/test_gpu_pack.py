@@ -93,7 +93,8 @@ def test_ragged_rows_under_every_activation(tmp_path, dt, act, coef):
 
 
 def test_the_choice_for_ragged_rows():
-    for (M, N, K, kernel) in [(2048, 50257, 768, "mfma_256x256_m16_k64"), (512, 1001, 1024, "mfma_128x128_m16_k128"),
+    for (M, N, K, kernel) in [(2048, 50257, 768, "mfma_256x256_m16_k64"), (512, 1001, 2048, "mfma_128x128_m16_k128"),
+                              (128, 1809, 320, "mfma_32x32_waves"), (304, 630, 512, "mfma_64x64"),
                               (512, 1001, 200, "mfma_32x32_waves")]:
         a, b = srt.Tensor(shape=[M, K], dtype=np.uint16), srt.Tensor(shape=[N, K], dtype=np.uint16)
         assert query_kernel(a, False, b, True, srt.Tensor(shape=[M, N], dtype=np.uint16)) == kernel
