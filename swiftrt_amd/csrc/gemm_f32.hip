@@ -759,6 +759,9 @@ static double splitk_us(const GemmProblem& p) {
 //   32 x 32 tiles, k split over the waves: every workgroup reads 64 x K x 4 bytes, at 42 / 50 / 38 / 43 bytes/ns (x . W /
 //   x . W^T / x^T . W / x^T . W^T) alone on its unit and 36 / 37 / 33 / 38 per unit when they share, + 3
 //                      (512^3 6.1 / 6.1 and 5.6 / 5.4, 512 x 512 x 2048 15.5 / 16.5 and 13.5 / 14.6, 1001^3 31 / 31 and 31 / 30)
+//   where units share, rounds count whole up to three from K = 512 on (816 x 768 x 704 18.0 / 18.0, against 15.6 in 64 x 64 tiles); with
+//   an A along m always, at 31 / 36 bytes/ns and 0.45 for a tile's fill and store (256 x 1728 x 1088 x^T . W 22.2 / 21.8, 20.2;
+//   1344 x 320 x 3648 58.6 / 64, 57.2)
 // Smaller tiles cost more per flop (more operand bytes per MFMA through L2 and LDS) and win by filling the device:
 // 1024^3 20 us on 256 tiles of 64 x 64 against 31-42 on 32 x 32 and 62 on 64 tiles of 128 x 128.
 // Returns 0: 128 x 128, 1: 64 x 128, 2: 64 x 64, 3: parts, 4: the 32 x 32 kernel.
@@ -784,7 +787,17 @@ static int ring_choice(const GemmProblem& p, double* us) {
     offer(3, (double)((tiles * s + cus - 1) / cus) * 59.0 * (double)(p.K / s) / 1024.0 + 4.0 +
                  (double)s * (double)p.M * (double)p.N * 8.0 / 6.0e6 + 5.0);
   }
-  if (f32_mfma_supported(p)) offer(4, splitk_us(p));
+  if (f32_mfma_supported(p)) {
+    double split = splitk_us(p);
+    const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch / cus;
+    const bool along_m = p.sak != 1;
+    if (splitk_vec_fits(p) && tiles > 1.0 && (along_m || p.K >= 512)) {
+      const double rate = along_m ? (p.sbn == 1 ? 31.0e3 : 36.0e3) : (p.sbn == 1 ? 36.0e3 : 37.0e3);
+      const double shared = (tiles <= 3.0 ? __builtin_ceil(tiles) : tiles) * 256.0 * (double)p.K / rate;
+      split = (shared > split - 3.0 ? shared : split - 3.0) + 3.0 + (along_m ? 0.45 * tiles : 0.0);
+    }
+    offer(4, split);
+  }
   return choice;
 }
 
