@@ -150,9 +150,10 @@ __device__ __forceinline__ void store_front(typename T::storage* p, const Pack<T
 
 // RAGGED: rows that are no whole number of aligned vectors (odd extents, pitches or bases), read at element alignment.  The last,
 // partial vector of a row is read whole, from the row's last V elements, moved to the front (what it read of its neighbour's elements,
-// which that lane may be overwriting, falls off), and its `V - over` results are stored one by one.  Rows of fewer than 1000 elements (RAGGED 1) are read without the streaming hint: a line that two waves share is wanted
-// twice (bias add f32 2^24 elements in rows of 255 36 -> 28 us; 5001 x 7001 f32 add with the hint 64, without 79).  Read by elements too, one after the other, it held a launch up by 0.2 us an element (bias add bf16 1040 x 63 4.6 us; element
-// by element throughout 3.6).
+// which that lane may be overwriting, falls off), and its `V - over` results are stored one by one.  (Read by elements too, one after
+// the other, it held a launch up by 0.2 us an element: bias add bf16 1040 x 63 4.6 us, element by element throughout 3.6.)
+// Rows of fewer than 1000 elements (RAGGED 1) are read without the streaming hint, because a line that two waves share is wanted twice
+// (bias add f32 2^24 elements in rows of 255 36 -> 28 us); longer ones (RAGGED 2) with it (5001 x 7001 f32 add 64 us, without 79).
 template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE, int RAGGED = 0>
 __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
   using SI = typename TI::storage;
@@ -250,8 +251,9 @@ __global__ __launch_bounds__(256) void copy_pair_kernel(Map m0, Map m1, uint32_t
 // reads such an operand along its own rows (16 bytes per lane), turns it in LDS and writes the result along the result's rows;
 // an operand that needs no turning is read where the result is written.
 //   bound   memory, both sides in whole 128-byte (16-bit) or 256-byte (fp32) row segments
-//   LDS     [64 rows of the result's dimension][64 + pad], one element per bank word or half word: pad 2 (16-bit) and 1 (fp32) put the
-//           eight (four) elements a lane gathers, and its neighbours', on different banks
+//   LDS     [64 rows of the result's dimension][64 + pad]: pad 2 (16-bit) and 1 (fp32) put the eight (four) elements a lane gathers on
+//           different banks; its neighbours' still meet (40 % of the LDS cycles are conflicts in 16 bits, 50 % in fp32, 4096^2), which the
+//           wait for memory hides (bf16 67 MB at 5.2 TB/s, fp32 134 MB at 4.7)
 constexpr int TURN = 64;
 
 struct TurnMap {

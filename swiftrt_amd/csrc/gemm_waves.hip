@@ -14,8 +14,10 @@
 //           one ds_read_b128; mn-contiguous [32 k][32 mn], 64 bytes per k row: two ds_read_b64_tr_b16, whose four k rows
 //           per half wave are 256 contiguous bytes
 //   sums    fp32; the eight partial tiles meet in LDS and are added pairwise, in a fixed order
-//   measured (before / now, us, bf16; before: 128 x 128 and 64 x 64 tiles, split-K, the streaming kernel): 136 x 448 x 576 9.9 / 3.8, 192 x 1536 x 2240 26.2 / 10.5, 128 x 112 x 8000 46 / 16, 152 x 257 x 1529 x . W^T 19.0 /
-//           6.3, 1176 x 384 x 3280 44 / 22, 1001^3 17.7 / 15.0, 32 x 2304 x 1469 13.7 / 5.3
+//   measured (before / now, us, bf16, where this is the choice; before: 64 x 64 tiles, by 16-byte loads or any) x . W^T 136 x 448 x 576 8.4 /
+//           3.8, 128 x 287 x 3376 27.8 / 7.5, 152 x 257 x 1529 21.6 / 6.2; x^T . W 128 x 440 x 656 18.5 / 3.9, 193 x 1535 x 2241 212 / 18;
+//           x . W 32 x 2304 x 1469 31 / 5.2, 192 x 1537 x 2241 85 / 21, 128 x 113 x 8001 342 / 26
+//   LDS     of the cycles it is busy, 24 % are bank conflicts with a k-contiguous operand (22 % with one of the two), none without
 #include "gemm_common.h"
 
 namespace srt {
