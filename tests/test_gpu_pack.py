@@ -3,6 +3,7 @@
 Integer operands, exact comparison (every partial sum is representable, so the kernel and its order of summation do not
 matter); operands framed by NaNs, results by a sentinel, so that a copy or a store past an edge shows."""
 import ctypes
+import os
 
 import numpy as np
 import pytest
@@ -124,6 +125,7 @@ def test_copied_fp32_views_without_a_unit_stride():
 # device-filling and small 16-bit products, fp32: the choice is the copies, and a stream under capture gives them no workspace
 @pytest.mark.parametrize("dt,M,N,K", [(H.BF16, 2049, 2051, 135), (H.F16, 2047, 2049, 257), (H.BF16, 1025, 1023, 1501),
                                       (H.F32, 1023, 2047, 1001)])
+@pytest.mark.skipif("debug" in os.environ.get("SWIFTRT_HIP_LIBRARY", ""), reason="the debug build synchronises after every launch")
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
 def test_without_workspace_the_operands_run_as_they_are(dt, M, N, K, ta, tb):
     g, L, q = H.rng(950), native.lib(), srt.current_queue()
