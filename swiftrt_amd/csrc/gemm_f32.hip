@@ -863,7 +863,8 @@ F32Any f32_any_choice(const GemmProblem& p, bool copies) {
   if (tiles(128) >= 256) per_k = mfma128_vec_fits(p) ? (t128 > 1 ? 78.0 : 86.0) * t128 : (t128 > 1 ? 92.0 : 120.0) * t128;
   const double as_is = per_k * (double)p.K / 1024.0 + 4.0;
   const double split = splitk_us(p) + 0.45 * tiles(32) / cus;
-  const double copied = copies ? packed_us(p) : 0.0;
+  // (a launch for the copies and the ring kernel's shortest problem are 11 already)
+  const double copied = copies && (as_is < split ? as_is : split) > 11.0 ? packed_us(p) : 0.0;
   if (copied > 0.0 && copied < as_is && copied < split) return F32Any::kPacked;
   return split < as_is ? F32Any::kSplitK : F32Any::kTile;
 }
