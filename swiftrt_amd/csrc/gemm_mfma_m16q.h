@@ -353,7 +353,7 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
     const int le = lane_id();
     constexpr bool LINEAR_BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_RELU || EPI == EPI_CLIPPED || EPI == EPI_SIGMOID ||
                                  EPI == EPI_TANH || EPI == EPI_ELU;
-    // What the epilogue needs of the problem is read from the kernel's arguments here: held from the start, it spilled scalar
+    // What the epilogue needs of the problem is read from the kernel's arguments here (the problem is the only one, at offset 0): held from the start, it spilled scalar
     // registers in the prologue, and two or three 128-deep units are mostly prologue and epilogue (us, held / read here: F16
     // 32 x 256^3 x . W^T 6.37 / 6.28, 512 x 4096 x 256 x . W 6.60 / 6.52, 640 x 896 x 768 8.67 / 8.55).  x^T . W has registers to
     // spare and is 1 % better off without (512^3 7.43 / 7.50).
