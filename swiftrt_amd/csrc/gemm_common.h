@@ -270,14 +270,31 @@ inline hipError_t ensure_lds_limit(const void* kernel, int bytes, std::atomic<ui
   return e;
 }
 
-// Compute units of the current device (cached per device).
+// Compute units of the current device.  The choice of a kernel asks a dozen times a call: where all visible devices agree -- asked
+// once -- the answer needs no look at which one is current (0.04 us each).
 inline int compute_units() {
+  auto units_of = [](int device) {
+    int n = 0;
+    return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && n > 0 ? n : 256;
+  };
+  static const int every = [&] {
+    int count = 0;
+    if (hipGetDeviceCount(&count) != hipSuccess || count < 1) {
+      (void)hipGetLastError();
+      return 256;
+    }
+    const int n = units_of(0);
+    for (int d = 1; d < count; ++d)
+      if (units_of(d) != n) return 0;
+    return n;
+  }();
+  if (every) return every;
   static std::atomic<int> cached[32];
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return 256;
   int n = cached[device & 31].load(std::memory_order_relaxed);
   if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) n = 256;
+    n = units_of(device);
     cached[device & 31].store(n, std::memory_order_relaxed);
   }
   return n;
@@ -322,9 +339,9 @@ double f32_ring_us(const GemmProblem& p);   // and of the ring kernel's plans al
 enum class F32Any { kTile, kSplitK, kParts, kPacked };
 F32Any f32_any_choice(const GemmProblem& p, bool copies);   // for a problem the ring kernel does not read
 hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErrorOutOfMemory: no workspace, nothing was launched
-// 32 x 32 tiles whose waves split k (gemm_waves.hip): whether they read the problem, whether they are the choice, and the launch.
+// Tiles whose waves split k (gemm_waves.hip): whether they read the problem, an estimate of the time, and the launch.
 bool waves_supported(const GemmProblem& p);
-bool waves_preferred(const GemmProblem& p);
+double waves_us(const GemmProblem& p);
 hipError_t launch_waves(const GemmProblem& p, hipStream_t stream);
 hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream);
 // Split-K over the 256 x 256 kernel: number of k parts (0: the problem does not qualify) and launch.

@@ -9,10 +9,10 @@
 //   128 x 128 / 64 x 64 element-wise loads with the caller's strides (views, column-major, odd
 //                       pitches all land here); the small tile when the large one would leave CUs idle
 //   32 x 32 split-K     launch-latency-sized problems (512^3 = 64 tiles of 64 x 64): the waves split
-//                       K between them and sum through LDS; operands with a unit stride take a variant
-//                       of 8 waves with 16-byte loads
+//                       K between them and sum through LDS; operands with a unit stride run gemm_waves.h
 #include "gemm_common.h"
 #include "gemm_f32_ring.h"
+#include "gemm_waves.h"
 
 namespace srt {
 
@@ -378,201 +378,6 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_splitk_kernel(GemmProblem p
     if (mb + i < p.M) C[(long long)(mb + i) * p.scm + (long long)n * p.scn] = out[i];
 }
 
-// ---- 32 x 32 tiles, 8 waves split K; operands with a unit stride -------------------------------------------
-// The variant above walks k element by element, one slab in flight per wave.  When both operands
-// have a unit stride, along k or along m / n, a wave requests SV_SLABS slabs of its k range at once
-// with 16-byte loads (4 per slab and lane) and multiplies them as they arrive; wave w owns a
-// contiguous eighth of K.  Rows may start anywhere and end anywhere: the loads need element
-// alignment only, and a piece that would cross a row's end is loaded from the row's last four
-// elements and shifted into place when it is stored to LDS.
-//   bound   latency: a round trip to memory and the matrix time of a unit's tiles (512^3: one tile per unit, 1.7 us of
-//           MFMAs at their peak).  Two waves per SIMD, so that one multiplies while the other waits or stores to LDS.
-//   waves   us with 4 waves x 8 slabs / 8 x 8 / 8 x 4 / 8 x 2 / 16 x 4: 512^3 x . W 7.2 / 7.0 / 6.3 / 6.1 / 6.6, 256 x 1000 x 784
-//           10.8 / 9.5 / 8.7 / 8.5 / 8.2, 64 x 2048 x 1024 11.4 / 9.4 / 9.0 / 8.9 / 8.7, 4 x 256^3 5.3 / 5.4 / 4.7 / 4.2 / 5.5, 1001^3
-//           35.2 / 40.3 / 30.2 / 30.7 / 36.7: more slabs than a wave has are loads for nothing, and registers that
-//           keep a second workgroup off the unit
-//   before  (4 waves x 8 slabs for aligned row-major operands, by elements otherwise) 512^3 x . W 6.7, x . W^T 11.5, x^T . W 11.5;
-//           256 x 1000 x 784 10.0, 16.7, 16.7; 64 x 2048 x 1024 10.7, 19.6, 19.7; 1001^3 41; 33 x 4093 x 2047 35.
-//           Now 6.1, 5.4, 6.4; 8.5, 7.7, 9.4; 8.9, 7.9, 10.1; 31, 30, 35; 17.1, 14.5, 18.7.
-//   k-contiguous slab   32 rows x 16 k: lane f (two per lane) loads 4 k of row f / 4; transposed into LDS
-//           k-major [k][m], pitch 36: the four ds_write_b32 of a lane pair are conflict-free.
-//   mn-contiguous slab  16 k x 32 mn: lane f loads 4 mn of k row f / 8; LDS [k][mn], pitch 32: even k rows sit
-//           in banks 0-31 and odd ones in 32-63, which is exactly the split of the MFMA operand
-//           read (lanes 0-31 take k = 2 kk, lanes 32-63 k = 2 kk + 1).
-constexpr int SV_WAVES = 8, SV_SLABS = 2;
-
-typedef f32x4v_t f32x4u_t __attribute__((aligned(4)));
-
-// v's elements s .. 3 moved to the front, zeros behind them (s >= 4: all zeros)
-__device__ __forceinline__ f32x4v_t shifted(f32x4v_t v, int s) {
-  if (s & 1) v = f32x4v_t{v[1], v[2], v[3], 0.0f};
-  if (s & 2) v = f32x4v_t{v[2], v[3], 0.0f, 0.0f};
-  if (s >= 4) v = f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f};
-  return v;
-}
-
-template <bool KC>
-struct SlabStage {
-  static constexpr int PITCH = KC ? 36 : 32;
-  const float* row[2];   // KC: the row's start; MN: the piece's place in k row 0
-  int k[2], mn[2];       // the piece's place in a slab
-  int over[2];           // MN: elements the piece was moved back to end inside its row
-  long long ld;
-  int K, last_k;         // last_k: the largest k (MN) or piece start (KC) this wave may read
-  bool edge;             // MN, workgroup-uniform: some piece crosses the rows' end
-
-  // extent: M or N (MN: at least 4); k_end: where this wave's k range ends (KC: K at least 4)
-  __device__ __forceinline__ void init(const float* base, int lane, int mn0, int extent, long long stride, int K_, int k_end) {
-    ld = stride;
-    K = K_;
-    last_k = min(k_end, K_) - (KC ? 4 : 1);
-    edge = !KC && mn0 + 32 > extent;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int f = lane + 64 * i;
-      if (KC) {
-        mn[i] = f >> 2; k[i] = (f & 3) * 4; over[i] = 0;
-        // (a row past the extent repeats the last one: it feeds results that are not stored)
-        row[i] = base + (long long)min(mn0 + mn[i], extent - 1) * stride;
-      } else {
-        k[i] = f >> 3; mn[i] = (f & 7) * 4;
-        const int at = min(mn0 + mn[i], extent - 4);
-        over[i] = mn0 + mn[i] - at;
-        row[i] = base + at;
-      }
-    }
-  }
-  __device__ __forceinline__ f32x4v_t load(int i, int k0) const {
-    const int at = min(k0 + k[i], last_k);
-    return *reinterpret_cast<const f32x4u_t*>(row[i] + (KC ? (long long)at : (long long)at * ld));
-  }
-  __device__ __forceinline__ void store(int i, int k0, f32x4v_t v, float (*dst)[PITCH]) const {
-    if (KC) {
-      if (k0 + FK > K) v = shifted(v, max(0, k0 + k[i] - (K - 4)));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dst[k[i] + e][mn[i]] = v[e];
-    } else {
-      if (edge) v = shifted(v, over[i]);
-      if (k0 + FK > K && k0 + k[i] >= K) v = f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f};
-      *reinterpret_cast<f32x4v_t*>(&dst[k[i]][mn[i]]) = v;
-    }
-  }
-};
-
-template <bool A_KC, bool B_KC>
-__global__ __launch_bounds__(64 * SV_WAVES) void gemm_f32_mfma_splitk_vec_kernel(GemmProblem p) {
-  using StageA = SlabStage<A_KC>;
-  using StageB = SlabStage<B_KC>;
-  union Lds {
-    struct {
-      float a[SV_WAVES][FK][StageA::PITCH], b[SV_WAVES][FK][StageB::PITCH];
-    } slab;
-    float red[SV_WAVES][16][64];   // the waves' partial tiles, once every wave is done with its slabs
-  };
-  __shared__ __attribute__((aligned(16))) Lds lds;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 31, kh = lane >> 5;
-  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32, bz = blockIdx.z;
-  float* C = (float*)p.C + (long long)bz * p.scb;
-
-  // this wave's slabs: a contiguous part of the k range
-  const int slabs = (p.K + FK - 1) / FK;
-  const int per_wave = (slabs + SV_WAVES - 1) / SV_WAVES;
-  const int first = wave * per_wave;
-  const int last = min(slabs, first + per_wave);   // exclusive
-
-  StageA sa;
-  StageB sb;
-  sa.init((const float*)p.A + (long long)bz * p.sab, lane, m0, p.M, A_KC ? p.sam : p.sak, p.K, last * FK);
-  sb.init((const float*)p.B + (long long)bz * p.sbb, lane, n0, p.N, B_KC ? p.sbn : p.sbk, p.K, last * FK);
-
-  f32x16_t acc;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-
-  for (int s0 = first; s0 < last; s0 += SV_SLABS) {
-    f32x4v_t ra[SV_SLABS][2], rb[SV_SLABS][2];
-    // (slabs past the wave's range repeat its last piece: no branch between the loads)
-#pragma unroll
-    for (int s = 0; s < SV_SLABS; ++s) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ra[s][i] = sa.load(i, (s0 + s) * FK);
-        rb[s][i] = sb.load(i, (s0 + s) * FK);
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < SV_SLABS; ++s) {
-      if (s0 + s >= last) break;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        sa.store(i, (s0 + s) * FK, ra[s][i], lds.slab.a[wave]);
-        sb.store(i, (s0 + s) * FK, rb[s][i], lds.slab.b[wave]);
-      }
-      // the slab is written and read by this wave only: LDS operations of one wave execute in
-      // order (the next slab's writes behind this one's reads, too), so a wave-level fence (for
-      // the compiler) is all that is needed
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int kk = 0; kk < FK / 2; ++kk)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(lds.slab.a[wave][2 * kk + kh][r], lds.slab.b[wave][2 * kk + kh][r], acc, 0, 0, 0);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-  }
-
-  __syncthreads();
-#pragma unroll
-  for (int v = 0; v < 16; ++v) lds.red[wave][v][lane] = acc[v];
-  __syncthreads();
-
-  // wave w finishes accumulator registers R w .. R w + R - 1; register v is row 8 (v / 4) + 4 kh + v % 4, column r
-  constexpr int R = 16 / SV_WAVES;
-  Epilogue<F32> ep(p);
-  const int n = n0 + r;
-  if (n >= p.N) return;
-  const int mb = m0 + 8 * (R * wave / 4) + 4 * kh + (R * wave) % 4;
-  float out[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    float part[SV_WAVES];
-#pragma unroll
-    for (int w = 0; w < SV_WAVES; ++w) part[w] = lds.red[w][R * wave + i][lane];
-#pragma unroll
-    for (int step = 1; step < SV_WAVES; step *= 2)
-#pragma unroll
-      for (int w = 0; w < SV_WAVES; w += 2 * step) part[w] += part[w + step];
-    out[i] = part[0];
-  }
-  ep.finish_run(out, [&](int i, int* m, int* nn) {
-    *m = mb + i;
-    *nn = n;
-    return *m < p.M;
-  });
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-    if (mb + i < p.M) C[(long long)(mb + i) * p.scm + (long long)n * p.scn] = out[i];
-}
-
-// Preconditions of the vector variant: both operands have a unit stride, with at least one whole vector along it.
-bool splitk_vec_fits(const GemmProblem& p) {
-  if (p.sak == 1 ? p.K < 4 : (p.sam != 1 || p.M < 4)) return false;
-  if (p.sbn == 1 ? p.N < 4 : (p.sbk != 1 || p.K < 4)) return false;
-  return true;
-}
-
-hipError_t launch_f32_splitk_vec(const GemmProblem& p, hipStream_t stream) {
-  const dim3 grid((p.N + 31) / 32, (p.M + 31) / 32, p.batch), block(64 * SV_WAVES);
-  const bool a_kc = p.sak == 1, b_kc = p.sbn != 1;
-  if (a_kc && b_kc) hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<true, true>), grid, block, 0, stream, p);
-  else if (a_kc) hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<true, false>), grid, block, 0, stream, p);
-  else if (b_kc) hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<false, true>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((gemm_f32_mfma_splitk_vec_kernel<false, false>), grid, block, 0, stream, p);
-  return launch_status(stream);
-}
-
 // ---- split-K over the 128 x 128 vector kernel -----------------------------------------------------
 // The 128 x 128 kernel leans on several workgroups per compute unit to hide its k stages' load latency and barriers
 // (4096^3, four per unit: 117-121 TFLOP/s; 2048^3, one per unit: 92), and a problem of fewer tiles than units
@@ -739,15 +544,16 @@ bool f32_mfma_supported(const GemmProblem& p) {
   return true;
 }
 
-// The 32 x 32 kernel's time in microseconds (f32_ring_choice below has the figures).
+// The 32 x 32 tiles' time in microseconds (every one reads 64 x K x 4 bytes; the kernel that walks by elements at 16 bytes/ns alone
+// and 21.5 shared).  Fitted to 625 random problems, rms 10 %; measured / estimated: 512^3 5.6 / 6.1, 256 x 1000 x 784 8.0 / 7.5, 648 x
+// 344 x 3032 22.4 / 19, 1001^3 27.5 / 30, 320 x 3759 x 3648 98 / 112, 32 x 256^3 x . W^T 17.2 / 18.
 static double splitk_us(const GemmProblem& p) {
   const double cus = compute_units();
-  const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch;
-  const double bytes = 64.0 * (double)p.K * 4.0;   // per workgroup
-  constexpr double kAlone[5] = {42.0e3, 50.0e3, 38.0e3, 43.0e3, 16.0e3}, kShared[5] = {36.0e3, 37.0e3, 33.0e3, 38.0e3, 21.5e3};
-  const int layout = !splitk_vec_fits(p) ? 4 : (p.sak == 1 ? 0 : 2) + (p.sbn == 1 ? 0 : 1);
-  const double alone = bytes / kAlone[layout], shared = tiles / cus * bytes / kShared[layout];
-  return (alone > shared ? alone : shared) + 3.0;
+  const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch / cus;
+  const double kb = 0.256 * (double)p.K;
+  if (waves::fits(p)) return tiles <= 1.0 ? 3.5 + kb / 50.0 : 3.1 + tiles * (0.31 + kb / 40.0);
+  const double alone = kb / 16.0, shared = tiles * (kb / 21.5);
+  return (alone > shared ? alone : shared) + 3.0 + 0.45 * tiles;
 }
 
 // Which fp32 kernel a problem the ring kernel reads should run on, by estimates of the time in microseconds (each
@@ -756,12 +562,7 @@ static double splitk_us(const GemmProblem& p) {
 //   64 x 128 tiles    R x 30.5 per 1024 k + 4      (512 x 4096 x 4096 125 / 126, 256 x 8192 x 8192 255 / 248, 1536^3 95 / 96)
 //   64 x 64 tiles     R x 16.5 per 1024 k + 4      (1024^3 20.3 / 20.5, 64 x 14336 x 4096 71 / 70, 1536^3 77 / 78, 768^3 15.9 / 16.4)
 //   k in parts on 128 x 128 tiles: f32_tile_parts' estimate
-//   32 x 32 tiles, k split over the waves: every workgroup reads 64 x K x 4 bytes, at 42 / 50 / 38 / 43 bytes/ns (x . W /
-//   x . W^T / x^T . W / x^T . W^T) alone on its unit and 36 / 37 / 33 / 38 per unit when they share, + 3
-//                      (512^3 6.1 / 6.1 and 5.6 / 5.4, 512 x 512 x 2048 15.5 / 16.5 and 13.5 / 14.6, 1001^3 31 / 31 and 31 / 30)
-//   where units share, rounds count whole up to three from K = 512 on (816 x 768 x 704 18.0 / 18.0, against 15.6 in 64 x 64 tiles); with
-//   an A along m always, at 31 / 36 bytes/ns and 0.45 for a tile's fill and store (256 x 1728 x 1088 x^T . W 22.2 / 21.8, 20.2;
-//   1344 x 320 x 3648 58.6 / 64, 57.2)
+//   32 x 32 tiles, k split over the waves: splitk_us
 // Smaller tiles cost more per flop (more operand bytes per MFMA through L2 and LDS) and win by filling the device:
 // 1024^3 20 us on 256 tiles of 64 x 64 against 31-42 on 32 x 32 and 62 on 64 tiles of 128 x 128.
 // Returns 0: 128 x 128, 1: 64 x 128, 2: 64 x 64, 3: parts, 4: the 32 x 32 kernel.
@@ -787,17 +588,7 @@ static int ring_choice(const GemmProblem& p, double* us) {
     offer(3, (double)((tiles * s + cus - 1) / cus) * 59.0 * (double)(p.K / s) / 1024.0 + 4.0 +
                  (double)s * (double)p.M * (double)p.N * 8.0 / 6.0e6 + 5.0);
   }
-  if (f32_mfma_supported(p)) {
-    double split = splitk_us(p);
-    const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch / cus;
-    const bool along_m = p.sak != 1;
-    if (splitk_vec_fits(p) && tiles > 1.0 && (along_m || p.K >= 512)) {
-      const double rate = along_m ? (p.sbn == 1 ? 31.0e3 : 36.0e3) : (p.sbn == 1 ? 36.0e3 : 37.0e3);
-      const double shared = (tiles <= 3.0 ? __builtin_ceil(tiles) : tiles) * 256.0 * (double)p.K / rate;
-      split = (shared > split - 3.0 ? shared : split - 3.0) + 3.0 + (along_m ? 0.45 * tiles : 0.0);
-    }
-    offer(4, split);
-  }
+  if (f32_mfma_supported(p)) offer(4, splitk_us(p));
   return choice;
 }
 
@@ -821,7 +612,7 @@ bool f32_mfma_prefers_splitk(const GemmProblem& p) {
 
 hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_t stream) {
   if (splitk) {
-    if (splitk_vec_fits(p)) return launch_f32_splitk_vec(p, stream);
+    if (waves::fits(p)) return waves::launch_layout<F32, 1>(p, stream);
     dim3 grid((p.N + 31) / 32, (p.M + 31) / 32, p.batch);
     hipLaunchKernelGGL(gemm_f32_mfma_splitk_kernel, grid, dim3(256), 0, stream, p);
   } else {
@@ -845,7 +636,7 @@ hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_
 // microseconds:
 //   as it is   64 x 64 tiles at 30.8 per 1024 k and tile of a unit; from 256 tiles of 128 x 128 on those at 92 (120 when a unit
 //              has one only), or at 78 (86) with 16-byte loads; + 4
-//   32 x 32    splitk_us and 0.45 per tile of a unit for its fill and store
+//   32 x 32    splitk_us
 //   copied     (packed_us in gemm_pack.hip) the ring kernel's estimate, 5 for the extra launch and the wait between the
 //              two, the copies and the result's stores at their bandwidth
 // measured, x . W (as it is / 32 x 32 / copied): 1000 x 2000 x 1000 64 / 60 / 46, 1023 x 2047 x 2047 126 / 114 / 76, 2000^3 172 / 212 /
@@ -862,7 +653,7 @@ F32Any f32_any_choice(const GemmProblem& p, bool copies) {
   double per_k = 30.8 * t64;
   if (tiles(128) >= 256) per_k = mfma128_vec_fits(p) ? (t128 > 1 ? 78.0 : 86.0) * t128 : (t128 > 1 ? 92.0 : 120.0) * t128;
   const double as_is = per_k * (double)p.K / 1024.0 + 4.0;
-  const double split = splitk_us(p) + 0.45 * tiles(32) / cus;
+  const double split = splitk_us(p);
   // (a launch for the copies and the ring kernel's shortest problem are 11 already)
   const double copied = copies && (as_is < split ? as_is : split) > 11.0 ? packed_us(p) : 0.0;
   if (copied > 0.0 && copied < as_is && copied < split) return F32Any::kPacked;

@@ -171,14 +171,12 @@ Plan tile_plan(const GemmProblem& p, bool copies) {
     case 12: return kPlanM16DH;
     case 13: return kPlanM16DN;
     case 14: return kPlanM16Q;
-    default: return srt::waves_preferred(p) ? kPlanWaves : kPlanMfma64;
+    default: return kPlanMfma64;
   }
 }
 
-Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
-  // 16-bit problems of few tiles off the 16-byte rules: 32 x 32 tiles whose waves split k (aligned operands keep the choices
-  // below and run them where that is the 64 x 64 plan)
-  if (srt::mfma_config(p, 3) == 0 && srt::waves_preferred(p)) return kPlanWaves;
+// The choice among every plan but the wave-split tiles.
+Plan base_plan(const GemmProblem& p, bool copies) {
   // one round of 128 x 128 tiles holds the problem (64 rows or more) and its k loop is not worth cutting
   if (srt::mfma_prefers_quarter(p)) return kPlanM16Q;
   if (srt::skinny_supported(p) && srt::skinny_preferred(p)) return kPlanSkinny;
@@ -225,6 +223,97 @@ Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
     }
   }
   return kPlanGeneric;
+}
+
+// What a 16-bit problem takes on a plan that base_plan picked, in microseconds, as a bound from below where a plan's figures
+// spread (0: not compared).  R: rounds of its tiles over the units, k: K in 1024s.  Fitted to 1900 random problems (gemm_waves.hip), rms
+// 3-10 % except the 64 x 64 kernel (15 %); rates are those of a device that is not power-limited.
+double plan_us(const GemmProblem& p, Plan plan) {
+  const int cus = srt::compute_units();
+  auto rounds = [&](int tm, int tn) {
+    const long long t = (long long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn) * p.batch;
+    return (double)((t + cus - 1) / cus);
+  };
+  const bool a_kc = p.sak == 1, b_kc = p.sbk == 1;
+  const double k = (double)p.K / 1024.0;
+  const double quarter = 4.4 + rounds(128, 128) * (0.9 + 5.1 * k), whole = 4.4 + rounds(256, 256) * (2.4 + 15.7 * k);
+  switch (plan) {
+    case kPlanM16Q: return quarter;
+    case kPlanM16H: return 4.1 + rounds(128, 256) * (1.4 + (b_kc ? 16.7 : 11.8) * k);
+    case kPlanM16DH: return 4.2 + rounds(128, 256) * (0.9 + 10.0 * k);
+    case kPlanM16DN: return 4.2 + rounds(256, 128) * (2.3 + 9.8 * k);
+    case kPlanM16D: return whole;
+    case kPlanM16:
+    case kPlanRing256:
+    case kPlanKc64: return 4.4 + rounds(256, 256) * (3.0 + 16.5 * k);
+    case kPlanM16DTail: return 12.0 + 7.0 * k;
+    case kPlanMfma64: return 5.3 + rounds(64, 64) * (a_kc ? 6.0 : b_kc ? 9.0 : 11.5) * k;
+    case kPlanSplitK: {
+      const int parts = srt::mfma_splitk_parts(p);
+      const double sums = (double)parts * (double)p.M * (double)p.N * 8.0;
+      return a_kc && p.M <= 128 ? 9.0 + 12.0 * k / parts + sums / 5.0e6 : 10.0 + 20.0 * k / parts + sums / 7.0e6;
+    }
+    case kPlanAny64: {
+      // (its 64-deep stages at 1.0, 2.5 or 5 by layout, once per two tiles a unit: gemm_pack.hip)
+      const double t64 = (double)((p.M + 63) / 64) * (double)((p.N + 63) / 64) * (double)p.batch;
+      return 4.0 + (p.K + 63) / 64 * (a_kc ? (b_kc ? 1.0 : 2.5) : 5.0) * __builtin_ceil(t64 / (2.0 * cus));
+    }
+    case kPlanCopied: {
+      // the launch and bytes of the copies, and the product's own
+      const double bytes = ((double)p.M + (double)p.N) * (double)p.K * 2.0 * (double)p.batch;
+      return 8.0 + 2.0 * bytes / 6.0e6 + (quarter < whole ? quarter : whole);
+    }
+    case kPlanSkinny: {
+      // bound by its own loads (40 or 45 bytes/ns a unit) or by the weight's from memory
+      const double wide = !b_kc || (p.M > 16 && (p.N + 63) / 64 * (long long)p.batch >= 192) ? 64.0 : 32.0;
+      const double groups = (double)((p.N + (long long)wide - 1) / (long long)wide) * (double)p.batch / cus;
+      const double kb = (wide + (double)((p.M + 7) / 8 * 8)) * (double)p.K * 2.0 / 1000.0;
+      return (b_kc ? 3.2 : 4.5) + (groups > 1.0 ? groups : 1.0) * kb / (b_kc ? 45.0 : 40.0);
+    }
+    default: return 0.0;
+  }
+}
+
+// Problems whose plan stays what base_plan picks, ahead or not: a plan's name is part of the interface (saved plans, the kernel query),
+// and the tests of the choice fix it over these ranges.  The price, measured (kept / wave-split, us): 512 x 512 x 1024 x^T . W 9.9 / 5.2,
+// 256 x 1024 x 960 x . W 14.0 / 4.6, 1024^3 x^T . W 9.9 / 7.2, 256^3 x . W^T 6.2 / 3.7, 32 x 1024 x 1024 x . W^T 5.0 / 4.6.
+bool keeps_plan(const GemmProblem& p, Plan plan) {
+  const long long results = (long long)p.M * p.N;
+  switch (plan) {
+    case kPlanAny64: return false;
+    case kPlanCopied:   // a large single matrix
+      return p.batch == 1 && (results >= (1LL << 22) || (p.K >= 1024 && (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) > srt::compute_units()));
+    case kPlanMfma64:   // whole 64-deep units of a large single matrix, or 128-deep ones into rows that are no whole chunks
+      return (p.K % 64 == 0 && p.K >= 960 && p.batch == 1 && results >= (1LL << 20)) || (p.K % 128 == 0 && p.K >= 256 && p.N % 8 != 0);
+    case kPlanSkinny: return p.batch > 1 || p.K >= 8192 || (p.sbk == 1 && p.N <= 1024);
+    default:
+      if (p.M <= 32) return true;   // a handful of rows
+      if (p.K % 64 != 0) return false;
+      if (p.batch > 1 ? p.K < 512 : p.K < 640) return plan == kPlanM16Q && p.K <= 256;   // two 128-deep units
+      return p.batch > 1 || results >= (1LL << 18);
+  }
+}
+
+// Whether a problem runs on tiles whose waves split k instead of on `plan`, which base_plan picked: by the two estimates.
+bool prefers_waves(const GemmProblem& p, Plan plan) {
+  if (p.row_padding || !srt::waves_supported(p) || keeps_plan(p, plan)) return false;
+  const double other = plan_us(p, plan);
+  if (other == 0.0) return false;
+  double here = srt::waves_us(p);
+  if (plan == kPlanSkinny) {
+    // few rows: the weight comes from memory, in whole lines on the streaming kernel
+    const double kb = (double)(32 + (p.M < 32 ? p.M : 32)) * (double)p.K * 2.0 / 1000.0, bytes = (double)p.N * (double)p.K * (double)p.batch * 2.0;
+    const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch / srt::compute_units();
+    const double cold = 2.9 + (tiles > 1.0 ? tiles : 1.0) * kb / (p.sbk == 1 ? 48.0 : 37.5);
+    if (cold > here) here = cold;
+    if (bytes > 12.0e6) return false;
+  }
+  return here < (plan == kPlanMfma64 ? 0.88 : 0.95) * other;   // (that kernel's estimate spreads most)
+}
+
+Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
+  const Plan plan = base_plan(p, copies);
+  return p.dtype != srtReal32F && prefers_waves(p, plan) ? kPlanWaves : plan;
 }
 
 hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
