@@ -58,11 +58,13 @@ class HipDeviceMemory:
     frees it when released; byte count padded to a multiple of 32 as the reference does."""
 
     def __init__(self, device_index, byte_count, queue):
+        self.pointer = None
         self.device_index = device_index
         self.byte_count = int(byte_count)
-        padded = (self.byte_count + 31) // 32 * 32
         p = ctypes.c_void_p()
-        check(native.lib().srtDeviceAllocate(ctypes.byref(p), max(padded, 32), queue.stream), "srtDeviceAllocate")
+        status = queue.lib.srtDeviceAllocate(ctypes.byref(p), max((self.byte_count + 31) // 32 * 32, 32), queue.stream)
+        if status:
+            check(status, "srtDeviceAllocate")
         self.pointer = p.value
         self.version = -1
         self.name = None
@@ -77,7 +79,7 @@ class HipDeviceMemory:
             if self.pointer:
                 if self.last_queue is not None and self.last_queue is not self.queue:
                     self.queue.wait(self.last_queue.record_event())
-                native.lib().srtDeviceFree(ctypes.c_void_p(self.pointer))
+                self.queue.lib.srtDeviceFree(self.pointer)
                 self.pointer = None
         except Exception:
             pass
@@ -96,14 +98,16 @@ class HipQueue:
         self.memory_type = "discrete"
         self.mode = "async"
         self.use_flat_forms = True   # dense element-wise operands go through the Flat entry points
-        L = native.lib()
+        self.lib = L = native.lib()
         check(L.srtSetDevice(gpu_id), "srtSetDevice")
         s = ctypes.c_void_p()
         check(L.srtStreamCreate(ctypes.byref(s)), "srtStreamCreate")
         self.stream = s
 
     def select(self):
-        check(native.lib().srtSetDevice(self.gpu_id), "srtSetDevice")
+        status = self.lib.srtSetDevice(self.gpu_id)
+        if status:
+            check(status, "srtSetDevice")
 
     # -- DeviceQueue protocol (platform/common/DeviceQueue.swift:22-82) -----------------------
     def allocate(self, byte_count, heap_index=0):
@@ -155,8 +159,8 @@ class HipQueue:
         b_ptr = rhs.device_read(self)
         bias_ptr = bias.device_read(self) if bias is not None else None
         o_ptr = result.device_write(self)
-        L = native.lib()
-        if bias is None and activation in (None, IDENTITY):
+        L = self.lib
+        if bias is None and (activation is None or activation == IDENTITY):
             st = L.srtMatmul(a_ptr, lhs.descriptor_ref(), int(transpose_lhs), b_ptr, rhs.descriptor_ref(), int(transpose_rhs),
                              o_ptr, result.descriptor_ref(), self.stream)
         else:
@@ -164,7 +168,8 @@ class HipQueue:
             st = L.srtMatmulBiasActivation(a_ptr, lhs.descriptor_ref(), int(transpose_lhs), b_ptr, rhs.descriptor_ref(),
                                            int(transpose_rhs), bias_ptr, bias.descriptor_ref() if bias is not None else None,
                                            act, float(coef), o_ptr, result.descriptor_ref(), self.stream)
-        check(st, "srtMatmul")
+        if st:
+            check(st, "srtMatmul")
         result.device_written()
 
     def tune_matmul(self, lhs, transpose_lhs, rhs, transpose_rhs, result, bias=None, activation=None, coef=0.0):

@@ -48,6 +48,27 @@ def strides_for(shape, order):
     return st
 
 
+# Dense layouts by (shape, order) and descriptors by layout: a step of a program makes results of the same few shapes over and over,
+# and working one out costs more than the call that uses it.  Both hold layouts only (no pointer, no tensor), are emptied when they
+# have grown to _LAYOUTS_MOST, and what a tensor took from them lives on with the tensor.
+_LAYOUTS_MOST = 4096
+_dense_layouts = {}
+_descriptors = {}
+
+
+def _dense_layout(shape, order):
+    """(shape, strides, count) of a dense tensor, as tuples of ints."""
+    dims = tuple(map(int, shape))
+    key = (dims, order._value_)
+    layout = _dense_layouts.get(key)
+    if layout is None:
+        layout = dims, tuple(strides_for(dims, order)), math.prod(dims)
+        if len(_dense_layouts) >= _LAYOUTS_MOST:
+            _dense_layouts.clear()
+        _dense_layouts[key] = layout
+    return layout
+
+
 class Tensor:
     """Shape + strides + storage offset over a flat storage buffer with a host replica and a
     lazily created device replica (the role of DiscreteStorage's per-device replicas with
@@ -96,11 +117,11 @@ class Tensor:
             else:
                 flat = np.ascontiguousarray(arr).reshape(-1).copy()
             self.storage = Tensor._Storage(flat)
+            self.shape, self.strides, _ = _dense_layout(shape, order)
         else:
-            self.storage = Tensor._Storage(dtype=dtype, size=math.prod(int(s) for s in shape))
+            self.shape, self.strides, size = _dense_layout(shape, order)
+            self.storage = Tensor._Storage(dtype=dtype, size=size)
         self.offset = 0
-        self.shape = tuple(int(s) for s in shape)
-        self.strides = tuple(strides_for(self.shape, order))
         self.order = order
         self._contiguous = True
 
@@ -146,11 +167,19 @@ class Tensor:
         return native.make_descriptor(_DTYPES[self.dtype], self.shape, self.strides, self.order.value)
 
     def descriptor_ref(self):
-        """The descriptor as an argument of a native call: made once and kept with the tensor.  For this module's own calls, which do not write to it; descriptor() makes one that the caller owns."""
-        if self._descriptor is None:
-            d, keep = self.descriptor()
-            self._descriptor = (ctypes.byref(d), d, keep)
-        return self._descriptor[0]
+        """The descriptor as an argument of a native call, one for all tensors of a layout.  For this module's own calls, which do not write to it; descriptor() makes one that the caller owns."""
+        made = self._descriptor
+        if made is None:
+            key = (_DTYPES[self.storage.dtype], self.shape, self.strides, self.order._value_)
+            made = _descriptors.get(key)
+            if made is None:
+                d, keep = self.descriptor()
+                made = (ctypes.byref(d), d, keep)
+                if len(_descriptors) >= _LAYOUTS_MOST:
+                    _descriptors.clear()
+                _descriptors[key] = made
+            self._descriptor = made
+        return made[0]
 
     @property
     def type_id(self):
@@ -229,8 +258,10 @@ class Tensor:
         """Pointer to this view's first element on the queue's device, copying host->device when
         the device replica is stale (Tensor.deviceRead, Tensor.swift:558-582)."""
         s = self.storage
-        self._ensure_device(queue)
         s.last_copy = None
+        if s.last_queue is queue and s.device_version >= s.host_version:   # resident, last used here
+            return s.device.pointer + self.offset * s.itemsize
+        self._ensure_device(queue)
         if s.device_version < s.host_version:
             if s._host is None:                  # zeros: made where they are read
                 queue.zero(s.device, s.nbytes)
@@ -251,14 +282,16 @@ class Tensor:
         reads none: when the view is the whole buffer, nothing is copied or cleared first (the values a 4096 x 11008 result
         was born with took three milliseconds to make and move).  device_written() follows once the call has been accepted."""
         s = self.storage
-        if self.offset == 0 and self.is_contiguous and self.count == s.size:
-            self._ensure_device(queue)
+        if self.offset == 0 and self.is_contiguous and math.prod(self.shape) == s.size:
+            if s.last_queue is not queue:
+                self._ensure_device(queue)
             return s.device.pointer
         return self.device_read(queue)
 
     def device_written(self):
         s = self.storage
-        s.device_version = max(s.device_version, s.host_version) + 1
+        device, host = s.device_version, s.host_version
+        s.device_version = (device if device > host else host) + 1
 
     def array(self):
         """Logical values as a numpy array in storage dtype, syncing device->host first if the
@@ -290,11 +323,12 @@ def matmul(lhs, rhs, transposed_lhs=False, transposed_rhs=False, bias=None):
     (operators/Matmul.swift:29-45, :57-72), rank 2, plus the rank-3 batched form whose queue
     function the reference keeps (CudaMatmul.swift:44-61).  The result is dense, in lhs.order.
     With `bias` the intended semantics are implemented (the reference drops the bias)."""
-    if lhs.rank != rhs.rank or lhs.rank not in (2, 3):
+    rank = len(lhs.shape)
+    if rank != len(rhs.shape) or rank not in (2, 3):
         raise ValueError("matmul takes two rank-2 or two rank-3 tensors")
     ls = _transposed_shape(lhs.shape, transposed_lhs)
     rs = _transposed_shape(rhs.shape, transposed_rhs)
-    if ls[-1] != rs[-2] or (lhs.rank == 3 and ls[0] != rs[0]):
+    if ls[-1] != rs[-2] or (rank == 3 and ls[0] != rs[0]):
         raise ValueError("matmul inner dimensions must be equal")
     result = Tensor(shape=ls[:-1] + [rs[-1]], dtype=lhs.dtype, order=lhs.order)
     current_queue().matmul(lhs, transposed_lhs, rhs, transposed_rhs, result, bias=bias)
