@@ -420,6 +420,17 @@ srtStatus srtLstmGates(const void* gates, const srtTensorDescriptor* gatesDesc, 
                        const srtTensorDescriptor* cellDesc, void* newCell, const srtTensorDescriptor* newCellDesc,
                        void* newHidden, const srtTensorDescriptor* newHiddenDesc, srtStream stream);
 
+/* One step of an LSTM cell in one launch (role of LSTMCell, SwiftRTLayers/Recurrent.swift:165-266): gates = [x, hidden] . weight + bias,
+ * rounded to the element type, then srtLstmGates' arithmetic.  x [B, I], hidden and cell [B, H], weight [I + H, 4 H], bias [4 H], results
+ * [B, H]; one element type (32F, 16F, 16BF) and row order for all.  srtErrorNotSupported -- nothing was launched, and the caller runs
+ * srtConcat, srtMatmulBiasActivation and srtLstmGates (or the element-wise calls) instead -- for other shapes, H not a multiple of 8,
+ * rows (except the cell's) that are not contiguous, results that share memory with an operand or each other, and cells
+ * large enough for the product's own kernels to be ahead. */
+srtStatus srtLstmCell(const void* x, const srtTensorDescriptor* xDesc, const void* hidden, const srtTensorDescriptor* hiddenDesc,
+                      const void* weight, const srtTensorDescriptor* weightDesc, const void* bias, const srtTensorDescriptor* biasDesc,
+                      const void* cell, const srtTensorDescriptor* cellDesc, void* newCell, const srtTensorDescriptor* newCellDesc,
+                      void* newHidden, const srtTensorDescriptor* newHiddenDesc, srtStream stream);
+
 /* ---- test helper ------------------------------------------------------------------------- */
 /* Replaces srtDelayStream, Modules/SwiftRTCuda/utilities_api.h:28: occupies `stream` for about
  * `seconds` (bounded spin on the device clock; at most 10 s). */

@@ -16,6 +16,7 @@
 #include <utility>
 
 #include "gemm_common.h"
+#include "lstm_gates.h"
 #include "status.h"
 
 namespace srt {
@@ -578,8 +579,6 @@ struct GateProblem {
 template <typename T, int V>
 __global__ __launch_bounds__(256) void lstm_gates_kernel(GateProblem p) {
   using S = typename T::storage;
-  using SigmoidT = std::conditional_t<T::dtype == srtReal32F, Sigmoid, SigmoidFast>;
-  using TanhT = std::conditional_t<T::dtype == srtReal32F, Tanh, TanhFast>;
   const uint32_t id = blockIdx.x * 256 + threadIdx.x;
   if (id >= p.rows * p.columns) return;
   const uint32_t row = id / p.columns, col = (id - row * p.columns) * V;
@@ -588,15 +587,9 @@ __global__ __launch_bounds__(256) void lstm_gates_kernel(GateProblem p) {
                    gf = load_pack<T, V, false>(g + 2 * p.part), go = load_pack<T, V, false>(g + 3 * p.part);
   const Pack<T, V> c = load_pack<T, V, false>((const S*)p.cell + (long long)row * p.cell_row + (long long)col * p.cell_col);
   Pack<T, V> nc, nh;
-  auto round = [](float x) { return T::to_float(T::from_float(x)); };
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
-    const float in = round(SigmoidT::apply(T::to_float(gi.v[i]), 0.0f)), up = round(TanhT::apply(T::to_float(gu.v[i]), 0.0f));
-    const float forget = round(SigmoidT::apply(T::to_float(gf.v[i]), 0.0f)), out = round(SigmoidT::apply(T::to_float(go.v[i]), 0.0f));
-    const float kept = round(T::to_float(c.v[i]) * forget), added = round(in * up);
-    nc.v[i] = T::from_float(kept + added);
-    nh.v[i] = T::from_float(round(TanhT::apply(T::to_float(nc.v[i]), 0.0f)) * out);
-  }
+  for (int i = 0; i < V; ++i)
+    lstm_gate<T>(T::to_float(gi.v[i]), T::to_float(gu.v[i]), T::to_float(gf.v[i]), T::to_float(go.v[i]), T::to_float(c.v[i]), &nc.v[i], &nh.v[i]);
   *reinterpret_cast<Pack<T, V>*>((S*)p.new_cell + (long long)row * p.new_cell_row + (long long)col * p.new_cell_col) = nc;
   *reinterpret_cast<Pack<T, V>*>((S*)p.new_hidden + (long long)row * p.new_hidden_row + (long long)col * p.new_hidden_col) = nh;
 }

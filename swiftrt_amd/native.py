@@ -105,6 +105,7 @@ SIGNATURES = {
     "srtCopyFlat": (_i32, [_i32, _vp, _i32, _vp, ctypes.c_size_t, _vp]),
     "srtFillFlat": (_i32, [_i32, _vp, _vp, ctypes.c_size_t, _vp]),
     "srtConcat": (_i32, [_vp, _descp, _vp, _descp, _i32, _vp, _descp, _vp]),
+    "srtLstmCell": (_i32, [_vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _vp]),
     "srtLstmGates": (_i32, [_vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _vp]),
 }
 # element-wise neighbours: tensor-tensor, tensor-element and unary forms share three signatures

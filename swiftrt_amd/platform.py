@@ -263,6 +263,22 @@ class HipQueue:
                                      self.stream), "srtConcat")
         out.device_written()
 
+    def lstm_cell(self, x, cell, hidden, weight, bias, new_cell, new_hidden):
+        """One step of an LSTMCell in one launch; False, with nothing launched, for a cell that is to run call by call."""
+        self.select()
+        pointers = [t.device_read(self) for t in (x, hidden, weight, bias, cell)]
+        nc_ptr, nh_ptr = new_cell.device_write(self), new_hidden.device_write(self)
+        status = self.lib.srtLstmCell(pointers[0], x.descriptor_ref(), pointers[1], hidden.descriptor_ref(), pointers[2], weight.descriptor_ref(),
+                                      pointers[3], bias.descriptor_ref(), pointers[4], cell.descriptor_ref(), nc_ptr, new_cell.descriptor_ref(),
+                                      nh_ptr, new_hidden.descriptor_ref(), self.stream)
+        if status == native.ERROR_NOT_SUPPORTED:
+            return False
+        if status:
+            check(status, "srtLstmCell")
+        new_cell.device_written()
+        new_hidden.device_written()
+        return True
+
     def lstm_gates(self, gates, cell, new_cell, new_hidden):
         """The gate arithmetic of LSTMCell (SwiftRTLayers/Recurrent.swift:255-266), one launch."""
         self.select()

@@ -472,6 +472,12 @@ class LSTMCell:
         return fused[:, i * h:(i + 1) * h]
 
     def __call__(self, x, cell, hidden):
+        # (a cell of another kind -- broadcast gates, more columns, another element type -- answers for itself below)
+        if len(x.shape) == 2 and cell.shape == hidden.shape and x.dtype == hidden.dtype == cell.dtype:
+            new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
+            new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
+            if current_queue().lstm_cell(x, cell, hidden, self.fused_weight, self.fused_bias, new_cell, new_hidden):
+                return new_cell, new_hidden
         gate_input = concatenate(x, hidden, axis=1)
         fused = matmul(gate_input, self.fused_weight, bias=self.fused_bias)
         if cell.rank != 2 or fused.shape != (cell.shape[0], 4 * cell.shape[1]):
