@@ -343,6 +343,10 @@ hipError_t launch_packed(const GemmProblem& p, hipStream_t stream);   // hipErro
 bool waves_supported(const GemmProblem& p);
 double waves_us(const GemmProblem& p);
 hipError_t launch_waves(const GemmProblem& p, hipStream_t stream);
+// 128 x 128 tiles for short k loops (gemm_short.hip): whether they are the kernel of a problem on 128 x 128 tiles, an estimate, the launch.
+bool short_supported(const GemmProblem& p);
+double short_us(const GemmProblem& p);
+hipError_t launch_short(const GemmProblem& p, hipStream_t stream);
 hipError_t launch_heuristic(const GemmProblem& p, hipStream_t stream);
 // Split-K over the 256 x 256 kernel: number of k parts (0: the problem does not qualify) and launch.
 int mfma_splitk_parts(const GemmProblem& p);

@@ -247,6 +247,8 @@ double plan_us(const GemmProblem& p, Plan plan) {
     case kPlanRing256:
     case kPlanKc64: return 4.4 + rounds(256, 256) * (3.0 + 16.5 * k);
     case kPlanM16DTail: return 12.0 + 7.0 * k;
+    case kPlanMfma128:
+    case kPlanAny128: return srt::short_supported(p) ? srt::short_us(p) : 0.0;
     case kPlanMfma64: return 5.3 + rounds(64, 64) * (a_kc ? 6.0 : b_kc ? 9.0 : 11.5) * k;
     case kPlanSplitK: {
       const int parts = srt::mfma_splitk_parts(p);
@@ -254,9 +256,9 @@ double plan_us(const GemmProblem& p, Plan plan) {
       return a_kc && p.M <= 128 ? 9.0 + 12.0 * k / parts + sums / 5.0e6 : 10.0 + 20.0 * k / parts + sums / 7.0e6;
     }
     case kPlanAny64: {
-      // (its 64-deep stages at 1.0, 2.5 or 5 by layout, once per two tiles a unit: gemm_pack.hip)
-      const double t64 = (double)((p.M + 63) / 64) * (double)((p.N + 63) / 64) * (double)p.batch;
-      return 4.0 + (p.K + 63) / 64 * (a_kc ? (b_kc ? 1.0 : 2.5) : 5.0) * __builtin_ceil(t64 / (2.0 * cus));
+      // (its stages and its stores, two tiles a unit: 512 x 3072 x 54 x . W^T 6.6 / 6.9, 346 x 5440 x 92 7.9 / 7.8, 12 x 768 x 320 x 53 7.8 / 7.8)
+      const double t64 = (double)((p.M + 63) / 64) * (double)((p.N + 63) / 64) * (double)p.batch / (2.0 * cus);
+      return 5.4 + 1.3 * t64 + (p.K + 63) / 64 * (a_kc ? (b_kc ? 0.55 : 2.2) : 4.5) * (t64 > 1.0 ? t64 : 1.0);
     }
     case kPlanCopied: {
       // the launch and bytes of the copies, and the product's own
@@ -280,7 +282,9 @@ double plan_us(const GemmProblem& p, Plan plan) {
 bool keeps_plan(const GemmProblem& p, Plan plan) {
   const long long results = (long long)p.M * p.N;
   switch (plan) {
-    case kPlanAny64: return false;
+    case kPlanAny64:
+    case kPlanAny128:
+    case kPlanMfma128: return false;
     case kPlanCopied:   // a large single matrix
       return p.batch == 1 && (results >= (1LL << 22) || (p.K >= 1024 && (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) > srt::compute_units()));
     case kPlanMfma64:   // whole 64-deep units of a large single matrix, or 128-deep ones into rows that are no whole chunks
@@ -311,8 +315,20 @@ bool prefers_waves(const GemmProblem& p, Plan plan) {
   return here < (plan == kPlanMfma64 ? 0.88 : 0.95) * other;   // (that kernel's estimate spreads most)
 }
 
+// Whether a problem with a short k loop runs on 128 x 128 tiles instead of on copies of its operands or small tiles: from five
+// quarters of a tile a unit -- at the first few past one, most units wait for those that have two --, below that where
+// the estimate is ahead of copies and of 64 x 64 tiles by elements.
+bool prefers_short(const GemmProblem& p, Plan plan) {
+  const bool others = plan == kPlanCopied || plan == kPlanAny64 || plan == kPlanAny128;
+  if ((!others && plan != kPlanMfma64) || !srt::short_supported(p)) return false;
+  const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, cus = srt::compute_units();
+  if (4 * tiles >= 5 * cus) return true;
+  return others && tiles <= cus && srt::short_us(p) < plan_us(p, plan);
+}
+
 Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
-  const Plan plan = base_plan(p, copies);
+  Plan plan = base_plan(p, copies);
+  if (p.dtype != srtReal32F && prefers_short(p, plan)) plan = srt::mfma_config(p, 2) != 0 ? kPlanMfma128 : kPlanAny128;
   return p.dtype != srtReal32F && prefers_waves(p, plan) ? kPlanWaves : plan;
 }
 
@@ -320,13 +336,13 @@ hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
   switch (plan) {
     case kPlanSkinny: return srt::launch_skinny(p, stream);
     case kPlanRing256: return srt::launch_mfma(p, srt::mfma_config(p, 1), stream);
-    case kPlanMfma128: return srt::launch_mfma(p, srt::mfma_config(p, 2), stream);
+    case kPlanMfma128: return srt::short_supported(p) ? srt::launch_short(p, stream) : srt::launch_mfma(p, srt::mfma_config(p, 2), stream);
     case kPlanMfma64: return srt::launch_mfma(p, srt::mfma_config(p, 3), stream);
     case kPlanKc64: return srt::launch_mfma(p, srt::mfma_config(p, 4), stream);
     case kPlanM16: return srt::launch_mfma(p, srt::mfma_config(p, 5), stream);
     case kPlanSplitK: return srt::launch_mfma_splitk(p, stream);
     case kPlanM16H: return srt::launch_mfma(p, srt::mfma_config(p, 6), stream);
-    case kPlanAny128: return srt::launch_mfma(p, srt::mfma_config(p, 7), stream);
+    case kPlanAny128: return srt::short_supported(p) ? srt::launch_short(p, stream) : srt::launch_mfma(p, srt::mfma_config(p, 7), stream);
     case kPlanAny64: return srt::launch_mfma(p, srt::mfma_config(p, 8), stream);
     case kPlanM16D: return srt::launch_mfma(p, srt::mfma_config(p, 9), stream);
     case kPlanM16DTail: return srt::launch_mfma(p, srt::mfma_config(p, 10), stream);
