@@ -414,12 +414,16 @@ hipError_t launch(const GemmProblem& p, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds_bytes, stream, p, walk);
     return launch_status(stream);
   };
-  static std::atomic<uint32_t> configured[3];
+  static std::atomic<uint32_t> configured[4];
   const bool several = walk.tiles > (uint32_t)compute_units();
   if constexpr (TILES == 1) {
     // operands of one XCD's L2 or less reach every unit in any order: the walk's arithmetic is 0.2 us for nothing
     const long long bytes = ((long long)p.M + p.N) * p.K * p.batch * (long long)sizeof(typename T::storage);
-    if (!walk.tiles || (!several && bytes <= (4LL << 20))) return go(gemm_waves_kernel<T, A_KC, B_KC, 1, 8, false>, 8, false, configured[0]);
+    const bool any_order = bytes <= (4LL << 20);
+    if (!walk.tiles || (!several && any_order)) return go(gemm_waves_kernel<T, A_KC, B_KC, 1, 8, false>, 8, false, configured[0]);
+    // (several tiles a unit and a k loop of two slabs: 2 x 720 x 344 x 48 4.16 us by walk, 3.43; longer ones share enough for it to pay,
+    // 384 x 1052 x 1234 7.0 and 8.7)
+    if (any_order && p.K <= 128) return go(gemm_waves_kernel<T, A_KC, B_KC, 1, 4, false>, 4, false, configured[3]);
   }
   if (several) return go(gemm_waves_kernel<T, A_KC, B_KC, TILES, 4, true>, 4, true, configured[1]);
   return go(gemm_waves_kernel<T, A_KC, B_KC, TILES, 8, true>, 8, true, configured[2]);
