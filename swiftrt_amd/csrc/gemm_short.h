@@ -2,7 +2,8 @@
 //
 // A k loop of one to four 64-deep slabs is over before a ring of prefetched stages has filled, and a kernel that takes a whole
 // compute unit has nothing else to run while its tile is stored: 64 x 512 x 512 x 64 x . W^T took 12.5 us for 42 MB.  Here a
-// workgroup needs 33 KB of LDS and 128 registers, so four share a unit, and one's stores run beside another's loads.
+// workgroup needs 33 KB of LDS and under 100 registers (one slab; 172 for more), so four (two or three) share a unit, and one's stores
+// run beside another's loads.
 //
 //   bound   the result's stores, then the operands' loads (each XCD's L2 holds what its neighbouring tiles share: the walk of
 //           gemm_waves.h)
@@ -12,6 +13,8 @@
 //   store   through LDS ([128 rows][16 chunks of 16 bytes], chunk c of row r at c ^ (r & 15)): 16 bytes a lane, whole rows of a tile
 //   bias    in LDS from the start, so that the epilogue waits for no load
 #pragma once
+#include <type_traits>
+
 #include "gemm_waves.h"
 
 namespace srt {
@@ -19,8 +22,9 @@ namespace shortk {
 
 constexpr int EDGE = 128, OPERAND = 4 * 4096, BIAS = 2 * OPERAND, LDS_BYTES = BIAS + EDGE * 4;
 
-template <typename T, bool A_KC, bool B_KC>
-__global__ __launch_bounds__(256, 2) void gemm_short_kernel(GemmProblem p, waves::Walk walk) {
+// ONE: a single slab, whose registers are free for the sums once it is in LDS: four workgroups a unit instead of two or three.
+template <typename T, bool A_KC, bool B_KC, bool ONE>
+__global__ __launch_bounds__(256, ONE ? 4 : 2) void gemm_short_kernel(GemmProblem p, waves::Walk walk) {
   using S = typename T::storage;
   using StageA = waves::Stage<T, A_KC, 1, A_KC || B_KC>;
   using StageB = waves::Stage<T, B_KC, 1, A_KC || B_KC>;
@@ -58,12 +62,12 @@ __global__ __launch_bounds__(256, 2) void gemm_short_kernel(GemmProblem p, waves
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
-  const int slabs = (p.K + DEPTH - 1) / DEPTH;
+  const int slabs = ONE ? 1 : (p.K + DEPTH - 1) / DEPTH;
   for (int s = 0; s < slabs; ++s) {
     sa.store(ra, s * DEPTH, my_a);
     sb.store(rb, s * DEPTH, my_b);
     __syncthreads();
-    if (s + 1 < slabs) {
+    if (!ONE && s + 1 < slabs) {
       sa.load(ra, (s + 1) * DEPTH);
       sb.load(rb, (s + 1) * DEPTH);
     }
@@ -130,13 +134,19 @@ __global__ __launch_bounds__(256, 2) void gemm_short_kernel(GemmProblem p, waves
   __syncthreads();
   S* C = (S*)p.C + (long long)bz * p.scb;
   const int c = tid & 15, n = n0 + 8 * c;
+  // rows of whole cache lines go past the caches, up to what those would hold of them in part (64 x 512 x 512 x 64 x . W^T 11.3 -> 10.8 us,
+  // x 128 14.8 -> 12.6); lines that two tiles share must meet in L2 (1064-column rows lost a third)
+  const bool stream = ((p.N | (int)p.scm | (int)p.scb) & 63) == 0 && (reinterpret_cast<uintptr_t>(p.C) & 127u) == 0 &&
+                      (long long)p.M * p.N * p.batch <= (64LL << 20);
 #pragma unroll
   for (int it = 0; it < 8; ++it) {
     const int row = 16 * it + (tid >> 4), m = m0 + row;
     if (m >= p.M || n >= p.N) continue;
     const waves::u32x4_t w = *reinterpret_cast<const SRT_LDS waves::u32x4_t*>(lds_a + (uint32_t)(row * 256 + ((c ^ (row & 15)) << 4)));
     S* dst = C + (long long)m * p.scm + n;
-    if (n + 8 <= p.N) {
+    if (stream) {
+      __builtin_nontemporal_store(w, reinterpret_cast<waves::u32x4_t*>(dst));
+    } else if (n + 8 <= p.N) {
       __builtin_memcpy(dst, &w, 16);
     } else {
 #pragma unroll
@@ -156,10 +166,15 @@ hipError_t launch(const GemmProblem& p, hipStream_t stream) {
   const waves::Walk walk = waves::make_walk(p.M, p.N, p.batch, EDGE);
   const dim3 grid(8 * walk.chunk), block(256);
   const bool a_kc = p.sak == 1, b_kc = p.sbn != 1;
-  if (a_kc && b_kc) hipLaunchKernelGGL((gemm_short_kernel<T, true, true>), grid, block, 0, stream, p, walk);
-  else if (a_kc) hipLaunchKernelGGL((gemm_short_kernel<T, true, false>), grid, block, 0, stream, p, walk);
-  else if (b_kc) hipLaunchKernelGGL((gemm_short_kernel<T, false, true>), grid, block, 0, stream, p, walk);
-  else hipLaunchKernelGGL((gemm_short_kernel<T, false, false>), grid, block, 0, stream, p, walk);
+  auto layout = [&](auto one) {
+    constexpr bool ONE = decltype(one)::value;
+    if (a_kc && b_kc) hipLaunchKernelGGL((gemm_short_kernel<T, true, true, ONE>), grid, block, 0, stream, p, walk);
+    else if (a_kc) hipLaunchKernelGGL((gemm_short_kernel<T, true, false, ONE>), grid, block, 0, stream, p, walk);
+    else if (b_kc) hipLaunchKernelGGL((gemm_short_kernel<T, false, true, ONE>), grid, block, 0, stream, p, walk);
+    else hipLaunchKernelGGL((gemm_short_kernel<T, false, false, ONE>), grid, block, 0, stream, p, walk);
+  };
+  if (p.K <= 64) layout(std::true_type{});
+  else layout(std::false_type{});
   return launch_status(stream);
 }
 

@@ -317,13 +317,17 @@ bool prefers_waves(const GemmProblem& p, Plan plan) {
 
 // Whether a problem with a short k loop runs on 128 x 128 tiles instead of on copies of its operands or small tiles: from five
 // quarters of a tile a unit -- at the first few past one, most units wait for those that have two --, below that where
-// the estimate is ahead of copies and of 64 x 64 tiles by elements.
+// the estimate is ahead of copies and of 64 x 64 tiles by elements.  A k loop of one slab: instead of the 256 x 256 kernels too, whose tiles
+// are all epilogue (365 random problems of 4 Mi results and more: 1.3x, none under 0.95x; 3072 x 6336 x 64 x . W 15.4 / 12.0,
+// 2544 x 4088 x 56 x . W^T 10.2 / 7.7), and of the 128 x 256 ones of a single matrix (1.1x; batches of small ones are even).
 bool prefers_short(const GemmProblem& p, Plan plan) {
-  const bool others = plan == kPlanCopied || plan == kPlanAny64 || plan == kPlanAny128;
-  if ((!others && plan != kPlanMfma64) || !srt::short_supported(p)) return false;
+  if (!srt::short_supported(p)) return false;
+  const bool one_slab = p.K <= 64 && (plan == kPlanM16 || plan == kPlanRing256 || plan == kPlanKc64 || (plan == kPlanM16H && p.batch == 1));
+  const bool others = one_slab || plan == kPlanCopied || plan == kPlanAny64 || plan == kPlanAny128;
+  if (!others && plan != kPlanMfma64) return false;
   const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, cus = srt::compute_units();
   if (4 * tiles >= 5 * cus) return true;
-  return others && tiles <= cus && srt::short_us(p) < plan_us(p, plan);
+  return others && tiles <= cus && srt::short_us(p) < 0.95 * plan_us(p, plan);
 }
 
 Plan heuristic_plan(const GemmProblem& p, bool copies = true) {

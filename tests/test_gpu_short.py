@@ -20,7 +20,7 @@ def clean_cache():
 # of a wave's quarter of one and of a chunk; a batch; more tiles than units; one row of tiles; aligned operands
 @pytest.mark.parametrize("M,N,K,batch,frame", [(128, 128, 64, 1, (0, 0)), (129, 255, 65, 1, (3, 2)), (33, 161, 13, 1, (3, 2)), (97, 31, 200, 3, (0, 0)),
                                                (300, 9, 256, 1, (3, 2)), (1500, 3001, 70, 1, (1, 0)), (20, 5003, 129, 1, (3, 2)), (260, 301, 350, 1, (0, 0)),
-                                               (2048, 2080, 40, 1, (8, 8)), (130, 8, 8, 2, (3, 2))])
+                                               (2048, 2080, 40, 1, (8, 8)), (700, 1088, 61, 2, (0, 0)), (130, 8, 8, 2, (3, 2))])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("dt", [H.BF16, H.F16])
 def test_exact_inside_the_view(tmp_path, dt, M, N, K, batch, frame, ta, tb):
