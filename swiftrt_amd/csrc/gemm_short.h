@@ -161,9 +161,20 @@ inline bool fits(const GemmProblem& p) {
   return (p.dtype == srtReal16BF || p.dtype == srtReal16F) && waves::fits(p) && p.scn == 1 && waves::make_walk(p.M, p.N, p.batch, EDGE).tiles != 0;
 }
 
+// Whether tiles that follow each other lie along the result's rows: where two of them share a line (rows of other than whole lines) and a
+// column of tiles is long, the second half of a line otherwise comes a column later, when L2 has written the first half out.  us, down
+// the columns / along the rows, bf16: 8192 x 9001 x 40 67.7 / 40.4, 8192 x 9001 x 64 x . W^T 68.3 / 39.9, 8192 x 12003 x 256 157 / 117, 7001 x 7400 x 33 40.7 /
+// 27.6, 6100 x 9001 x 150 62.9 / 56.2, 4200 x 9001 x 40 25.2 / 22.6, 4 x 3000 x 3333 x 64 27.5 / 25.1, 6 x 3501 x 3502 x 64 54.2 / 39.6.  Fewer
+// results stay in L2 either way, and down the columns neighbours do not write one line at a time: 3072 x 9001 x 150 31.6 / 33.7, 4000 x 4999 x
+// 130 21.8 / 23.3, 2048 x 2049 x 40 7.5 / 8.2.  (Rows of whole lines share none: 8192^2 x 64 30.2 / 32.0, though 3712 x 16384 x 64 39.8 / 27.4.)
+inline bool along_rows(const GemmProblem& p) {
+  const bool whole_lines = ((p.N | (int)p.scm | (int)p.scb) & 63) == 0 && (reinterpret_cast<uintptr_t>(p.C) & 127u) == 0;
+  return !whole_lines && p.M > 20 * EDGE && (long long)p.M * p.N * p.batch >= (32LL << 20);
+}
+
 template <typename T>
 hipError_t launch(const GemmProblem& p, hipStream_t stream) {
-  const waves::Walk walk = waves::make_walk(p.M, p.N, p.batch, EDGE);
+  const waves::Walk walk = waves::make_walk(p.M, p.N, p.batch, EDGE, along_rows(p));
   const dim3 grid(8 * walk.chunk), block(256);
   const bool a_kc = p.sak == 1, b_kc = p.sbn != 1;
   auto layout = [&](auto one) {

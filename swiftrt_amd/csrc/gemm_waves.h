@@ -216,17 +216,18 @@ struct Stage {
 };
 
 // The walk over the tiles: workgroup id runs on XCD id % 8 (each has its own L2), which takes the id / 8-th of its consecutive
-// eighth of the tiles, the shorter side of the grid of tiles fastest, so that an XCD's tiles share rows and columns.
+// eighth of the tiles, the shorter side of the grid of tiles fastest, so that an XCD's tiles share rows and columns (along_rows: always
+// the columns of tiles fastest).
 struct Walk {
   uint32_t tiles, chunk;    // in total, per XCD
   uint32_t fast, slow;      // extents of the grid of tiles, in walk order
   uint32_t fast_rcp, slow_rcp;   // ceil(2^32 / extent): quotients of indexes below 2^16 by one multiplication (0: divide)
   int fast_is_m;
 };
-inline Walk make_walk(int M, int N, int batch, int edge) {
+inline Walk make_walk(int M, int N, int batch, int edge, bool along_rows = false) {
   Walk w;
   const uint32_t tm = (uint32_t)((M + edge - 1) / edge), tn = (uint32_t)((N + edge - 1) / edge);
-  w.fast_is_m = tm <= tn;
+  w.fast_is_m = tm <= tn && !along_rows;
   w.fast = w.fast_is_m ? tm : tn;
   w.slow = w.fast_is_m ? tn : tm;
   const unsigned long long all = (unsigned long long)tm * tn * (unsigned long long)batch;

@@ -47,3 +47,16 @@ def test_epilogues(act, order):
     # one rounding to bf16 (eight significant bits: half a step is at most 2^-8 of the value), the sum's own error (90 x 2^-24 x the
     # products' magnitudes, under 40) and the fast forms' 2^-14
     assert np.all(np.abs(got - want) <= (2.0 ** -8 + 2.0 ** -14) * np.abs(want) + 90 * 2.0 ** -24 * 40)
+
+
+def test_tiles_along_the_rows():
+    """Results of 32 Mi and more in rows of other than whole lines: every tile once, the last ones of either side partial.  Sums of 24 products of
+    -1, 0 and 1 and a bias up to 3 are exact in bf16."""
+    M, N, K = 2690, 12501, 24
+    g = H.rng(31)
+    x, w, b = g.integers(-1, 2, (M, K)), g.integers(-1, 2, (K, N)), g.integers(-3, 4, N)
+    xt, wt, bt = (srt.Tensor(H.encode(v.astype(np.float64), H.BF16)) for v in (x, w, b))
+    with H.pinned("mfma_128x128_any", H.BF16, M, N, K, 25, (1 | (int(srt.ActivationType.identity) << 1),)):
+        got = srt.Dense(wt, bt, srt.ActivationType.identity)(xt).array()
+    want = x.astype(np.float32) @ w.astype(np.float32) + b.astype(np.float32)
+    assert np.array_equal(got, (want.view(np.uint32) >> 16).astype(np.uint16))
