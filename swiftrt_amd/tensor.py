@@ -473,6 +473,7 @@ class LSTMCell:
 
     def __call__(self, x, cell, hidden):
         # (a cell of another kind -- broadcast gates, more columns, another element type -- answers for itself below)
+        new_cell = new_hidden = None
         if len(x.shape) == 2 and cell.shape == hidden.shape and x.dtype == hidden.dtype == cell.dtype:
             new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
             new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
@@ -484,7 +485,8 @@ class LSTMCell:
             # gates broadcast against the cell's shape, or a weight with columns past the fourth part: operator by operator
             new_cell = (cell * sigmoid(self.part(2, fused)) + sigmoid(self.part(0, fused)) * tanh(self.part(1, fused)))
             return new_cell, tanh(new_cell) * sigmoid(self.part(3, fused))
-        new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
-        new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
+        if new_cell is None:
+            new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
+            new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
         current_queue().lstm_gates(fused, cell, new_cell, new_hidden)
         return new_cell, new_hidden
