@@ -472,9 +472,9 @@ class LSTMCell:
         return fused[:, i * h:(i + 1) * h]
 
     def __call__(self, x, cell, hidden):
-        # (a cell of another kind -- broadcast gates, more columns, another element type -- answers for itself below)
+        # (a cell of another kind -- no bias, broadcast gates, more columns, another element type -- answers for itself below)
         new_cell = new_hidden = None
-        if len(x.shape) == 2 and cell.shape == hidden.shape and x.dtype == hidden.dtype == cell.dtype:
+        if self.fused_bias is not None and len(x.shape) == 2 and cell.shape == hidden.shape and x.dtype == hidden.dtype == cell.dtype:
             new_cell = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
             new_hidden = Tensor(shape=cell.shape, dtype=cell.dtype, order=cell.order)
             if current_queue().lstm_cell(x, cell, hidden, self.fused_weight, self.fused_bias, new_cell, new_hidden):

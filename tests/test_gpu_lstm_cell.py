@@ -69,3 +69,15 @@ def test_cells_left_to_the_three_calls():
     new = srt.Tensor(shape=[8, 16], dtype=np.float32)
     for nc, nh in ((cell, new), (new, hidden), (new, new), (new, x)):   # other workgroups still read what one would store
         assert not q().lstm_cell(x, cell, hidden, weight, bias, nc, nh)
+
+
+@pytest.mark.parametrize("dt", [H.F32, H.BF16])
+def test_a_cell_without_a_bias(dt):
+    x, cell, hidden, weight, _ = cell_inputs(dt, 9, 24, 16, 5)
+    layer = srt.LSTMCell(weight, None)
+    got = layer(x, cell, hidden)
+    gates = srt.matmul(srt.concatenate(x, hidden, 1), weight)
+    update, add, keep, out = (layer.part(i, gates) for i in range(4))
+    new_cell = cell * srt.sigmoid(keep) + srt.sigmoid(update) * srt.tanh(add)
+    for a, w in zip(got, (new_cell, srt.tanh(new_cell) * srt.sigmoid(out))):
+        assert np.array_equal(bits(a), bits(w))
