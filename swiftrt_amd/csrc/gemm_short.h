@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256, ONE ? 4 : 2) void gemm_short_kernel(GemmProble
 
 // Unit strides along k or along m / n, as the wave-split tiles; the result's rows contiguous.
 inline bool fits(const GemmProblem& p) {
-  return (p.dtype == srtReal16BF || p.dtype == srtReal16F) && waves::fits(p) && p.scn == 1 && waves::make_walk(p.M, p.N, p.batch, EDGE).tiles != 0;
+  return (p.dtype == srtReal16BF || p.dtype == srtReal16F) && waves::reads(p) && p.scn == 1 && waves::make_walk(p.M, p.N, p.batch, EDGE).tiles != 0;
 }
 
 // Whether tiles that follow each other lie along the result's rows: where two of them share a line (rows of other than whole lines) and a

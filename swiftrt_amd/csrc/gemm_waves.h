@@ -27,6 +27,7 @@
 //           320 x 3759 x 3648 159 / 98
 #pragma once
 #include "gemm_common.h"
+#include "walk.h"
 
 namespace srt {
 namespace waves {
@@ -215,30 +216,6 @@ struct Stage {
   }
 };
 
-// The walk over the tiles: workgroup id runs on XCD id % 8 (each has its own L2), which takes the id / 8-th of its consecutive
-// eighth of the tiles, the shorter side of the grid of tiles fastest, so that an XCD's tiles share rows and columns (along_rows: always
-// the columns of tiles fastest).
-struct Walk {
-  uint32_t tiles, chunk;    // in total, per XCD
-  uint32_t fast, slow;      // extents of the grid of tiles, in walk order
-  uint32_t fast_rcp, slow_rcp;   // ceil(2^32 / extent): quotients of indexes below 2^16 by one multiplication (0: divide)
-  int fast_is_m;
-};
-inline Walk make_walk(int M, int N, int batch, int edge, bool along_rows = false) {
-  Walk w;
-  const uint32_t tm = (uint32_t)((M + edge - 1) / edge), tn = (uint32_t)((N + edge - 1) / edge);
-  w.fast_is_m = tm <= tn && !along_rows;
-  w.fast = w.fast_is_m ? tm : tn;
-  w.slow = w.fast_is_m ? tn : tm;
-  const unsigned long long all = (unsigned long long)tm * tn * (unsigned long long)batch;
-  w.tiles = all < (1u << 30) ? (uint32_t)all : 0u;   // (0: too many for the walk's one grid dimension)
-  w.chunk = (w.tiles + 7) / 8;
-  // (exact while index x extent < 2^32: the reciprocal is too large by less than extent / 2^32)
-  auto rcp = [&](uint32_t d) { return w.tiles <= 0xffffu && d > 1 ? (uint32_t)((0x100000000ull + d - 1) / d) : 0u; };
-  w.fast_rcp = rcp(w.fast);
-  w.slow_rcp = rcp(w.slow);
-  return w;
-}
 __device__ __forceinline__ uint32_t quotient(uint32_t n, uint32_t d, uint32_t rcp) { return rcp ? __umulhi(n, rcp) : d == 1 ? n : n / d; }
 
 // WALK: workgroups take tiles by `walk`; otherwise the grid is (columns, rows, matrices) of tiles.
@@ -439,7 +416,7 @@ hipError_t launch_layout(const GemmProblem& p, hipStream_t stream) {
 }
 
 // Both operands have a unit stride, with at least one whole vector along it, and a pitch below 2^31; there is something to sum.
-inline bool fits(const GemmProblem& p) {
+inline bool reads(const GemmProblem& p) {
   const int per = p.dtype == srtReal32F ? 4 : 8;
   if (p.K < 1) return false;
   if (p.sak == 1 ? p.K < per : (p.sam != 1 || p.M < per)) return false;
@@ -447,6 +424,11 @@ inline bool fits(const GemmProblem& p) {
   const long long lda = p.sak == 1 ? p.sam : p.sak, ldb = p.sbn == 1 ? p.sbk : p.sbn;
   if (lda < 0 || lda > 0x7fffffffLL || ldb < 0 || ldb > 0x7fffffffLL) return false;
   return (p.M + 31) / 32 <= 65535 && p.batch <= 65535;
+}
+// And some grid holds the 32 x 32 tiles: the walk's, or (columns, rows, matrices) of them with eight waves each.
+inline bool fits(const GemmProblem& p) {
+  if (!reads(p)) return false;
+  return make_walk(p.M, p.N, p.batch, 32).tiles != 0 || ((uint64_t)p.N + 31) / 32 * 512 <= kMostThreads;
 }
 
 }  // namespace waves
