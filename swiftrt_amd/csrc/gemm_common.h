@@ -249,10 +249,24 @@ struct Epilogue {
           if (at(q, &m, &n)) b[q] = T::to_float(bias[(long long)(per_row ? m : n) * sbias]);
         }
       }
+      // (one switch a run, not one an element: half a microsecond of a launch-sized problem's tiles under sigmoid or tanh)
+      constexpr bool FAST = sizeof(typename T::storage) == 2;
+      auto each = [&](auto f) {
 #pragma unroll
-      for (int q = 0; q < COUNT; ++q)
-        v[q] = sizeof(typename T::storage) == 2 ? apply_activation_16(activation, coef, v[q] + b[q])
-                                                : apply_activation(activation, coef, v[q] + b[q]);
+        for (int q = 0; q < COUNT; ++q) v[q] = f(v[q] + b[q]);
+      };
+      switch (activation) {
+        case srtActivationSigmoid:
+          each([&](float x) { return FAST ? activation16_ct<srtActivationSigmoid>(coef, x) : activation_ct<srtActivationSigmoid>(coef, x); });
+          break;
+        case srtActivationTanh:
+          each([&](float x) { return FAST ? activation16_ct<srtActivationTanh>(coef, x) : activation_ct<srtActivationTanh>(coef, x); });
+          break;
+        case srtActivationElu:
+          each([&](float x) { return FAST ? activation16_ct<srtActivationElu>(coef, x) : activation_ct<srtActivationElu>(coef, x); });
+          break;
+        default: each([&](float x) { return activation_ct<srtActivationClippedRelu>(coef, x); }); break;
+      }
     }
   }
 };

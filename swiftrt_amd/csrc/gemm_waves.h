@@ -342,39 +342,46 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_waves_kernel(GemmProblem p, W
 
   Epilogue<T> ep(p);
   S* C = (S*)p.C + (long long)bz * p.scb;
-  constexpr int CHUNKS = 8 * TILES;   // chunks of four columns in a row of the tile
+  // every lane has a share, two consecutive columns where eight waves finish one 32 x 32 tile: four columns of half the lanes were 0.2-0.4 us
+  // more under libm's activations (fp32 7 x 64 x 72 x 64 x . W^T, tanh: 4.4 and 3.9)
+  constexpr int COLS = EDGE * EDGE / 4 < 64 * WAVES ? 2 : 4, PIECES = EDGE / COLS;   // pieces of COLS columns in a row of the tile
+  static_assert(EDGE * PIECES % (64 * WAVES) == 0, "whole rounds of the lanes");
+  typedef float piece_t __attribute__((ext_vector_type(COLS)));
 #pragma unroll
-  for (int id = 0; id < EDGE * CHUNKS; id += 64 * WAVES) {
+  for (int id = 0; id < EDGE * PIECES; id += 64 * WAVES) {
     const int q = id + tid;
-    if (EDGE * CHUNKS < 64 * WAVES && q >= EDGE * CHUNKS) return;
-    const int row = q / CHUNKS, c = q % CHUNKS, r = row & 31;
-    const int m = m0 + row, n = n0 + 4 * c;
+    const int row = q / PIECES, c = q % PIECES * COLS, r = row & 31;
+    const int m = m0 + row, n = n0 + c;
     if (m >= p.M || n >= p.N) continue;
-    const uint32_t at = lds + (uint32_t)(((row >> 5) * TILES + (c >> 3)) * TILE + r * 128 + (((c & 7) ^ ((r >> 1) & 7)) << 4));
-    f32x4_t part[WAVES];
+    const uint32_t at = lds + (uint32_t)(((row >> 5) * TILES + (c >> 5)) * TILE + r * 128 + ((((c >> 2) & 7) ^ ((r >> 1) & 7)) << 4) + (c & 3) * 4);
+    piece_t part[WAVES];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) part[w] = *reinterpret_cast<const SRT_LDS f32x4_t*>(at + (uint32_t)(w * PART));
+    for (int w = 0; w < WAVES; ++w) part[w] = *reinterpret_cast<const SRT_LDS piece_t*>(at + (uint32_t)(w * PART));
 #pragma unroll
     for (int step = 1; step < WAVES; step *= 2)
 #pragma unroll
       for (int w = 0; w < WAVES; w += 2 * step) part[w] += part[w + step];
-    float out[4] = {part[0][0], part[0][1], part[0][2], part[0][3]};
+    float out[COLS];
+#pragma unroll
+    for (int e = 0; e < COLS; ++e) out[e] = part[0][e];
     ep.finish_run(out, [&](int e, int* mm, int* nn) {
       *mm = m;
       *nn = n + e;
       return n + e < p.N;
     });
     S* dst = C + (long long)m * p.scm + (long long)n * p.scn;
-    if (p.scn == 1 && n + 4 <= p.N) {   // one store, at whatever alignment the row has
+    if (p.scn == 1 && n + COLS <= p.N) {   // one store, at whatever alignment the row has
       if constexpr (sizeof(S) == 2) {
-        const u32x2_t w = {T::template pack2<true>(out[0], out[1]), T::template pack2<true>(out[2], out[3])};
-        __builtin_memcpy(dst, &w, 8);
+        uint32_t w[COLS / 2];
+#pragma unroll
+        for (int e = 0; e < COLS; e += 2) w[e / 2] = T::template pack2<true>(out[e], out[e + 1]);
+        __builtin_memcpy(dst, w, sizeof(w));
       } else {
-        __builtin_memcpy(dst, out, 16);
+        __builtin_memcpy(dst, out, sizeof(out));
       }
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < COLS; ++e)
         if (n + e < p.N) dst[(long long)e * p.scn] = T::from_float(out[e]);
     }
   }
