@@ -315,6 +315,23 @@ bool prefers_waves(const GemmProblem& p, Plan plan) {
   return here < (plan == kPlanMfma64 ? 0.88 : 0.95) * other;   // (that kernel's estimate spreads most)
 }
 
+bool curved(int activation) { return activation == srtActivationSigmoid || activation == srtActivationTanh || activation == srtActivationElu; }
+
+// Whether copied operands are ahead of the 128 x 128 tiles for short k loops after all: their 256 x 256 tiles read an operand half as often, which
+// tells once a unit has many tiles of three slabs or more and the larger ones come out in whole rounds (11 us each into whole lines, 13.4 into
+// whole chunks, 15.5 into others).  230 random problems whose other plan is copies, us, copies / those tiles: 12191 x 5312 x 216 x^T . W^T 54 / 67,
+// 8512 x 9280 x 143 62 / 73, 2963 x 9728 x 256 29 / 35, 9712 x 8251 x 256 x . W 81 / 104, 15996 x 2709 x 221 51 / 60; not 6510 x 5768 x 256
+// x^T . W^T 48 / 42, 6562 x 8768 x 192 x^T . W 47 / 44, nor under an activation with an exponential, 5760 x 7032 x 156 tanh 83 / 50.
+bool copies_ahead(const GemmProblem& p) {
+  const double cus = srt::compute_units(), slabs = (p.K + 63) / 64;
+  auto tiles = [&](int edge) { return (double)((p.M + edge - 1) / edge) * (double)((p.N + edge - 1) / edge) * (double)p.batch / cus; };
+  const bool chunks = srt::c_whole_chunks(p), lines = ((p.N | (int)p.scm | (int)p.scb) & 63) == 0 && (reinterpret_cast<uintptr_t>(p.C) & 127u) == 0;
+  const double t = tiles(128);
+  if (curved(p.activation) || t < 6.0 || slabs < (chunks ? 3.0 : 4.0)) return false;
+  const double here = 4.6 + t * (1.26 + 0.73 * slabs + (chunks ? 0.0 : 0.9));
+  return 8.0 + __builtin_ceil(tiles(256)) * (lines ? 11.0 : chunks ? 13.4 : 15.5) < 0.93 * here;
+}
+
 // Whether a problem with a short k loop runs on 128 x 128 tiles instead of on copies of its operands or small tiles: from five
 // quarters of a tile a unit -- at the first few past one, most units wait for those that have two --, below that where
 // the estimate is ahead of copies and of 64 x 64 tiles by elements.  A k loop of one slab: instead of the 256 x 256 kernels too, whose tiles
@@ -326,7 +343,7 @@ bool prefers_short(const GemmProblem& p, Plan plan) {
   const bool others = one_slab || plan == kPlanCopied || plan == kPlanAny64 || plan == kPlanAny128;
   if (!others && plan != kPlanMfma64) return false;
   const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, cus = srt::compute_units();
-  if (4 * tiles >= 5 * cus) return true;
+  if (4 * tiles >= 5 * cus) return plan != kPlanCopied || !copies_ahead(p);
   return others && tiles <= cus && srt::short_us(p) < 0.95 * plan_us(p, plan);
 }
 

@@ -1,0 +1,30 @@
+"""The kernel chosen where two are close: problems measured on both, by the kernel query."""
+import ctypes
+
+import pytest
+
+from swiftrt_amd import native
+
+BF16, F16, F32 = native.REAL16BF, native.REAL16F, native.REAL32F
+
+
+def query(dt, M, N, K, ta=False, tb=False, batch=1):
+    def descriptor(rows, columns):
+        if batch == 1:
+            return native.make_descriptor(dt, (rows, columns), (columns, 1), native.ORDER_ROW)
+        return native.make_descriptor(dt, (batch, rows, columns), (rows * columns, columns, 1), native.ORDER_ROW)
+
+    (ad, k1), (bd, k2), (od, k3) = descriptor(*((K, M) if ta else (M, K))), descriptor(*((N, K) if tb else (K, N))), descriptor(M, N)
+    buf, p = ctypes.create_string_buffer(64), ctypes.c_void_p(256)
+    assert native.lib().srtMatmulQueryKernel(ctypes.byref(ad), int(ta), ctypes.byref(bd), int(tb), ctypes.byref(od), p, p, p, buf, 64) == 0
+    return buf.value.decode()
+
+
+# us, copies / 128 x 128 tiles for short k loops
+@pytest.mark.parametrize("dt,M,N,K,ta,tb,plan", [
+    (BF16, 12191, 5312, 216, True, True, "copied"), (BF16, 8512, 9280, 143, True, True, "copied"),           # 54 / 67, 62 / 73
+    (BF16, 2963, 9728, 256, True, True, "copied"), (F16, 9712, 8251, 256, False, False, "copied"),           # 29 / 35, 81 / 104
+    (BF16, 6510, 5768, 256, True, True, "mfma_128x128_any"), (F16, 6562, 8768, 192, True, False, "mfma_128x128_any"),   # 48 / 42, 47 / 44
+    (BF16, 4288, 7769, 104, False, True, "mfma_128x128"), (BF16, 2772, 2023, 120, True, False, "mfma_128x128_any")])   # 62 / 28, 22 / 9.5
+def test_copies_and_short_k_loops(dt, M, N, K, ta, tb, plan):
+    assert query(dt, M, N, K, ta, tb) == plan
