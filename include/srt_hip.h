@@ -425,7 +425,7 @@ srtStatus srtLstmGates(const void* gates, const srtTensorDescriptor* gatesDesc, 
  * [B, H]; one element type (32F, 16F, 16BF) and row order for all.  srtErrorNotSupported -- nothing was launched, and the caller runs
  * srtConcat, srtMatmulBiasActivation and srtLstmGates (or the element-wise calls) instead -- for other shapes, H not a multiple of 8,
  * rows (except the cell's) that are not contiguous, results that share memory with an operand or each other, and cells
- * large enough for the product's own kernels to be ahead. */
+ * whose rows, columns or depth I + H put the product's own kernels ahead. */
 srtStatus srtLstmCell(const void* x, const srtTensorDescriptor* xDesc, const void* hidden, const srtTensorDescriptor* hiddenDesc,
                       const void* weight, const srtTensorDescriptor* weightDesc, const void* bias, const srtTensorDescriptor* biasDesc,
                       const void* cell, const srtTensorDescriptor* cellDesc, void* newCell, const srtTensorDescriptor* newCellDesc,

@@ -166,11 +166,17 @@ hipError_t launch(const CellProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
-// Whether one launch is ahead of the three: while a unit has two of its tiles at most (128 x 1024 x 1024, fp32 34.5 us in three, 32.8 in
-// one; bf16 21.5 and 21.9; 256 x 1024 x 512 26.7 / 24.3 and 19.4 / 17.6).  Beyond that the product alone runs on larger tiles, which
-// read the operands less often.
-bool launch_choice(const CellProblem& p) {
-  return (long long)((p.rows + 31) / 32) * (p.hidden / GROUP) <= 2LL * compute_units();
+// Whether one launch is ahead of the three: while k is short against the product's own kernels, which cut a long one over idle units and
+// read the weight in larger tiles.  By the depth D = I + H and the slabs a unit walks (D times its tiles), device times of 8000 random cells
+// of 1-1024 x 8-16384 x 8-4096, three / one, us, bf16: 32 x 1024 x 1024 18.8 / 9.5, 8 x 2048 x 1024 21.7 / 12.3, 128 x 512 x 1024 18.4 / 17.8, but
+// 64 x 512 x 2048 24.2 / 30.4, 128 x 4096 x 1024 27.5 / 50.7, 8 x 8192 x 256 26.4 / 36.9; fp32 64 x 1024 x 1024 21.0 / 18.8, 32 x 4096 x 1024 39.9 / 38.6,
+// but 64 x 64 x 2048 33.7 / 37.7, 64 x 8192 x 2048 122 / 214.  Up to four groups of columns a product of few columns idles as well: 64 x 16384 x 8
+// 55.9 / 21.9.  1 cell in 60 that this takes is more than 5 % behind its three calls (the bound of two tiles a unit alone: 1 in 5).
+bool launch_choice(const CellProblem& p, bool f32) {
+  const long long tiles = (long long)((p.rows + 31) / 32) * (p.hidden / GROUP), cus = compute_units();
+  const long long depth = (long long)p.inputs + p.hidden, walk = depth * tiles;
+  if (tiles > 2 * cus || (depth > (f32 ? 8192 : 4096) && p.hidden > 32)) return false;
+  return walk <= (f32 || depth <= 1300 ? 2600 : 1800) * cus;
 }
 
 bool row_ok(long long stride) { return stride >= 0 && stride <= 0x7fffffffLL; }
@@ -211,7 +217,7 @@ extern "C" srtStatus srtLstmCell(const void* x, const srtTensorDescriptor* xDesc
   p.bias_step = (long long)biasDesc->strides[0];
   p.cell_row = (long long)cellDesc->strides[0]; p.cell_col = (long long)cellDesc->strides[1];
   p.new_cell_row = (long long)newCellDesc->strides[0]; p.new_hidden_row = (long long)newHiddenDesc->strides[0];
-  if (!srt::launch_choice(p) || (rows + 31) / 32 > 65535) return srtErrorNotSupported;
+  if (!srt::launch_choice(p, per == 4) || (rows + 31) / 32 > 65535) return srtErrorNotSupported;
 
   // workgroups read x, h and the weight while others store: the results share no memory with any operand, nor with one another
   const size_t es = per == 4 ? 4 : 2;
