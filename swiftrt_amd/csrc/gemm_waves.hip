@@ -7,7 +7,9 @@ namespace {
 // Estimates in microseconds (256 units), fitted to 1900 random problems of 1-64 matrices, 1-8192 x 32-16384 x 32-8192, all layouts; a
 // tile reads 128 K (32 x 32) or 256 K (64 x 64) bytes, an operand whose rows are off the 16-byte boundaries costs a sixth more, a third along m / n:
 //   32 x 32   one tile a unit 3.4 + its bytes at 97 a ns; several 3.3 + each 0.26 + its bytes at 70
-//   64 x 64   4.6 + bytes at 77; 2.9 + each 1.8 + bytes at 59
+//   64 x 64   4.6 + bytes at 77; 4.4 + each 1.8 + bytes at 65.  (Several a unit, refitted to 400 problems of two slabs and more: with 2.9 and 59,
+//             15 % low, k loops of three to eight slabs ran on them that 32 x 32 tiles finish sooner, us: 1280 x 784 x 312 x . W^T 8.6 / 6.0, 256 x 8320 x 320
+//             13.4 / 9.8, 973 x 1088 x 174 7.2 / 5.6)
 // Half of the estimates are within 6 %, 19 of 20 within 25 %; the better of the two by them is within 2 % of the better one on average.
 double traffic(const GemmProblem& p) {
   const bool a_kc = p.sak == 1, b_kc = p.sbn != 1;
@@ -26,7 +28,7 @@ double small_us(const GemmProblem& p) {
 }
 double large_us(const GemmProblem& p) {
   const double tiles = per_unit(p, 64), kb = 0.256 * traffic(p);
-  return tiles <= 1.0 ? 4.6 + kb / 77.0 : 2.9 + tiles * (1.77 + kb / 58.9);
+  return tiles <= 1.0 ? 4.6 + kb / 77.0 : 4.4 + tiles * (1.77 + kb / 65.0);
 }
 
 }  // namespace

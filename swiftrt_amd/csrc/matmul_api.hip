@@ -312,7 +312,7 @@ bool prefers_waves(const GemmProblem& p, Plan plan) {
     if (cold > here) here = cold;
     if (bytes > 12.0e6) return false;
   }
-  return here < (plan == kPlanMfma64 ? 0.88 : 0.95) * other;   // (that kernel's estimate spreads most)
+  return here < 0.95 * other;
 }
 
 bool curved(int activation) { return activation == srtActivationSigmoid || activation == srtActivationTanh || activation == srtActivationElu; }
