@@ -225,6 +225,21 @@ Plan base_plan(const GemmProblem& p, bool copies) {
   return kPlanGeneric;
 }
 
+bool curved(int activation) { return activation == srtActivationSigmoid || activation == srtActivationTanh || activation == srtActivationElu; }
+
+// What an activation with an exponential adds to the 128 x 128 tiles for short k loops, whose lanes put 64 results through it, in microseconds.
+// A round of the other tiles: 0.6 of that (128 x 128 and 64 x 64 ones), 3.3 times (128 x 256), 5.7 times (256 x 256, 1664 x 2368 x 8 11.2, sigmoid
+// 23.6, tanh 28.7).
+double curved_us(const GemmProblem& p) { return !curved(p.activation) ? 0.0 : p.activation == srtActivationTanh ? 3.0 : 2.0; }
+
+// The wave-split tiles spread over more workgroups, and add 0.15 a tile of a unit: us, 128 x 128 tiles for short k loops / wave-split, 3321 x 384 x 64
+// x^T . W tanh 9.0 / 6.3, 4864 x 298 x 128 tanh 11.9 / 8.0, 1492 x 988 x 32 sigmoid 8.2 / 7.0, but 10240 x 336 x 8 sigmoid 8.3 / 11.8.
+double short_time(const GemmProblem& p) { return srt::short_us(p) + curved_us(p); }
+double waves_time(const GemmProblem& p) {
+  const double tiles = (double)((p.M + 31) / 32) * (double)((p.N + 31) / 32) * (double)p.batch / srt::compute_units();
+  return srt::waves_us(p) + (curved(p.activation) ? 0.15 * tiles : 0.0);
+}
+
 // What a 16-bit problem takes on a plan that base_plan picked, in microseconds, as a bound from below where a plan's figures
 // spread (0: not compared).  R: rounds of its tiles over the units, k: K in 1024s.  Fitted to 1900 random problems (gemm_waves.hip), rms
 // 3-10 % except the 64 x 64 kernel (15 %); rates are those of a device that is not power-limited.
@@ -236,20 +251,21 @@ double plan_us(const GemmProblem& p, Plan plan) {
   };
   const bool a_kc = p.sak == 1, b_kc = p.sbk == 1;
   const double k = (double)p.K / 1024.0;
-  const double quarter = 4.4 + rounds(128, 128) * (0.9 + 5.1 * k), whole = 4.4 + rounds(256, 256) * (2.4 + 15.7 * k);
+  const double act = curved_us(p);
+  const double quarter = 4.4 + rounds(128, 128) * (0.9 + 5.1 * k + 0.6 * act), whole = 4.4 + rounds(256, 256) * (2.4 + 15.7 * k + 5.7 * act);
   switch (plan) {
     case kPlanM16Q: return quarter;
-    case kPlanM16H: return 4.1 + rounds(128, 256) * (1.4 + (b_kc ? 16.7 : 11.8) * k);
-    case kPlanM16DH: return 4.2 + rounds(128, 256) * (0.9 + 10.0 * k);
-    case kPlanM16DN: return 4.2 + rounds(256, 128) * (2.3 + 9.8 * k);
+    case kPlanM16H: return 4.1 + rounds(128, 256) * (1.4 + (b_kc ? 16.7 : 11.8) * k + 3.3 * act);
+    case kPlanM16DH: return 4.2 + rounds(128, 256) * (0.9 + 10.0 * k + 3.3 * act);
+    case kPlanM16DN: return 4.2 + rounds(256, 128) * (2.3 + 9.8 * k + 3.3 * act);
     case kPlanM16D: return whole;
     case kPlanM16:
     case kPlanRing256:
-    case kPlanKc64: return 4.4 + rounds(256, 256) * (3.0 + 16.5 * k);
+    case kPlanKc64: return 4.4 + rounds(256, 256) * (3.0 + 16.5 * k + 5.7 * act);
     case kPlanM16DTail: return 12.0 + 7.0 * k;
     case kPlanMfma128:
-    case kPlanAny128: return srt::short_supported(p) ? srt::short_us(p) : 0.0;
-    case kPlanMfma64: return 5.3 + rounds(64, 64) * (a_kc ? 6.0 : b_kc ? 9.0 : 11.5) * k;
+    case kPlanAny128: return srt::short_supported(p) ? short_time(p) : 0.0;
+    case kPlanMfma64: return 5.3 + rounds(64, 64) * (a_kc ? 6.0 : b_kc ? 9.0 : 11.5) * k + 0.6 * act;
     case kPlanSplitK: {
       const int parts = srt::mfma_splitk_parts(p);
       const double sums = (double)parts * (double)p.M * (double)p.N * 8.0;
@@ -258,7 +274,7 @@ double plan_us(const GemmProblem& p, Plan plan) {
     case kPlanAny64: {
       // (its stages and its stores, two tiles a unit: 512 x 3072 x 54 x . W^T 6.6 / 6.9, 346 x 5440 x 92 7.9 / 7.8, 12 x 768 x 320 x 53 7.8 / 7.8)
       const double t64 = (double)((p.M + 63) / 64) * (double)((p.N + 63) / 64) * (double)p.batch / (2.0 * cus);
-      return 5.4 + 1.3 * t64 + (p.K + 63) / 64 * (a_kc ? (b_kc ? 0.55 : 2.2) : 4.5) * (t64 > 1.0 ? t64 : 1.0);
+      return 5.4 + 0.5 * act + 1.3 * t64 + (p.K + 63) / 64 * (a_kc ? (b_kc ? 0.55 : 2.2) : 4.5) * (t64 > 1.0 ? t64 : 1.0);
     }
     case kPlanCopied: {
       // the launch and bytes of the copies, and the product's own
@@ -303,7 +319,7 @@ bool prefers_waves(const GemmProblem& p, Plan plan) {
   if (p.row_padding || !srt::waves_supported(p) || keeps_plan(p, plan)) return false;
   const double other = plan_us(p, plan);
   if (other == 0.0) return false;
-  double here = srt::waves_us(p);
+  double here = waves_time(p);
   if (plan == kPlanSkinny) {
     // few rows: the weight comes from memory, in whole lines on the streaming kernel
     const double kb = (double)(32 + (p.M < 32 ? p.M : 32)) * (double)p.K * 2.0 / 1000.0, bytes = (double)p.N * (double)p.K * (double)p.batch * 2.0;
@@ -314,8 +330,6 @@ bool prefers_waves(const GemmProblem& p, Plan plan) {
   }
   return here < 0.95 * other;
 }
-
-bool curved(int activation) { return activation == srtActivationSigmoid || activation == srtActivationTanh || activation == srtActivationElu; }
 
 // Whether copied operands are ahead of the 128 x 128 tiles for short k loops after all: their 256 x 256 tiles read an operand half as often, which
 // tells once a unit has many tiles of three slabs or more and the larger ones come out in whole rounds (11 us each into whole lines, 13.4 into
@@ -344,7 +358,7 @@ bool prefers_short(const GemmProblem& p, Plan plan) {
   if (!others && plan != kPlanMfma64) return false;
   const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, cus = srt::compute_units();
   if (4 * tiles >= 5 * cus) return plan != kPlanCopied || !copies_ahead(p);
-  return others && tiles <= cus && srt::short_us(p) < 0.95 * plan_us(p, plan);
+  return others && tiles <= cus && short_time(p) < 0.95 * plan_us(p, plan);
 }
 
 Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
