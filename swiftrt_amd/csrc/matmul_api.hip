@@ -265,7 +265,10 @@ double plan_us(const GemmProblem& p, Plan plan) {
     case kPlanM16DTail: return 12.0 + 7.0 * k;
     case kPlanMfma128:
     case kPlanAny128: return srt::short_supported(p) ? short_time(p) : 0.0;
-    case kPlanMfma64: return 5.3 + rounds(64, 64) * (a_kc ? 6.0 : b_kc ? 9.0 : 11.5) * k + 0.6 * act;
+    case kPlanMfma64:
+      // (up to sixteen columns in one slab: us, 64 x 64 / wave-split, 48 x 856 x 8 x 64 x . W^T 3.8 / 4.8, 56 x 960 x 8 x 64 5.0 / 6.8, 39 x 848 x 8 x 8 4.0 / 4.9)
+      if (p.N <= 16 && p.K <= 64) return 3.3 + 0.4 * rounds(64, 64) + 0.6 * act;
+      return 5.3 + rounds(64, 64) * (a_kc ? 6.0 : b_kc ? 9.0 : 11.5) * k + 0.6 * act;
     case kPlanSplitK: {
       const int parts = srt::mfma_splitk_parts(p);
       const double sums = (double)parts * (double)p.M * (double)p.N * 8.0;
@@ -355,7 +358,8 @@ bool prefers_short(const GemmProblem& p, Plan plan) {
   if (!srt::short_supported(p)) return false;
   const bool one_slab = p.K <= 64 && (plan == kPlanM16 || plan == kPlanRing256 || plan == kPlanKc64 || (plan == kPlanM16H && p.batch == 1));
   const bool others = one_slab || plan == kPlanCopied || plan == kPlanAny64 || plan == kPlanAny128;
-  if (!others && plan != kPlanMfma64) return false;
+  // (nor instead of 64 x 64 tiles where more than half of a tile is padding: 40 x 976 x 56 x 32 x . W^T 5.9 / 7.4)
+  if (!others && (plan != kPlanMfma64 || p.N <= 64)) return false;
   const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch, cus = srt::compute_units();
   if (4 * tiles >= 5 * cus) return plan != kPlanCopied || !copies_ahead(p);
   return others && tiles <= cus && short_time(p) < 0.95 * plan_us(p, plan);

@@ -28,3 +28,11 @@ def query(dt, M, N, K, ta=False, tb=False, batch=1):
     (BF16, 4288, 7769, 104, False, True, "mfma_128x128"), (BF16, 2772, 2023, 120, True, False, "mfma_128x128_any")])   # 62 / 28, 22 / 9.5
 def test_copies_and_short_k_loops(dt, M, N, K, ta, tb, plan):
     assert query(dt, M, N, K, ta, tb) == plan
+
+
+# us, 64 x 64 tiles / wave-split ones: a handful of columns and one slab; columns that fill less than half of a 128 x 128 tile
+@pytest.mark.parametrize("dt,batch,M,N,K,plan", [
+    (F16, 48, 856, 8, 64, "mfma_64x64"), (BF16, 56, 960, 8, 64, "mfma_64x64"), (F16, 39, 848, 8, 8, "mfma_64x64"),   # 3.8 / 4.8, 5.0 / 6.8, 4.0 / 4.9
+    (F16, 40, 976, 56, 32, "mfma_64x64")])                                                                           # 5.9 / 7.4
+def test_narrow_batches(dt, batch, M, N, K, plan):
+    assert query(dt, M, N, K, tb=True, batch=batch) == plan
