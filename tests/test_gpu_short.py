@@ -60,3 +60,13 @@ def test_tiles_along_the_rows():
         got = srt.Dense(wt, bt, srt.ActivationType.identity)(xt).array()
     want = x.astype(np.float32) @ w.astype(np.float32) + b.astype(np.float32)
     assert np.array_equal(got, (want.view(np.uint32) >> 16).astype(np.uint16))
+
+
+# k loops past the short kernel's, many tiles: the register-staged 128 x 128 tiles of the same two plans, off and on the 16-byte rules
+@pytest.mark.parametrize("M,N,K,frame", [(2049, 2051, 353, (0, 0)), (2050, 2049, 396, (3, 2)), (1500, 3001, 369, (1, 0)), (2040, 2056, 264, (1, 2)),
+                                         (2040, 2056, 392, (8, 8))])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_longer_k_loops_on_register_staged_tiles(tmp_path, M, N, K, frame, ta, tb):
+    plans = ("mfma_128x128_any", "mfma_128x128") if frame == (8, 8) else ("mfma_128x128_any",)
+    assert run_matmul_case(tmp_path, H.BF16 if M % 2 else H.F16, M, N, K, 1, ta, tb, plans, 1900 + M + K, left=frame[0], right=frame[1],
+                           operand_sentinel=NAN_BITS, with_bias=K % 2 == 0, relu=M % 2 == 0) == list(plans)
