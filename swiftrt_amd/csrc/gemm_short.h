@@ -2,8 +2,9 @@
 //
 // A k loop of one to four 64-deep slabs is over before a ring of prefetched stages has filled, and a kernel that takes a whole
 // compute unit has nothing else to run while its tile is stored: 64 x 512 x 512 x 64 x . W^T took 12.5 us for 42 MB.  Here a
-// workgroup needs 33 KB of LDS and under 100 registers (one slab; 172 for more), so four (two or three) share a unit, and one's stores
-// run beside another's loads.
+// workgroup needs 33 KB of LDS and under 100 registers (one slab; 172 for more), so four (two or three) share a unit, and in a grid of
+// several rounds one's stores run beside another's loads.  A grid of one round, as that one of four workgroups a unit, loads first and
+// stores last: what it gained (12.5 -> 9.5 us) it gained with its operands in the caches.
 //
 //   bound   the result's stores, then the operands' loads (each XCD's L2 holds what its neighbouring tiles share: the walk of
 //           gemm_waves.h)

@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_waves_kernel(GemmProblem p, W
   using StageB = Stage<T, B_KC, TILES, A_KC || B_KC>;
   constexpr int DEPTH = StageA::DEPTH, LOADS = StageA::LOADS, EDGE = 32 * TILES;
   constexpr int SLAB = StageA::BYTES + StageB::BYTES;       // a wave's share of LDS
-  // fp32: two chains of sums a wave, eight or sixteen a result: no sum is longer than an eighth of K, or 16 products
+  // fp32: two chains of sums a wave, eight or sixteen a result, each 16 ceil(ceil(K / 32) / WAVES) products long
   constexpr int CHAINS = sizeof(S) == 4 ? 2 : 1;
   extern __shared__ __attribute__((aligned(1024))) unsigned char waves_lds[];
   const uint32_t lds = (uint32_t)(uintptr_t)(SRT_LDS unsigned char*)waves_lds;

@@ -295,8 +295,8 @@ double plan_us(const GemmProblem& p, Plan plan) {
   }
 }
 
-// Problems whose plan stays what base_plan picks, ahead or not: a plan's name is part of the interface (saved plans, the kernel query),
-// and the tests of the choice fix it over these ranges.  The price, measured (kept / wave-split, us): 512 x 512 x 1024 x^T . W 9.9 / 5.2,
+// Problems whose plan stays what base_plan picks, ahead or not: not by speed, but because the tests of the choice assert its name in these
+// ranges (a pinned or saved name is good whatever is picked here).  The price, measured (kept / wave-split, us): 512 x 512 x 1024 x^T . W 9.9 / 5.2,
 // 256 x 1024 x 960 x . W 14.0 / 4.6, 1024^3 x^T . W 9.9 / 7.2, 256^3 x . W^T 6.2 / 3.7, 32 x 1024 x 1024 x . W^T 5.0 / 4.6.
 bool keeps_plan(const GemmProblem& p, Plan plan) {
   const long long results = (long long)p.M * p.N;
