@@ -166,17 +166,18 @@ hipError_t launch(const CellProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
-// Whether one launch is ahead of the three: while k is short against the product's own kernels, which cut a long one over idle units and
-// read the weight in larger tiles.  By the depth D = I + H and the slabs a unit walks (D times its tiles), device times of 8000 random cells
-// of 1-1024 x 8-16384 x 8-4096, three / one, us, bf16: 32 x 1024 x 1024 18.8 / 9.5, 8 x 2048 x 1024 21.7 / 12.3, 128 x 512 x 1024 18.4 / 17.8, but
-// 64 x 512 x 2048 24.2 / 30.4, 128 x 4096 x 1024 27.5 / 50.7, 8 x 8192 x 256 26.4 / 36.9; fp32 64 x 1024 x 1024 21.0 / 18.8, 32 x 4096 x 1024 39.9 / 38.6,
-// but 64 x 64 x 2048 33.7 / 37.7, 64 x 8192 x 2048 122 / 214.  Up to four groups of columns a product of few columns idles as well: 64 x 16384 x 8
-// 55.9 / 21.9.  1 cell in 60 that this takes is more than 5 % behind its three calls (the bound of two tiles a unit alone: 1 in 5).
+// Whether one launch is ahead of the three.  On the device it is while k is short against the product's own kernels, which cut a long one over idle
+// units and read the weight in larger tiles; a program's step is ahead up to 35 us of it, which its own three calls take on the host (37 us, of
+// which one call takes 20).  By the depth D = I + H and the slabs a unit walks (D times its tiles); device times of 420 cells of 1-512 x 64-16384 x
+// 8-2048, three / one, us, bf16: 32 x 1024 x 1024 18.8 / 9.5, 8 x 2048 x 1024 21.7 / 12.3, 64 x 512 x 2048 24.2 / 30.4 (taken: under 35), but 128 x
+// 4096 x 1024 27.5 / 50.7, 8 x 8192 x 256 26.4 / 36.9; fp32 64 x 1024 x 1024 21.0 / 18.8, 128 x 1024 x 1024 36.3 / 33.4, but 64 x 1024 x 2048 41.5 / 48.5,
+// 64 x 8192 x 2048 122 / 214.  Up to four groups of columns a product of few columns idles as well: 64 x 16384 x 8 55.9 / 21.9.  A program's
+// step is 0.4 % (bf16) and 0.2 % (fp32) behind the better of the two in the mean, 10 % and 5 % by the bound of two tiles a unit alone.
 bool launch_choice(const CellProblem& p, bool f32) {
   const long long tiles = (long long)((p.rows + 31) / 32) * (p.hidden / GROUP), cus = compute_units();
-  const long long depth = (long long)p.inputs + p.hidden, walk = depth * tiles;
-  if (tiles > 2 * cus || (depth > (f32 ? 8192 : 4096) && p.hidden > 32)) return false;
-  return walk <= (f32 || depth <= 1300 ? 2600 : 1800) * cus;
+  const long long depth = (long long)p.inputs + p.hidden;
+  if (tiles > 2 * cus || (depth > (f32 ? 8192 : 5200) && p.hidden > 32)) return false;
+  return depth * tiles <= (f32 ? 4200 : 5200) * cus;
 }
 
 bool row_ok(long long stride) { return stride >= 0 && stride <= 0x7fffffffLL; }

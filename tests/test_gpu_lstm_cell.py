@@ -83,11 +83,11 @@ def test_a_cell_without_a_bias(dt):
         assert np.array_equal(bits(a), bits(w))
 
 
-# device us, three launches / one: a cell is taken where one is ahead
+# device us, three launches / one: a cell is taken where one is ahead, there or (under 35 us) for a program that makes the three calls
 @pytest.mark.parametrize("dt,b,i,h,taken", [
-    (H.BF16, 32, 1024, 1024, True), (H.BF16, 64, 512, 2048, False), (H.BF16, 128, 512, 1024, False),        # 18.8 / 9.5, 24.2 / 30.4, 18.4 / 17.8
+    (H.BF16, 32, 1024, 1024, True), (H.BF16, 128, 1024, 1024, True), (H.BF16, 64, 512, 2048, True),         # 18.8 / 9.5, 20.9 / 22.1, 24.2 / 30.4
     (H.BF16, 128, 4096, 1024, False), (H.BF16, 8, 8192, 256, False), (H.F16, 64, 16384, 8, True),           # 27.5 / 50.7, 26.4 / 36.9, 55.9 / 21.9
-    (H.F32, 64, 1024, 1024, True), (H.F32, 64, 64, 2048, False), (H.F32, 64, 16384, 256, False)])           # 21.0 / 18.8, 33.7 / 37.7, 90.8 / 103.6
+    (H.F32, 128, 1024, 1024, True), (H.F32, 64, 1024, 2048, False), (H.F32, 64, 16384, 256, False)])        # 36.3 / 33.4, 41.5 / 48.5, 90.8 / 103.6
 def test_cells_are_taken_where_one_launch_is_ahead(dt, b, i, h, taken):
     dtype = H.encode(np.zeros(1), dt).dtype
     make = lambda *shape: srt.Tensor(shape=shape, dtype=dtype)   # noqa: E731
