@@ -373,6 +373,11 @@ bool skinny_supported(const GemmProblem& p);
 bool skinny_preferred(const GemmProblem& p);   // the heuristic's choice among the problems it supports
 hipError_t launch_skinny(const GemmProblem& p, hipStream_t stream);
 
+// Up to 32 rows against an n-contiguous weight, 16-bit types (gemm_stream.hip): whether it reads the problem, an estimate, the launch.
+bool stream_supported(const GemmProblem& p);
+double stream_us(const GemmProblem& p);
+hipError_t launch_stream(const GemmProblem& p, hipStream_t stream);
+
 bool f32_mfma_supported(const GemmProblem& p);
 bool f32_mfma_prefers_splitk(const GemmProblem& p);
 hipError_t launch_f32_mfma_variant(const GemmProblem& p, bool splitk, hipStream_t stream);

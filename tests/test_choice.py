@@ -36,3 +36,11 @@ def test_copies_and_short_k_loops(dt, M, N, K, ta, tb, plan):
     (F16, 40, 976, 56, 32, "mfma_64x64")])                                                                           # 5.9 / 7.4
 def test_narrow_batches(dt, batch, M, N, K, plan):
     assert query(dt, M, N, K, tb=True, batch=batch) == plan
+
+
+# a few rows against an n-contiguous weight; us, streaming kernel / wave-split tiles
+@pytest.mark.parametrize("dt,M,N,K,plan", [
+    (BF16, 8, 9776, 6216, "skinny"), (BF16, 32, 11008, 4096 + 8, "skinny"), (F16, 16, 21760, 4123, "skinny"),    # 28 / 42, 22 / 33, 35 / 56
+    (BF16, 32, 7096, 1992, "mfma_32x32_waves"), (BF16, 2, 3808, 3520, "mfma_32x32_waves"), (F16, 8, 17008, 960, "mfma_32x32_waves")])   # 12.8 / 8.7, 11.3 / 8.1, 11.0 / 8.9
+def test_a_few_rows(dt, M, N, K, plan):
+    assert query(dt, M, N, K) == plan
