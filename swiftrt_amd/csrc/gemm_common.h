@@ -367,6 +367,7 @@ int mfma_splitk_parts(const GemmProblem& p);
 bool mfma_prefers_splitk(const GemmProblem& p);
 bool mfma_prefers_tail(const GemmProblem& p);
 bool mfma_prefers_quarter(const GemmProblem& p);
+bool mfma_quarter_depth(const GemmProblem& p);
 hipError_t launch_mfma_splitk(const GemmProblem& p, hipStream_t stream);
 
 bool skinny_supported(const GemmProblem& p);

@@ -688,7 +688,7 @@ int mfma_config(const GemmProblem& p, int tile) {
   if ((tile == 1 || tile >= 4) && !(stores_any ? ring_reach_problem(p, (layout & 2) != 0, (layout & 1) != 0)
                                                : ring_fits_problem(p, (layout & 2) != 0, (layout & 1) != 0))) return 0;
   if ((tile == 9 || tile == 12 || tile == 13) && !(p.K % 64 == 0 && p.K >= 256)) return 0;   // whole 64-deep units, at least four
-  if (tile == 14 && !(p.K % 128 == 0 && p.K >= 256)) return 0;   // whole 128-deep units, at least two
+  if (tile == 14 && p.K <= 128) return 0;   // at least two 128-deep units, the last one of any depth
   if (tile == 10) {   // left-over tiles to share, k in whole quads, no transcendental activation
     const bool trans = p.activation == srtActivationSigmoid || p.activation == srtActivationTanh || p.activation == srtActivationElu;
     if (trans || !m16d_tail_fits_BF16_xx(p)) return 0;
@@ -751,9 +751,10 @@ static int ragged_store_config(const GemmProblem& p) {
     const long long t = (long long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn) * p.batch;
     return (double)((t + cus - 1) / cus);
   };
-  const int configs[4] = {mfma_config(p, 9), mfma_config(p, 12), mfma_config(p, 13), mfma_config(p, 14)};
+  const int configs[4] = {mfma_config(p, 9), mfma_config(p, 12), mfma_config(p, 13), p.K % 128 == 0 || (mfma_quarter_depth(p) && rounds(128, 128) == 1.0) ? mfma_config(p, 14) : 0};
   const double r[4] = {rounds(256, 256), rounds(128, 256), rounds(256, 128), rounds(128, 128)};
-  const double times[4] = {r[0], 0.6 * r[1], 0.6 * r[2], 0.29 * r[3]};
+  // (past one round the quarter tiles' operand traffic sets the pace: 4097 x 4099 x 4096 x . W^T 152 us in five rounds of them, 143 in halves)
+  const double times[4] = {r[0], 0.6 * r[1], 0.6 * r[2], (r[3] > 1.0 ? 0.4 : 0.29) * r[3]};
   int best = -1;
   for (int i = 0; i < 4; ++i)
     if (configs[i] && (best < 0 || times[i] < times[best])) best = i;
@@ -1055,6 +1056,17 @@ bool mfma_prefers_splitk(const GemmProblem& p) {
   return parts >= 8 || (parts >= 4 && (p.K >= 8192 || p.M <= 192 || th <= 96));
 }
 
+// Whether the k range suits the quarter tile's 128-deep units: whole ones, or a last one of any depth where the tiles are at least three quarters full
+// (us, the plans before / quarter tiles: 2048 x 2048 x 2008 x . W 30.2 / 20.4, x . W^T 40.4 / 20.9, x^T . W 43.8 / 20.9, 1600 x 2112 x 1600 20.6 /
+// 15.9, 700 x 3000 x 400 11.3 / 8.7).  Whole tiles of a k in whole 64s, or of a batch, stay with the half tiles: not by speed, but because the tests of the choice assert
+// the name there (2048 x 2048 x 1984 x . W 24.2 / 20.0).
+bool mfma_quarter_depth(const GemmProblem& p) {
+  if (p.K % 128 == 0) return true;
+  if (p.K < 256) return false;   // (two units' fixed costs: 2908 x 624 x 160 x . W 7.8 us in half tiles, 10.1)
+  const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128);
+  return (p.M % 128 != 0 || p.N % 128 != 0 || (p.K % 64 != 0 && p.batch == 1)) && 4LL * p.M * p.N >= 3 * tiles * 16384;
+}
+
 // Whether the 128 x 128 quarter tile is the choice: when one round of them holds the problem -- at most a quarter of
 // a device's worth of whole tiles -- and the k loop is not so long that cutting it over more units does better.  A
 // quarter tile's k loop runs 4.8 us per 1024 k on top of 5 us of launch, first fill and epilogue whatever the tile
@@ -1076,7 +1088,7 @@ bool mfma_prefers_splitk(const GemmProblem& p) {
 bool mfma_prefers_quarter(const GemmProblem& p) {
   const int config = mfma_config(p, 14);
   const bool a_kc = (config & 2) != 0, b_kc = (config & 1) != 0;
-  if (config == 0 || p.N < 64) return false;
+  if (config == 0 || p.N < 64 || !mfma_quarter_depth(p)) return false;
   if (!c_whole_chunks(p) && !p.row_padding) return false;   // (ragged_store_config weighs it against 64 x 64 tiles)
   // (33-63 rows against an n-contiguous weight and a k loop of two or three units: 48 x 4712 x 256 6.6 us against 7.7 in half
   // tiles, 43 x 472 x 256 6.2 against 7.2 streamed; at K = 640 the streaming kernel is ahead again, 24 x 384 x 640 6.3 against 8.1)

@@ -300,6 +300,8 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
   // WHOLE: N is a multiple of 8 and rows are aligned (checked on the host).  Otherwise the result is stored through its
   // address instead of a descriptor: 16 bytes at 2-byte alignment where the chunk lies inside the row, elements at its end
   const bool n_rd_ok = n_rd < p.N && (TN == 8 || (rd_chunk < 2 * TN && n_rd < n_end));
+  const bool n_rd_full = n_rd_ok && n_rd + 8 <= p.N;
+  const bool row_ends = !WHOLE && wave_n0 < p.N && p.N < wave_n0 + 128 && (p.N & 7) != 0;   // (the same for every lane; tiles start at whole chunks)
 
   // staging address of accumulator tile (ii, j): row 16 ii + jn, chunk (2 j + g / 2) ^ jn -- the lane's part of
   // it is the same for every ii (a row group is 4096 bytes further: an immediate offset of the write)
@@ -370,11 +372,17 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
         if constexpr (WHOLE) {
           const uint32_t off = (n_rd_ok && m < p.M) ? (uint32_t)(m * ldc2 + n_rd * 2) : OOB;
           __builtin_amdgcn_raw_buffer_store_b128(v[q], rc, (int)off, 0, SRT_STORE_AUX);
-        } else if (n_rd_ok && m < p.M) {
-          S* dst = C + (long long)m * p.scm + n_rd;
-          if (n_rd + 8 <= p.N) {
-            __builtin_memcpy(dst, &v[q], 16);
-          } else {
+        } else if (n_rd_full && m < p.M) {
+          // (a 32-bit offset from a scalar base: the results are within reach of one)
+          __builtin_memcpy(reinterpret_cast<char*>(C) + (uint32_t)(m * ldc2 + n_rd * 2), &v[q], 16);
+        }
+      }
+      if (!WHOLE && row_ends) {   // the tile in which the rows end inside a chunk
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int m = wave_m0 + ROWS * half + rd_row + 4 * (4 * it4 + q);
+          if (n_rd_ok && !n_rd_full && m < p.M) {
+            S* dst = C + (long long)m * p.scm + n_rd;
 #pragma unroll
             for (int e = 0; e < 7; ++e)
               if (n_rd + e < p.N) dst[e] = (S)(v[q][e >> 1] >> (16 * (e & 1)));

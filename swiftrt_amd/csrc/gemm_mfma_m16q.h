@@ -9,8 +9,8 @@
 // 16 MFMAs = 256 cycles, and two things follow.
 //   * A unit of staging is 128 rows (or columns) x 128 k = 32 KiB, twice as deep as the 256-wide kernels': a
 //     super-stage -- four slices, 64 MFMAs per wave -- then lasts as long as the 128 x 256 half tile's, and two of them
-//     cover the load latency.  K must be a multiple of 128 and at least 256 (with two or three units per tile every
-//     request of the main loop already belongs to the workgroup's next tile).
+//     cover the load latency.  K must fill more than one unit (with two or three units per tile every request of the
+//     main loop already belongs to the workgroup's next tile); the last one may be ragged (RAGGED).
 //   * The fragments of a slice cannot wait for registers to fall free inside it (the 256-wide kernels re-read each
 //     B tile "right behind its last MFMA", 32 MFMAs ahead of its next use; here that would be 8).  There are
 //     registers to spare instead: two fragment sets, the next slice's eight fragments read into the idle set while
@@ -74,6 +74,26 @@ struct Loader {
   // bytes between so[0] and so[1]: 16 rows
   static __device__ __forceinline__ uint32_t step(long long ld) { return (uint32_t)(16 * ld * 2); }
 
+  // Where a load of the last unit starts at or beyond K (all ones: its lane offset becomes OOB, and it reads zeros): by load mod 4 (KC: by
+  // chunk), or by load (MN: by k row).
+  static constexpr int ENDS = KC ? 4 : 8;
+  uint32_t end[ENDS];
+  static constexpr int eindex(int i) { return KC ? (i & 3) : i; }
+  __device__ __forceinline__ void init_end(int wave, int lane, int krem) {
+#pragma unroll
+    for (int i = 0; i < ENDS; ++i) {
+      const int row = wave * 32 + (i & 3) * 4 + (lane >> 4) + (i >= 4 ? 16 : 0);
+      const int k = KC ? ((lane & 15) ^ (row & 15)) * 8 : row;
+      end[i] = k >= krem ? ~0u : 0u;
+    }
+  }
+
+  // load i's lane offset in a request of the last unit (mask: all ones) or of another (0)
+  __device__ __forceinline__ uint32_t aimed(int i, uint32_t mask) const {
+    const uint32_t m = end[eindex(i)] & mask;
+    return (voff[vindex(i)] & ~m) | (OOB & m);
+  }
+
   // ld: elements between rows (KC: rows are m or n; MN: rows are k)
   __device__ __forceinline__ void init(int wave, int lane, long long ld) {
 #pragma unroll
@@ -131,7 +151,10 @@ struct FragReader<false> {
 #define SRT_ARGS __attribute__((address_space(4)))
 
 // WHOLE: the result's rows are whole aligned 16-byte chunks (c_whole_chunks), stored through a descriptor; false: any rows.
-template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE>
+// RAGGED: K need not fill the last unit.  What lies past K must come as zeros in both operands (a k-contiguous operand's next row follows there, and a batch's next
+// matrix), so the lanes of a last unit's loads that start at or past K aim out of range: two instructions a load, in the slices before it,
+// in the shadow of their MFMAs.
+template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE, bool RAGGED>
 __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];
   const uint32_t lds = (uint32_t)(uintptr_t)(SRT_LDS unsigned char*)lds_raw;
@@ -167,7 +190,8 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
   const uint32_t kstep_a = A_KC ? (uint32_t)(DK * 2) : (uint32_t)(DK * lda * 2);   // bytes per super-stage
   const uint32_t kstep_b = B_KC ? (uint32_t)(DK * 2) : (uint32_t)(DK * ldb * 2);
   const uint32_t lstep_a = Loader<A_KC>::step(lda), lstep_b = Loader<B_KC>::step(ldb);
-  const int S = p.K / DK;   // super-stages per tile (the host admits whole ones only, at least two)
+  const int S = RAGGED ? (p.K + DK - 1) / DK : p.K / DK;   // super-stages per tile (the host admits at least two)
+  const int krem = p.K - (S - 1) * DK;                     // k of the last one
 
   // per-XCD start of the k walk for an A stored k x m (see gemm_ring_kernel)
   const int rot = !A_KC ? (int)(((unsigned)(blockIdx.x & 7) * (unsigned)S) / 8u) : 0;
@@ -182,17 +206,22 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
   TileRef cur_tile = locate(v);
 
   // the eight loads of one unit, outside the main loop (first fill, and B_1 after an epilogue)
-  auto issue_a = [&](const Loader<A_KC>& l, uint32_t slot, uint32_t base) {
+  // (at: the unit's place among the tile's, for a ragged last one)
+  auto issue_a = [&](const Loader<A_KC>& l, uint32_t slot, uint32_t tile_off, int at) {
+    const uint32_t base = tile_off + (uint32_t)at * kstep_a, mask = at == S - 1 ? ~0u : 0u;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       ring::load_to_lds(ra, slot + Loader<A_KC>::wave_share(wave) + Loader<A_KC>::landing(i),
-                        l.voff[Loader<A_KC>::vindex(i)], base + (uint32_t)Loader<A_KC>::sindex(i) * lstep_a);
+                        RAGGED ? l.aimed(i, mask) : l.voff[Loader<A_KC>::vindex(i)],
+                        base + (uint32_t)Loader<A_KC>::sindex(i) * lstep_a);
   };
-  auto issue_b = [&](const Loader<B_KC>& l, uint32_t slot, uint32_t base) {
+  auto issue_b = [&](const Loader<B_KC>& l, uint32_t slot, uint32_t tile_off, int at) {
+    const uint32_t base = tile_off + (uint32_t)at * kstep_b, mask = at == S - 1 ? ~0u : 0u;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       ring::load_to_lds(rb, slot + Loader<B_KC>::wave_share(wave) + Loader<B_KC>::landing(i),
-                        l.voff[Loader<B_KC>::vindex(i)], base + (uint32_t)Loader<B_KC>::sindex(i) * lstep_b);
+                        RAGGED ? l.aimed(i, mask) : l.voff[Loader<B_KC>::vindex(i)],
+                        base + (uint32_t)Loader<B_KC>::sindex(i) * lstep_b);
   };
 
   uint32_t x = lds;   // slot of A_s; B_s follows it, then A_{s+1}, B_{s+1}, A_{s+2} (B_{s+2} goes where A_s is)
@@ -207,17 +236,21 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
     const int lane = lane_id();
     la.init(wave, lane, lda);
     lb.init(wave, lane, ldb);
+    if constexpr (RAGGED) {
+      la.init_end(wave, lane, krem);
+      lb.init_end(wave, lane, krem);
+    }
     fa.init(lane, wm0);
     fb.init(lane, wn0);
     uint32_t xb = wrap(x + UNIT), xa1 = wrap(x + 2 * UNIT), xb1 = wrap(x + 3 * UNIT);
     if (first_tile) {
-      issue_a(la, x, cur_tile.offa + (uint32_t)stage_of(0) * kstep_a);
-      issue_b(lb, xb, cur_tile.offb + (uint32_t)stage_of(0) * kstep_b);
-      issue_a(la, xa1, cur_tile.offa + (uint32_t)stage_of(1) * kstep_a);
-      issue_b(lb, xb1, cur_tile.offb + (uint32_t)stage_of(1) * kstep_b);
+      issue_a(la, x, cur_tile.offa, stage_of(0));
+      issue_b(lb, xb, cur_tile.offb, stage_of(0));
+      issue_a(la, xa1, cur_tile.offa, stage_of(1));
+      issue_b(lb, xb1, cur_tile.offb, stage_of(1));
       asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
     } else {
-      issue_b(lb, xb1, cur_tile.offb + (uint32_t)stage_of(1) * kstep_b);
+      issue_b(lb, xb1, cur_tile.offb, stage_of(1));
     }
     first_tile = false;
     SRT_FENCE();
@@ -239,6 +272,9 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
 
     int e_req = stage_of(2);   // k index of request s + 2
     uint32_t ea_off = (uint32_t)e_req * kstep_a, eb_off = (uint32_t)e_req * kstep_b;
+
+    // RAGGED: the lane offsets of this super-stage's requests (load i: entry eindex(i))
+    uint32_t va[8], vb[8], mask = 0;
 
     auto set_target = [](auto imm_tag, uint32_t base) __attribute__((always_inline)) {
       ring::set_lds_target<decltype(imm_tag)::value>(base);
@@ -279,8 +315,8 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
           if (ld >= 0) {
             SRT_FENCE();
             const uint32_t so = (ld >> 2) == 0 ? so0 : so1;
-            if (LOADS == 3) ring::load_to_lds_at_m0(rb, lb.voff[ld & 3], so);
-            else ring::load_to_lds_at_m0(ra, la.voff[ld & 3], so);
+            if (LOADS == 3) ring::load_to_lds_at_m0(rb, RAGGED ? vb[Loader<B_KC>::eindex(ld & 7)] : lb.voff[ld & 3], so);
+            else ring::load_to_lds_at_m0(ra, RAGGED ? va[Loader<A_KC>::eindex(ld & 7)] : la.voff[ld & 3], so);
           }
           if ((u & 1) == 0) {
             const int f = u >> 1;
@@ -311,17 +347,30 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
         if (u == 9) ta = xa2 + Loader<A_KC>::wave_share(wave);
         if (u == 11) so_a0 = soa;
         if (u == 13) so_a1 = select_lt(r, limit_a, soa + lstep_a, OOB);
+        if constexpr (RAGGED) {
+          // (a request that is none already aims out of range, by its scalar offset: two such offsets would add up to one in range)
+          if (u == 0) mask = select_lt(e_req, S - 1, 0u, select_lt(r, limit_a, ~0u, 0u));
+          if ((u & 1) == 0 && u >= 2 && (u >> 1) - 1 < Loader<A_KC>::ENDS) {
+            const int i = (u >> 1) - 1;
+            va[i] = la.aimed(i, mask);
+          }
+          if (Loader<A_KC>::ENDS == 8 && u == 15) va[7] = la.aimed(7, mask);
+        }
       });
       // ---- slice 1: loads 0-3 of A_{s+2} ----
       slice(C1{}, std::false_type{}, C2{}, C1{}, x, xb, ta, so_a0, so_a1, [&](int u) __attribute__((always_inline)) {
         if (u == 3) sel = select_lt(r, S, cur_tile.offb, next_tile.offb);
         if (u == 7) sob = select_lt(r, limit_b, sel + eb_off, OOB);
+        if (RAGGED && u == 11) mask = select_lt(r, limit_b, mask, 0u);
       });
       // ---- slice 2: loads 4-7 of A_{s+2} ----
       slice(C0{}, std::false_type{}, C3{}, C2{}, x, xb, ta, so_a0, so_a1, [&](int u) __attribute__((always_inline)) {
         if (u == 3) so_b0 = sob;
         if (u == 7) so_b1 = select_lt(r, limit_b, sob + lstep_b, OOB);
         if (u == 11) tb = x + Loader<B_KC>::wave_share(wave);
+        if constexpr (RAGGED) {
+          if ((u & 1) == 0 && (u >> 1) < Loader<B_KC>::ENDS) vb[u >> 1] = lb.aimed(u >> 1, mask);
+        }
       });
       // ---- sync: all of super-stage s is in registers, A_{s+1} and B_{s+1} have landed ----
       asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -382,15 +431,15 @@ __device__ __forceinline__ void gemm_m16q_body(const GemmProblem& p) {
 
 #undef SRT_FENCE
 
-template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE>
+template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE, bool RAGGED>
 __global__ __launch_bounds__(NT) void gemm_m16q_kernel(GemmProblem p) {
-  gemm_m16q_body<T, A_KC, B_KC, EPI, WHOLE>(p);
+  gemm_m16q_body<T, A_KC, B_KC, EPI, WHOLE, RAGGED>(p);
 }
 
 // ---- host side ---------------------------------------------------------------------------------------
-template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE>
+template <typename T, bool A_KC, bool B_KC, int EPI, bool WHOLE, bool RAGGED>
 hipError_t launch_kernel(const GemmProblem& p, hipStream_t stream) {
-  auto kernel = gemm_m16q_kernel<T, A_KC, B_KC, EPI, WHOLE>;
+  auto kernel = gemm_m16q_kernel<T, A_KC, B_KC, EPI, WHOLE, RAGGED>;
   constexpr int lds_bytes = UNITS * UNIT;
   static std::atomic<uint32_t> configured{0};
   if (hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kernel), lds_bytes, configured); e != hipSuccess) return e;
@@ -400,23 +449,25 @@ hipError_t launch_kernel(const GemmProblem& p, hipStream_t stream) {
   return launch_status(stream);
 }
 
-template <typename T, bool A_KC, bool B_KC, bool WHOLE>
+template <typename T, bool A_KC, bool B_KC, bool WHOLE, bool RAGGED>
 hipError_t launch_as(const GemmProblem& p, hipStream_t stream) {
-  if (p.activation == srtActivationSigmoid) return launch_kernel<T, A_KC, B_KC, EPI_SIGMOID, WHOLE>(p, stream);
-  if (p.activation == srtActivationTanh) return launch_kernel<T, A_KC, B_KC, EPI_TANH, WHOLE>(p, stream);
-  if (p.activation == srtActivationElu) return launch_kernel<T, A_KC, B_KC, EPI_ELU, WHOLE>(p, stream);
-  if (p.activation == srtActivationClippedRelu) return launch_kernel<T, A_KC, B_KC, EPI_CLIPPED, WHOLE>(p, stream);
+  if (p.activation == srtActivationSigmoid) return launch_kernel<T, A_KC, B_KC, EPI_SIGMOID, WHOLE, RAGGED>(p, stream);
+  if (p.activation == srtActivationTanh) return launch_kernel<T, A_KC, B_KC, EPI_TANH, WHOLE, RAGGED>(p, stream);
+  if (p.activation == srtActivationElu) return launch_kernel<T, A_KC, B_KC, EPI_ELU, WHOLE, RAGGED>(p, stream);
+  if (p.activation == srtActivationClippedRelu) return launch_kernel<T, A_KC, B_KC, EPI_CLIPPED, WHOLE, RAGGED>(p, stream);
   if (p.activation == srtActivationRelu) {
-    if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS_RELU, WHOLE>(p, stream);
-    return launch_kernel<T, A_KC, B_KC, EPI_RELU, WHOLE>(p, stream);
+    if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS_RELU, WHOLE, RAGGED>(p, stream);
+    return launch_kernel<T, A_KC, B_KC, EPI_RELU, WHOLE, RAGGED>(p, stream);
   }
-  if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS, WHOLE>(p, stream);
-  return launch_kernel<T, A_KC, B_KC, EPI_PLAIN, WHOLE>(p, stream);
+  if (p.bias) return launch_kernel<T, A_KC, B_KC, EPI_BIAS, WHOLE, RAGGED>(p, stream);
+  return launch_kernel<T, A_KC, B_KC, EPI_PLAIN, WHOLE, RAGGED>(p, stream);
 }
 
 template <typename T, bool A_KC, bool B_KC>
 hipError_t launch(const GemmProblem& p, hipStream_t stream) {
-  return c_whole_chunks(p) ? launch_as<T, A_KC, B_KC, true>(p, stream) : launch_as<T, A_KC, B_KC, false>(p, stream);
+  // (ragged on whole units costs 4 % in the mean of 850 problems)
+  if (p.K % DK == 0) return c_whole_chunks(p) ? launch_as<T, A_KC, B_KC, true, false>(p, stream) : launch_as<T, A_KC, B_KC, false, false>(p, stream);
+  return c_whole_chunks(p) ? launch_as<T, A_KC, B_KC, true, true>(p, stream) : launch_as<T, A_KC, B_KC, false, true>(p, stream);
 }
 
 }  // namespace m16q

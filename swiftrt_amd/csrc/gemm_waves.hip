@@ -27,7 +27,10 @@ double small_us(const GemmProblem& p) {
   return tiles <= 1.0 ? 3.4 + kb / 97.0 : 3.3 + tiles * (0.26 + kb / 70.0);
 }
 double large_us(const GemmProblem& p) {
-  const double tiles = per_unit(p, 64), kb = 0.256 * traffic(p);
+  double tiles = per_unit(p, 64), kb = 0.256 * traffic(p);
+  // long k loops: the first tiles past one a unit cost nearly a round (104 x 9152 x 4736 x^T . W^T, 286 tiles, 40 us), x^T . W reads slower (512 x 600 x 6656 35)
+  if (p.K >= 2048 && tiles > 1.0 && tiles < 1.45) tiles = 1.45;
+  if (p.K >= 4096 && p.sak != 1 && p.sbn == 1) kb *= 1.5;
   return tiles <= 1.0 ? 4.6 + kb / 77.0 : 4.4 + tiles * (1.77 + kb / 65.0);
 }
 

@@ -254,7 +254,12 @@ double plan_us(const GemmProblem& p, Plan plan) {
   const double act = curved_us(p);
   const double quarter = 4.4 + rounds(128, 128) * (0.9 + 5.1 * k + 0.6 * act), whole = 4.4 + rounds(256, 256) * (2.4 + 15.7 * k + 5.7 * act);
   switch (plan) {
-    case kPlanM16Q: return quarter;
+    case kPlanM16Q: {
+      // a ragged last unit: whole to the matrix cores, and its masks; in a batch or a second round the operands' traffic sets the pace
+      if (p.K % 128 == 0) return quarter;
+      const double r = rounds(128, 128), per_k = p.batch > 1 ? 9.0 : r > 1.0 ? 8.3 : 5.6;
+      return 5.0 + r * (0.9 + per_k * ((p.K + 127) / 128) / 8.0 + 0.6 * act + (srt::c_whole_chunks(p) ? 0.0 : 1.5));
+    }
     case kPlanM16H: return 4.1 + rounds(128, 256) * (1.4 + (b_kc ? 16.7 : 11.8) * k + 3.3 * act);
     case kPlanM16DH: return 4.2 + rounds(128, 256) * (0.9 + 10.0 * k + 3.3 * act);
     case kPlanM16DN: return 4.2 + rounds(256, 128) * (2.3 + 9.8 * k + 3.3 * act);
@@ -300,6 +305,8 @@ double plan_us(const GemmProblem& p, Plan plan) {
 // 256 x 1024 x 960 x . W 14.0 / 4.6, 1024^3 x^T . W 9.9 / 7.2, 256^3 x . W^T 6.2 / 3.7, 32 x 1024 x 1024 x . W^T 5.0 / 4.6.
 bool keeps_plan(const GemmProblem& p, Plan plan) {
   const long long results = (long long)p.M * p.N;
+// (others by speed: 1344 x 760 x 3008 x . W 35.3 us on half tiles, 16.1 on wave-split ones)
+  const bool whole = p.M <= 64 || (p.M % 128 == 0 && (p.N % 128 == 0 || plan == kPlanM16Q)) || (plan == kPlanM16Q && p.K < 768);
   switch (plan) {
     case kPlanAny64:
     case kPlanAny128:
@@ -307,13 +314,15 @@ bool keeps_plan(const GemmProblem& p, Plan plan) {
     case kPlanCopied:   // a large single matrix
       return p.batch == 1 && (results >= (1LL << 22) || (p.K >= 1024 && (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) > srt::compute_units()));
     case kPlanMfma64:   // whole 64-deep units of a large single matrix, or 128-deep ones into rows that are no whole chunks
-      return (p.K % 64 == 0 && p.K >= 960 && p.batch == 1 && results >= (1LL << 20)) || (p.K % 128 == 0 && p.K >= 256 && p.N % 8 != 0);
+      return (p.K % 64 == 0 && p.K >= 960 && p.batch == 1 && whole && results >= (1LL << 20)) || (p.K % 128 == 0 && p.K >= 256 && p.N % 8 != 0);
     case kPlanSkinny: return p.batch > 1 || p.K >= 8192 || (p.sbk == 1 && p.N <= 1024);
     default:
+      if (plan == kPlanM16Q && p.K % 128 != 0) return false;
       if (p.M <= 32) return true;   // a handful of rows
       if (p.K % 64 != 0) return false;
-      if (p.batch > 1 ? p.K < 512 : p.K < 640) return plan == kPlanM16Q && p.K <= 256;   // two 128-deep units
-      return p.batch > 1 || results >= (1LL << 18);
+      if (plan == kPlanSplitK && p.K >= 8192 && results >= (1LL << 18)) return true;   // long k loops in parts
+      if (p.batch > 1 ? p.K < 512 : p.K < 640) return plan == kPlanM16Q && p.K <= 256 && whole;   // two 128-deep units
+      return p.batch > 1 || (whole && results >= (1LL << 18));
   }
 }
 
@@ -367,7 +376,7 @@ bool prefers_short(const GemmProblem& p, Plan plan) {
 
 // Up to 32 rows against an n-contiguous weight: the streaming kernel (gemm_stream.hip) or the wave-split tiles, by what the two take (2100 random
 // problems of 1-32 x 256-24000 x 128-8192, operands out of the caches or not in turn: 1.16x in the mean over the choice before, one in 30 more than 5 %
-// behind it).  From 50 MB the weight comes from memory, and tiles of 64-byte pieces are no match: 8 x 14336 x 4096 34 us against 22.5.  What base_plan
+// behind it).  From 50 MB and a tile a unit, or 85, the weight comes from memory, and tiles of 64-byte pieces are no match: 8 x 14336 x 4096 34 us against 22.5.  What base_plan
 // picks stays for whole 256-column tiles and a k in 1024s, where the tests assert its name (the streaming kernel runs under "skinny" and, in
 // parts, under the split-K plan's name, too); that costs most with many such tiles and a short k loop: 8 x 28672 x 1024 15.2 us in half tiles against 13.5.
 bool few_rows(const GemmProblem& p, Plan* plan) {
@@ -375,7 +384,7 @@ bool few_rows(const GemmProblem& p, Plan* plan) {
   const double bytes = 2.0 * p.N * p.K, tiles = (double)((p.N + 31) / 32) / srt::compute_units();
   const double kb = 0.128 * p.K * (1.0 + ((p.sbk % 8 != 0) ? 0.3 : 0.0) + ((p.sam % 8 != 0) ? 0.17 : 0.0));
   const double waves = (tiles <= 1.0 ? 3.2 + kb / 97.0 : 3.3 + tiles * (0.26 + kb / 70.0)) + bytes / 32.0e6;
-  const bool stream = !srt::waves_supported(p) || bytes > 50.0e6 || srt::stream_us(p) < waves;
+  const bool stream = !srt::waves_supported(p) || (bytes > 50.0e6 && (tiles > 1.0 || bytes > 85.0e6)) || (p.K >= 512 && srt::stream_us(p) < 0.95 * waves);
   *plan = stream ? kPlanSkinny : kPlanWaves;
   return true;
 }
@@ -384,6 +393,11 @@ Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
   Plan plan;
   if (few_rows(p, &plan)) return plan;
   plan = base_plan(p, copies);
+  // k ranges off the 64-deep units: two rounds of quarter tiles instead of the 32-deep kernels where the estimates say so (1848 x 4352 x 1512 x^T . W 35.6 us in
+  // whole tiles, 30.8; not x . W, which has half tiles: x 552 14.5 / 16.9, x 5480 88 / 94)
+  if ((plan == kPlanM16H || plan == kPlanM16 || plan == kPlanRing256 || plan == kPlanKc64) && p.K % 64 != 0 && srt::mfma_config(p, 14) != 0 &&
+      srt::mfma_quarter_depth(p) && plan_us(p, kPlanM16Q) < 0.95 * plan_us(p, plan))
+    plan = kPlanM16Q;
   if (p.dtype != srtReal32F && prefers_short(p, plan)) plan = srt::mfma_config(p, 2) != 0 ? kPlanMfma128 : kPlanAny128;
   return p.dtype != srtReal32F && prefers_waves(p, plan) ? kPlanWaves : plan;
 }

@@ -44,3 +44,12 @@ def test_narrow_batches(dt, batch, M, N, K, plan):
     (BF16, 32, 7096, 1992, "mfma_32x32_waves"), (BF16, 2, 3808, 3520, "mfma_32x32_waves"), (F16, 8, 17008, 960, "mfma_32x32_waves")])   # 12.8 / 8.7, 11.3 / 8.1, 11.0 / 8.9
 def test_a_few_rows(dt, M, N, K, plan):
     assert query(dt, M, N, K) == plan
+
+
+# a ragged last 128-deep unit, and tiles whose waves split k where quarter or half tiles would be padded; us, the plan before / this one
+@pytest.mark.parametrize("dt,M,N,K,ta,tb,plan", [
+    (BF16, 2048, 2048, 2008, True, False, "mfma_128x128_m16_k128"), (BF16, 1600, 2112, 1600, False, True, "mfma_128x128_m16_k128"),   # 43.8 / 20.9, 20.8 / 15.2
+    (F16, 700, 3000, 400, False, False, "mfma_128x128_m16_k128"), (BF16, 2908, 624, 160, False, False, "mfma_128x256_m16"),          # 11.3 / 8.7; 7.8 (10.1 in quarters)
+    (BF16, 1344, 760, 3008, False, False, "mfma_32x32_waves"), (F16, 1000, 1000, 1024, False, True, "mfma_32x32_waves")])           # 35.3 / 16.1
+def test_depths_off_the_units(dt, M, N, K, ta, tb, plan):
+    assert query(dt, M, N, K, ta, tb) == plan
