@@ -165,6 +165,9 @@ srtStatus srtEventElapsedTime(float* milliseconds, srtEvent start, srtEvent stop
  * does for cross-queue reads, DiscreteStorage.swift:271-296).  Thread safe.  The caller owns the
  * pointer; the library keeps no reference to tensor memory. */
 srtStatus srtDeviceAllocate(void** devPtr, size_t size, srtStream stream);
+/* The same for a queue that makes a result: selects `device` for the calling thread (srtSetDevice) and returns the block, or NULL
+ * where srtDeviceAllocate would not return srtSuccess.  One call instead of three.  No counterpart in the reference. */
+void* srtQueueAllocate(int32_t device, size_t size, srtStream stream);
 srtStatus srtDeviceFree(void* devPtr);
 /* Returns every cached (free) block of every device to the driver. */
 srtStatus srtDeviceEmptyCache(void);
@@ -306,6 +309,19 @@ srtStatus srtActivationBackwardBias(const void* y, const srtTensorDescriptor* yD
                                     srtActivation activation, double coef,
                                     void* dx, const srtTensorDescriptor* dxDesc,
                                     void* dbias, const srtTensorDescriptor* dbiasDesc, srtStream stream);
+
+/* The whole pullback of a Dense layer in one call: dz = dy * activation'(y) with dbias as above, dx = dz . W^T and dw = x^T . dz
+ * (_vjpMatmul...bias and matmulGradients, differentiable/MathDerivatives.swift:460-482, :520-554).  x [M, K], w [K, N], y, dy [M, N],
+ * dx [M, K], dw [K, N]: rank 2; dbias: rank 1, N elements, or NULL.  The same bits as srtActivationBackwardBias into a tensor of y's order
+ * and two srtMatmul; dz is a stream-ordered workspace of M x N elements. */
+srtStatus srtDenseBackward(const void* x, const srtTensorDescriptor* xDesc,
+                           const void* w, const srtTensorDescriptor* wDesc,
+                           const void* y, const srtTensorDescriptor* yDesc,
+                           const void* dy, const srtTensorDescriptor* dyDesc,
+                           srtActivation activation, double coef,
+                           void* dx, const srtTensorDescriptor* dxDesc,
+                           void* dw, const srtTensorDescriptor* dwDesc,
+                           void* dbias, const srtTensorDescriptor* dbiasDesc, srtStream stream);
 
 /* The same computation for callers that cannot allocate (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Identical arguments and

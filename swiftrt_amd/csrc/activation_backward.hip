@@ -350,3 +350,38 @@ extern "C" srtStatus srtActivationBackwardBiasNoAlloc(const void* y, const srtTe
                                                       srtStream stream) {
   return activation_backward_bias(y, yDesc, dy, dyDesc, activation, coef, dx, dxDesc, dbias, dbiasDesc, stream, true);
 }
+
+// The products read dz as a tensor of y's order would be read: same kernels, same bits.  (A program's step made four tensors and three
+// calls of it: forward and pullback of 256 x 784 x 1000 in fp32 39 us of host time, 32 in one.)
+extern "C" srtStatus srtDenseBackward(const void* x, const srtTensorDescriptor* xDesc, const void* w, const srtTensorDescriptor* wDesc, const void* y,
+                                      const srtTensorDescriptor* yDesc, const void* dy, const srtTensorDescriptor* dyDesc, srtActivation activation,
+                                      double coef, void* dx, const srtTensorDescriptor* dxDesc, void* dw, const srtTensorDescriptor* dwDesc, void* dbias,
+                                      const srtTensorDescriptor* dbiasDesc, srtStream stream) {
+  if (!yDesc || !yDesc->shape) return srtErrorInvalidValue;
+  if (yDesc->rank != 2) return srtErrorNotSupported;
+  size_t es = 0;
+  switch (yDesc->type) {
+    case srtReal32F: es = 4; break;
+    case srtReal16F:
+    case srtReal16BF: es = 2; break;
+    default: return srtErrorNotSupported;
+  }
+  size_t shape[2] = {yDesc->shape[0], yDesc->shape[1]};
+  const bool columns = yDesc->order == srtOrderCol;
+  size_t strides[2] = {columns ? 1 : shape[1], columns ? shape[0] : 1}, logical[2] = {shape[1], 1};
+  const size_t count = shape[0] * shape[1];
+  if (shape[1] != 0 && (count / shape[1] != shape[0] || count > ((size_t)1 << 60))) return srtErrorOutOfMemory;
+  srtTensorDescriptor dzDesc = *yDesc;
+  dzDesc.count = dzDesc.spanCount = count;
+  dzDesc.shape = shape;
+  dzDesc.strides = strides;
+  dzDesc.logicalStrides = logical;
+  void* dz = nullptr;
+  srtStatus s = srtDeviceAllocate(&dz, count * es < 32 ? 32 : count * es, stream);
+  if (s != srtSuccess) return s;
+  s = srtActivationBackwardBias(y, yDesc, dy, dyDesc, activation, coef, dz, &dzDesc, dbias, dbiasDesc, stream);
+  if (s == srtSuccess) s = srtMatmul(dz, &dzDesc, 0, w, wDesc, 1, dx, dxDesc, stream);
+  if (s == srtSuccess) s = srtMatmul(x, xDesc, 1, dz, &dzDesc, 0, dw, dwDesc, stream);
+  (void)srtDeviceFree(dz);   // stream-ordered: reused only by work queued after the products
+  return s;
+}

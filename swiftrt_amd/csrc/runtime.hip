@@ -358,6 +358,15 @@ srtStatus srtDeviceAllocate(void** devPtr, size_t size, srtStream stream) {
   return allocator().allocate(devPtr, size, hs(stream));
 }
 
+void* srtQueueAllocate(int32_t device, size_t size, srtStream stream) {
+  void* p = nullptr;
+  if (hipSetDevice(device) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return allocator().allocate(&p, size, hs(stream)) == srtSuccess ? p : nullptr;
+}
+
 srtStatus srtDeviceFree(void* devPtr) { return allocator().release(devPtr); }
 
 srtStatus srtDeviceEmptyCache(void) { return allocator().empty_cache(); }

@@ -80,6 +80,7 @@ SIGNATURES = {
     "srtEventQuery": (_i32, [_vp]),
     "srtEventElapsedTime": (_i32, [ctypes.POINTER(ctypes.c_float), _vp, _vp]),
     "srtDeviceAllocate": (_i32, [ctypes.POINTER(_vp), ctypes.c_size_t, _vp]),
+    "srtQueueAllocate": (_vp, [_i32, ctypes.c_size_t, _vp]),
     "srtDeviceFree": (_i32, [_vp]),
     "srtDeviceEmptyCache": (_i32, []),
     "srtHostAllocate": (_i32, [ctypes.POINTER(_vp), ctypes.c_size_t]),
@@ -96,6 +97,8 @@ SIGNATURES = {
                                           _vp, _descp, _vp]),
     "srtActivationBackwardBiasNoAlloc": (_i32, [_vp, _descp, _vp, _descp, _i32, ctypes.c_double, _vp, _descp,
                                                  _vp, _descp, _vp]),
+    "srtDenseBackward": (_i32, [_vp, _descp, _vp, _descp, _vp, _descp, _vp, _descp, _i32, ctypes.c_double, _vp, _descp, _vp, _descp,
+                                _vp, _descp, _vp]),
     "srtMatmulTune": (_i32, [_vp, _descp, _i32, _vp, _descp, _i32, _vp, _descp, _i32, ctypes.c_double, _vp, _descp,
                               _vp, ctypes.c_char_p, ctypes.c_size_t]),
     "srtPlanCacheClear": (_i32, []),

@@ -57,17 +57,20 @@ class HipDeviceMemory:
     """Role of CudaDeviceMemory (CudaDevice.swift:96-162): the host object owns the pointer and
     frees it when released; byte count padded to a multiple of 32 as the reference does."""
 
+    version = -1
+    name = None
+
     def __init__(self, device_index, byte_count, queue):
         self.pointer = None
         self.device_index = device_index
-        self.byte_count = int(byte_count)
-        p = ctypes.c_void_p()
-        status = queue.lib.srtDeviceAllocate(ctypes.byref(p), max((self.byte_count + 31) // 32 * 32, 32), queue.stream)
-        if status:
-            check(status, "srtDeviceAllocate")
-        self.pointer = p.value
-        self.version = -1
-        self.name = None
+        self.byte_count = byte_count = int(byte_count)
+        size = (byte_count + 31 & -32) or 32
+        pointer = queue.lib.srtQueueAllocate(queue.gpu_id, size, queue.stream)   # (selects the device)
+        if pointer is None:   # once more, for the reason
+            p = ctypes.c_void_p()
+            check(queue.lib.srtDeviceAllocate(ctypes.byref(p), size, queue.stream), "srtDeviceAllocate")
+            pointer = p.value
+        self.pointer = pointer
         self.queue = queue          # the allocator hands the block back to this queue's stream at once
         self.last_queue = queue     # the queue that used the block last (kept up to date by the tensor)
 
@@ -111,7 +114,6 @@ class HipQueue:
 
     # -- DeviceQueue protocol (platform/common/DeviceQueue.swift:22-82) -----------------------
     def allocate(self, byte_count, heap_index=0):
-        self.select()
         return HipDeviceMemory(self.device_index, byte_count, self)
 
     def copy_to_device(self, host_ptr, dst, byte_count):
@@ -318,6 +320,21 @@ class HipQueue:
         if dbias is not None:
             dbias.device_written()
 
+    def dense_backward(self, x, weight, y, dy, activation, coef, dx, dweight, dbias=None):
+        """The pullback of a Dense layer in one native call (activation_backward and the two products of matmulGradients)."""
+        self.select()
+        x_ptr, w_ptr, y_ptr, dy_ptr = x.device_read(self), weight.device_read(self), y.device_read(self), dy.device_read(self)
+        dx_ptr, dw_ptr = dx.device_write(self), dweight.device_write(self)
+        db_ptr, db_desc = (dbias.device_write(self), dbias.descriptor_ref()) if dbias is not None else (None, None)
+        st = self.lib.srtDenseBackward(x_ptr, x.descriptor_ref(), w_ptr, weight.descriptor_ref(), y_ptr, y.descriptor_ref(), dy_ptr, dy.descriptor_ref(),
+                                       activation, coef, dx_ptr, dx.descriptor_ref(), dw_ptr, dweight.descriptor_ref(), db_ptr, db_desc, self.stream)
+        if st:
+            check(st, "srtDenseBackward")
+        dx.device_written()
+        dweight.device_written()
+        if dbias is not None:
+            dbias.device_written()
+
     def __del__(self):
         try:
             if self.stream:
@@ -364,6 +381,8 @@ class HipPlatform:
 
     @classmethod
     def local(cls):
+        if cls._local is not None:   # (set once, below)
+            return cls._local
         with cls._lock:
             if cls._local is None:
                 cls._local = HipPlatform()
@@ -376,7 +395,8 @@ class HipPlatform:
 
 def current_queue():
     """`currentQueue` (platform/common/Platform.swift:78-80)."""
-    return HipPlatform.local().current_queue
+    platform = HipPlatform._local
+    return (HipPlatform.local() if platform is None else platform).queue_stack[-1]
 
 
 class using:

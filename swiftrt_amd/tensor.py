@@ -432,6 +432,15 @@ def dense_backward(layer, x, y, out_grad):
     (HipQueue.activation_backward); dx = dz W^T and dW = x^T dz are matmuls with transpose flags
     (matmulGradients' (false, false) row).  Fills the bias pullbacks the reference leaves as
     fatalError() (MathDerivatives.swift:520-554)."""
+    weight = layer.weight
+    if len(x.shape) == len(y.shape) == len(out_grad.shape) == 2:   # one native call, dz its workspace
+        if y.shape[1] != weight.shape[1] or x.shape[0] != y.shape[0]:
+            raise ValueError("matmul inner dimensions must be equal")
+        dx = Tensor(shape=(y.shape[0], weight.shape[0]), dtype=y.dtype, order=y.order)
+        dw = Tensor(shape=(x.shape[1], y.shape[1]), dtype=x.dtype, order=x.order)
+        dbias = Tensor(shape=(y.shape[1],), dtype=y.dtype) if layer.bias is not None else None
+        current_queue().dense_backward(x, weight, y, out_grad, int(layer.activation), float(layer.coef), dx, dw, dbias)
+        return dx, dw, dbias
     dz = Tensor(shape=y.shape, dtype=y.dtype, order=y.order)
     dbias = Tensor(shape=[y.shape[1]], dtype=y.dtype) if layer.bias is not None else None
     current_queue().activation_backward(y, out_grad, layer.activation, layer.coef, dz, dbias)
