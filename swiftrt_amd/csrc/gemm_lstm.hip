@@ -7,6 +7,7 @@
 //
 //   bound   latency, as those tiles: a round trip to memory per slab of a wave, the sums, the gates
 //   k       x's slabs, then h's: each range ends with its own masked slab, and W's rows go on where x's end
+//   width   8, or any from 16 up: a last group of fewer than 8 columns (1 x 384 x 1020 f16, a program's step: 39.7 us as three calls, 18.7)
 //   W       n-contiguous: a lane's 16 bytes are 8 columns of one gate (fp32: 4, two lanes a gate), so a k row of the tile is 16
 //           or 32 bytes in each of four lines, which the neighbouring workgroups share through L2
 //   sums    fp32; bias added in fp32 and rounded to the element type, as the product's result is; then lstm_gate
@@ -31,6 +32,7 @@ struct CellProblem {
 };
 
 constexpr int WAVES = 8, GROUP = 8;   // hidden columns of a workgroup
+__host__ __device__ constexpr int groups_of(int hidden) { return (hidden + GROUP - 1) / GROUP; }
 
 template <typename T>
 __global__ __launch_bounds__(64 * WAVES) void lstm_cell_kernel(CellProblem p) {
@@ -43,7 +45,7 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_cell_kernel(CellProblem p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // workgroup x runs on XCD x % 8, which takes its consecutive eighth of the groups: neighbours share W's lines
-  const int per_xcd = (p.hidden / GROUP + 7) / 8, group = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  const int per_xcd = (groups_of(p.hidden) + 7) / 8, group = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
   if (group * GROUP >= p.hidden) return;
   const int m0 = blockIdx.y * 32, j0 = group * GROUP;
   const uint32_t lds_a = lds + (uint32_t)(wave * SLAB), lds_b = lds_a + StageA::BYTES;
@@ -55,8 +57,12 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_cell_kernel(CellProblem p) {
   auto stages = [&](const void* a, long long a_row, const S* b, int depth, StageA* sa, StageB* sb) {
     sa->init((const S*)a, lane, m0, p.rows, a_row, depth);
     sb->init(b, lane, 0, 4 * p.hidden, p.w_row, depth);
-    sb->ptr[0] = b + column;   // (H is a multiple of 8: every piece is whole)
-    sb->edge = false;
+    // a last group of fewer than 8 columns reads into the next gate's, for results that are not stored; behind the fourth gate a row ends, and a
+    // piece that would cross that end is moved back inside and shifted into place
+    const int at = min(column, 4 * p.hidden - EPC);
+    sb->ptr[0] = b + at;
+    sb->over = column - at;
+    sb->edge = j0 + GROUP > p.hidden;
   };
   StageA ax, ah;
   StageB bx, bh;
@@ -135,16 +141,17 @@ __global__ __launch_bounds__(64 * WAVES) void lstm_cell_kernel(CellProblem p) {
     for (int step = 1; step < WAVES; step *= 2)
 #pragma unroll
       for (int i = 0; i < WAVES; i += 2 * step) part[i] += part[i + step];
-    const S* bias = (const S*)p.bias + (long long)((c >> 1) * p.hidden + j0 + (c & 1) * 4) * p.bias_step;
+    const int j = j0 + (c & 1) * 4;
+    const S* bias = (const S*)p.bias + (long long)((c >> 1) * p.hidden) * p.bias_step;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       *reinterpret_cast<SRT_LDS float*>(sums + (uint32_t)((row * 33 + 4 * c + e) * 4)) =
-          T::to_float(T::from_float(part[0][e] + T::to_float(bias[(long long)e * p.bias_step])));
+          T::to_float(T::from_float(part[0][e] + T::to_float(bias[(long long)min(j + e, p.hidden - 1) * p.bias_step])));
   }
   __syncthreads();
   if (tid < 256) {
     const int row = tid >> 3, j = tid & 7, m = m0 + row, n = j0 + j;
-    if (m >= p.rows) return;
+    if (m >= p.rows || n >= p.hidden) return;
     float gate[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) gate[g] = *reinterpret_cast<const SRT_LDS float*>(sums + (uint32_t)((row * 33 + 8 * g + j) * 4));
@@ -162,7 +169,7 @@ hipError_t launch(const CellProblem& p, hipStream_t stream) {
   static std::atomic<uint32_t> configured{0};
   const void* kernel = reinterpret_cast<const void*>(lstm_cell_kernel<T>);
   if (hipError_t e = ensure_lds_limit(kernel, lds_bytes, configured); e != hipSuccess) return e;
-  hipLaunchKernelGGL(lstm_cell_kernel<T>, dim3(8 * ((p.hidden / GROUP + 7) / 8), (p.rows + 31) / 32), dim3(64 * WAVES), lds_bytes, stream, p);
+  hipLaunchKernelGGL(lstm_cell_kernel<T>, dim3(8 * ((groups_of(p.hidden) + 7) / 8), (p.rows + 31) / 32), dim3(64 * WAVES), lds_bytes, stream, p);
   return launch_status(stream);
 }
 
@@ -174,7 +181,7 @@ hipError_t launch(const CellProblem& p, hipStream_t stream) {
 // 64 x 8192 x 2048 122 / 214.  Up to four groups of columns a product of few columns idles as well: 64 x 16384 x 8 55.9 / 21.9.  A program's
 // step is 0.4 % (bf16) and 0.2 % (fp32) behind the better of the two in the mean, 10 % and 5 % by the bound of two tiles a unit alone.
 bool launch_choice(const CellProblem& p, bool f32) {
-  const long long tiles = (long long)((p.rows + 31) / 32) * (p.hidden / GROUP), cus = compute_units();
+  const long long tiles = (long long)((p.rows + 31) / 32) * groups_of(p.hidden), cus = compute_units();
   const long long depth = (long long)p.inputs + p.hidden;
   if (tiles > 2 * cus || (depth > (f32 ? 8192 : 5200) && p.hidden > 32)) return false;
   return depth * tiles <= (f32 ? 4200 : 5200) * cus;
@@ -205,7 +212,7 @@ extern "C" srtStatus srtLstmCell(const void* x, const srtTensorDescriptor* xDesc
   for (const srtTensorDescriptor* d : {cellDesc, newCellDesc, newHiddenDesc})
     if (d->shape[0] != rows || d->shape[1] != units) return srtErrorNotSupported;
   const size_t per = xDesc->type == srtReal32F ? 4 : 8, lim = 1u << 26;
-  if (rows == 0 || rows > lim || inputs > lim || units > lim || inputs < per || units < 8 || units % 8 != 0) return srtErrorNotSupported;
+  if (rows == 0 || rows > lim || inputs > lim || units > lim || inputs < per || units < 8 || (units % 8 != 0 && units < 16)) return srtErrorNotSupported;
   for (const srtTensorDescriptor* d : {xDesc, hiddenDesc, weightDesc, newCellDesc, newHiddenDesc})
     if (d->strides[1] != 1 || !srt::row_ok((long long)d->strides[0])) return srtErrorNotSupported;
   if (!x || !hidden || !weight || !bias || !cell || !newCell || !newHidden) return srtErrorInvalidValue;
