@@ -30,6 +30,12 @@ constexpr int kVectorsPerLane = 4;   // (two: sigmoid 32.2 -> 30.7 us, bias-broa
 // x 4096 (16 MB) 4.3 / 7.2, sigmoid f32 2048 x 2000 (33 MB) 6.8 / 8.7, bias add and tanh bf16 4096^2 (67 MB) 12.2 / 13.9 and 11.9 /
 // 13.2, add bf16 4096^2 (100 MB) 18.5 / 17.9, cast bf16 4096^2 to f32 (100 MB) 19.8 / 18.0, add f32 4096^2 (201 MB) 36.9 / 33.2.
 constexpr unsigned long long kOneVectorBytes = 80000000;
+// From the last-level cache's 256 MiB of traffic two vectors a lane, and the results stored with the streaming hint: nothing of them would be
+// there for the next reader, and what the hint leaves out is their way through L2.  Four a lane and plain stores / two and the hint, us: tanh
+// bf16 8192^2 (268 MB) 50.1 / 44.0, f32 94.4 / 84.9, add 71.8 / 63.9 and 142 / 132, bias add f32 4096 x 11008 (361 MB) 67.5 / 59.7, bias add and
+// tanh of its sum f32 8192^2 178 / 172; below the line the sum stays for its reader (bf16 8192 x 4096, 134 MB each, 46.6 / 49.6).
+constexpr unsigned long long kCachedBytes = 256ull << 20;
+constexpr int kVectorsPerLanePast = 2;
 
 // ---- operations -----------------------------------------------------------------------------
 struct Add { static constexpr bool binary = true; static __device__ __forceinline__ float apply(float a, float b) { return a + b; } };
@@ -107,9 +113,21 @@ __device__ __forceinline__ Pack<T, V> load_pack(const typename T::storage* p) {
     return *reinterpret_cast<const Pack<T, V>*>(p);
   }
 }
-template <typename T, int V>
-__device__ __forceinline__ void store_pack_anywhere(typename T::storage* p, const Pack<T, V>& v) {
-  __builtin_memcpy(p, &v, sizeof(v));
+// One vector of results; STREAM and ANYWHERE as above.
+template <typename T, int V, bool STREAM, bool ANYWHERE>
+__device__ __forceinline__ void store_pack(typename T::storage* p, const Pack<T, V>& v) {
+  using S = typename T::storage;
+  constexpr int BYTES = V * (int)sizeof(S);
+  if constexpr (STREAM && BYTES >= 8) {
+    typedef uint32_t whole_t __attribute__((ext_vector_type(BYTES / 4)));
+    typedef uint32_t loose_t __attribute__((ext_vector_type(BYTES / 4), aligned(sizeof(S))));
+    using words_t = std::conditional_t<ANYWHERE, loose_t, whole_t>;
+    __builtin_nontemporal_store(__builtin_bit_cast(whole_t, v), reinterpret_cast<words_t*>(p));
+  } else if constexpr (ANYWHERE) {
+    __builtin_memcpy(p, &v, sizeof(v));
+  } else {
+    *reinterpret_cast<Pack<T, V>*>(p) = v;
+  }
 }
 
 // V results of an operation, rounded to the element type.
@@ -163,7 +181,7 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
   const SI* b = (const SI*)m.b;
   SO* o = (SO*)m.o;
   const int inner = m.rank - 1;
-  // four vectors per lane, a block apart, one after the other: few registers (36), eight waves per SIMD.  On
+  // PER_LANE vectors per lane, a block apart, one after the other: few registers (36), eight waves per SIMD.  On
   // this device the memory parallelism of a streaming kernel comes from the waves: the same kernel with all
   // four vectors' loads issued before the first use needs 92 registers (five waves) and ran 15-20 % slower,
   // and four consecutive rows per lane with a row-broadcast operand loaded once were no faster either.
@@ -229,8 +247,7 @@ __device__ __forceinline__ void map_block(const Map& m, uint32_t block) {
     }
     const Pack<TO, V> po = apply_pack<TO, Op, V>(fa, fb);
     if (RAGGED && over) store_front<TO, V>(o + oo, po, over);
-    else if constexpr (RAGGED) store_pack_anywhere<TO, V>(o + oo, po);
-    else *reinterpret_cast<Pack<TO, V>*>(o + oo) = po;
+    else store_pack<TO, V, PER_LANE == kVectorsPerLanePast, RAGGED != 0>(o + oo, po);
   }
 }
 
@@ -266,7 +283,9 @@ struct TurnMap {
 
 //   STREAM  the turned operand's reads carry the streaming hint once the map is past kOneVectorBytes: f32 4096^2 32.5 -> 28.5 us, but
 //           bf16 4096^2 13.0 -> 15.3
-template <typename TI, typename TO, typename Op, bool STREAM>
+//   PAST    the results' stores as well, from kCachedBytes and with every row of the result on whole 128-byte lines: f32 4096 x 11008 81.4 -> 71.7
+//           us, 8192^2 112 -> 97, bf16 55.7 -> 50.4; rows off the lines, which two workgroups fill in parts, lose (bf16 16384 x 8200 123 -> 156)
+template <typename TI, typename TO, typename Op, bool STREAM, bool PAST>
 __global__ __launch_bounds__(256) void turn_kernel(TurnMap t) {
   using SI = typename TI::storage;
   using SO = typename TO::storage;
@@ -354,7 +373,7 @@ __global__ __launch_bounds__(256) void turn_kernel(TurnMap t) {
     const Pack<TO, V> po = apply_pack<TO, Op, V>(fa, fb);
     SO* dst = o + (long long)row * m.so[t.across] + col;
     if (col + V <= ni) {
-      store_pack_anywhere<TO, V>(dst, po);
+      store_pack<TO, V, PAST, !PAST>(dst, po);
     } else {
 #pragma unroll
       for (int e = 0; e < V; ++e)
@@ -396,28 +415,35 @@ bool plan_turn(const Map& m, TurnMap* t) {
   return fill >= (!halves ? 0.55 : whole && (all_turned || m.total >= 4000000) ? 0.25 : all_turned ? 0.5 : 0.6);
 }
 
+template <typename TI, typename TO, typename Op, int V, bool B_CACHED, int PER_LANE, int RAGGED>
+hipError_t launch_lanes(const Map& m, hipStream_t stream) {
+  const unsigned long long blocks = (m.total + 256 * PER_LANE - 1) / (256 * PER_LANE);
+  if (blocks == 0) return hipSuccess;
+  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, B_CACHED, PER_LANE, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
+  return launch_status(stream);
+}
+
 template <typename TI, typename TO, typename Op, int V, int RAGGED>
 hipError_t launch_v(const Map& m, hipStream_t stream) {
   unsigned long long vector_bytes = V * sizeof(typename TO::storage);
   if (!m.fill) vector_bytes += V * sizeof(typename TI::storage) * (m.b && !m.b_reused ? 2 : 1);
   // (single elements, 2-byte accesses: from a million of them four each, bias add bf16 4095^2 34.0 us against 37.8)
-  const int per_lane = m.total * vector_bytes <= (V == 1 ? kOneVectorBytes / 16 : kOneVectorBytes) ? 1 : kVectorsPerLane;
-  const unsigned long long blocks = (m.total + 256 * per_lane - 1) / (256 * per_lane);
-  if (blocks == 0) return hipSuccess;
-  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-  if (per_lane == 1) {
-    hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, false, 1, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
-    return launch_status(stream);
-  }
+  const unsigned long long bytes = m.total * vector_bytes;
+  if (bytes <= (V == 1 ? kOneVectorBytes / 16 : kOneVectorBytes)) return launch_lanes<TI, TO, Op, V, false, 1, RAGGED>(m, stream);
   // (a run-time choice between the two kinds of load inside one kernel cost every operation 14 %)
-  if constexpr (V > 1 && Op::binary) {
-    if (m.b_reused) {
-      hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, true, kVectorsPerLane, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
-      return launch_status(stream);
+  if constexpr (V > 1) {
+    if (bytes >= kCachedBytes) {
+      if constexpr (Op::binary) {
+        if (m.b_reused) return launch_lanes<TI, TO, Op, V, true, kVectorsPerLanePast, RAGGED>(m, stream);
+      }
+      return launch_lanes<TI, TO, Op, V, false, kVectorsPerLanePast, RAGGED>(m, stream);
+    }
+    if constexpr (Op::binary) {
+      if (m.b_reused) return launch_lanes<TI, TO, Op, V, true, kVectorsPerLane, RAGGED>(m, stream);
     }
   }
-  hipLaunchKernelGGL((map_kernel<TI, TO, Op, V, false, kVectorsPerLane, RAGGED>), dim3((unsigned)blocks), dim3(256), 0, stream, m);
-  return launch_status(stream);
+  return launch_lanes<TI, TO, Op, V, false, kVectorsPerLane, RAGGED>(m, stream);
 }
 
 // Vector width the layout allows: the innermost dimension must be contiguous in the result and
@@ -492,8 +518,11 @@ hipError_t launch_t(Map m, hipStream_t stream) {
     const unsigned long long blocks = others * t.tiles_inner * t.tiles_across;
     if (blocks <= 0x7fffffffull) {
       const unsigned long long bytes = m.total * (sizeof(typename TO::storage) + sizeof(typename TI::storage) * (m.b && !m.b_reused ? 2 : 1));
-      if (bytes > kOneVectorBytes) hipLaunchKernelGGL((turn_kernel<TI, TO, Op, true>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
-      else hipLaunchKernelGGL((turn_kernel<TI, TO, Op, false>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+      bool lines = (uintptr_t)m.o % 128 == 0;
+      for (int d = 0; d < inner; ++d) lines = lines && m.so[d] * (long long)sizeof(typename TO::storage) % 128 == 0;
+      if (bytes >= kCachedBytes && lines) hipLaunchKernelGGL((turn_kernel<TI, TO, Op, true, true>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+      else if (bytes > kOneVectorBytes) hipLaunchKernelGGL((turn_kernel<TI, TO, Op, true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+      else hipLaunchKernelGGL((turn_kernel<TI, TO, Op, false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
       return launch_status(stream);
     }
   }
