@@ -11,14 +11,20 @@
 //   layout    the operand keeps its orientation (rows along its unit stride; a view without one takes its smaller stride as
 //             the row), rows padded to a multiple of 64 elements, zero behind the extent; k is padded to the unit of the
 //             kernel that will read it (pack_depth), as zero columns or zero rows
-//   lanes     one 16-byte chunk of the copy each, four per lane a workgroup apart
+//   lanes     one 16-byte chunk of the copy each, two per lane a workgroup apart (four / two, the whole product, us: 512 x 11007 x 4096 88.5 /
+//             87.4, 8191^3 794 / 786, the rest within a percent)
 #include "gemm_common.h"
 #include "status.h"
 
 namespace srt {
 namespace {
 
-constexpr int kChunksPerLane = 4;
+constexpr int kChunksPerLane = 2;
+// Copies of this much and more read their sources with the streaming hint: that large they are not in the caches, and are read once.  Without /
+// with it, the whole product, us: x . W^T 2048 x 768 x 50257 (283 MB of copies) 484 / 425, x . W 512 x 11007 x 4096 (94 MB) 87.4 / 80.9, 2048 x
+// 50257 x 768 (77 MB) 183.3 / 181.5; smaller sources mostly are, and two rows share their lines: 4096 x 4095 x 4095 (67 MB) 121.4 / 125.7, 2048 x
+// 2047 x 2049 32.5 / 37.8.
+constexpr size_t kStreamedCopies = 75000000;
 // The copies of a call take at most this much, in blocks of a power of two: the allocator keeps a freed block for the next call of
 // its size, so calls of many odd shapes share a dozen blocks instead of leaving one each (two operands that the 256 x 256 kernels'
 // 32-bit offsets reach are 4 GiB; larger ones run as they are).
@@ -40,7 +46,7 @@ struct Element<2> { using type = uint16_t; };
 template <>
 struct Element<4> { using type = uint32_t; };
 
-template <int ES>
+template <int ES, bool STREAM>
 __global__ __launch_bounds__(256) void pack_kernel(PackJob a, PackJob b, uint32_t blocks_a) {
   using E = typename Element<ES>::type;
   constexpr uint32_t PER = 16 / ES;   // elements of a chunk
@@ -60,7 +66,13 @@ __global__ __launch_bounds__(256) void pack_kernel(PackJob a, PackJob b, uint32_
       const E* src = (const E*)j.src + (long long)bz * j.batch + (long long)row * j.ld + (long long)col * j.inner;
       const uint32_t n = j.cols - col;
       if (j.inner == 1 && n >= PER) {
-        __builtin_memcpy(&x, src, 16);
+        if constexpr (STREAM) {
+          typedef uint32_t words_t __attribute__((ext_vector_type(4), aligned(2)));   // (from any element's address)
+          const words_t w = __builtin_nontemporal_load(reinterpret_cast<const words_t*>(src));
+          __builtin_memcpy(&x, &w, 16);
+        } else {
+          __builtin_memcpy(&x, src, 16);
+        }
       } else {
 #pragma unroll
         for (uint32_t e = 0; e < PER; ++e)
@@ -193,8 +205,10 @@ hipError_t launch_packed(const GemmProblem& p, hipStream_t stream) {
   if (t.bytes_b) t.q.B = t.b.dst = (char*)workspace + t.at_b();
   auto blocks = [](const PackJob& j) { return (j.total + 256 * kChunksPerLane - 1) / (256 * kChunksPerLane); };
   const dim3 grid(blocks(t.a) + blocks(t.b));
-  if (p.dtype == srtReal32F) hipLaunchKernelGGL(pack_kernel<4>, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a));
-  else hipLaunchKernelGGL(pack_kernel<2>, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a));
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a)); };
+  const bool streamed = t.bytes_a + t.bytes_b >= kStreamedCopies;
+  if (p.dtype == srtReal32F) streamed ? launch(pack_kernel<4, true>) : launch(pack_kernel<4, false>);
+  else streamed ? launch(pack_kernel<2, true>) : launch(pack_kernel<2, false>);
   hipError_t e = launch_status(stream);
   if (e == hipSuccess) e = launch_heuristic(t.q, stream);
   (void)srtDeviceFree(workspace);   // stream-ordered: reused only by work queued after the kernels above
