@@ -301,6 +301,12 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
   // address instead of a descriptor: 16 bytes at 2-byte alignment where the chunk lies inside the row, elements at its end
   const bool n_rd_ok = n_rd < p.N && (TN == 8 || (rd_chunk < 2 * TN && n_rd < n_end));
   const bool n_rd_full = n_rd_ok && n_rd + 8 <= p.N;
+  // Long rows off whole chunks leave past the caches from 100 MB of results at a short k against a k-contiguous B, where the stores are what
+  // the launch waits for.  Cached / past, bf16 x . W^T, us: 2048 x 50257 x 768 177 / 154, 2048 x 25001 x 768 (102 MB) 99 / 87, 1024 x 50257 x 768
+  // 95 / 86, 8192 x 16001 x 960 243 / 221, 2048 x 50260 x 256 99 / 93, x^T . W^T 176 / 156; a longer k 108 / 111 (1024 x 50257 x 1024) and 274 /
+  // 283 (2048 x 50257 x 1600), shorter rows 76 / 85 (16384 x 5001 x 256), an n-contiguous W 134 / 141 (2048 x 40001 x 768).
+  const bool past = !WHOLE && p.N >= 16000 && p.K < 1024 && p.sbk == 1 &&
+                    (unsigned long long)p.M * (unsigned)p.N * (unsigned)p.batch >= 50000000u;
   const bool row_ends = !WHOLE && wave_n0 < p.N && p.N < wave_n0 + 128 && (p.N & 7) != 0;   // (the same for every lane; tiles start at whole chunks)
 
   // staging address of accumulator tile (ii, j): row 16 ii + jn, chunk (2 j + g / 2) ^ jn -- the lane's part of
@@ -365,16 +371,27 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[q][e] = ring::canonical_nans_bf16x2(v[q][e]);
       }
+      typedef uint32_t loose_t __attribute__((ext_vector_type(4), aligned(2)));
+      if (past) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int row = rd_row + 4 * (4 * it4 + q);
-        const int m = wave_m0 + ROWS * half + row;
-        if constexpr (WHOLE) {
-          const uint32_t off = (n_rd_ok && m < p.M) ? (uint32_t)(m * ldc2 + n_rd * 2) : OOB;
-          __builtin_amdgcn_raw_buffer_store_b128(v[q], rc, (int)off, 0, SRT_STORE_AUX);
-        } else if (n_rd_full && m < p.M) {
-          // (a 32-bit offset from a scalar base: the results are within reach of one)
-          __builtin_memcpy(reinterpret_cast<char*>(C) + (uint32_t)(m * ldc2 + n_rd * 2), &v[q], 16);
+        for (int q = 0; q < 4; ++q) {
+          const int m = wave_m0 + ROWS * half + rd_row + 4 * (4 * it4 + q);
+          if (n_rd_full && m < p.M)
+            __builtin_nontemporal_store(v[q], reinterpret_cast<loose_t*>(reinterpret_cast<char*>(C) + (uint32_t)(m * ldc2 + n_rd * 2)));
+        }
+        __builtin_amdgcn_sched_barrier(0);   // (the compiler would make one store of the two branches' and drop the hint)
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int row = rd_row + 4 * (4 * it4 + q);
+          const int m = wave_m0 + ROWS * half + row;
+          if constexpr (WHOLE) {
+            const uint32_t off = (n_rd_ok && m < p.M) ? (uint32_t)(m * ldc2 + n_rd * 2) : OOB;
+            __builtin_amdgcn_raw_buffer_store_b128(v[q], rc, (int)off, 0, SRT_STORE_AUX);
+          } else if (n_rd_full && m < p.M) {
+            // (a 32-bit offset from a scalar base: the results are within reach of one)
+            *reinterpret_cast<loose_t*>(reinterpret_cast<char*>(C) + (uint32_t)(m * ldc2 + n_rd * 2)) = v[q];
+          }
         }
       }
       if (!WHOLE && row_ends) {   // the tile in which the rows end inside a chunk
