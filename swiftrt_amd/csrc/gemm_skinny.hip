@@ -16,7 +16,7 @@
 //           vector-memory instructions are global->LDS loads and its only register-producing
 //           loads are LDS reads.
 //   grid    ceil(N / 32) x batch workgroups of 60-72 KiB LDS: two per CU, all resident at once.
-//   W[K,N]  An n-contiguous weight (x . W, the Dense layer's own layout) streams the same way with 64
+//   W[K,N]  An n-contiguous weight (x . W; one matrix of up to 32 16-bit rows is gemm_stream.hip's) streams the same way with 64
 //           columns per workgroup: a k row of the block is then 128 contiguous bytes, one load
 //           instruction fetches 8 k rows, and a k block of 64 rows lands as [64 k][8 chunks of 16 B],
 //           chunk c of k row k at c ^ (((k >> 1) & 1) << 2).  The MFMA operand (lane l: column l % 32,
