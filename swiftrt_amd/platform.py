@@ -66,7 +66,8 @@ class HipDeviceMemory:
         self.byte_count = byte_count = int(byte_count)
         size = (byte_count + 31 & -32) or 32
         pointer = queue.lib.srtQueueAllocate(queue.gpu_id, size, queue.stream)   # (selects the device)
-        if pointer is None:   # once more, for the reason
+        if pointer is None:   # once more, for the reason; on this queue's device, or not at all
+            queue.select()
             p = ctypes.c_void_p()
             check(queue.lib.srtDeviceAllocate(ctypes.byref(p), size, queue.stream), "srtDeviceAllocate")
             pointer = p.value
