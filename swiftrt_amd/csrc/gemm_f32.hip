@@ -514,7 +514,7 @@ hipError_t launch_f32_tile_parts(const GemmProblem& p, hipStream_t stream) {
   if (parts < 2) return hipErrorInvalidValue;
   void* workspace = nullptr;
   const size_t bytes = (size_t)parts * p.M * p.N * sizeof(float);
-  if (srtDeviceAllocate(&workspace, bytes, reinterpret_cast<srtStream>(stream)) != srtSuccess) return hipErrorOutOfMemory;
+  if (hipError_t e = take_workspace(&workspace, bytes, stream); e != hipSuccess) return e;
   GemmProblem q = p;
   q.K = p.K / parts;
   q.batch = parts;

@@ -1206,7 +1206,7 @@ hipError_t launch_mfma_splitk(const GemmProblem& p, hipStream_t stream) {
   const bool a_kc = (layout & 2) != 0, b_kc = (layout & 1) != 0;
   void* workspace = nullptr;
   const size_t bytes = (size_t)parts * p.M * p.N * sizeof(float);
-  if (srtDeviceAllocate(&workspace, bytes, reinterpret_cast<srtStream>(stream)) != srtSuccess) return hipErrorOutOfMemory;
+  if (hipError_t e = take_workspace(&workspace, bytes, stream); e != hipSuccess) return e;
   GemmProblem q = p;
   q.K = p.K / parts;
   q.batch = parts;

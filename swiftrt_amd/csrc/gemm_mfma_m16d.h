@@ -1008,10 +1008,7 @@ hipError_t launch_tail_kernel(const GemmProblem& p, hipStream_t stream) {
   void* workspace = nullptr;
   // flags (and, in checking builds, the store counts behind them), then a partial per piece
   const size_t bytes = TAIL_FLAG_BYTES + (size_t)plan.left * plan.parts * TAIL_PARTIAL_BYTES;
-  // (nor for a stream under capture: every replay would carry the same epoch, and find the flags of the one before raised)
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return hipErrorOutOfMemory;
-  if (srtDeviceAllocate(&workspace, bytes, reinterpret_cast<srtStream>(stream)) != srtSuccess) return hipErrorOutOfMemory;
+  if (hipError_t e = take_workspace(&workspace, bytes, stream); e != hipSuccess) return e;
   TailShare ts;
   ts.parts = plan.parts;
   ts.cut1 = plan.cut1;

@@ -196,11 +196,8 @@ bool pack_preferred(const GemmProblem& p) {
 hipError_t launch_packed(const GemmProblem& p, hipStream_t stream) {
   PackPlan t;
   if (!plan_pack(p, &t)) return hipErrorInvalidValue;
-  // a stream under capture takes no workspace: the block would go back to the allocator while the graph still writes it
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return hipErrorOutOfMemory;
   void* workspace = nullptr;
-  if (srtDeviceAllocate(&workspace, t.workspace(), reinterpret_cast<srtStream>(stream)) != srtSuccess) return hipErrorOutOfMemory;
+  if (hipError_t e = take_workspace(&workspace, t.workspace(), stream); e != hipSuccess) return e;
   if (t.bytes_a) t.q.A = t.a.dst = workspace;
   if (t.bytes_b) t.q.B = t.b.dst = (char*)workspace + t.at_b();
   auto blocks = [](const PackJob& j) { return (j.total + 256 * kChunksPerLane - 1) / (256 * kChunksPerLane); };

@@ -272,10 +272,8 @@ hipError_t launch_rows(const GemmProblem& p, hipStream_t stream) {
   if (share.parts > 1) {
     const size_t flag_bytes = ((size_t)strips * share.parts * sizeof(unsigned long long) + 255) / 256 * 256;
     const size_t bytes = flag_bytes + (size_t)strips * share.parts * MT * 8192;
-    // a stream under capture takes no workspace (a replay would find the flags of the last one raised), nor does a full device: the whole k range a workgroup
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
-        srtDeviceAllocate(&workspace, bytes, reinterpret_cast<srtStream>(stream)) != srtSuccess) {
+    // without a workspace: the whole k range a workgroup
+    if (take_workspace(&workspace, bytes, stream) != hipSuccess) {
       share.parts = 1;
     } else {
       share.flags = reinterpret_cast<unsigned long long*>(workspace);

@@ -433,7 +433,8 @@ hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
   }
 }
 
-// A plan that finds no room for its workspace (nothing that matters was launched) gives way to the plan that needs none.
+// A plan that gets no workspace (a full device, a stream under capture; nothing that matters was launched) gives way to the next best, which may
+// want one too: copies to what runs the operands as they are, tiles with shared left-overs to whole ones, parts of k to the whole range.
 hipError_t launch_or_fall_back(const GemmProblem& p, Plan plan, hipStream_t stream) {
   const hipError_t e = launch_plan(p, plan, stream);
   if (e != hipErrorOutOfMemory) return e;
@@ -446,7 +447,7 @@ hipError_t launch_or_fall_back(const GemmProblem& p, Plan plan, hipStream_t stre
     default: return e;
   }
   (void)hipGetLastError();
-  return launch_plan(p, plan_supported(p, next) ? next : kPlanGeneric, stream);
+  return launch_or_fall_back(p, plan_supported(p, next) ? next : kPlanGeneric, stream);
 }
 
 struct PlanKey {
