@@ -303,25 +303,14 @@ srtStatus srtPlanCacheLoad(const char* path);
  * y, dy, dx: rank 2, [M, N], one element type (32F, 16F, 16BF), any strides; dbias: rank 1, N
  * elements.  Sums are fp32 in a fixed order (results do not vary from run to run).
  * With dbias, takes a stream-ordered workspace of at most max(8 MiB, 4 N bytes) from the library's
- * allocator for the duration of the call's kernels.  srtErrorNotSupported for other ranks or element types. */
+ * allocator for the duration of the call's kernels; on a stream under capture it is the fixed array of
+ * srtActivationBackwardBiasNoAlloc instead, under that call's rules (N beyond its limit: srtErrorNotSupported).
+ * srtErrorNotSupported for other ranks or element types. */
 srtStatus srtActivationBackwardBias(const void* y, const srtTensorDescriptor* yDesc,
                                     const void* dy, const srtTensorDescriptor* dyDesc,
                                     srtActivation activation, double coef,
                                     void* dx, const srtTensorDescriptor* dxDesc,
                                     void* dbias, const srtTensorDescriptor* dbiasDesc, srtStream stream);
-
-/* The whole pullback of a Dense layer in one call: dz = dy * activation'(y) with dbias as above, dx = dz . W^T and dw = x^T . dz
- * (_vjpMatmul...bias and matmulGradients, differentiable/MathDerivatives.swift:460-482, :520-554).  x [M, K], w [K, N], y, dy [M, N],
- * dx [M, K], dw [K, N]: rank 2; dbias: rank 1, N elements, or NULL.  The same bits as srtActivationBackwardBias into a tensor of y's order
- * and two srtMatmul; dz is a stream-ordered workspace of M x N elements. */
-srtStatus srtDenseBackward(const void* x, const srtTensorDescriptor* xDesc,
-                           const void* w, const srtTensorDescriptor* wDesc,
-                           const void* y, const srtTensorDescriptor* yDesc,
-                           const void* dy, const srtTensorDescriptor* dyDesc,
-                           srtActivation activation, double coef,
-                           void* dx, const srtTensorDescriptor* dxDesc,
-                           void* dw, const srtTensorDescriptor* dwDesc,
-                           void* dbias, const srtTensorDescriptor* dbiasDesc, srtStream stream);
 
 /* The same computation for callers that cannot allocate (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Identical arguments and
@@ -341,6 +330,19 @@ srtStatus srtActivationBackwardBiasNoAlloc(const void* y, const srtTensorDescrip
                                            srtActivation activation, double coef,
                                            void* dx, const srtTensorDescriptor* dxDesc,
                                            void* dbias, const srtTensorDescriptor* dbiasDesc, srtStream stream);
+
+/* The whole pullback of a Dense layer in one call: dz = dy * activation'(y) with dbias as above, dx = dz . W^T and dw = x^T . dz
+ * (_vjpMatmul...bias and matmulGradients, differentiable/MathDerivatives.swift:460-482, :520-554).  x [M, K], w [K, N], y, dy [M, N],
+ * dx [M, K], dw [K, N]: rank 2; dbias: rank 1, N elements, or NULL.  The same bits as srtActivationBackwardBias into a tensor of y's order
+ * and two srtMatmul; dz is a stream-ordered workspace of M x N elements. */
+srtStatus srtDenseBackward(const void* x, const srtTensorDescriptor* xDesc,
+                           const void* w, const srtTensorDescriptor* wDesc,
+                           const void* y, const srtTensorDescriptor* yDesc,
+                           const void* dy, const srtTensorDescriptor* dyDesc,
+                           srtActivation activation, double coef,
+                           void* dx, const srtTensorDescriptor* dxDesc,
+                           void* dw, const srtTensorDescriptor* dwDesc,
+                           void* dbias, const srtTensorDescriptor* dbiasDesc, srtStream stream);
 
 /* ---- element-wise neighbours of the path ---------------------------------------------------------
  * Same names, argument order and conventions as the reference's native module

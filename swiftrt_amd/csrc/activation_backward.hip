@@ -216,7 +216,8 @@ float* scratch_of_stream(hipStream_t stream, srtStatus* status) {
   return scratch_of_device(device, status);
 }
 
-// fixed_workspace: false -- the partial rows come from the library's stream-ordered allocator;
+// fixed_workspace: false -- the partial rows come from the library's stream-ordered allocator, or, on a stream
+// under capture (whose graph would keep the address of a block given back), from the static array;
 // true -- from the device's static scratch array (nothing is allocated or freed), and a problem
 // whose partial rows exceed it is refused.
 template <typename T>
@@ -245,8 +246,10 @@ srtStatus run(BackwardProblem p, void* dbias, long long dbias_stride, hipStream_
   chunks = (p.M + p.rows_per_chunk - 1) / p.rows_per_chunk;
 
   void* workspace = nullptr;
+  const bool captured = dbias && !fixed_workspace && capturing(stream);
+  if (captured) fixed_workspace = true;
   if (dbias && fixed_workspace) {
-    if ((size_t)chunks * p.N * sizeof(float) > kScratchBytes) return srtErrorInvalidValue;
+    if ((size_t)chunks * p.N * sizeof(float) > kScratchBytes) return captured ? srtErrorNotSupported : srtErrorInvalidValue;
     srtStatus s;
     workspace = scratch_of_stream(stream, &s);
     if (!workspace) return s;

@@ -335,13 +335,14 @@ inline unsigned long long next_launch_epoch() {
 // Workspace for the kernels of one call, given back with srtDeviceFree behind their launches (stream-ordered: reused only by work queued after
 // them).  A stream under capture gets none: the block would go to the allocator's next caller while every replay still writes it, and launch-unique
 // flags in it would come again.  hipErrorOutOfMemory: the plan gives way to one that needs none (launch_or_fall_back).
-inline hipError_t take_workspace(void** workspace, size_t bytes, hipStream_t stream) {
+inline bool capturing(hipStream_t stream) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
-    (void)hipGetLastError();
-    return hipErrorOutOfMemory;
-  }
-  if (capture != hipStreamCaptureStatusNone) return hipErrorOutOfMemory;
+  if (hipStreamIsCapturing(stream, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();   // (the null stream beside another stream's capture: as one under capture)
+  return true;
+}
+inline hipError_t take_workspace(void** workspace, size_t bytes, hipStream_t stream) {
+  if (capturing(stream)) return hipErrorOutOfMemory;
   return srtDeviceAllocate(workspace, bytes, reinterpret_cast<srtStream>(stream)) == srtSuccess ? hipSuccess : hipErrorOutOfMemory;
 }
 

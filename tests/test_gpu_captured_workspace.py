@@ -73,3 +73,33 @@ def test_replays_leave_other_tensors_alone(plan, dt, M, N, K, tb):
         for t in held:
             assert np.all(t.array() == 7.0)
         assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
+
+
+@pytest.mark.parametrize("dt,M,N", [(H.F32, 700, 1000), (H.BF16, 4099, 264)])
+def test_captured_bias_gradient(dt, M, N):
+    """Its partial rows are the fixed array's under capture: the eager call's bits, and no other tensor is written."""
+    g, L, q = H.rng(53), native.lib(), srt.current_queue()
+    sources = [srt.Tensor(H.encode(g.standard_normal((M, N)), dt)) for _ in range(3)]
+    y, dy = srt.Tensor(H.encode(g.standard_normal((M, N)), dt)), srt.Tensor(H.encode(g.standard_normal((M, N)), dt))
+    dx, db, want_dx, want_db = (srt.Tensor(shape=s, dtype=H.NP_STORAGE[dt]) for s in ([M, N], [N]) * 2)
+
+    def call(dx, db):
+        q.activation_backward(y, dy, srt.ActivationType.tanh, 0.0, dx, db)
+    call(dx, db)
+    graph, run = captured(q, lambda: call(dx, db))
+    held = [srt.Tensor(shape=[1 << s], dtype=np.float32) for s in range(12, 23) for _ in range(2)]
+    held += [srt.Tensor(shape=[chunks * N], dtype=np.float32) for chunks in range(1, 257)]   # a row of sums a chunk of 16 rows or more
+    for t in held:
+        q.fill(t, 7.0)
+    for source in sources:
+        q.copy(source, dy)
+        call(want_dx, want_db)
+        q.fill(dx, 0.0)
+        q.fill(db, 0.0)
+        assert L.hipGraphLaunch(run, q.stream) == 0
+        dx.device_written()
+        db.device_written()
+        assert dx.array().tobytes() == want_dx.array().tobytes() and db.array().tobytes() == want_db.array().tobytes()
+    for t in held:
+        assert np.all(t.array() == 7.0)
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
