@@ -334,7 +334,8 @@ srtStatus srtActivationBackwardBiasNoAlloc(const void* y, const srtTensorDescrip
 /* The whole pullback of a Dense layer in one call: dz = dy * activation'(y) with dbias as above, dx = dz . W^T and dw = x^T . dz
  * (_vjpMatmul...bias and matmulGradients, differentiable/MathDerivatives.swift:460-482, :520-554).  x [M, K], w [K, N], y, dy [M, N],
  * dx [M, K], dw [K, N]: rank 2; dbias: rank 1, N elements, or NULL.  The same bits as srtActivationBackwardBias into a tensor of y's order
- * and two srtMatmul; dz is a stream-ordered workspace of M x N elements. */
+ * and two srtMatmul; dz is a stream-ordered workspace of M x N elements.  Not for graphs: on a stream under capture srtErrorNotSupported, with
+ * nothing launched (the three calls, with a dz of the caller's, can be captured). */
 srtStatus srtDenseBackward(const void* x, const srtTensorDescriptor* xDesc,
                            const void* w, const srtTensorDescriptor* wDesc,
                            const void* y, const srtTensorDescriptor* yDesc,

@@ -379,6 +379,7 @@ extern "C" srtStatus srtDenseBackward(const void* x, const srtTensorDescriptor* 
   dzDesc.shape = shape;
   dzDesc.strides = strides;
   dzDesc.logicalStrides = logical;
+  if (srt::capturing(reinterpret_cast<hipStream_t>(stream))) return srtErrorNotSupported;   // a graph would keep dz's address, and the allocator reuse it
   void* dz = nullptr;
   srtStatus s = srtDeviceAllocate(&dz, count * es < 32 ? 32 : count * es, stream);
   if (s != srtSuccess) return s;

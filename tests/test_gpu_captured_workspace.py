@@ -103,3 +103,26 @@ def test_captured_bias_gradient(dt, M, N):
     for t in held:
         assert np.all(t.array() == 7.0)
     assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
+
+
+def test_a_captured_pullback_is_refused_with_nothing_launched():
+    g, L, q = H.rng(54), native.lib(), srt.current_queue()
+    t = lambda *s: srt.Tensor(H.encode(g.standard_normal(s), H.F32))
+    layer = srt.Dense(t(48, 64), t(64), srt.ActivationType.relu)
+    x, dy = t(32, 48), t(32, 64)
+    y = layer(x)
+    dx, dw, db = (srt.Tensor(shape=s, dtype=np.float32) for s in ([32, 48], [48, 64], [64]))
+    for out in (dx, dw, db):
+        q.fill(out, 7.0)
+    for tensor in (x, dy, layer.weight):
+        tensor.device_read(q)
+
+    def call():
+        with pytest.raises(native.NotSupportedError):
+            q.dense_backward(x, layer.weight, y, dy, int(layer.activation), 0.0, dx, dw, db)
+    graph, run = captured(q, call)
+    nodes = ctypes.c_size_t()
+    assert L.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 0
+    for out in (dx, dw, db):
+        assert np.all(out.array() == 7.0)
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
