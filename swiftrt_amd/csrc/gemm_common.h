@@ -388,10 +388,11 @@ bool skinny_supported(const GemmProblem& p);
 bool skinny_preferred(const GemmProblem& p);   // the heuristic's choice among the problems it supports
 hipError_t launch_skinny(const GemmProblem& p, hipStream_t stream);
 
-// Up to 32 rows against an n-contiguous weight, 16-bit types (gemm_stream.hip): whether it reads the problem, an estimate, the launch.
+// Up to 32 rows against an n-contiguous weight, 16-bit types (gemm_stream.hip): whether it reads the problem, an estimate, the launch (whole: the
+// whole k range a workgroup; else hipErrorOutOfMemory where k is in parts and there is no workspace for them to meet in).
 bool stream_supported(const GemmProblem& p);
 double stream_us(const GemmProblem& p);
-hipError_t launch_stream(const GemmProblem& p, hipStream_t stream);
+hipError_t launch_stream(const GemmProblem& p, hipStream_t stream, bool whole = false);
 
 bool f32_mfma_supported(const GemmProblem& p);
 bool f32_mfma_prefers_splitk(const GemmProblem& p);

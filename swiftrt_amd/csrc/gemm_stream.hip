@@ -264,22 +264,18 @@ int stream_parts(const GemmProblem& p) {
 }
 
 template <typename T, int MT>
-hipError_t launch_rows(const GemmProblem& p, hipStream_t stream) {
+hipError_t launch_rows(const GemmProblem& p, hipStream_t stream, bool whole) {
   const int strips = (p.N + STRIP - 1) / STRIP;
   Share share{};
-  share.parts = stream_parts(p);
+  share.parts = whole ? 1 : stream_parts(p);
   void* workspace = nullptr;
   if (share.parts > 1) {
     const size_t flag_bytes = ((size_t)strips * share.parts * sizeof(unsigned long long) + 255) / 256 * 256;
     const size_t bytes = flag_bytes + (size_t)strips * share.parts * MT * 8192;
-    // without a workspace: the whole k range a workgroup
-    if (take_workspace(&workspace, bytes, stream) != hipSuccess) {
-      share.parts = 1;
-    } else {
-      share.flags = reinterpret_cast<unsigned long long*>(workspace);
-      share.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + flag_bytes);
-      share.epoch = next_launch_epoch();
-    }
+    if (hipError_t e = take_workspace(&workspace, bytes, stream); e != hipSuccess) return e;
+    share.flags = reinterpret_cast<unsigned long long*>(workspace);
+    share.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + flag_bytes);
+    share.epoch = next_launch_epoch();
   }
   hipLaunchKernelGGL((gemm_stream_kernel<T, MT>), dim3(strips, share.parts), dim3(64 * WAVES), 0, stream, p, share);
   const hipError_t e = launch_status(stream);
@@ -307,10 +303,10 @@ double stream_us(const GemmProblem& p) {
   return (parts > 1 ? 7.0 : 3.3) + (p.M > 16 ? 0.7 : 0.0) + (a_unit > memory ? a_unit : memory);
 }
 
-hipError_t launch_stream(const GemmProblem& p, hipStream_t stream) {
+hipError_t launch_stream(const GemmProblem& p, hipStream_t stream, bool whole) {
   const bool bf16 = p.dtype == srtReal16BF;
-  if (p.M <= 16) return bf16 ? launch_rows<BF16, 1>(p, stream) : launch_rows<F16, 1>(p, stream);
-  return bf16 ? launch_rows<BF16, 2>(p, stream) : launch_rows<F16, 2>(p, stream);
+  if (p.M <= 16) return bf16 ? launch_rows<BF16, 1>(p, stream, whole) : launch_rows<F16, 1>(p, stream, whole);
+  return bf16 ? launch_rows<BF16, 2>(p, stream, whole) : launch_rows<F16, 2>(p, stream, whole);
 }
 
 }  // namespace srt

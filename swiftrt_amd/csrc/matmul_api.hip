@@ -433,12 +433,25 @@ hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
   }
 }
 
+// Up to 32 rows against an n-contiguous weight where the streaming kernel would cut k and gets no workspace: in one part a quarter to half of the
+// units would read.  From 50 MB of weight and a tile a unit the kernel that stages it through LDS, 64 columns a workgroup, else wave-split tiles
+// (us, one part / LDS / wave-split, weights from memory: 8 x 9776 x 6216 49.7 / 39.0 / 42.4, 32 x 11008 x 4096 33.3 / 24.4 / 33.4, 8 x 4096 x 8192 51.5
+// / 37.0 / 31.4, 8 x 1024 x 2056 15.7 / 12.4 / 10.1; 3643 random problems: within 0.4 % of the best of the three in the mean, one part 82 % behind).
+hipError_t launch_whole_range(const GemmProblem& p, hipStream_t stream) {
+  if (srt::skinny_supported(p) && p.N > 32 * srt::compute_units() && 2.0 * p.N * p.K > 50.0e6) return srt::launch_skinny(p, stream);
+  return srt::waves_supported(p) ? srt::launch_waves(p, stream) : srt::launch_stream(p, stream, true);
+}
+
 // A plan that gets no workspace (a full device, a stream under capture; nothing that matters was launched) gives way to the next best, which may
 // want one too: copies to what runs the operands as they are, tiles with shared left-overs to whole ones, parts of k to the whole range.
 hipError_t launch_or_fall_back(const GemmProblem& p, Plan plan, hipStream_t stream) {
   const hipError_t e = launch_plan(p, plan, stream);
   if (e != hipErrorOutOfMemory) return e;
   Plan next;
+  if ((plan == kPlanSkinny || plan == kPlanSplitK) && srt::stream_supported(p)) {
+    (void)hipGetLastError();
+    return launch_whole_range(p, stream);
+  }
   switch (plan) {
     case kPlanSplitK: next = tile_plan(p, false); break;
     case kPlanM16DTail: next = kPlanM16D; break;
@@ -712,7 +725,7 @@ srtStatus srtMatmulTune(const void* a, const srtTensorDescriptor* aDesc, int32_t
     if (plan == kPlanGeneric && fallback != kPlanGeneric && 2.0 * p.M * p.N * p.K * p.batch > 1e9) continue;
     const int warm = 2, reps = 8;
     for (int i = 0; i < warm && err == hipSuccess; ++i) err = launch_plan(p, plan, hs);
-    if ((plan == kPlanSplitK || plan == kPlanM16DTail || plan == kPlanF32Parts || plan == kPlanCopied) && err == hipErrorOutOfMemory) {
+    if ((plan == kPlanSkinny || plan == kPlanSplitK || plan == kPlanM16DTail || plan == kPlanF32Parts || plan == kPlanCopied) && err == hipErrorOutOfMemory) {
       // no room for this plan's workspace (nothing was launched): it is not a candidate, as in run()
       (void)hipGetLastError();
       err = hipSuccess;

@@ -1,5 +1,5 @@
 """The streaming kernel for a few rows against an n-contiguous weight (gemm_stream.hip): exact on integers, nothing outside a view, one set of bits
-whichever workgroup adds the parts, every epilogue within one rounding, the whole k range a workgroup under capture."""
+whichever workgroup adds the parts, every epilogue within one rounding, another kernel where k would be cut under capture."""
 import ctypes
 import os
 
@@ -89,3 +89,53 @@ def test_replays_of_a_captured_call():
                 out.device_written()
                 assert np.array_equal(out.array(), want)
         assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
+
+
+class KernelNode(ctypes.Structure):
+    """hipKernelNodeParams."""
+    _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
+
+# k in one part already; parts, a weight past 50 MB in rows of a tile a unit: 64 columns a workgroup; parts, other weights: neither of the two
+@pytest.mark.skipif("debug" in os.environ.get("SWIFTRT_HIP_LIBRARY", ""), reason="the debug build synchronises after every launch")
+@pytest.mark.parametrize("M,N,K,groups", [(5, 16500, 520, 129), (8, 8712, 2880, 137), (32, 8200, 3080, 129), (8, 8184, 3080, None), (3, 12001, 2200, None),
+                                          (17, 1024, 2056, None)])
+def test_the_kernel_of_a_captured_call(M, N, K, groups):
+    g, L, q = H.rng(48), native.lib(), srt.current_queue()
+    x, w = (g.integers(-2, 3, s).astype(np.float32) for s in ((M, K), (K, N)))
+    xt, wt, out = srt.Tensor(H.encode(x, H.BF16)), srt.Tensor(H.encode(w, H.BF16)), srt.Tensor(shape=[M, N], dtype=np.uint16)
+    want = H.encode(x @ w, H.BF16)   # (sums below 2^24: exact in any order)
+    (ad, k1), (bd, k2), (od, k3) = xt.descriptor(), wt.descriptor(), out.descriptor()
+    a, b, o = xt.device_read(q), wt.device_read(q), out.device_read_write(q)
+
+    def call():
+        native.check(L.srtMatmul(a, ctypes.byref(ad), 0, b, ctypes.byref(bd), 0, o, ctypes.byref(od), q.stream))
+    with H.pinned("skinny", H.BF16, M, N, K, 25 | (64 if K % 8 == 0 and N % 8 == 0 else 0)):
+        call()
+        out.device_written()
+        assert np.array_equal(out.array(), want)
+        graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+        assert L.hipStreamBeginCapture(q.stream, 1) == 0
+        try:
+            call()
+        finally:
+            assert L.hipStreamEndCapture(q.stream, ctypes.byref(graph)) == 0
+    count, node, kernel = ctypes.c_size_t(1), ctypes.c_void_p(), KernelNode()
+    assert L.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0 and count.value == 1
+    assert L.hipGraphGetNodes(graph, ctypes.byref(node), ctypes.byref(count)) == 0
+    assert L.hipGraphKernelNodeGetParams(node, ctypes.byref(kernel)) == 0
+    if groups is None:
+        assert tuple(kernel.grid)[0] not in ((N + 127) // 128, (N + 63) // 64)
+    else:
+        assert tuple(kernel.grid) == (groups, 1, 1)
+    assert L.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        q.fill(out, 0.0)
+        assert L.hipGraphLaunch(run, q.stream) == 0
+        out.device_written()
+        assert np.array_equal(out.array(), want)
+        call()
+        out.device_written()
+        assert np.array_equal(out.array(), want)
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
