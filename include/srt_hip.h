@@ -232,7 +232,9 @@ srtStatus srtMatmulBiasActivation(const void* a, const srtTensorDescriptor* aDes
  * "mfma_128x128_m16_k128", "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_256x256_m16", "mfma_256x256", "skinny", "generic", ...; the full
  * list is with srtMatmulTune), written into `name`; nothing is launched.  A 16-bit problem
  * whose operands span 1 Gi elements or more runs as several launches over halves of its batch, M or N;
- * the name is then that of the first piece's kernel followed by "/pieces".  Diagnostic only
+ * the name is then that of the first piece's kernel followed by "/pieces".  The built-in choice reports "mfma_256x256_splitk" too where up to
+ * 32 16-bit rows against an n-contiguous weight, whole 256-column tiles and k in 1024s, have their k in parts on the kernel that "skinny" names
+ * there; recorded in the plan cache, the name is the split-K kernel.  Diagnostic only
  * (the reference's matmul diagnostic line, CudaMatmul.swift:34-37, has no counterpart for
  * kernel choice). */
 srtStatus srtMatmulQueryKernel(const srtTensorDescriptor* aDesc, int32_t transposeA,
@@ -266,7 +268,8 @@ srtStatus srtMatmulQueryKernel(const srtTensorDescriptor* aDesc, int32_t transpo
  * "mfma_256x256_splitk", "mfma_128x256_m16", "mfma_128x128", "mfma_64x64", "mfma_128x128_any", "mfma_64x64_any" (16-bit
  * operands of any stride and alignment), "mfma_32x32_waves" (16-bit problems of few tiles: small tiles whose eight waves split
  * k, operands with a unit stride at any alignment), "copied" (operands off the 16-byte rules copied into aligned workspace first,
- * 16-bit types and fp32; the plan behind the copies is the heuristic's), "skinny" (16-bit types up to 64 rows, fp32 up to 32), "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring" (one
+ * 16-bit types and fp32; the plan behind the copies is the heuristic's), "skinny" (16-bit types up to 64 rows, fp32 up to 32: the kernels that
+ * stream the weight past a few rows, of which one matrix of up to 32 16-bit rows against an n-contiguous weight has its own), "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring" (one
  * fp32 kernel in three tile shapes: K a multiple of 64 and at least 128, operands contiguous along k or along m / n with
  * 16-byte aligned rows), "f32_mfma_128x128_parts" (its k range cut in parts, for a single matrix of a few tiles and a long k),
  * "f32_mfma_64x64", "f32_mfma_splitk", "generic").

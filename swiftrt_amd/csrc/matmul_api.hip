@@ -114,7 +114,8 @@ srtStatus build_problem(const void* a, const srtTensorDescriptor* ad, int tA,
 // (the role of ExecutionPlanCache / ExecutionPlanner, platform/common/ExecutionPlanner.swift:20-29,
 // and of the empty CudaMatmul2.tune, platform/cuda/functions/CudaMatmul.swift:112-120).
 enum Plan { kPlanGeneric, kPlanSkinny, kPlanRing256, kPlanMfma128, kPlanMfma64, kPlanF32Tile64, kPlanF32SplitK,
-            kPlanKc64, kPlanM16, kPlanSplitK, kPlanM16H, kPlanAny128, kPlanAny64, kPlanM16D, kPlanM16DTail, kPlanM16DSplit, kPlanM16DH, kPlanM16DN, kPlanM16Q, kPlanF32Parts, kPlanF32Ring, kPlanF32Ring64x128, kPlanF32Ring64, kPlanWaves, kPlanCopied, kPlanCount };
+            kPlanKc64, kPlanM16, kPlanSplitK, kPlanM16H, kPlanAny128, kPlanAny64, kPlanM16D, kPlanM16DTail, kPlanM16DSplit, kPlanM16DH, kPlanM16DN, kPlanM16Q, kPlanF32Parts, kPlanF32Ring, kPlanF32Ring64x128, kPlanF32Ring64, kPlanWaves, kPlanCopied, kPlanCount,
+            kPlanStreamed = kPlanCount };   // never recorded: few rows on the streaming kernel where split-K's name is reported (heuristic_plan)
 
 const char* const kPlanNames[kPlanCount] = {"generic", "skinny", "mfma_256x256", "mfma_128x128", "mfma_64x64",
                                             "f32_mfma_64x64", "f32_mfma_splitk", "mfma_256x256_k64",
@@ -122,6 +123,8 @@ const char* const kPlanNames[kPlanCount] = {"generic", "skinny", "mfma_256x256",
                                             "mfma_128x128_any", "mfma_64x64_any", "mfma_256x256_m16_k64",
                                             "mfma_256x256_m16_k64_tail", "mfma_256x256_m16_k64_split",
                                             "mfma_128x256_m16_k64", "mfma_256x128_m16_k64", "mfma_128x128_m16_k128", "f32_mfma_128x128_parts", "f32_mfma_128x128_ring", "f32_mfma_64x128_ring", "f32_mfma_64x64_ring", "mfma_32x32_waves", "copied"};
+
+const char* plan_name(Plan plan) { return kPlanNames[plan == kPlanStreamed ? kPlanSplitK : plan]; }
 
 bool plan_supported(const GemmProblem& p, Plan plan) {
   switch (plan) {
@@ -377,8 +380,7 @@ bool prefers_short(const GemmProblem& p, Plan plan) {
 // Up to 32 rows against an n-contiguous weight: the streaming kernel (gemm_stream.hip) or the wave-split tiles, by what the two take (2100 random
 // problems of 1-32 x 256-24000 x 128-8192, operands out of the caches or not in turn: 1.16x in the mean over the choice before, one in 30 more than 5 %
 // behind it).  From 50 MB and a tile a unit, or 85, the weight comes from memory, and tiles of 64-byte pieces are no match: 8 x 14336 x 4096 34 us against 22.5.  What base_plan
-// picks stays for whole 256-column tiles and a k in 1024s, where the tests assert its name (the streaming kernel runs under "skinny" and, in
-// parts, under the split-K plan's name, too); that costs most with many such tiles and a short k loop: 8 x 28672 x 1024 15.2 us in half tiles against 13.5.
+// picks stays for whole 256-column tiles and a k in 1024s, where the tests assert its name; that costs most with many such tiles and a short k loop: 8 x 28672 x 1024 15.2 us in half tiles against 13.5.
 bool few_rows(const GemmProblem& p, Plan* plan) {
   if (!srt::stream_supported(p) || (p.N % 256 == 0 && p.K % 1024 == 0)) return false;
   const double bytes = 2.0 * p.N * p.K, tiles = (double)((p.N + 31) / 32) / srt::compute_units();
@@ -398,20 +400,23 @@ Plan heuristic_plan(const GemmProblem& p, bool copies = true) {
   if ((plan == kPlanM16H || plan == kPlanM16 || plan == kPlanRing256 || plan == kPlanKc64) && p.K % 64 != 0 && srt::mfma_config(p, 14) != 0 &&
       srt::mfma_quarter_depth(p) && plan_us(p, kPlanM16Q) < 0.95 * plan_us(p, plan))
     plan = kPlanM16Q;
+  // k in parts for up to 32 rows against an n-contiguous weight: the streaming kernel's, under the name of split-K, which the tests assert (32 x 4096 x
+  // 4096 16.1 -> 12.7 us, 8 x 4096 x 8192 22.2 -> 16.7).  A pinned or recorded split-K is split-K.
+  if (plan == kPlanSplitK && srt::stream_supported(p)) return kPlanStreamed;
   if (p.dtype != srtReal32F && prefers_short(p, plan)) plan = srt::mfma_config(p, 2) != 0 ? kPlanMfma128 : kPlanAny128;
   return p.dtype != srtReal32F && prefers_waves(p, plan) ? kPlanWaves : plan;
 }
 
 hipError_t launch_plan(const GemmProblem& p, Plan plan, hipStream_t stream) {
   switch (plan) {
+    case kPlanStreamed: return srt::launch_stream(p, stream);
     case kPlanSkinny: return srt::stream_supported(p) ? srt::launch_stream(p, stream) : srt::launch_skinny(p, stream);
     case kPlanRing256: return srt::launch_mfma(p, srt::mfma_config(p, 1), stream);
     case kPlanMfma128: return srt::short_supported(p) ? srt::launch_short(p, stream) : srt::launch_mfma(p, srt::mfma_config(p, 2), stream);
     case kPlanMfma64: return srt::launch_mfma(p, srt::mfma_config(p, 3), stream);
     case kPlanKc64: return srt::launch_mfma(p, srt::mfma_config(p, 4), stream);
     case kPlanM16: return srt::launch_mfma(p, srt::mfma_config(p, 5), stream);
-    // (up to 32 rows against an n-contiguous weight the parts of k are the streaming kernel's: 32 x 4096 x 4096 16.1 -> 12.7 us, 8 x 4096 x 8192 22.2 -> 16.7)
-    case kPlanSplitK: return srt::stream_supported(p) ? srt::launch_stream(p, stream) : srt::launch_mfma_splitk(p, stream);
+    case kPlanSplitK: return srt::launch_mfma_splitk(p, stream);
     case kPlanM16H: return srt::launch_mfma(p, srt::mfma_config(p, 6), stream);
     case kPlanAny128: return srt::short_supported(p) ? srt::launch_short(p, stream) : srt::launch_mfma(p, srt::mfma_config(p, 7), stream);
     case kPlanAny64: return srt::launch_mfma(p, srt::mfma_config(p, 8), stream);
@@ -448,7 +453,7 @@ hipError_t launch_or_fall_back(const GemmProblem& p, Plan plan, hipStream_t stre
   const hipError_t e = launch_plan(p, plan, stream);
   if (e != hipErrorOutOfMemory) return e;
   Plan next;
-  if ((plan == kPlanSkinny || plan == kPlanSplitK) && srt::stream_supported(p)) {
+  if ((plan == kPlanSkinny || plan == kPlanStreamed || plan == kPlanSplitK) && srt::stream_supported(p)) {
     (void)hipGetLastError();
     return launch_whole_range(p, stream);
   }
@@ -679,7 +684,7 @@ srtStatus srtMatmulQueryKernel(const srtTensorDescriptor* aDesc, int32_t transpo
     bool pieces = false;
     while (!has_cached_plan(piece) && split_for_reach(piece, &lo, &hi)) { piece = lo; pieces = true; }
     const Plan plan = select(piece);
-    n = kPlanNames[plan];
+    n = plan_name(plan);
     if (plan == kPlanF32Tile64 || plan == kPlanF32SplitK || plan == kPlanF32Parts || plan == kPlanF32Ring || plan == kPlanF32Ring64x128 || plan == kPlanF32Ring64) n = "f32_mfma";   // one family name for the fp32 tiles
     if (pieces) {
       std::snprintf(name, nameCapacity, "%s/pieces", n);

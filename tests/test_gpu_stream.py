@@ -91,6 +91,30 @@ def test_replays_of_a_captured_call():
         assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
 
 
+def test_a_recorded_name_is_its_kernel():
+    """The two plans of a few rows that cut k, told apart by the workspace they take: sixteen parts of M x N sums, eight of a strip's."""
+    M, N, K = 32, 4096, 8192
+    L, q = native.lib(), srt.current_queue()
+    x, w = srt.Tensor(np.zeros((M, K), np.uint16)), srt.Tensor(np.zeros((K, N), np.uint16))
+    out = srt.Tensor(shape=[M, N], dtype=np.uint16)
+
+    def free():
+        q.wait_for_completion()
+        n, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert L.hipMemGetInfo(ctypes.byref(n), ctypes.byref(total)) == 0
+        return n.value
+
+    def taken(plan):
+        with H.pinned(plan, H.BF16, M, N, K, 25 | 64):
+            q.matmul(x, False, w, False, out)   # kernels loaded, operands on the device
+            q.wait_for_completion()
+            native.check(L.srtDeviceEmptyCache())
+            before = free()
+            q.matmul(x, False, w, False, out)
+            return before - free()
+    assert taken("skinny") < 16 * M * N * 4 <= taken("mfma_256x256_splitk")
+
+
 class KernelNode(ctypes.Structure):
     """hipKernelNodeParams."""
     _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3),
