@@ -23,14 +23,18 @@ double per_unit(const GemmProblem& p, int edge) {
   return (double)((p.M + edge - 1) / edge) * (double)((p.N + edge - 1) / edge) * (double)p.batch / compute_units();
 }
 double small_us(const GemmProblem& p) {
-  const double tiles = per_unit(p, 32), kb = 0.128 * traffic(p);
+  const double tiles = per_unit(p, 32);
+  double kb = 0.128 * traffic(p);
+  // x^T . W past a short k: 64-byte pieces of both operands (32 x 32 / 64 x 64 tiles, us: 512 x 1280 x 8101 67 / 33, 704 x 1024 x 5769 44 / 23, 1578 x 384 x
+  // 5776 51 / 28; 106 problems between 2048 and 8192 deep 1.1x)
+  if (p.K >= 2048 && p.sak != 1 && p.sbn == 1 && p.M > 32 && p.N > 32) kb *= 1.5;
   return tiles <= 1.0 ? 3.4 + kb / 97.0 : 3.3 + tiles * (0.26 + kb / 70.0);
 }
 double large_us(const GemmProblem& p) {
-  double tiles = per_unit(p, 64), kb = 0.256 * traffic(p);
-  // long k loops: the first tiles past one a unit cost nearly a round (104 x 9152 x 4736 x^T . W^T, 286 tiles, 40 us), x^T . W reads slower (512 x 600 x 6656 35)
+  double tiles = per_unit(p, 64);
+  const double kb = 0.256 * traffic(p);
+  // long k loops: the first tiles past one a unit cost nearly a round (104 x 9152 x 4736 x^T . W^T, 286 tiles, 40 us)
   if (p.K >= 2048 && tiles > 1.0 && tiles < 1.45) tiles = 1.45;
-  if (p.K >= 4096 && p.sak != 1 && p.sbn == 1) kb *= 1.5;
   return tiles <= 1.0 ? 4.6 + kb / 77.0 : 4.4 + tiles * (1.77 + kb / 65.0);
 }
 
