@@ -62,6 +62,8 @@ def test_a_few_rows_off_whole_lines(M, N, K, plan):
 @pytest.mark.parametrize("dt,M,N,K,ta,tb,plan", [
     (BF16, 2048, 2048, 2008, True, False, "mfma_128x128_m16_k128"), (BF16, 1600, 2112, 1600, False, True, "mfma_128x128_m16_k128"),   # 43.8 / 20.9, 20.8 / 15.2
     (F16, 700, 3000, 400, False, False, "mfma_128x128_m16_k128"), (BF16, 2908, 624, 160, False, False, "mfma_128x256_m16"),          # 11.3 / 8.7; 7.8 (10.1 in quarters)
-    (BF16, 1344, 760, 3008, False, False, "mfma_32x32_waves"), (F16, 1000, 1000, 1024, False, True, "mfma_32x32_waves")])           # 35.3 / 16.1
+    (BF16, 1344, 760, 3008, False, False, "mfma_32x32_waves"), (F16, 1000, 1000, 1024, False, True, "mfma_32x32_waves"),            # 35.3 / 16.1
+    (BF16, 1024, 1780, 448, True, True, "mfma_32x32_waves"), (F16, 2560, 674, 320, True, True, "mfma_32x32_waves"),                  # quarters 11.0 / 8.0, 10.8 / 8.2
+    (BF16, 336, 2752, 2448, False, False, "mfma_32x32_waves")])   # 25.7 / 19.5
 def test_depths_off_the_units(dt, M, N, K, ta, tb, plan):
     assert query(dt, M, N, K, ta, tb) == plan
