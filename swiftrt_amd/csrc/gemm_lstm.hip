@@ -7,7 +7,8 @@
 //
 //   bound   latency, as those tiles: a round trip to memory per slab of a wave, the sums, the gates
 //   k       x's slabs, then h's: each range ends with its own masked slab, and W's rows go on where x's end
-//   width   8, or any from 16 up: a last group of fewer than 8 columns (1 x 384 x 1020 f16, a program's step: 39.7 us as three calls, 18.7)
+//   width   8, or any from 16 up (9 to 15, never measured here, are left to the three calls): a last group of fewer than 8 columns (1 x 384 x 1020
+//           f16, a program's step: 39.7 us as three calls, 18.7)
 //   W       n-contiguous: a lane's 16 bytes are 8 columns of one gate (fp32: 4, two lanes a gate), so a k row of the tile is 16
 //           or 32 bytes in each of four lines, which the neighbouring workgroups share through L2
 //   sums    fp32; bias added in fp32 and rounded to the element type, as the product's result is; then lstm_gate

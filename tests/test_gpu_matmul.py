@@ -462,9 +462,10 @@ def test_skinny_up_to_64_rows_integer_exact_bias_and_choice(dt, tmp_path):
 
 @pytest.mark.parametrize("dt", [H.F16, H.BF16])
 def test_skinny_n_contiguous_weight_integer_exact_bias_and_batch(dt, tmp_path):
-    """x[M, K] . W[K, N] (no transposes) with up to 64 rows of x: the streaming kernel reads W through the
-    transposing LDS read.  Every staged row count, N ending inside a 64-column group, K ending inside a k block,
-    bias + ReLU, a batch, and random data against fp64."""
+    """x[M, K] . W[K, N] (no transposes) with up to 64 rows of x, on what the plan "skinny" launches: one matrix of up to 32
+    rows and 128 columns or more on gemm_stream.hip, the others through the transposing LDS read of gemm_skinny.hip
+    (its smaller staged row counts: test_gpu_skinny_batches.py).  N ending inside a 64-column group, K ending inside a
+    k block, bias + ReLU, a batch, and random data against fp64."""
     r = H.rng(43)
     relu = srt.ActivationType.relu
     for (M, N, K) in [(1, 64, 8), (5, 104, 72), (8, 1000, 520), (16, 4096, 64), (17, 12328, 200), (32, 264, 4096),
