@@ -303,9 +303,11 @@ __device__ __forceinline__ void store_tile(const GemmProblem& p, const f32x4_t (
   const bool n_rd_full = n_rd_ok && n_rd + 8 <= p.N;
   // Long rows off whole chunks leave past the caches from 100 MB of results at a short k against a k-contiguous B, where the stores are what
   // the launch waits for.  Cached / past, bf16 x . W^T, us: 2048 x 50257 x 768 177 / 154, 2048 x 25001 x 768 (102 MB) 99 / 87, 1024 x 50257 x 768
-  // 95 / 86, 8192 x 16001 x 960 243 / 221, 2048 x 50260 x 256 99 / 93, x^T . W^T 176 / 156; a longer k 108 / 111 (1024 x 50257 x 1024) and 274 /
-  // 283 (2048 x 50257 x 1600), shorter rows 76 / 85 (16384 x 5001 x 256), an n-contiguous W 134 / 141 (2048 x 40001 x 768).
-  const bool past = !WHOLE && p.N >= 16000 && p.K < 1024 && p.sbk == 1 &&
+  // 95 / 86, 8192 x 16001 x 960 243 / 221, x^T . W^T 176 / 156; a longer k 108 / 111 (1024 x 50257 x 1024) and 274 / 283 (2048 x 50257 x 1600), shorter
+  // rows 76 / 85 (16384 x 5001 x 256; nothing was measured between 5001 and 16001 columns), an n-contiguous W 134 / 141 (2048 x 40001 x 768).  820 random
+  // problems from K = 320: 1.10x with three sets of operands, 1.01x with all of them from memory, most where the plain stores take half as
+  // long again (1964 x 33025 x 896 187 / 116); shorter k loops lose, 270 problems 1.00x and 0.94x (5793 x 28089 x 224 136 / 168).
+  const bool past = !WHOLE && p.N >= 16000 && p.K >= 320 && p.K < 1024 && p.sbk == 1 &&
                     (unsigned long long)p.M * (unsigned)p.N * (unsigned)p.batch >= 50000000u;
   const bool row_ends = !WHOLE && wave_n0 < p.N && p.N < wave_n0 + 128 && (p.N & 7) != 0;   // (the same for every lane; tiles start at whole chunks)
 
