@@ -20,10 +20,11 @@ namespace srt {
 namespace {
 
 constexpr int kChunksPerLane = 2;
-// Copies of this much and more read their sources with the streaming hint: that large they are not in the caches, and are read once.  Without /
-// with it, the whole product, us: x . W^T 2048 x 768 x 50257 (283 MB of copies) 484 / 425, x . W 512 x 11007 x 4096 (94 MB) 87.4 / 80.9, 2048 x
-// 50257 x 768 (77 MB) 183.3 / 181.5; smaller sources mostly are, and two rows share their lines: 4096 x 4095 x 4095 (67 MB) 121.4 / 125.7, 2048 x
-// 2047 x 2049 32.5 / 37.8.
+// Copies of this much and more read their sources with the streaming hint: source and copy together then fill the last-level cache, and the source is
+// read once.  Without / with it, the whole product, us: x . W^T 2048 x 768 x 50257 (283 MB of copies) 484 / 425, x . W 512 x 11007 x 4096 (94 MB) 87.4 /
+// 80.9, 320 x 7714 x 5888 (91 MB) 87 / 74; small sources are in the caches, and two rows share their lines: 4096 x 4095 x 4095 (67 MB) 121.4 / 125.7,
+// 2048 x 2047 x 2049 32.5 / 37.8.  The line is a middle: between 75 and 134 MB it is worth up to 15 % for a long x . W with operands read again,
+// costs 1-3 % elsewhere (2048 x 50257 x 768, 77 MB, even) and 0.7 % in the mean of 2326 problems.
 constexpr size_t kStreamedCopies = 75000000;
 // The copies of a call take at most this much, in blocks of a power of two: the allocator keeps a freed block for the next call of
 // its size, so calls of many odd shapes share a dozen blocks instead of leaving one each (two operands that the 256 x 256 kernels'
