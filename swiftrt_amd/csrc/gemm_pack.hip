@@ -20,12 +20,11 @@ namespace srt {
 namespace {
 
 constexpr int kChunksPerLane = 2;
-// Copies of this much and more read their sources with the streaming hint: source and copy together then fill the last-level cache, and the source is
-// read once.  Without / with it, the whole product, us: x . W^T 2048 x 768 x 50257 (283 MB of copies) 484 / 425, x . W 512 x 11007 x 4096 (94 MB) 87.4 /
-// 80.9, 320 x 7714 x 5888 (91 MB) 87 / 74; small sources are in the caches, and two rows share their lines: 4096 x 4095 x 4095 (67 MB) 121.4 / 125.7,
-// 2048 x 2047 x 2049 32.5 / 37.8.  The line is a middle: between 75 and 134 MB it is worth up to 15 % for a long x . W with operands read again,
-// costs 1-3 % elsewhere (2048 x 50257 x 768, 77 MB, even) and 0.7 % in the mean of 2326 problems.
-constexpr size_t kStreamedCopies = 75000000;
+// Copies that fit the last-level cache (256 MiB) only if their sources stay out of it read the sources with the streaming hint, so that the product
+// finds the copies there.  What the hint is worth, 2611 random problems, by megabytes of copies, single matrices / batches: 75-130 0.985 / 0.966,
+// 130-150 0.993 / 0.966, 150-165 1.03 / 0.97, 165-180 1.07 / 0.99, 180-200 1.10 / 1.00, 200-270 1.13 / 1.03, 270-300 1.03 / 1.01, beyond 0.98 / 0.98: two
+// rows share lines that the hint drops, most where batches have short ones (40 x 1920 x 384 x 767 x . W^T, 142 MB, 120 us without it, 160).
+constexpr size_t kStreamedFrom = 160000000, kStreamedTo = 290000000;
 // The copies of a call take at most this much, in blocks of a power of two: the allocator keeps a freed block for the next call of
 // its size, so calls of many odd shapes share a dozen blocks instead of leaving one each (two operands that the 256 x 256 kernels'
 // 32-bit offsets reach are 4 GiB; larger ones run as they are).
@@ -204,7 +203,8 @@ hipError_t launch_packed(const GemmProblem& p, hipStream_t stream) {
   auto blocks = [](const PackJob& j) { return (j.total + 256 * kChunksPerLane - 1) / (256 * kChunksPerLane); };
   const dim3 grid(blocks(t.a) + blocks(t.b));
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a)); };
-  const bool streamed = t.bytes_a + t.bytes_b >= kStreamedCopies;
+  const size_t copies = t.bytes_a + t.bytes_b;
+  const bool streamed = copies >= kStreamedFrom && copies < kStreamedTo;
   if (p.dtype == srtReal32F) streamed ? launch(pack_kernel<4, true>) : launch(pack_kernel<4, false>);
   else streamed ? launch(pack_kernel<2, true>) : launch(pack_kernel<2, false>);
   hipError_t e = launch_status(stream);

@@ -1,5 +1,5 @@
-"""Copies of 75 MB and more, whose sources are read with the streaming hint: rows off every vector, inside a frame of NaNs, each layout of the
-right operand, one that is just below.  Small integers, so the products are exact."""
+"""Large copies, from 160 to 290 MB of which the sources are read with the streaming hint: rows off every vector, inside a frame of NaNs, each layout
+of the right operand, sizes below and between the two.  Small integers, so the products are exact."""
 import numpy as np
 import pytest
 
@@ -26,3 +26,9 @@ def test_large_copies(dt, m, n, k, transposed):
         got = srt.matmul(x, wt, transposed_rhs=transposed)
         assert query_kernel(x, False, wt, transposed, got) == "copied"
     assert np.array_equal(got.array(), H.encode(want, dt))
+
+
+@pytest.mark.parametrize("dt,m,n,k,transposed", [(H.BF16, 129, 81003, 1001, False), (H.F32, 65, 41003, 1001, True), (H.F16, 66, 90001, 1001, True)])
+def test_copies_read_with_the_hint(dt, m, n, k, transposed):
+    assert 160e6 < n * k * (4 if dt == H.F32 else 2) < 270e6
+    test_large_copies(dt, m, n, k, transposed)
