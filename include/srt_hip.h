@@ -445,7 +445,7 @@ srtStatus srtLstmGates(const void* gates, const srtTensorDescriptor* gatesDesc, 
 /* One step of an LSTM cell in one launch (role of LSTMCell, SwiftRTLayers/Recurrent.swift:165-266): gates = [x, hidden] . weight + bias,
  * rounded to the element type, then srtLstmGates' arithmetic.  x [B, I], hidden and cell [B, H], weight [I + H, 4 H], bias [4 H], results
  * [B, H]; one element type (32F, 16F, 16BF) and row order for all.  srtErrorNotSupported -- nothing was launched, and the caller runs
- * srtConcat, srtMatmulBiasActivation and srtLstmGates (or the element-wise calls) instead -- for other shapes, H not a multiple of 8,
+ * srtConcat, srtMatmulBiasActivation and srtLstmGates (or the element-wise calls) instead -- for other shapes, H under 16 other than 8,
  * rows (except the cell's) that are not contiguous, results that share memory with an operand or each other, and cells
  * whose rows, columns or depth I + H put the product's own kernels ahead. */
 srtStatus srtLstmCell(const void* x, const srtTensorDescriptor* xDesc, const void* hidden, const srtTensorDescriptor* hiddenDesc,

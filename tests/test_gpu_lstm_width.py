@@ -41,3 +41,13 @@ def test_between_nans(dt):
     for o, want in zip(outs, by_calls(*dense)):
         got = H.to64(o.array())
         assert np.array_equal(got[:, 1:1 + h], H.to64(want.array())) and (got[:, [0, *range(1 + h, h + 4)]] == 7.0).all()
+
+
+# a program's step, us, one launch / three calls
+@pytest.mark.parametrize("dt,b,i,h,taken", [
+    (H.BF16, 6, 2975, 2079, False), (H.F16, 2, 1245, 2415, False), (H.F32, 78, 2842, 663, False),     # 75 / 37, 55 / 35, 55 / 36
+    (H.F16, 1, 384, 1020, True), (H.BF16, 6, 975, 2078, True), (H.F32, 64, 512, 511, True)])          # 19 / 40; 28 / 36
+def test_cells_are_taken_where_one_launch_is_ahead(dt, b, i, h, taken):
+    dtype = H.encode(np.zeros(1), dt).dtype
+    make = lambda *shape: srt.Tensor(shape=shape, dtype=dtype)   # noqa: E731
+    assert srt.current_queue().lstm_cell(make(b, i), make(b, h), make(b, h), make(i + h, 4 * h), make(4 * h), make(b, h), make(b, h)) == taken
