@@ -166,7 +166,8 @@ srtStatus srtEventElapsedTime(float* milliseconds, srtEvent start, srtEvent stop
  * pointer; the library keeps no reference to tensor memory. */
 srtStatus srtDeviceAllocate(void** devPtr, size_t size, srtStream stream);
 /* The same for a queue that makes a result: selects `device` for the calling thread (srtSetDevice) and returns the block, or NULL
- * where srtDeviceAllocate would not return srtSuccess.  One call instead of three.  No counterpart in the reference. */
+ * where the device cannot be selected or srtDeviceAllocate would not return srtSuccess (srtSetDevice and srtDeviceAllocate tell which).
+ * One call instead of three.  No counterpart in the reference. */
 void* srtQueueAllocate(int32_t device, size_t size, srtStream stream);
 srtStatus srtDeviceFree(void* devPtr);
 /* Returns every cached (free) block of every device to the driver. */
