@@ -20,11 +20,13 @@ namespace srt {
 namespace {
 
 constexpr int kChunksPerLane = 2;
-// Copies that fit the last-level cache (256 MiB) only if their sources stay out of it read the sources with the streaming hint, so that the product
-// finds the copies there.  What the hint is worth, 2611 random problems, by megabytes of copies, single matrices / batches: 75-130 0.985 / 0.966,
-// 130-150 0.993 / 0.966, 150-165 1.03 / 0.97, 165-180 1.07 / 0.99, 180-200 1.10 / 1.00, 200-270 1.13 / 1.03, 270-300 1.03 / 1.01, beyond 0.98 / 0.98: two
-// rows share lines that the hint drops, most where batches have short ones (40 x 1920 x 384 x 767 x . W^T, 142 MB, 120 us without it, 160).
-constexpr size_t kStreamedFrom = 160000000, kStreamedTo = 290000000;
+// Copies that fit the last-level cache (256 MiB) better if their sources stay out of it read the sources with the streaming hint, so that the product
+// finds the copies there.  What the hint is worth, by megabytes of copies, in passes that follow each other over three sets of operands / in the first
+// pass over new ones, 410 random problems: single matrices 50-75 0.983 / 0.992, 75-100 0.992 / 1.013, 100-130 1.01 / 1.025, 130-160 1.00 / 1.046,
+// 160-200 1.01 / 1.07, 200-270 1.04 / 1.065, 270-300 1.01 / 1.01, beyond 0.99 / 0.985; batches 75-130 0.957 / 0.987, 130-160 0.97 / 1.02, 160-200 0.98 / 1.025,
+// 200-270 1.01 / 1.02: two rows share lines that the hint drops, most where batches have short ones (40 x 1920 x 384 x 767 x . W^T, 142 MB, 120 us
+// without it, 160).  2048 x 50257 x 768 (77 MB) 190 / 191 us, the first pass over new operands 214 / 203; x . W^T 2048 x 768 x 50257 (283 MB) 484 / 425.
+constexpr size_t kStreamedFrom = 75000000, kStreamedBatchFrom = 160000000, kStreamedTo = 290000000;
 // The copies of a call take at most this much, in blocks of a power of two: the allocator keeps a freed block for the next call of
 // its size, so calls of many odd shapes share a dozen blocks instead of leaving one each (two operands that the 256 x 256 kernels'
 // 32-bit offsets reach are 4 GiB; larger ones run as they are).
@@ -204,7 +206,7 @@ hipError_t launch_packed(const GemmProblem& p, hipStream_t stream) {
   const dim3 grid(blocks(t.a) + blocks(t.b));
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, t.a, t.b, blocks(t.a)); };
   const size_t copies = t.bytes_a + t.bytes_b;
-  const bool streamed = copies >= kStreamedFrom && copies < kStreamedTo;
+  const bool streamed = copies >= (p.batch == 1 ? kStreamedFrom : kStreamedBatchFrom) && copies < kStreamedTo;
   if (p.dtype == srtReal32F) streamed ? launch(pack_kernel<4, true>) : launch(pack_kernel<4, false>);
   else streamed ? launch(pack_kernel<2, true>) : launch(pack_kernel<2, false>);
   hipError_t e = launch_status(stream);

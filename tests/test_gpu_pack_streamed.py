@@ -1,5 +1,5 @@
-"""Large copies, from 160 to 290 MB of which the sources are read with the streaming hint: rows off every vector, inside a frame of NaNs, each layout
-of the right operand, sizes below and between the two.  Small integers, so the products are exact."""
+"""Copies of 75 MB and more, whose sources are read with the streaming hint: rows off every vector, inside a frame of NaNs, each layout of the
+right operand, one that is just below.  Small integers, so the products are exact."""
 import numpy as np
 import pytest
 
