@@ -258,13 +258,14 @@ double plan_us(const GemmProblem& p, Plan plan) {
   const double quarter = 4.4 + rounds(128, 128) * (0.9 + 5.1 * k + 0.6 * act), whole = 4.4 + rounds(256, 256) * (2.4 + 15.7 * k + 5.7 * act);
   switch (plan) {
     case kPlanM16Q: {
-      // a ragged last unit: whole to the matrix cores, and its masks; in a batch or a second round the operands' traffic sets the pace; one round
-      // against wave-split tiles, refitted to 2400 problems out of the caches or not in turn (with 1.5 for ragged rows and no factor one in twenty of
-      // them was more than 10 % behind: 1024 x 1780 x 448 x^T . W^T 11.0 / 8.0 us, 336 x 2752 x 2448 x . W 25.7 / 19.5 from memory)
+      // a ragged last unit: whole to the matrix cores, and its masks; in a batch or a second round the operands' traffic sets the pace; one round of a
+      // single matrix as 2400 problems in turn measure against wave-split tiles, passes that follow each other, from memory and on new operands (with
+      // 1.5 for ragged rows there and no factor 1024 x 1780 x 448 x^T . W^T ran 11.0 us for 8.0; a factor of 1.1 to 1.15 gains another tenth from memory
+      // and loses a twentieth out of the caches, 1688 x 840 x 7360 x . W 50.6 / 60.4; in batches both lose, 9 x 448 x 704 x 400 10.0 / 13.3)
       if (p.K % 128 == 0) return quarter;
       const double r = rounds(128, 128), per_k = p.batch > 1 ? 9.0 : r > 1.0 ? 8.3 : 5.6;
-      const double t = 5.0 + r * (0.9 + per_k * ((p.K + 127) / 128) / 8.0 + 0.6 * act + (srt::c_whole_chunks(p) ? 0.0 : 3.3));
-      return r > 1.0 || !a_kc ? t : t * (b_kc ? 1.1 : 1.15);
+      const double t = 5.0 + r * (0.9 + per_k * ((p.K + 127) / 128) / 8.0 + 0.6 * act + (srt::c_whole_chunks(p) ? 0.0 : p.batch > 1 ? 1.5 : 3.3));
+      return r > 1.0 || !a_kc || p.batch > 1 ? t : 1.05 * t;
     }
     case kPlanM16H: return 4.1 + rounds(128, 256) * (1.4 + (b_kc ? 16.7 : 11.8) * k + 3.3 * act);
     case kPlanM16DH: return 4.2 + rounds(128, 256) * (0.9 + 10.0 * k + 3.3 * act);
