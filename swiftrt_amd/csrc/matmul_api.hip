@@ -381,31 +381,31 @@ bool prefers_short(const GemmProblem& p, Plan plan) {
   return others && tiles <= cus && short_time(p) < 0.95 * plan_us(p, plan);
 }
 
-// Whether few rows stay on `plan`, which base_plan picked, where the streaming kernel is behind it: weights past 85 MB, most in rows off 128-byte lines,
-// of which a strip's 256 bytes take three instead of two.  Off whole lines: split-K from 150 MB where the strips get one part or two (us, streaming /
-// split-K: 8 x 18072 x 8128 72.4 / 64.1, 4 x 14424 x 12544 75.2 / 63.5, 45 random problems 1.12x); the 32-deep half tiles where the strips take twice
-// their rounds over the units (8 x 37432 x 4024 84.5 / 60.6, 32 x 50888 x 944 27.7 / 20.9, 42 problems 1.26x) or, past 16 rows, more rounds (32 x 91408
-// x 1032 53.8 / 43.4); the 64-deep ones at twice the rounds past 16 rows (32 x 124344 x 1984 118 / 94, 23 problems 1.08x).  In whole lines the 32-deep
-// ones at twice the rounds past 16 rows (32 x 41472 x 3664 73.3 / 62.7, nine problems 1.10x); else the streaming kernel is ahead (split-K 1.17x, half
-// tiles 1.3x).
+// Whether few rows stay on `plan`, which base_plan picked, where the streaming kernel is behind it: weights past 85 MB in rows off 128-byte lines, of
+// which a strip's 256 bytes take three instead of two.  Split-K from 150 MB where the strips get one part or two (us, streaming / split-K: 8 x 18072 x
+// 8128 72.4 / 64.1, 4 x 14424 x 12544 75.2 / 63.5; 33 random problems 1.11x); the 32-deep half tiles, past the shortest k loops, where the strips take
+// twice their rounds over the units (8 x 37432 x 4024 84.5 / 60.6, 32 x 50888 x 944 27.7 / 20.9) or, past 16 rows, more rounds (32 x 91408 x 1032 53.8
+// / 43.4; 49 problems 1.2x, 9 x 129936 x 392 not: 31.8 / 43.3); the 64-deep ones at twice the rounds past 16 rows (32 x 124344 x 1984 118 / 94; 36
+// problems 1.1x).  In whole lines the streaming kernel is ahead (split-K 1.17x, half tiles 1.3x) or, past 16 rows at twice the rounds, even.
 bool few_rows_keep(const GemmProblem& p, Plan plan) {
   const double bytes = 2.0 * p.N * p.K;
-  if (bytes < 85.0e6) return false;
+  if (bytes < 85.0e6 || p.sbk % 64 == 0) return false;
   const long long cus = srt::compute_units(), strips = (p.N + 127) / 128, halves = (p.N + 255) / 256;
   const long long strip_rounds = (strips + cus - 1) / cus, half_rounds = (halves + cus - 1) / cus;
-  const bool twice = strip_rounds >= 2 * half_rounds, two_tiles = p.M > 16, lines = p.sbk % 64 == 0;
-  if (plan == kPlanM16H) return lines ? twice && two_tiles : twice || (two_tiles && strip_rounds > half_rounds);
-  if (lines) return false;
+  const bool twice = strip_rounds >= 2 * half_rounds, two_tiles = p.M > 16;
   if (plan == kPlanSplitK) return bytes >= 150.0e6 && strip_rounds == 1 && 3 * strips > cus;
+  if (plan == kPlanM16H) return p.K >= 640 && (twice || (two_tiles && strip_rounds > half_rounds));
   return plan == kPlanM16DH && twice && two_tiles;
 }
 
-// Up to 32 rows against an n-contiguous weight: the streaming kernel (gemm_stream.hip) or the wave-split tiles, by what the two take (4920 random
-// problems of 1-32 x 128-140000 x 32-16384 that ran on another kernel before there was a streaming one, operands out of the caches or not in turn: 1.57x in
-// the mean over that kernel, one in 65 more than 5 % behind it, one in 230 more than 10 %).  Past some size the weight comes from memory, and tiles of 64-byte pieces are no match: from 30 MB with too few of them
-// for half the units (us, tiles / streaming: 4 x 3584 x 10752 41 / 17), else from 40 MB in rows of whole 128-byte lines (50 while every unit has a tile at
-// most; 1 x 10752 x 2176 18.9 / 12.2, 8 x 14336 x 4096 34 / 22.5), from 100 in others, whose strips read a half more (8 x 15784 x 1792 15.7 / 16.8, 11.4 / 16.2
-// out of the caches).  What base_plan picks stays for whole 256-column tiles and a k in 1024s, where the tests assert its name; that costs
+// Up to 32 rows against an n-contiguous weight: the streaming kernel (gemm_stream.hip) or the wave-split tiles, by what the two take.  Against the kernels
+// before there was a streaming one, 500 random problems of 1-32 x 128-140000 x 32-16384 that changed: 1.59x in passes that follow each other over three
+// weights, 1.55x from memory, 1.32x in the first pass on a new weight; nine more than 5 % behind in the mean of the three.  Past some size the weight
+// comes from memory, and tiles of 64-byte pieces are no match, but out of the caches they stay ahead longer; the lines lie where the mean of the three
+// is even (380 random problems): from 35 MB with too few tiles for half the units (us, tiles / streaming: 4 x 3584 x 10752 41 / 17), 65 with a tile a
+// unit at most, 40 with three rounds of them and up to 16 rows, else 50 (8 x 14336 x 4096 34 / 22.5; 1 x 6976 x 3712 9.9 / 13.2 out of the caches, 15.0 /
+// 14.4 from memory); in rows off whole 128-byte lines, of which the strips read a half more, from 40 and 85 (8 x 15784 x 1792 15.7 / 16.8 from memory,
+// 11.4 / 16.2 out of the caches).  What base_plan picks stays for whole 256-column tiles and a k in 1024s, where the tests assert its name; that costs
 // most with many such tiles and a short k loop: 8 x 28672 x 1024 15.2 us in half tiles against 13.5.
 bool few_rows(const GemmProblem& p, Plan* plan) {
   if (!srt::stream_supported(p) || (p.N % 256 == 0 && p.K % 1024 == 0)) return false;
@@ -415,7 +415,7 @@ bool few_rows(const GemmProblem& p, Plan* plan) {
   if (few_rows_keep(p, *plan)) return true;
   const double kb = 0.128 * p.K * (1.0 + ((p.sbk % 8 != 0) ? 0.3 : 0.0) + ((p.sam % 8 != 0) ? 0.17 : 0.0));
   const double waves = (tiles <= 1.0 ? 3.2 + kb / 97.0 : 3.3 + tiles * (0.26 + kb / 70.0)) + bytes / 32.0e6;
-  const double memory = tiles <= 0.5 ? 30.0e6 : !lines ? 100.0e6 : tiles > 1.0 ? 40.0e6 : 50.0e6;
+  const double memory = !lines ? (tiles <= 0.5 ? 40.0e6 : 85.0e6) : tiles <= 0.5 ? 35.0e6 : tiles <= 1.0 ? 65.0e6 : tiles > 2.0 && p.M <= 16 ? 40.0e6 : 50.0e6;
   const bool stream = !srt::waves_supported(p) || bytes > memory || (p.K >= 512 && srt::stream_us(p) < 0.95 * waves);
   *plan = stream ? kPlanSkinny : kPlanWaves;
   return true;

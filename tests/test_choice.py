@@ -42,7 +42,8 @@ def test_narrow_batches(dt, batch, M, N, K, plan):
 @pytest.mark.parametrize("dt,M,N,K,plan", [
     (BF16, 8, 9776, 6216, "skinny"), (BF16, 32, 11008, 4096 + 8, "skinny"), (F16, 16, 21760, 4123, "skinny"),    # 28 / 42, 22 / 33, 35 / 56
     (BF16, 32, 7096, 1992, "mfma_32x32_waves"), (BF16, 2, 3808, 3520, "mfma_32x32_waves"), (F16, 8, 17008, 960, "mfma_32x32_waves"),   # 12.8 / 8.7, 11.3 / 8.1, 11.0 / 8.9
-    (BF16, 1, 10752, 2176, "skinny"), (BF16, 4, 3584, 10752, "skinny"),                                          # weights from memory: 12.2 / 18.9, 17 / 41
+    (BF16, 16, 19072, 1088, "skinny"), (BF16, 4, 3584, 10752, "skinny"),                                         # weights from memory: 12.6 / 15.4, 17 / 41
+    (F16, 1, 6976, 3712, "mfma_32x32_waves"), (BF16, 2, 6784, 3784, "mfma_32x32_waves"),                          # out of the caches 13.2 / 9.9, 13.0 / 10.4
     (BF16, 8, 15784, 1792, "mfma_32x32_waves"), (BF16, 1, 15384, 2039, "mfma_32x32_waves")])                     # off whole lines: 16.2 / 11.4, 17.1 / 12.1
 def test_a_few_rows(dt, M, N, K, plan):
     assert query(dt, M, N, K) == plan
@@ -52,7 +53,7 @@ def test_a_few_rows(dt, M, N, K, plan):
 @pytest.mark.parametrize("M,N,K,plan", [
     (8, 18072, 8128, "mfma_256x256_splitk"), (4, 14424, 12544, "mfma_256x256_splitk"), (8, 18048, 8128, "skinny"),          # 72 / 64, 75 / 63
     (8, 37432, 4024, "mfma_128x256_m16"), (32, 50888, 944, "mfma_128x256_m16"), (16, 50880, 944, "skinny"),                 # 84 / 61, 28 / 21
-    (32, 91408, 1032, "mfma_128x256_m16"), (32, 41472, 3664, "mfma_128x256_m16"), (16, 41472, 3664, "skinny"),              # 54 / 43, 73 / 63
+    (32, 91408, 1032, "mfma_128x256_m16"), (9, 129936, 392, "skinny"), (16, 41472, 3664, "skinny"),                         # 54 / 43, 32 / 43
     (32, 124344, 1984, "mfma_128x256_m16_k64"), (16, 124344, 1984, "skinny"), (8, 70008, 1608, "skinny")])                  # 118 / 94; three rounds of strips for two
 def test_a_few_rows_off_whole_lines(M, N, K, plan):
     assert query(BF16, M, N, K) == plan
