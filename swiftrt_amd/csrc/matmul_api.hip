@@ -264,8 +264,9 @@ double plan_us(const GemmProblem& p, Plan plan) {
       // and loses a twentieth out of the caches, 1688 x 840 x 7360 x . W 50.6 / 60.4; in batches both lose, 9 x 448 x 704 x 400 10.0 / 13.3)
       if (p.K % 128 == 0) return quarter;
       const double r = rounds(128, 128), per_k = p.batch > 1 ? 9.0 : r > 1.0 ? 8.3 : 5.6;
-      const double t = 5.0 + r * (0.9 + per_k * ((p.K + 127) / 128) / 8.0 + 0.6 * act + (srt::c_whole_chunks(p) ? 0.0 : p.batch > 1 ? 1.5 : 3.3));
-      return r > 1.0 || !a_kc || p.batch > 1 ? t : 1.05 * t;
+      const bool low = p.batch > 1 || p.K >= 4096;   // (the wave-split tiles' estimate is a fifth low past there: 1193 x 1193 x 5672 x . W^T 44.6 us, 56.4 on them)
+      const double t = 5.0 + r * (0.9 + per_k * ((p.K + 127) / 128) / 8.0 + 0.6 * act + (srt::c_whole_chunks(p) ? 0.0 : low ? 1.5 : 3.3));
+      return r > 1.0 || !a_kc || low ? t : 1.05 * t;
     }
     case kPlanM16H: return 4.1 + rounds(128, 256) * (1.4 + (b_kc ? 16.7 : 11.8) * k + 3.3 * act);
     case kPlanM16DH: return 4.2 + rounds(128, 256) * (0.9 + 10.0 * k + 3.3 * act);
