@@ -185,10 +185,10 @@ bool launch_choice(const CellProblem& p, bool f32) {
   const long long tiles = (long long)((p.rows + 31) / 32) * groups_of(p.hidden), cus = compute_units();
   const long long depth = (long long)p.inputs + p.hidden;
   if (tiles > 2 * cus || (depth > (f32 ? 8192 : 5200) && p.hidden > 32)) return false;
-  // (widths off the groups of eight, whose weight rows are mostly off 16 bytes, take up to twice as long: by the other widths' bounds 3.3 % of 6757
-  // programs' steps were more than 5 % behind the three calls, one / three, us: bf16 6 x 2975 x 2079 75 / 37, f16 2 x 1245 x 2415 55 / 35, f32 78 x
-  // 2842 x 663 55 / 36; by these 0.1 % of 5002, at 1.76x in the mean)
-  if (p.hidden % 8 != 0) return depth * tiles <= (f32 ? 2800 : p.hidden % 2 != 0 && tiles > cus ? 2600 : 3800) * cus;
+  // (widths off the groups of eight, whose weight rows are mostly off 16 bytes, take up to twice as long, one / three, us: bf16 6 x 2975 x 2079 75 / 37,
+  // f16 2 x 1245 x 2415 55 / 35, f32 78 x 2842 x 663 55 / 36.  84 programs' steps between these bounds and the other widths': three calls 1.11x as
+  // fast in steps that follow each other, and in the first one on new operands 1.05x in 16 bits, 0.87x in fp32)
+  if (p.hidden % 8 != 0) return depth * tiles <= (f32 ? 3400 : p.hidden % 2 == 0 ? 4500 : tiles > cus ? 3400 : 3800) * cus;
   return depth * tiles <= (f32 ? 4200 : 5200) * cus;
 }
 
